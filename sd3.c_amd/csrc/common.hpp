@@ -37,6 +37,20 @@ inline int launch_status(const char* what) {
     return SD3_OK;
 }
 
+// compute units of the current device (0 after a failed query, which has set the error message)
+inline int compute_units() {
+    static int cus = 0;
+    if (!cus) {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+            fail(SD3_ERR_HIP, "cannot query the number of compute units");
+            return 0;
+        }
+        cus = n;
+    }
+    return cus;
+}
+
 // ---- bf16 as raw 16-bit storage ----
 typedef uint16_t bf16_t;
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
@@ -87,6 +101,42 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// ---- direct global -> LDS loads and the tile order of the GEMM kernels ----
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+typedef const __attribute__((address_space(1))) void* glb_ptr_t;
+
+// s_waitcnt vmcnt(n) with the other counters left unconstrained (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[15:14])
+template <int N>
+__device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+
+// Workgroup -> output tile. The hardware hands consecutive workgroup ids to the 8 XCDs in turn, and each XCD has its own L2, so
+// the workgroups that land on one XCD should share as few A row panels and W column panels as possible. When the tile grid
+// divides that way, the XCDs take a 4 x 2 arrangement of rectangular blocks of it (for 32 x 24 tiles: 8 x 12 each, 8 + 12 panels
+// through that L2 instead of 4 + 24 with contiguous runs of tile rows), walked in bands of 4 tile rows so that the 32 tiles an XCD
+// works on at a time form a 4 x 8 patch. Otherwise every XCD gets a contiguous run of tiles, walked in bands of 2 tile rows
+// (measured over 1, 2, 3, 4, 8, 16 on the 24-block forward).
+__device__ __forceinline__ void tile_of_workgroup(int wg, int tiles_m, int tiles_n, int& tile_m, int& tile_n) {
+    constexpr int XCDS = 8, XR = 4, XC = 2, BAND = 4, GROUP_M = 2;
+    const int total = tiles_m * tiles_n;
+    const int xcd = wg % XCDS, local = wg / XCDS;
+    if (tiles_m % (XR * BAND) == 0 && tiles_n % XC == 0) {
+        const int bm = tiles_m / XR, bc = tiles_n / XC;  // the XCD's block: bm x bc tiles, exactly total / 8
+        const int band = local / (BAND * bc), r = local % (BAND * bc);
+        tile_m = (xcd / XC) * bm + band * BAND + r % BAND;
+        tile_n = (xcd % XC) * bc + r / BAND;
+        return;
+    }
+    const int per = (total + XCDS - 1) / XCDS, tall = (total % XCDS) ? (total % XCDS) : XCDS;  // `tall` XCDs get `per` tiles, the rest per-1
+    const int t = (xcd < tall) ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+    const int in_group = GROUP_M * tiles_n, group = t / in_group, first_m = group * GROUP_M;
+    const int gsize = min(tiles_m - first_m, GROUP_M);
+    tile_m = first_m + (t % in_group) % gsize;
+    tile_n = (t % in_group) / gsize;
+}
+
 // ---- epilogues of the GEMM kernels ----
 enum Epilogue : int {
     EPI_BIAS = 0,         // out = acc + bias
@@ -112,6 +162,16 @@ struct GemmEpilogueArgs {
 // fp32 GEMM on the fp32 MFMA units: out(M,N) = A(M,K; lda) @ W(K, ldw)[:, n0:n0+N] (+ epilogue); out fp32 with row stride ldc.
 int gemm_f32(const float* A, int lda, const float* W, int ldw, int n0, float* out, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
              hipStream_t st);
+// Up to three independent fp32 GEMMs with the same epilogue kind: one launch where all rows are made of whole 16-byte chunks.
+struct GemmF32Problem {
+    const float* A;
+    const float* W;
+    float* out;
+    int lda, ldw, n0, ldc, M, N, K;
+    GemmEpilogueArgs ea;
+};
+int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st);
+extern int g_gemm_f32_tile;
 // bf16 GEMM: A bf16 (M,K) row-major; Wp = packed weight, bf16 (N,K) K-contiguous; out bf16 (out_is_f32 = 0) or fp32.
 int gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* out, int out_is_f32, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
               hipStream_t st);

@@ -302,8 +302,8 @@ int linear_layer(sd3_ctx* ctx, int prec, const void* A, const float* W, const fl
     return gemm_bf16((const bf16_t*)A, (const bf16_t*)wp, out, out_f32, ldc, M, N, K, epi, ea, ctx->stream);
 }
 
-// The same layer of the latent stream and of the context stream (different weights and rows, same kind): on the bf16
-// path both go into one launch, so that the few context rows ride along instead of paying a launch of their own.
+// The same layer of the latent stream and of the context stream (different weights and rows, same kind): both
+// go into one launch, so that the few context rows ride along instead of paying a launch of their own.
 struct LayerCall {
     const void* A;
     const float* W;
@@ -313,15 +313,25 @@ struct LayerCall {
     GemmEpilogueArgs ea;
 };
 int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f32, int epi) {
+    if (n > 3) return fail(SD3_ERR_INVALID_ARG, "linear_pair: at most three layers per group");
     if (!is_bf(prec)) {
+        GemmF32Problem probs[3];
+        int m = 0;
+        double flop = 0;
         for (int i = 0; i < n; i++) {
             const LayerCall& c = calls[i];
-            if (c.M > 0) SD3_TRY(linear_layer(ctx, prec, c.A, c.W, c.bias, c.out, out_f32, c.ldc, c.M, c.N, c.K, epi, c.ea));
+            if (c.M <= 0) continue;
+            if (!c.W) return fail(SD3_ERR_MISSING_PARAM, "a weight needed by this configuration is not bound (N=%d K=%d)", c.N, c.K);
+            probs[m] = GemmF32Problem{(const float*)c.A, c.W, (float*)c.out, c.K, c.N, 0, c.ldc, c.M, c.N, c.K, c.ea};
+            probs[m].ea.bias = c.bias;
+            flop += 2.0 * c.M * c.N * c.K;
+            m++;
         }
-        return SD3_OK;
+        if (m == 0) return SD3_OK;
+        ProfScope ps(ctx, SD3_PROF_GEMM, flop);
+        return gemm_f32_grouped(probs, m, epi, ctx->stream);
     }
     GemmBf16Problem probs[3];
-    if (n > 3) return fail(SD3_ERR_INVALID_ARG, "linear_pair: at most three layers per group");
     int m = 0;
     double flop = 0;
     for (int i = 0; i < n; i++) {
@@ -1356,6 +1366,11 @@ int sd3_tune(const char* name, int value) {
     if (!std::strcmp(name, "gemm_bf16_tile")) return sd3_gemm_bf16_force_tile(value);
     if (!std::strcmp(name, "gemm_bf16_row_split")) {
         g_gemm_bf16_row_split = value != 0;
+        return SD3_OK;
+    }
+    if (!std::strcmp(name, "gemm_f32_tile")) {
+        SD3_REQUIRE(value >= -1 && value <= 4, "sd3_tune(%s): -1 (automatic) or 0..4 (got %d)", name, value);
+        g_gemm_f32_tile = value;
         return SD3_OK;
     }
     if (!std::strcmp(name, "attention_context_splits")) {

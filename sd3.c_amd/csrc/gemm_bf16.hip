@@ -16,9 +16,6 @@ namespace {
 
 constexpr int BK = 64;  // bf16 elements per K tile = 128 bytes per LDS row
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef const __attribute__((address_space(1))) void* glb_ptr_t;
-
 struct EpiDev {
     const float* a_scale;  // fp8 operands: one factor per row of A (null: 1)
     const float* w_scale;  // fp8 operands: one factor per output column (null: 1)
@@ -40,38 +37,6 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // eight 16-byte slots of a half. (With swz() that pattern hits every slot twice: the bank-conflict counter read 47 % of the LDS
 // cycles; the 32x32 layout, lane l: row l % 32, is conflict-free with swz() and would not be with this key.)
 __device__ __forceinline__ int swz16(int row) { return row & 6; }
-
-// s_waitcnt vmcnt(n) with the other counters left unconstrained (gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[15:14])
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// Workgroup -> output tile. The hardware hands consecutive workgroup ids to the 8 XCDs in turn, and each XCD has its own L2, so
-// the workgroups that land on one XCD should share as few A row panels and W column panels as possible. When the tile grid
-// divides that way, the XCDs take a 4 x 2 arrangement of rectangular blocks of it (for 32 x 24 tiles: 8 x 12 each, 8 + 12 panels
-// through that L2 instead of 4 + 24 with contiguous runs of tile rows), walked in bands of 4 tile rows so that the 32 tiles an XCD
-// works on at a time form a 4 x 8 patch. Otherwise every XCD gets a contiguous run of tiles, walked in bands of 2 tile rows
-// (measured over 1, 2, 3, 4, 8, 16 on the 24-block forward).
-__device__ __forceinline__ void tile_of_workgroup(int wg, int tiles_m, int tiles_n, int& tile_m, int& tile_n) {
-    constexpr int XCDS = 8, XR = 4, XC = 2, BAND = 4, GROUP_M = 2;
-    const int total = tiles_m * tiles_n;
-    const int xcd = wg % XCDS, local = wg / XCDS;
-    if (tiles_m % (XR * BAND) == 0 && tiles_n % XC == 0) {
-        const int bm = tiles_m / XR, bc = tiles_n / XC;  // the XCD's block: bm x bc tiles, exactly total / 8
-        const int band = local / (BAND * bc), r = local % (BAND * bc);
-        tile_m = (xcd / XC) * bm + band * BAND + r % BAND;
-        tile_n = (xcd % XC) * bc + r / BAND;
-        return;
-    }
-    const int per = (total + XCDS - 1) / XCDS, tall = (total % XCDS) ? (total % XCDS) : XCDS;  // `tall` XCDs get `per` tiles, the rest per-1
-    const int t = (xcd < tall) ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
-    const int in_group = GROUP_M * tiles_n, group = t / in_group, first_m = group * GROUP_M;
-    const int gsize = min(tiles_m - first_m, GROUP_M);
-    tile_m = first_m + (t % in_group) % gsize;
-    tile_n = (t % in_group) / gsize;
-}
 
 // LDS bytes of a configuration: the tile ring, or the epilogue staging slabs if those are larger
 template <int BM, int BN, int WM, int WN, int STAGES>
@@ -543,20 +508,6 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet ar
         gemm_tile<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8>(args.p[which], w - (which ? args.end[which - 1] : 0), smem);
         __syncthreads();  // the staging slabs of this tile's epilogue alias the ring the next tile fills
     }
-}
-
-// compute units of the current device (0 after a failed query, which has set the error message)
-int compute_units() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-            fail(SD3_ERR_HIP, "gemm_bf16: cannot query the number of compute units");
-            return 0;
-        }
-        cus = n;
-    }
-    return cus;
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false>

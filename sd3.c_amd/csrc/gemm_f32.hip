@@ -1,14 +1,17 @@
-// fp32 GEMM on the gfx950 fp32 matrix cores (v_mfma_f32_32x32x2_f32), for the fp32 parity path:
+// fp32 GEMM on the gfx950 fp32 matrix cores, for the fp32 parity path and the fp32 operators:
 //   out(M,N) = A(M,K) @ W(K,N)[:, n0:n0+N] + epilogue
 // replacing linear / partial_linear of the reference (modules.cpp:475-511, naive triple loops).
-// Tile: 128x128x16 per workgroup of 4 wavefronts (2x2), each wavefront owns 64x64 = 2x2 MFMA blocks.
-// Any M, N, K: out-of-range elements are zero-filled on load and masked on store.
+//
+// gemm_f32_tile_kernel (v_mfma_f32_16x16x4_f32) takes everything whose rows are made of whole 16-byte chunks, up to three problems
+// per launch; gemm_f32_kernel (v_mfma_f32_32x32x2_f32, 128x128x16 tiles, element-wise loads) takes any other stride or alignment.
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace sd3 {
 
 namespace {
-constexpr int BM = 128, BN = 128, BK = 16;
+constexpr int BM = 128, BN = 128, BK = 16;  // tile of the any-stride kernel
 constexpr int A_PITCH = BM + 4;  // As[k][m]: 4*(BM+4) = 528 = 16 mod 64 -> the four k-quads of a wave hit disjoint banks on store
 constexpr int B_PITCH = BN + 4;
 
@@ -36,7 +39,7 @@ __device__ __forceinline__ float apply_epilogue(float acc, int m, int n, int n_g
     return v;
 }
 
-template <int EPI, bool ALIGNED>
+template <int EPI>
 __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, int n0,
                                                        float* __restrict__ out, int ldc, int M, int N, int K, EpiDev epi) {
     __shared__ float As[BK * A_PITCH];
@@ -55,24 +58,15 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__
         for (int i = 0; i < 2; i++) {
             const int m = m_blk + a_row + i * 64;
             const int k = k0 + a_kq;
-            if (ALIGNED) {
-                ra[i] = (m < M && k < K) ? *reinterpret_cast<const float4*>(A + (long long)m * lda + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-            } else {
-                float t[4];
+            float t[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) t[j] = (m < M && k + j < K) ? A[(long long)m * lda + k + j] : 0.f;
-                ra[i] = make_float4(t[0], t[1], t[2], t[3]);
-            }
+            for (int j = 0; j < 4; j++) t[j] = (m < M && k + j < K) ? A[(long long)m * lda + k + j] : 0.f;
+            ra[i] = make_float4(t[0], t[1], t[2], t[3]);
             const int kk = k0 + b_k + i * 8;
             const int n = n_blk + b_n;
-            if (ALIGNED) {
-                rb[i] = (kk < K && n < N) ? *reinterpret_cast<const float4*>(W + (long long)kk * ldw + n0 + n) : make_float4(0.f, 0.f, 0.f, 0.f);
-            } else {
-                float t[4];
 #pragma unroll
-                for (int j = 0; j < 4; j++) t[j] = (kk < K && n + j < N) ? W[(long long)kk * ldw + n0 + n + j] : 0.f;
-                rb[i] = make_float4(t[0], t[1], t[2], t[3]);
-            }
+            for (int j = 0; j < 4; j++) t[j] = (kk < K && n + j < N) ? W[(long long)kk * ldw + n0 + n + j] : 0.f;
+            rb[i] = make_float4(t[0], t[1], t[2], t[3]);
         }
     };
     auto store_tiles = [&]() {
@@ -133,32 +127,340 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__
             }
         }
 }
+
+// ---- the tile kernel ----
+// fp32 matrix instructions are slow (64 FLOP per cycle and SIMD: a 64x64 wavefront tile works 2048 cycles on 16 k values), so the
+// matrix unit is the bound as soon as every SIMD has a tile; LDS and global traffic are not. What costs is SIMDs without work: the
+// layers of a 512 x 512 image are 96 tiles of 128x128 on 256 compute units. Hence a range of tile shapes down to 32x32, chosen per
+// launch by the number of rounds (pick_tile), and one launch for the layers of the same kind of both token streams.
+//
+// Both operands go global -> LDS by direct loads. A tile rows are 128 bytes (32 k values), 16-byte chunks XOR-swizzled by the row as
+// in the bf16 kernel's 16x16 layout: lane l reads chunk 4h + l/16 of row l%16, i.e. k values 16h + 4(l/16) .. +3 of one half h of the
+// tile, and matrix instruction s of the half contracts k = 16h + 4g + s, g = 0..3 (the same order of k whatever the tile shape:
+// a row's result depends on neither the shape nor the grouping). W stays N-contiguous as the reference stores it: lane l reads the NJ
+// consecutive columns NJ*(l%16) .. of its k row, one for each of its NJ column blocks, so column block j holds columns NJ*c + j and
+// a lane ends with NJ consecutive columns of a row: the epilogue stores straight from the accumulators, 16 lanes covering 16*NJ columns.
+struct TileProb {
+    const float* A;
+    const float* W;
+    float* out;
+    int lda, ldw, ldc, M, N, K, n0;
+    EpiDev epi;
+};
+constexpr int MAX_PROBS = 3;
+struct TileProbSet {
+    TileProb p[MAX_PROBS];
+    int end[MAX_PROBS];  // running totals of tiles
+};
+constexpr int TK = 32;  // k values per tile = 128-byte rows of A in LDS
+__device__ __align__(16) float zero_chunk[4];  // source of the k values beyond K (A and W)
+
+template <int NJ>
+struct Cols;  // NJ consecutive floats, loaded and stored as one
+template <>
+struct Cols<4> { typedef f32x4_t type; };
+template <>
+struct Cols<2> { typedef f32x2_t type; };
+template <>
+struct Cols<1> { typedef float type; };
+template <int NJ>
+__device__ __forceinline__ void load_cols(const float* p, float (&v)[NJ]) {
+    typedef typename Cols<NJ>::type T;
+    const T t = *reinterpret_cast<const T*>(p);
+    __builtin_memcpy(v, &t, sizeof(T));
+}
+template <int NJ>
+__device__ __forceinline__ void store_cols(float* p, const float (&v)[NJ]) {
+    typedef typename Cols<NJ>::type T;
+    T t;
+    __builtin_memcpy(&t, v, sizeof(T));
+    *reinterpret_cast<T*>(p) = t;
+}
+
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
+__global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const TileProbSet set) {
+    constexpr int NT = WM * WN * 64, TI = TM / WM / 16, NJ = TN / WN / 16;
+    constexpr int A_BYTES = TM * 128, STAGE_BYTES = A_BYTES + TK * TN * 4;
+    constexpr int LA = TM * 8 / NT, LB = TN * 8 / NT, CPR = TN / 4;  // 16-byte chunks per thread and tile; chunks per W row
+    static_assert(TM * 8 % NT == 0 && TN * 8 % NT == 0 && TI >= 1 && (NJ == 1 || NJ == 2 || NJ == 4), "tile shape");
+    // W rows whose k differs by 4 are read together; with fewer than 64 columns per wavefront their chunks are moved apart
+    constexpr int WX = NJ == 4 ? 0 : NJ == 2 ? 8 : 4, WXM = NJ == 2 ? 1 : 3;
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    const int w = blockIdx.x;
+    const int which = (w >= set.end[0]) + (w >= set.end[1]);
+    const TileProb& pr = set.p[which];
+    const int M = pr.M, N = pr.N, K = pr.K;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    int tile_m, tile_n;
+    tile_of_workgroup(w - (which ? set.end[which - 1] : 0), (M + TM - 1) / TM, (N + TN - 1) / TN, tile_m, tile_n);
+    const int m_blk = tile_m * TM, n_blk = tile_n * TN;
+
+    const float* ga[LA];
+    const float* gb[LB];
+    int ka[LA], kb[LB];  // k of the chunk within its tile
+#pragma unroll
+    for (int i = 0; i < LA; i++) {
+        const int q = i * NT + tid, row = q >> 3;
+        ka[i] = ((q & 7) ^ (row & 6)) * 4;
+        ga[i] = pr.A + (long long)min(m_blk + row, M - 1) * pr.lda + ka[i];  // rows beyond M re-read the last one and are never stored
+    }
+#pragma unroll
+    for (int i = 0; i < LB; i++) {
+        const int q = i * NT + tid;
+        kb[i] = q / CPR;
+        const int c = (q % CPR) ^ ((((kb[i] >> 2) & WXM) * WX) & (CPR - 1));
+        gb[i] = pr.W + (long long)kb[i] * pr.ldw + pr.n0 + min(n_blk + c * 4, N - 4);
+    }
+    const long long b_step = (long long)TK * pr.ldw;
+    const int nkt = (K + TK - 1) / TK;
+    const float* zeros = zero_chunk;
+    asm volatile("" : "+s"(zeros));  // (kept in registers: the compiler would fetch the address anew inside the loop)
+    // requests the next tile (the pointers advance with every call); past the last one zeros, into a stage that nobody reads again.
+    // No branches, so that the requests can be spread over the matrix instructions.
+    auto issue_tile = [&](int kt, int stage) {
+        const int left = K - kt * TK;
+        char* sa = smem + stage * STAGE_BYTES + wave * 1024;
+        char* sb = sa + A_BYTES;
+#pragma unroll
+        for (int i = 0; i < LA; i++) {
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(ka[i] < left ? ga[i] : zeros), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+            ga[i] += TK;
+        }
+#pragma unroll
+        for (int i = 0; i < LB; i++) {
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(kb[i] < left ? gb[i] : zeros), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+            gb[i] += b_step;
+        }
+    };
+
+    f32x4_t acc[TI][NJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[i][j][r] = 0.f;
+
+    static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "the loads in flight must fit the 6-bit counter");
+    f32x4_t a[2][TI];
+    float b[2][4][NJ];
+    // The operands of one half (16 k values) of a tile. They are fetched while the matrix unit works on the half before, across the
+    // barrier between tiles too: fetched when they are needed, their latency cost a quarter of the time of a lone workgroup.
+    auto fetch = [&](int stage, int h) {
+        const char* sa = smem + stage * STAGE_BYTES + (wm * (TM / WM) + lr) * 128;
+        const float* sb = reinterpret_cast<const float*>(smem + stage * STAGE_BYTES + A_BYTES);
+        const int col = (wn * (TN / WN) + NJ * lr) ^ ((((4 * h + lg) & WXM) * WX * 4) & (TN - 1));
+#pragma unroll
+        for (int i = 0; i < TI; i++) a[h][i] = *reinterpret_cast<const f32x4_t*>(sa + i * 16 * 128 + (((4 * h + lg) ^ (lr & 6)) * 16));
+#pragma unroll
+        for (int s = 0; s < 4; s++) load_cols<NJ>(sb + (16 * h + 4 * lg + s) * TN + col, b[h][s]);
+    };
+    auto multiply = [&](int h) {
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][i][s], b[h][s][j], acc[i][j], 0, 0, 0);
+    };
+    // Schedule of a half: an LDS read behind each of the first matrix instructions, then one direct load behind every second. Issued in
+    // one go the four wavefronts queue up for the LDS and the address unit while the matrix units stand still (4096 x 6144 x 1536: 618 -> 559 us, 125 -> 138 TFLOP/s).
+    auto spread = [&](auto loads_tag) {
+        constexpr int NM = TI * NJ * 4, R = TI + 4, LOADS = decltype(loads_tag)::value ? LA + LB : 0;
+        constexpr int PER_READ = NM / 2 >= R * 2 ? 2 : 1;                    // matrix instructions in front of a read
+        constexpr int USED = R * PER_READ < NM ? R * PER_READ : NM;
+        constexpr int PER_LOAD = (NM - USED) / (LA + LB) > 0 ? (NM - USED) / (LA + LB) : 1;
+#pragma unroll
+        for (int x = 0; x < R; x++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, PER_READ, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+#pragma unroll
+        for (int x = 0; x < LOADS; x++) {
+            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, PER_LOAD, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES; s++) issue_tile(s, s);
+    wait_vmcnt<(STAGES - 1) * (LA + LB)>();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch(0, 0);
+    for (int kt = 0, stage = 0; kt < nkt; kt++) {
+        fetch(stage, 1);
+        multiply(0);
+        spread(std::false_type{});
+        // this thread's loads of tile kt+1 have landed and its LDS reads of tile kt are done; behind the barrier that holds for everyone
+        constexpr int INFLIGHT = (STAGES - 2) * (LA + LB);
+        __builtin_amdgcn_s_waitcnt((INFLIGHT & 15) | (7 << 4) | ((INFLIGHT >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int freed = stage;
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+        fetch(stage, 0);
+        issue_tile(kt + STAGES, freed);
+        multiply(1);
+        spread(std::true_type{});
+    }
+    wait_vmcnt<0>();  // no direct load may still be on its way into this workgroup's LDS when it ends
+    // C layout of a 16x16 block: lane = column l%16 (of block j: column NJ*(l%16) + j), register r = row 4*(l/16) + r
+    const int n = n_blk + wn * (TN / WN) + NJ * lr;
+    if (n >= N) return;  // (N is a multiple of 4, so a lane's columns are all inside or all outside)
+    const EpiDev& e = pr.epi;
+    float bias[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) bias[j] = e.bias ? e.bias[pr.n0 + n + j] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = m_blk + wm * (TM / WM) + i * 16 + 4 * lg + r;
+            if (m >= M) continue;
+            const long long idx = (long long)m * pr.ldc + n;
+            float v[NJ], g[NJ], t[NJ];
+            if (EPI == EPI_GATE_RESID) {
+                load_cols<NJ>(e.gate + (long long)(m / e.rows_per_batch) * e.gate_ld + n, g);
+                load_cols<NJ>(e.resid + idx, t);
+            } else if (EPI == EPI_BIAS_ROWADD) {
+                load_cols<NJ>(e.table + (long long)(m % e.rows_per_batch) * e.gate_ld + n, t);
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                v[j] = acc[i][j][r] + bias[j];
+                if (EPI == EPI_BIAS_GELU) v[j] = gelu_tanh_precise(v[j]);
+                else if (EPI == EPI_BIAS_SILU) v[j] = silu_precise(v[j]);
+                else if (EPI == EPI_GATE_RESID) v[j] = v[j] * g[j] + t[j];
+                else if (EPI == EPI_BIAS_ROWADD) v[j] += t[j];
+            }
+            store_cols<NJ>(pr.out + idx, v);
+        }
+}
+
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
+int launch_tile(TileProbSet& set, int n, hipStream_t st) {
+    auto kern = gemm_f32_tile_kernel<TM, TN, WM, WN, STAGES, EPI>;
+    constexpr int smem = STAGES * (TM * 128 + TK * TN * 4);
+    static bool attr_done = false;  // raising the dynamic LDS limit is a per-function, per-process setting
+    if (smem > 65536 && !attr_done) {
+        SD3_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+        attr_done = true;
+    }
+    int total = 0;
+    for (int i = 0; i < MAX_PROBS; i++) {
+        if (i < n) total += ((set.p[i].M + TM - 1) / TM) * ((set.p[i].N + TN - 1) / TN);
+        set.end[i] = total;
+    }
+    hipLaunchKernelGGL(kern, dim3(total), dim3(WM * WN * 64), smem, st, set);
+    return launch_status("gemm_f32");
+}
+
+// The tile shapes, largest first, and what one K tile (32 k values) of one output tile costs in cycles, measured over N = 1536 .. 6144
+// and K = 1536, 6144: alone on its compute unit, and with two or three workgroups sharing one (the matrix instructions alone: TM*TN/4).
+struct TileShape {
+    int tm, tn;
+    double alone, shared;
+};
+constexpr TileShape TILE_SHAPES[] = {{128, 128, 4690, 4660}, {128, 64, 2560, 2430}, {64, 64, 1480, 1300}, {32, 64, 890, 720}, {32, 32, 580, 410}};
+
+template <int EPI>
+int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
+    switch (shape) {
+        // (rings no deeper than that two or three workgroups fit a compute unit: they hide each other's waits better than a deeper ring)
+        case 0: return launch_tile<128, 128, 2, 2, 2, EPI>(set, n, st);
+        case 1: return launch_tile<128, 64, 4, 1, 3, EPI>(set, n, st);
+        case 2: return launch_tile<64, 64, 2, 2, 3, EPI>(set, n, st);
+        case 3: return launch_tile<32, 64, 2, 2, 4, EPI>(set, n, st);
+        default: return launch_tile<32, 32, 2, 2, 5, EPI>(set, n, st);
+    }
+}
+
+// The shape whose busiest compute unit is done first: with r output tiles on it, r * shared cycles per K tile (alone for r = 1).
+// 1024 x 1536 x 6144 (96 / 192 / 384 / 768 / 1536 tiles): 378 / 211 / 211 / 186 / 202 us.
+int pick_tile(const TileProbSet& set, int n, int cus) {
+    int best = 0;
+    double best_cost = 0;
+    for (int s = 0; s < (int)(sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0])); s++) {
+        const TileShape t = TILE_SHAPES[s];
+        long long tiles = 0, depth = 0;
+        for (int i = 0; i < n; i++) {
+            const long long c = (long long)((set.p[i].M + t.tm - 1) / t.tm) * ((set.p[i].N + t.tn - 1) / t.tn);
+            tiles += c;
+            depth += c * set.p[i].K;
+        }
+        const long long r = (tiles + cus - 1) / cus;
+        const double cost = (double)depth / tiles * (r == 1 ? t.alone : r * t.shared);
+        if (s == 0 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+bool whole_chunks(const GemmF32Problem& q, int epi) {
+    auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    if (!al(q.A) || !al(q.W) || !al(q.out) || q.lda % 4 || q.ldw % 4 || q.ldc % 4 || q.n0 % 4 || q.K % 4 || q.N % 4) return false;
+    if (epi == EPI_GATE_RESID) return al(q.ea.gate) && al(q.ea.resid) && q.ea.gate_ld % 4 == 0;
+    if (epi == EPI_BIAS_ROWADD) return al(q.ea.table);
+    return true;
+}
 }  // namespace
+
+int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st) {
+    if (n < 1 || n > MAX_PROBS) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: 1 to %d problems (got %d)", MAX_PROBS, n);
+    TileProbSet set{};
+    int m = 0;
+    for (int i = 0; i < n; i++) {
+        const GemmF32Problem& q = probs[i];
+        if (q.M <= 0 || q.N <= 0) continue;
+        if (q.K <= 0) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: K must be positive");
+        EpiDev e{q.ea.bias, q.ea.gate, q.ea.resid, q.ea.table, q.ea.gate_ld, q.ea.rows_per_batch > 0 ? q.ea.rows_per_batch : 1};
+        if (epi == EPI_BIAS_ROWADD) e.gate_ld = q.N;
+        if (!whole_chunks(q, epi)) {
+            dim3 grid((q.N + BN - 1) / BN, (q.M + BM - 1) / BM), block(256);
+#define SD3_GEMM_F32_LAUNCH(E) \
+    case E: hipLaunchKernelGGL((gemm_f32_kernel<E>), grid, block, 0, st, q.A, q.lda, q.W, q.ldw, q.n0, q.out, q.ldc, q.M, q.N, q.K, e); break
+            switch (epi) {
+                SD3_GEMM_F32_LAUNCH(EPI_BIAS);
+                SD3_GEMM_F32_LAUNCH(EPI_BIAS_GELU);
+                SD3_GEMM_F32_LAUNCH(EPI_BIAS_SILU);
+                SD3_GEMM_F32_LAUNCH(EPI_GATE_RESID);
+                SD3_GEMM_F32_LAUNCH(EPI_BIAS_ROWADD);
+                default: return fail(SD3_ERR_INVALID_ARG, "gemm_f32: unknown epilogue %d", epi);
+            }
+#undef SD3_GEMM_F32_LAUNCH
+            SD3_TRY(launch_status("gemm_f32"));
+            continue;
+        }
+        set.p[m++] = TileProb{q.A, q.W, q.out, q.lda, q.ldw, q.ldc, q.M, q.N, q.K, q.n0, e};
+    }
+    if (m == 0) return SD3_OK;
+    const int cus = compute_units();
+    if (cus <= 0) return SD3_ERR_HIP;
+    const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile : pick_tile(set, m, cus);
+    switch (epi) {
+        case EPI_BIAS: return launch_shape<EPI_BIAS>(shape, set, m, st);
+        case EPI_BIAS_GELU: return launch_shape<EPI_BIAS_GELU>(shape, set, m, st);
+        case EPI_BIAS_SILU: return launch_shape<EPI_BIAS_SILU>(shape, set, m, st);
+        case EPI_GATE_RESID: return launch_shape<EPI_GATE_RESID>(shape, set, m, st);
+        case EPI_BIAS_ROWADD: return launch_shape<EPI_BIAS_ROWADD>(shape, set, m, st);
+        default: return fail(SD3_ERR_INVALID_ARG, "gemm_f32: unknown epilogue %d", epi);
+    }
+}
 
 int gemm_f32(const float* A, int lda, const float* W, int ldw, int n0, float* out, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
              hipStream_t st) {
-    if (M <= 0 || N <= 0) return SD3_OK;
-    if (K <= 0) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: K must be positive");
-    EpiDev e{ea.bias, ea.gate, ea.resid, ea.table, ea.gate_ld, ea.rows_per_batch > 0 ? ea.rows_per_batch : 1};
-    if (epi == EPI_BIAS_ROWADD) e.gate_ld = N;
-    const bool aligned = (lda % 4 == 0) && (ldw % 4 == 0) && (n0 % 4 == 0) && (K % 4 == 0) && (N % 4 == 0) &&
-                         ((reinterpret_cast<uintptr_t>(A) & 15) == 0) && ((reinterpret_cast<uintptr_t>(W) & 15) == 0);
-    dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM), block(256);
-#define SD3_GEMM_F32_LAUNCH(E)                                                                                                               \
-    do {                                                                                                                                     \
-        if (aligned) hipLaunchKernelGGL((gemm_f32_kernel<E, true>), grid, block, 0, st, A, lda, W, ldw, n0, out, ldc, M, N, K, e);             \
-        else hipLaunchKernelGGL((gemm_f32_kernel<E, false>), grid, block, 0, st, A, lda, W, ldw, n0, out, ldc, M, N, K, e);                    \
-    } while (0)
-    switch (epi) {
-        case EPI_BIAS: SD3_GEMM_F32_LAUNCH(EPI_BIAS); break;
-        case EPI_BIAS_GELU: SD3_GEMM_F32_LAUNCH(EPI_BIAS_GELU); break;
-        case EPI_BIAS_SILU: SD3_GEMM_F32_LAUNCH(EPI_BIAS_SILU); break;
-        case EPI_GATE_RESID: SD3_GEMM_F32_LAUNCH(EPI_GATE_RESID); break;
-        case EPI_BIAS_ROWADD: SD3_GEMM_F32_LAUNCH(EPI_BIAS_ROWADD); break;
-        default: return fail(SD3_ERR_INVALID_ARG, "gemm_f32: unknown epilogue %d", epi);
-    }
-#undef SD3_GEMM_F32_LAUNCH
-    return launch_status("gemm_f32");
+    const GemmF32Problem q{A, W, out, lda, ldw, n0, ldc, M, N, K, ea};
+    return gemm_f32_grouped(&q, 1, epi, st);
 }
+
+int g_gemm_f32_tile = -1;  // -1: chosen from the sizes; 0..4: that entry of TILE_SHAPES (sd3_tune)
 
 }  // namespace sd3
