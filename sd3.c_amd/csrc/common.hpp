@@ -223,6 +223,13 @@ int layernorm_full(const float* x, float* y, float* mean, float* rstd, const flo
 // RMSNorm over groups of `hs` consecutive values inside rows of stride `ld` (in place allowed): x[r*ld + g*hs + i], g < groups
 int rmsnorm_rows(const float* x, float* y, const float* w, float* rms, float eps, long long rows, int groups, int hs, int ld_in, int ld_out,
                  hipStream_t st);
+// In-place per-head RMSNorm of the q and k thirds of packed q|k|v rows (3 * heads * hs values, row stride ld), several buffers per launch
+struct QkNormJob {
+    float* qkv;
+    const float *wq, *wk;
+    long long rows;
+};
+int qk_norm_rows(const QkNormJob* jobs, int n, float eps, int heads, int hs, int ld, hipStream_t st);
 int unary_op(const float* in, float* out, long long n, int act, hipStream_t st);
 int add_op(const float* a, const float* b, float* out, long long n, hipStream_t st);
 int add_silu_op(const float* a, const float* b, float* out, long long n, hipStream_t st);

@@ -481,10 +481,8 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     // ---- joint attention over [context ; latent] (modules.cpp:1427-1432); fp32 path: qk-norm in place first
     auto seg_ptr = [&](void* base, int third) -> void* { return (char*)base + (size_t)third * C * es; };
     if (!bf && d.qk) {
-        SD3_TRY(rmsnorm_rows((float*)c_qkv, (float*)c_qkv, w.c_rms_q, nullptr, 1e-6f, mc, d.NH, d.HS, 3 * C, 3 * C, st));
-        SD3_TRY(rmsnorm_rows((float*)seg_ptr(c_qkv, 1), (float*)seg_ptr(c_qkv, 1), w.c_rms_k, nullptr, 1e-6f, mc, d.NH, d.HS, 3 * C, 3 * C, st));
-        SD3_TRY(rmsnorm_rows((float*)x_qkv, (float*)x_qkv, w.x_rms_q, nullptr, 1e-6f, mx, d.NH, d.HS, 3 * C, 3 * C, st));
-        SD3_TRY(rmsnorm_rows((float*)seg_ptr(x_qkv, 1), (float*)seg_ptr(x_qkv, 1), w.x_rms_k, nullptr, 1e-6f, mx, d.NH, d.HS, 3 * C, 3 * C, st));
+        const QkNormJob norms[3] = {{(float*)x_qkv, w.x_rms_q, w.x_rms_k, mx}, {(float*)c_qkv, w.c_rms_q, w.c_rms_k, mc}, {(float*)x_qkv2, w.x2_rms_q, w.x2_rms_k, mx}};
+        SD3_TRY(qk_norm_rows(norms, d.dual ? 3 : 2, 1e-6f, d.NH, d.HS, 3 * C, st));
     }
     AttnSegments joint{}, dual_set{};
     joint.q[0] = c_qkv; joint.k[0] = seg_ptr(c_qkv, 1); joint.v[0] = seg_ptr(c_qkv, 2); joint.out[0] = d.discard ? nullptr : c_att;
@@ -541,10 +539,6 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
 
     // ---- extra self-attention over the latent tokens (modules.cpp:1440-1453, 1486)
     if (d.dual) {
-        if (!bf && d.qk) {
-            SD3_TRY(rmsnorm_rows((float*)x_qkv2, (float*)x_qkv2, w.x2_rms_q, nullptr, 1e-6f, mx, d.NH, d.HS, 3 * C, 3 * C, st));
-            SD3_TRY(rmsnorm_rows((float*)seg_ptr(x_qkv2, 1), (float*)seg_ptr(x_qkv2, 1), w.x2_rms_k, nullptr, 1e-6f, mx, d.NH, d.HS, 3 * C, 3 * C, st));
-        }
         if (!bf) SD3_TRY(attention(ctx, dual_set, B, d.NH, d.HS, bf));
         GemmEpilogueArgs g2;
         g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;

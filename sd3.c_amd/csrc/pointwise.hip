@@ -255,6 +255,70 @@ int rmsnorm_rows(const float* x, float* y, const float* w, float* rms, float eps
     return launch_status("rmsnorm");
 }
 
+// The in-place norms of the q and k thirds of up to three packed q|k|v buffers (the two streams and the dual branch): one launch instead
+// of two per buffer. Heads of 64 or 128 values (whole chunks): a lane holds its hs / 16 values in registers, read and written once.
+struct QkNormDev {
+    QkNormJob j[3];
+    long long end[3];  // running totals of (row, head) pairs, q and k counted separately
+};
+template <int NV>  // float4 per lane
+__global__ void __launch_bounds__(256) qk_norm_kernel(const QkNormDev jobs, float eps, int heads, int ld) {
+    const int sub = threadIdx.x & 15;
+    long long g = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 4;
+    if (g >= jobs.end[2]) return;  // whole 16-lane groups
+    const int which = (g >= jobs.end[0]) + (g >= jobs.end[1]);
+    const QkNormJob& job = jobs.j[which];
+    if (which) g -= jobs.end[which - 1];
+    const int per_row = 2 * heads;
+    const long long row = g / per_row;
+    const int col = (int)(g % per_row);  // q heads, then k heads: consecutive thirds of the row
+    float4* p = reinterpret_cast<float4*>(job.qkv + row * ld + (long long)col * (NV * 64));
+    const float4* w = reinterpret_cast<const float4*>(col < heads ? job.wq : job.wk);
+    float4 v[NV];
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        v[i] = p[sub + 16 * i];
+        s += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+    }
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
+    const float inv = 1.0f / sqrtf(eps + s / (NV * 64));
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const float4 a = w[sub + 16 * i];
+        p[sub + 16 * i] = make_float4(v[i].x * inv * a.x, v[i].y * inv * a.y, v[i].z * inv * a.z, v[i].w * inv * a.w);
+    }
+}
+
+int qk_norm_rows(const QkNormJob* jobs, int n, float eps, int heads, int hs, int ld, hipStream_t st) {
+    auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    bool vec = (hs == 64 || hs == 128) && ld % 4 == 0 && n <= 3;
+    for (int i = 0; i < n; i++) vec = vec && al(jobs[i].qkv) && al(jobs[i].wq) && al(jobs[i].wk);
+    if (!vec) {
+        for (int i = 0; i < n; i++) {
+            SD3_TRY(rmsnorm_rows(jobs[i].qkv, jobs[i].qkv, jobs[i].wq, nullptr, eps, jobs[i].rows, heads, hs, ld, ld, st));
+            float* k = jobs[i].qkv + (long long)heads * hs;
+            SD3_TRY(rmsnorm_rows(k, k, jobs[i].wk, nullptr, eps, jobs[i].rows, heads, hs, ld, ld, st));
+        }
+        return SD3_OK;
+    }
+    QkNormDev d{};
+    long long total = 0;
+    for (int i = 0; i < 3; i++) {
+        if (i < n) {
+            d.j[i] = jobs[i];
+            total += jobs[i].rows * 2 * heads;
+        }
+        d.end[i] = total;
+    }
+    if (total == 0) return SD3_OK;
+    dim3 grid((unsigned)((total * 16 + 255) / 256)), block(256);
+    if (hs == 64) hipLaunchKernelGGL(qk_norm_kernel<1>, grid, block, 0, st, d, eps, heads, ld);
+    else hipLaunchKernelGGL(qk_norm_kernel<2>, grid, block, 0, st, d, eps, heads, ld);
+    return launch_status("qk_norm");
+}
+
 // ---- elementwise ----
 template <int OP>  // 0 silu, 1 gelu_tanh, 2 gelu (erf form, modules.cpp:280-285)
 __global__ void __launch_bounds__(256) unary_kernel(const float* __restrict__ in, float* __restrict__ out, long long n) {
