@@ -1,4 +1,4 @@
-// bf16 GEMM on the gfx950 matrix cores (v_mfma_f32_32x32x16_bf16), fp32 accumulation:
+// bf16 GEMM on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16), fp32 accumulation:
 //   out(M,N) = A(M,K) @ Wp^T + epilogue,  A bf16 row-major, Wp bf16 (N,K) row-major (the reference's (K,N) fp32
 //   weight transposed and rounded once by pack_weight_bf16), so that both operands are K-contiguous.
 // It replaces linear / partial_linear of the reference (modules.cpp:475-511) for the QKV, out-projection and MLP
@@ -7,6 +7,8 @@
 // Data path: global -> LDS with direct loads (global_load_lds_dwordx4: no registers, no VALU), a ring of STAGES
 // LDS buffers with one workgroup barrier per 64-deep K tile; LDS rows are 128 bytes with the 16-byte chunk index
 // XOR-swizzled by a key of the row, which makes both the linear LDS fill and the 16-byte MFMA operand reads conflict-free.
+// Two kernels: gemm_bf16_kernel (256x256 tiles by persistent workgroups; also the fp8 form) for launches that fill the device with
+// them, gemm_bf16_ring_kernel (64x64 to 256x128 tiles) for the others; tile_shapes says where the line is.
 #include "common.hpp"
 
 #include <type_traits>
@@ -37,6 +39,24 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // eight 16-byte slots of a half. (With swz() that pattern hits every slot twice: the bank-conflict counter read 47 % of the LDS
 // cycles; the 32x32 layout, lane l: row l % 32, is conflict-free with swz() and would not be with this key.)
 __device__ __forceinline__ int swz16(int row) { return row & 6; }
+
+// RMSNorm of one head of one token (modules.cpp:192-198) held by 16 consecutive lanes, four columns each
+__device__ __forceinline__ void qk_norm4(float (&v)[4], const float4 w4) {
+    // explicit fused multiply-adds: left to the compiler, each unrolled copy of this code may pick a different product to fuse, and a row's
+    // result would depend on where in the tile it sits
+    float ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
+    // butterfly over the 16 lanes with data-parallel-primitive moves (no trip through the LDS crossbar): lanes ^1 and ^2 by quad permutes;
+    // after those every quad holds one value, so mirroring the half row (i <-> 7-i) and then the row (i <-> 15-i) pairs the same
+    // partial sums as lanes ^4 and ^8 would
+    ss += dpp_move<0xB1>(ss);   // quad_perm [1,0,3,2]
+    ss += dpp_move<0x4E>(ss);   // quad_perm [2,3,0,1]
+    ss += dpp_move<0x141>(ss);  // row_half_mirror
+    ss += dpp_move<0x140>(ss);  // row_mirror
+    // (the hardware's reciprocal square root, 1 ulp: a divide and a square root here cost 0.2 ms per forward of the 1024x1024 pair, and
+    // the result is rounded to bf16 anyway)
+    const float inv = __builtin_amdgcn_rsqf(1e-6f + ss * (1.0f / 64.0f));
+    v[0] = (v[0] * inv) * w4.x; v[1] = (v[1] * inv) * w4.y; v[2] = (v[2] * inv) * w4.z; v[3] = (v[3] * inv) * w4.w;
+}
 
 // LDS bytes of a configuration: the tile ring, or the epilogue staging slabs if those are larger
 template <int BM, int BN, int WM, int WN, int STAGES>
@@ -79,9 +99,9 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
     constexpr int A_BYTES = BM * 128, STAGE_BYTES = (BM + BN) * 128;
     constexpr int LA = BM * 8 / NT, LB = BN * 8 / NT;        // 16-byte chunks per thread per tile
     static_assert(BM * 8 % NT == 0 && BN * 8 % NT == 0, "tile rows must divide evenly over the threads");
-    static_assert(BM % (WM * 16) == 0 && BN % (WN * 16) == 0 && (BM == 256 || (BM % (WM * 32) == 0 && BN % (WN * 32) == 0)), "wavefront tiles are made of 16x16 (256-row tiles) or 32x32 blocks");
+    static_assert(BM % (WM * 16) == 0 && BN % (WN * 16) == 0 && (!FP8 || (BM % (WM * 32) == 0 && BN % (WN * 32) == 0)), "wavefront tiles are made of 16x16 (bf16) or 32x32 (fp8) blocks");
 
-    constexpr bool M16 = (BM == 256) && !FP8;  // 16x16x32 matrix instructions (see below)
+    constexpr bool M16 = !FP8;  // bf16: 16x16x32 matrix instructions (see below); fp8: 32x32x64
     auto key = [](int row) { return M16 ? swz16(row) : swz(row); };
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS destinations of the direct loads are then scalar
@@ -115,10 +135,9 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
         for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + kt * 128), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
     };
 
-    // Two matrix instructions. 256x256 tiles use v_mfma_f32_16x16x32_bf16: on this device the clock under matrix load is set by
-    // the power limit, and measured on random operands the 16x16x32 form sustains 15-24 % more than 32x32x16 at the same nominal
-    // rate (half as many accumulator updates per product). 128x128 tiles keep v_mfma_f32_32x32x16_bf16: with four wavefronts per
-    // workgroup the finer instruction stream measured 5-15 % slower there. Both forms give bit-identical results.
+    // bf16 uses v_mfma_f32_16x16x32_bf16: on this device the clock under matrix load is set by the power limit, and measured on
+    // random operands the 16x16x32 form sustains 15-24 % more than 32x32x16 at the same nominal rate (half as many accumulator
+    // updates per product). Both forms give bit-identical results.
     constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;      // 16x16 blocks per wavefront
     f32x16_t acc[M16 ? 1 : TM][M16 ? 1 : TN];
     f32x4_t acc16[M16 ? MI : 1][M16 ? NJ : 1];
@@ -268,20 +287,15 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
         k_tile(nkt - 1, std::false_type{});
     } else {
         // operand addresses inside a stage: row*128 + (chunk ^ sw)*16 with sw = swz(row) = swz(l32) (block offsets are multiples of 16).
-        // bf16: k-step ks (16 deep) takes chunk 2*ks + lk; fp8: k-step ks (64 deep) takes the two chunks 4*ks + 2*lk, +1
+        // k-step ks (64 deep) takes the two chunks 4*ks + 2*lk, +1
         const int sw = swz(l32);
         const int a_off = (wm * (BM / WM) + l32) * 128, b_off = A_BYTES + (wn * (BN / WN) + l32) * 128;
         // operand fragments of k-step ks live in buffer ks&1; those of step ks+1 are fetched from LDS while the matrix cores work on step ks
-        using frag_t = std::conditional_t<FP8, i32x8_t, bf16x8_t>;
-        frag_t a[2][TM], b[2][TN];
-        auto read_frag = [&](const char* row, int ks) -> frag_t {
-            if constexpr (FP8) {
-                const i32x4_t lo = *reinterpret_cast<const i32x4_t*>(row + (((4 * ks + 2 * lk) ^ sw) * 16));
-                const i32x4_t hi = *reinterpret_cast<const i32x4_t*>(row + (((4 * ks + 2 * lk + 1) ^ sw) * 16));
-                return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-            } else {
-                return *reinterpret_cast<const bf16x8_t*>(row + (((2 * ks + lk) ^ sw) * 16));
-            }
+        i32x8_t a[2][TM], b[2][TN];
+        auto read_frag = [&](const char* row, int ks) -> i32x8_t {
+            const i32x4_t lo = *reinterpret_cast<const i32x4_t*>(row + (((4 * ks + 2 * lk) ^ sw) * 16));
+            const i32x4_t hi = *reinterpret_cast<const i32x4_t*>(row + (((4 * ks + 2 * lk + 1) ^ sw) * 16));
+            return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         };
         auto fetch = [&](const char* st, int ks, int buf) {
 #pragma unroll
@@ -289,7 +303,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
 #pragma unroll
             for (int j = 0; j < TN; j++) b[buf][j] = read_frag(st + b_off + j * 32 * 128, ks);
         };
-        constexpr int DSR = FP8 ? 2 : 1;  // LDS reads per fragment
+        constexpr int DSR = 2;  // LDS reads per fragment
 
         // Every stage is filled up front and exactly one tile is requested per K tile after that (past the end: the last tile
         // once more, into a buffer nobody reads again), so "tile kt+1 has landed" is always "all but the newest STAGES-2 tiles".
@@ -303,7 +317,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
         fetch(smem, 0, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, DSR * (TM + TN), 0);
 
-        constexpr int KS = FP8 ? 2 : 4;  // k-steps per 128-byte K tile
+        constexpr int KS = 2;  // k-steps per 128-byte K tile
         // One K tile. The workgroup barrier sits in front of the LAST k-step of a tile, not behind it: by then every fragment
         // of tile kt is in registers (or on its way: waited for), so its buffer can be handed to the loads of tile kt+2, and the
         // loads' issue and the first fragment reads of tile kt+1 are interleaved with the matrix instructions of that last
@@ -316,10 +330,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
 #pragma unroll
                 for (int i = 0; i < TM; i++)
 #pragma unroll
-                    for (int j = 0; j < TN; j++) {
-                        if constexpr (FP8) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0, 0, 0, 0);
-                        else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0);
-                    }
+                    for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0, 0, 0, 0);
             };
             // scheduling pattern of a step: behind each of the first matrix instructions one LDS fragment read of the next step
             // (and, in the last step, one direct global->LDS load of the tile after next), so that their issue and latency are
@@ -453,21 +464,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
                     // 16 consecutive lanes hold 64 consecutive columns of this row = one head of one token (modules.cpp:192-198, fused)
                     const int third = n0 / epi.gate_ld;  // 0 = q, 1 = k, 2 = v (uniform over the 16 lanes: C is a multiple of 64)
                     if (third < 2) {
-                        // explicit fused multiply-adds: left to the compiler, each unrolled copy of this code may pick a different
-                        // product to fuse, and a row's result would depend on where in the tile it sits
-                        float ss = fmaf(v[3], v[3], fmaf(v[2], v[2], fmaf(v[1], v[1], v[0] * v[0])));
-                        // butterfly over the 16 lanes with data-parallel-primitive moves (no trip through the LDS crossbar): lanes ^1 and ^2
-                        // by quad permutes; after those every quad holds one value, so mirroring the half row (i <-> 7-i) and then the
-                        // row (i <-> 15-i) pairs the same partial sums as lanes ^4 and ^8 would
-                        ss += dpp_move<0xB1>(ss);   // quad_perm [1,0,3,2]
-                        ss += dpp_move<0x4E>(ss);   // quad_perm [2,3,0,1]
-                        ss += dpp_move<0x141>(ss);  // row_half_mirror
-                        ss += dpp_move<0x140>(ss);  // row_mirror
-                        // (the hardware's reciprocal square root, 1 ulp: a divide and a square root here cost 0.2 ms per forward,
-                        // and the result is rounded to bf16 anyway)
-                        const float inv = __builtin_amdgcn_rsqf(1e-6f + ss * (1.0f / 64.0f));
-                        const float4 w4 = *reinterpret_cast<const float4*>((third == 0 ? epi.gate : epi.resid) + (n0 & 63));
-                        v[0] = (v[0] * inv) * w4.x; v[1] = (v[1] * inv) * w4.y; v[2] = (v[2] * inv) * w4.z; v[3] = (v[3] * inv) * w4.w;
+                        qk_norm4(v, *reinterpret_cast<const float4*>((third == 0 ? epi.gate : epi.resid) + (n0 & 63)));
                     }
                 }
                 res[p] = make_float4(v[0], v[1], v[2], v[3]);
@@ -544,13 +541,289 @@ int launch_epi_fp8(int variant, ProbSet& args, int n, hipStream_t st) {
     return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32, true>(args, n, st);
 }
 
+// ---- launches that do not fill the device with 256x256 tiles ----
+// A layer of a few hundred to a few thousand rows is fewer 256x256 tiles than there are compute units, and what it waits for is its
+// weights, which nobody has touched yet: the K loop's pace is set by how many compute units take part and by the bytes each has in
+// flight, less by the matrix instructions. So: a range of smaller tiles (64-column wavefronts: one attention head, so that the qk-norm
+// stays inside a wavefront), one workgroup per tile, eight wavefronts for all but the smallest (two per SIMD: 128x128 tiles of 8 against 4
+// wavefronts, mlp-2 of 2356 rows, 59 against 65 us), a ring of stages as deep as the LDS allows, fragments fetched a whole K tile (or half
+// of one) ahead of their matrix instructions, one barrier per K tile. mlp-2 with cold weights, rows 333 / 1178 / 2356 / 4250: 64 -> 31,
+// 86 -> 44, 86 -> 60, 99 -> 83 us.
+// Lane l of a 16-column block of W holds row l%16 of its LDS block; the loader puts output column NJ*(l%16) + j there (block j), so a lane
+// ends with NJ consecutive columns of a row and the epilogue stores straight from the accumulators.
+// The order of k is that of the other tiles (bit-identical results).
+// waits until all but the newest `ahead` tiles (at most MAX, PER loads of this thread each) have landed
+template <int MAX, int PER>
+__device__ __forceinline__ void wait_tiles(int ahead) {
+    if constexpr (MAX == 0) wait_vmcnt<0>();
+    else if (ahead >= MAX) wait_vmcnt<MAX * PER>();
+    else wait_tiles<MAX - 1, PER>(ahead);
+}
+template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_F32>
+__global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const ProbSet args) {
+    constexpr int NT = WM * WN * 64, TI = TM / WM / 16, WC = TN / WN, NJ = WC / 16;
+    constexpr int A_BYTES = TM * 128, STAGE_BYTES = (TM + TN) * 128;
+    constexpr int LA = TM * 8 / NT, LB = TN * 8 / NT;
+    static_assert(NJ == 4 && TI >= 1 && TM * 8 % NT == 0 && TN * 8 % NT == 0, "tile shape");
+    static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "the loads in flight must fit the 6-bit counter");
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    const int w = blockIdx.x;
+    const int which = (w >= args.end[0]) + (w >= args.end[1]);
+    const Prob& pr = args.p[which];
+    const int M = pr.M, N = pr.N, K = pr.K, ldc = pr.ldc;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+    int tile_m, tile_n;
+    tile_of_workgroup(w - (which ? args.end[which - 1] : 0), (M + TM - 1) / TM, (N + TN - 1) / TN, tile_m, tile_n);
+    const int m_blk = tile_m * TM, n_blk = tile_n * TN;
+
+    const char* ga[LA];
+    const char* gb[LB];
+#pragma unroll
+    for (int i = 0; i < LA; i++) {
+        const int q = i * NT + tid, row = q >> 3;
+        ga[i] = reinterpret_cast<const char*>(pr.A + (long long)min(m_blk + row, M - 1) * K) + ((q & 7) ^ swz16(row)) * 16;
+    }
+#pragma unroll
+    for (int i = 0; i < LB; i++) {
+        const int q = i * NT + tid, row = q >> 3;
+        const int n = n_blk + row / WC * WC + NJ * (row % 16) + row % WC / 16;
+        gb[i] = reinterpret_cast<const char*>(pr.Wp + (long long)min(n, N - 1) * K) + ((q & 7) ^ swz16(row)) * 16;
+    }
+    const int nkt = K / BK;
+    auto issue_tile = [&](int kt, int stage) {
+        char* sa = smem + stage * STAGE_BYTES + wave * 1024;
+        char* sb = sa + A_BYTES;
+        const int off = kt * 128;
+#pragma unroll
+        for (int i = 0; i < LA; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(ga[i] + off), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + off), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+    };
+    f32x4_t acc[TI][NJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    // Fragments are fetched ahead of their matrix instructions: a whole K tile ahead where it fits the registers, else one 32-deep half
+    constexpr bool WHOLE = TI * NJ < 16 && MW <= 2;
+    bf16x8_t a[WHOLE ? 2 : 1][2][TI], b[WHOLE ? 2 : 1][2][NJ];  // [buffer][half]
+    auto fetch_half = [&](int stage, int buf, int h) {
+        const char* st = smem + stage * STAGE_BYTES;
+        const int chunk = ((4 * h + lg) ^ swz16(lr)) * 16;
+#pragma unroll
+        for (int i = 0; i < TI; i++) a[buf][h][i] = *reinterpret_cast<const bf16x8_t*>(st + (wm * (TM / WM) + i * 16 + lr) * 128 + chunk);
+#pragma unroll
+        for (int j = 0; j < NJ; j++) b[buf][h][j] = *reinterpret_cast<const bf16x8_t*>(st + A_BYTES + (wn * WC + j * 16 + lr) * 128 + chunk);
+    };
+    auto multiply_half = [&](int buf, int h) {
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[buf][h][i], b[buf][h][j], acc[i][j], 0, 0, 0);
+    };
+    // schedule: NR LDS reads behind the first matrix instructions, then (with LOADS) one direct load behind each of the next ones
+    auto spread = [&](auto nm_tag, auto nr_tag, auto loads_tag) {
+        constexpr int NM = decltype(nm_tag)::value, NR = decltype(nr_tag)::value, PER = (NR + NM - 1) / NM, SLOTS = (NR + PER - 1) / PER;
+#pragma unroll
+        for (int x = 0; x < SLOTS; x++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, PER, 0);
+        }
+        if (decltype(loads_tag)::value)
+#pragma unroll
+            for (int x = 0; x < LA + LB; x++) {
+                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int s = 0; s < STAGES; s++)
+        if (s < nkt) issue_tile(s, s);
+    wait_tiles<STAGES - 1, LA + LB>(nkt - 1);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch_half(0, 0, 0);
+    if (WHOLE) fetch_half(0, 0, 1);
+    int stage = 0;
+    // One K tile: once its fragments are in registers hand its stage back, request the tile STAGES ahead into it, and fetch the next tile's
+    // fragments beside the matrix instructions. (Past the end nothing is requested: a deep ring's surplus tiles would be a quarter of the
+    // traffic of a launch with 24 K tiles.)
+    auto k_tile = [&](int kt, auto buf_tag, auto more_tag) {
+        constexpr bool MORE = decltype(more_tag)::value;
+        constexpr int BUF = WHOLE ? decltype(buf_tag)::value : 0;
+        using std::integral_constant;
+        if constexpr (!WHOLE) {
+            fetch_half(stage, 0, 1);
+            multiply_half(0, 0);
+            spread(integral_constant<int, TI * NJ>{}, integral_constant<int, TI + NJ>{}, std::false_type{});
+        }
+        if (MORE) wait_tiles<STAGES - 2, LA + LB>(STAGES - 2);
+        else wait_tiles<STAGES - 2, LA + LB>(nkt - 2 - kt);  // tile kt+1 has landed ...
+        __builtin_amdgcn_s_waitcnt(0xc07f);                  // ... and this thread's LDS reads of tile kt are done (lgkmcnt(0))
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int freed = stage;
+        stage = stage + 1 == STAGES ? 0 : stage + 1;
+        fetch_half(stage, WHOLE ? BUF ^ 1 : 0, 0);
+        if (WHOLE) fetch_half(stage, BUF ^ 1, 1);
+        if (MORE) issue_tile(kt + STAGES, freed);
+        if constexpr (WHOLE) {
+            multiply_half(BUF, 0);
+            multiply_half(BUF, 1);
+            spread(integral_constant<int, 2 * TI * NJ>{}, integral_constant<int, 2 * (TI + NJ)>{}, more_tag);
+        } else {
+            multiply_half(0, 1);
+            spread(integral_constant<int, TI * NJ>{}, integral_constant<int, TI + NJ>{}, more_tag);
+        }
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    int kt = 0;
+    for (; kt + 1 + STAGES < nkt; kt += 2) {
+        k_tile(kt, even, std::true_type{});
+        k_tile(kt + 1, odd, std::true_type{});
+    }
+    if (kt + STAGES < nkt) {
+        k_tile(kt++, even, std::true_type{});
+#pragma unroll 1
+        for (; kt < nkt; kt += 2) {
+            k_tile(kt, odd, std::false_type{});
+            if (kt + 1 < nkt) k_tile(kt + 1, even, std::false_type{});
+        }
+    } else {
+#pragma unroll 1
+        for (; kt < nkt; kt += 2) {
+            k_tile(kt, even, std::false_type{});
+            if (kt + 1 < nkt) k_tile(kt + 1, odd, std::false_type{});
+        }
+    }
+    wait_vmcnt<0>();
+
+    const int n0 = n_blk + wn * WC + NJ * lr;
+    if (n0 >= N) return;  // (N is a multiple of 4)
+    const EpiDev& epi = pr.epi;
+    const int rpb = epi.rows_per_batch;
+    float bias4[4] = {0.f, 0.f, 0.f, 0.f};
+    if (epi.bias)
+#pragma unroll
+        for (int c = 0; c < 4; c++) bias4[c] = epi.bias[n0 + c];
+    float4 norm_w = make_float4(1.f, 1.f, 1.f, 1.f);
+    const int third = EPI == EPI_QKV_NORM ? n0 / epi.gate_ld : 0;
+    if (EPI == EPI_QKV_NORM && third < 2) norm_w = *reinterpret_cast<const float4*>((third == 0 ? epi.gate : epi.resid) + (n0 & 63));
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = m_blk + wm * (TM / WM) + i * 16 + 4 * lg + r;  // (uniform over the 16 lanes that share a head)
+            if (m >= M) continue;
+            const long long idx = (long long)m * ldc + n0;
+            float v[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = acc[i][c][r] + bias4[c];
+            if (EPI == EPI_BIAS_GELU) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) v[c] = gelu_tanh_f(v[c]);
+            } else if (EPI == EPI_BIAS_SILU) {
+#pragma unroll
+                for (int c = 0; c < 4; c++) v[c] = v[c] / (1.0f + __expf(-v[c]));
+            } else if (EPI == EPI_GATE_RESID) {
+                const float4 g4 = *reinterpret_cast<const float4*>(epi.gate + (long long)(m / rpb) * epi.gate_ld + n0);
+                const float4 r4 = *reinterpret_cast<const float4*>(epi.resid + idx);
+                v[0] = r4.x + g4.x * v[0]; v[1] = r4.y + g4.y * v[1]; v[2] = r4.z + g4.z * v[2]; v[3] = r4.w + g4.w * v[3];
+            } else if (EPI == EPI_BIAS_ROWADD) {
+                const float4 t4 = *reinterpret_cast<const float4*>(epi.table + (long long)(m % rpb) * epi.gate_ld + n0);
+                v[0] += t4.x; v[1] += t4.y; v[2] += t4.z; v[3] += t4.w;
+            } else if (EPI == EPI_QKV_NORM && third < 2) {
+                qk_norm4(v, norm_w);
+            }
+            if (OUT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(pr.out) + idx) = make_float4(v[0], v[1], v[2], v[3]);
+            else *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(pr.out) + idx) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        }
+}
+
+template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_F32>
+int launch_ring(ProbSet& args, int n, hipStream_t st) {
+    auto kern = gemm_bf16_ring_kernel<TM, TN, WM, WN, STAGES, MW, EPI, OUT_F32>;
+    constexpr int smem = STAGES * (TM + TN) * 128;
+    static bool attr_done = false;  // raising the dynamic LDS limit is a per-function, per-process setting
+    if (smem > 65536 && !attr_done) {
+        SD3_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
+        attr_done = true;
+    }
+    int total = 0;
+    for (int i = 0; i < MAX_PROBS; i++) {
+        if (i < n) total += ((args.p[i].N + TN - 1) / TN) * ((args.p[i].M + TM - 1) / TM);
+        args.end[i] = total;
+    }
+    hipLaunchKernelGGL(kern, dim3(total), dim3(WM * WN * 64), smem, st, args);
+    g_gemm_bf16_launches.fetch_add(1, std::memory_order_relaxed);
+    return launch_status("gemm_bf16");
+}
+
+// The tile shapes of the bf16 GEMM, smallest first, and what an output tile costs its compute unit in microseconds: `fixed` + `per_k` for
+// each K tile of 64. Fitted to launches with cold weights at K = 1536 and 6144, 333 to 4250 rows, N = 1536 .. 6144 (a constant for the
+// first round, the same for all shapes, left out); what they stand for is the traffic of (tm + tn) * 128 bytes per K tile through one
+// compute unit's load path and, from 128x128 on, the matrix instructions.
+struct TileShape {
+    int tm, tn;
+    double fixed, per_k;
+};
+enum { TILE_64, TILE_128_64, TILE_64_128, TILE_128, TILE_256_128, TILE_256, TILE_SHAPES };
+constexpr TileShape tile_shapes[TILE_SHAPES] = {{64, 64, 1.3, 0.19},    {128, 64, 2.3, 0.285},  {64, 128, 2.3, 0.285},
+                                                {128, 128, 7.3, 0.403}, {256, 128, 11.3, 0.59}, {256, 256, 11.3, 1.28}};
+
+long long tiles_of(const Prob& q, int shape) {
+    const TileShape& t = tile_shapes[shape];
+    return (long long)((q.M + t.tm - 1) / t.tm) * ((q.N + t.tn - 1) / t.tn);
+}
+double launch_cost(const ProbSet& set, int n, int shape, int cus) {
+    long long tiles = 0, depth = 0;
+    for (int i = 0; i < n; i++) {
+        const long long c = tiles_of(set.p[i], shape);
+        tiles += c;
+        depth += c * (set.p[i].K / BK);
+    }
+    const TileShape& t = tile_shapes[shape];
+    return (double)((tiles + cus - 1) / cus) * (t.fixed + t.per_k * ((double)depth / tiles));
+}
+int cheapest_shape(const ProbSet& set, int n, int cus, double& cost) {
+    int best = TILE_256;
+    cost = launch_cost(set, n, TILE_256, cus);
+    for (int s = TILE_256 - 1; s >= 0; s--) {
+        const double c = launch_cost(set, n, s, cus);
+        if (c < cost) {
+            best = s;
+            cost = c;
+        }
+    }
+    return best;
+}
+
+// Rings: as deep as one workgroup per compute unit allows where a launch is a single round; 64x64 tiles and, with more than one round, the
+// next two shapes leave room for a second workgroup (mlp-2 of 1178 rows as 64x128 tiles: one round 45 against 49 us, two rounds of
+// 2356 rows 90 against 81).
 template <int EPI, bool OUT_F32>
-int launch_epi(int variant, ProbSet& args, int n, hipStream_t st) {
-    switch (variant) {
-        case 4: return launch_cfg<256, 256, 2, 4, 2, EPI, OUT_F32>(args, n, st);
-        case 5: return launch_cfg<256, 192, 2, 4, 2, EPI, OUT_F32>(args, n, st);
-        case 1: return launch_cfg<128, 128, 2, 2, 4, EPI, OUT_F32>(args, n, st);
-        default: return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32>(args, n, st);
+int launch_shape(int shape, ProbSet& args, int n, int cus, hipStream_t st) {
+    long long tiles = 0;
+    for (int i = 0; i < n; i++) tiles += tiles_of(args.p[i], shape);
+    const bool one_round = tiles <= cus;
+    switch (shape) {
+        case TILE_64: return launch_ring<64, 64, 4, 1, 5, 2, EPI, OUT_F32>(args, n, st);
+        case TILE_128_64:
+            if (one_round) return launch_ring<128, 64, 8, 1, 6, 2, EPI, OUT_F32>(args, n, st);
+            return launch_ring<128, 64, 8, 1, 3, 4, EPI, OUT_F32>(args, n, st);
+        case TILE_64_128:
+            if (one_round) return launch_ring<64, 128, 4, 2, 6, 2, EPI, OUT_F32>(args, n, st);
+            return launch_ring<64, 128, 4, 2, 3, 4, EPI, OUT_F32>(args, n, st);
+        case TILE_128: return launch_ring<128, 128, 4, 2, 4, 2, EPI, OUT_F32>(args, n, st);
+        case TILE_256_128: return launch_ring<256, 128, 4, 2, 3, 2, EPI, OUT_F32>(args, n, st);
+        default: return launch_cfg<256, 256, 2, 4, 2, EPI, OUT_F32>(args, n, st);
     }
 }
 
@@ -558,7 +831,70 @@ int launch_epi(int variant, ProbSet& args, int n, hipStream_t st) {
 
 std::atomic<long long> g_gemm_bf16_launches{0};
 int g_gemm_bf16_row_split = 1;  // 0: never split a problem's rows over two launches (sd3_tune)
-int g_gemm_bf16_variant = -1;  // -1: choose by shape; 0 / 4: forced 128x128 / 256x256 tiles (sd3_gemm_bf16_force_tile); 1: 128x128 with a ring of four stages
+int g_gemm_bf16_tile = 0;       // 0: chosen from the sizes; else a forced tile shape (sd3_gemm_bf16_force_tile)
+
+// the shape behind a value of sd3_gemm_bf16_force_tile (-1: none): 128 or 256 for those squares, else rows * 1000 + columns
+static int forced_shape(int tile) {
+    if (tile == 128 || tile == 256) tile *= 1001;
+    for (int s = 0; s < TILE_SHAPES; s++)
+        if (tile == tile_shapes[s].tm * 1000 + tile_shapes[s].tn) return s;
+    return -1;
+}
+static bool ring_can(const Prob& q, int epi) {
+    auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    if (q.N % 4 || q.ldc % 4 || !al(q.out)) return false;
+    if (epi == EPI_GATE_RESID) return al(q.epi.gate) && al(q.epi.resid) && q.epi.gate_ld % 4 == 0;
+    if (epi == EPI_BIAS_ROWADD) return al(q.epi.table);
+    return true;
+}
+
+// fp8 operands: 256x256 (one workgroup per compute unit) or 128x128 tiles (two), by rounds: measured on full rounds, a round of 128x128
+// tiles takes 0.62 of one of 256x256 tiles, a launch of its own for problems with few rows about 0.38
+static int fp8_launches(ProbSet& args, int m, int out_is_f32, int epi, int cus, hipStream_t st) {
+    auto launch = [&](ProbSet& pp, int count, int v) -> int {
+#define SD3_GEMM_FP8_LAUNCH(E) return out_is_f32 ? launch_epi_fp8<E, true>(v, pp, count, st) : launch_epi_fp8<E, false>(v, pp, count, st)
+        switch (epi) {
+            case EPI_BIAS: SD3_GEMM_FP8_LAUNCH(EPI_BIAS);
+            case EPI_BIAS_GELU: SD3_GEMM_FP8_LAUNCH(EPI_BIAS_GELU);
+            case EPI_GATE_RESID: SD3_GEMM_FP8_LAUNCH(EPI_GATE_RESID);
+            case EPI_QKV_NORM: SD3_GEMM_FP8_LAUNCH(EPI_QKV_NORM);
+            default: return fail(SD3_ERR_UNSUPPORTED, "gemm_fp8: epilogue %d is not built for fp8 operands", epi);
+        }
+#undef SD3_GEMM_FP8_LAUNCH
+    };
+    if (g_gemm_bf16_tile) return launch(args, m, g_gemm_bf16_tile == 256 ? 4 : 0);
+    constexpr double ROUND128 = 0.62, SMALL_LAUNCH = 0.38;
+    auto tiles = [](const Prob& q, int t) { return ((q.M + t - 1) / t) * ((q.N + t - 1) / t); };
+    auto rounds = [](long long t, int slots) { return (double)((t + slots - 1) / slots); };
+    ProbSet big{}, small{};
+    int nb = 0, ns = 0;
+    long long big256 = 0, big128 = 0, small256 = 0, small128 = 0;
+    for (int i = 0; i < m; i++) {
+        if (args.p[i].M < 1024) {
+            small.p[ns++] = args.p[i];
+            small256 += tiles(args.p[i], 256);
+            small128 += tiles(args.p[i], 128);
+        } else {
+            big.p[nb++] = args.p[i];
+            big256 += tiles(args.p[i], 256);
+            big128 += tiles(args.p[i], 128);
+        }
+    }
+    if (nb == 0) return launch(args, m, 0);
+    const double together256 = rounds(big256 + small256, cus), together128 = ROUND128 * rounds(big128 + small128, 2 * cus);
+    double best = together256 <= together128 ? together256 : together128;
+    int plan = together256 <= together128 ? 0 : 1;  // 0/1: one launch with 256/128 tiles; 2/3: the small problems first, alone
+    if (ns > 0) {
+        const double apart256 = rounds(big256, cus) + SMALL_LAUNCH, apart128 = ROUND128 * rounds(big128, 2 * cus) + SMALL_LAUNCH;
+        if (apart256 < best) { best = apart256; plan = 2; }
+        if (apart128 < best) { best = apart128; plan = 3; }
+    }
+    if (plan >= 2) {
+        SD3_TRY(launch(small, ns, 0));
+        return launch(big, nb, plan == 2 ? 4 : 0);
+    }
+    return launch(args, m, plan == 0 ? 4 : 0);
+}
 
 static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, bool fp8, hipStream_t st) {
     if (n < 1 || n > MAX_PROBS) return fail(SD3_ERR_INVALID_ARG, "gemm_bf16_grouped: 1 to %d problems (got %d)", MAX_PROBS, n);
@@ -584,19 +920,11 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         if (q.M > max_M) max_M = q.M;
     }
     if (m == 0) return SD3_OK;
-    auto launch = [&](ProbSet& pp, int count, int v) -> int {
-        if (fp8) {
-#define SD3_GEMM_FP8_LAUNCH(E) return out_is_f32 ? launch_epi_fp8<E, true>(v, pp, count, st) : launch_epi_fp8<E, false>(v, pp, count, st)
-            switch (epi) {
-                case EPI_BIAS: SD3_GEMM_FP8_LAUNCH(EPI_BIAS);
-                case EPI_BIAS_GELU: SD3_GEMM_FP8_LAUNCH(EPI_BIAS_GELU);
-                case EPI_GATE_RESID: SD3_GEMM_FP8_LAUNCH(EPI_GATE_RESID);
-                case EPI_QKV_NORM: SD3_GEMM_FP8_LAUNCH(EPI_QKV_NORM);
-                default: return fail(SD3_ERR_UNSUPPORTED, "gemm_fp8: epilogue %d is not built for fp8 operands", epi);
-            }
-#undef SD3_GEMM_FP8_LAUNCH
-        }
-#define SD3_GEMM_BF16_LAUNCH(E) return out_is_f32 ? launch_epi<E, true>(v, pp, count, st) : launch_epi<E, false>(v, pp, count, st)
+    const int cus = compute_units();
+    if (cus <= 0) return SD3_ERR_HIP;
+    if (fp8) return fp8_launches(args, m, out_is_f32, epi, cus, st);
+    auto launch = [&](ProbSet& pp, int count, int shape) -> int {
+#define SD3_GEMM_BF16_LAUNCH(E) return out_is_f32 ? launch_shape<E, true>(shape, pp, count, cus, st) : launch_shape<E, false>(shape, pp, count, cus, st)
         switch (epi) {
             case EPI_BIAS: SD3_GEMM_BF16_LAUNCH(EPI_BIAS);
             case EPI_BIAS_GELU: SD3_GEMM_BF16_LAUNCH(EPI_BIAS_GELU);
@@ -608,77 +936,82 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         }
 #undef SD3_GEMM_BF16_LAUNCH
     };
-    if (g_gemm_bf16_variant >= 0) return launch(args, m, fp8 && g_gemm_bf16_variant != 4 ? 0 : g_gemm_bf16_variant);
-    // Tile shape and grouping by a small cost model. A persistent launch takes ceil(tiles / resident workgroups) rounds; the unit
-    // of cost is one round of 256x256 tiles (8 wavefronts, one workgroup per compute unit). Measured on full rounds, a round of
-    // 128x128 tiles (4 wavefronts, two workgroups per unit) takes 0.62 of that for a quarter of the outputs per tile, and a launch
-    // of its own for problems with few rows (a short round of small tiles, bound by per-tile overhead) about 0.38.
-    const int cus = compute_units();
-    if (cus <= 0) return SD3_ERR_HIP;
-    constexpr double ROUND128 = 0.62, SMALL_LAUNCH = 0.38;
-    auto tiles = [](const Prob& q, int t) { return ((q.M + t - 1) / t) * ((q.N + t - 1) / t); };
-    auto rounds = [](long long t, int slots) { return (double)((t + slots - 1) / slots); };
+    // the ring kernel stores four columns at a time; rows that are not made of such chunks take the 256x256 tiles
+    bool whole_chunks = true;
+    for (int i = 0; i < m; i++) whole_chunks = whole_chunks && ring_can(args.p[i], epi);
+    if (g_gemm_bf16_tile == 192) {
+        if (epi == EPI_QKV_NORM) return fail(SD3_ERR_UNSUPPORTED, "gemm_bf16: this tile shape cannot fuse the qk-norm");
+#define SD3_GEMM_BF16_192(E) \
+    case E: return out_is_f32 ? launch_cfg<256, 192, 2, 4, 2, E, true>(args, m, st) : launch_cfg<256, 192, 2, 4, 2, E, false>(args, m, st)
+        switch (epi) {
+            SD3_GEMM_BF16_192(EPI_BIAS);
+            SD3_GEMM_BF16_192(EPI_BIAS_GELU);
+            SD3_GEMM_BF16_192(EPI_BIAS_SILU);
+            SD3_GEMM_BF16_192(EPI_GATE_RESID);
+            SD3_GEMM_BF16_192(EPI_BIAS_ROWADD);
+            default: return fail(SD3_ERR_INVALID_ARG, "gemm_bf16: unknown epilogue %d", epi);
+        }
+#undef SD3_GEMM_BF16_192
+    }
+    if (!whole_chunks) return launch(args, m, TILE_256);
+    if (g_gemm_bf16_tile) return launch(args, m, forced_shape(g_gemm_bf16_tile));
+    // One launch with the cheapest shape, or two: the many-row problems apart from the few-row ones (a launch of its own costs LAUNCH), or
+    // full rounds of 256x256 tiles first and the last rows of the last many-row problem with the few-row problems behind them. The
+    // latter only for epilogues that do not look at the row index (a row split would shift the batch boundaries).
+    constexpr double LAUNCH = 5.0;
+    double best;
+    const int together = cheapest_shape(args, m, cus, best);
     ProbSet big{}, small{};
     int nb = 0, ns = 0;
-    long long big256 = 0, big128 = 0, small256 = 0, small128 = 0;
     for (int i = 0; i < m; i++) {
-        if (args.p[i].M < 1024) {
-            small.p[ns++] = args.p[i];
-            small256 += tiles(args.p[i], 256);
-            small128 += tiles(args.p[i], 128);
-        } else {
-            big.p[nb++] = args.p[i];
-            big256 += tiles(args.p[i], 256);
-            big128 += tiles(args.p[i], 128);
+        if (args.p[i].M < 1024) small.p[ns++] = args.p[i];
+        else big.p[nb++] = args.p[i];
+    }
+    int apart_big = -1, apart_small = -1;
+    if (nb > 0 && ns > 0) {
+        double cb, cs;
+        const int sb = cheapest_shape(big, nb, cus, cb), ss = cheapest_shape(small, ns, cus, cs);
+        if (cb + cs + LAUNCH < best) {
+            best = cb + cs + LAUNCH;
+            apart_big = sb;
+            apart_small = ss;
         }
     }
-    // only problems with few rows: small tiles; with no more tiles than compute units one workgroup per unit, so that LDS can hold
-    // a ring of four stages
-    const int v_small = small128 <= cus ? 1 : 0;
-    if (nb == 0) return launch(args, m, v_small);
-    const double together256 = rounds(big256 + small256, cus), together128 = ROUND128 * rounds(big128 + small128, 2 * cus);
-    double best = together256 <= together128 ? together256 : together128;
-    int plan = together256 <= together128 ? 0 : 1;  // 0/1: one launch with 256/128 tiles; 2/3: the small problems first, alone
-    if (ns > 0) {
-        const double apart256 = rounds(big256, cus) + SMALL_LAUNCH, apart128 = ROUND128 * rounds(big128, 2 * cus) + SMALL_LAUNCH;
-        if (apart256 < best) { best = apart256; plan = 2; }
-        if (apart128 < best) { best = apart128; plan = 3; }
-    }
-    // One more plan when the 256x256 tiles of the many-row problems fill R >= 1 rounds and leave a partial one: everything up to the
-    // last row tile of the last many-row problem that still fits R rounds as 256x256 tiles, the remaining rows of that problem
-    // together with the few-row problems as 128x128 tiles in a second launch (a round of those costs 0.62). Only for epilogues that do
-    // not look at the row index (a row split would shift the batch boundaries).
-    if (g_gemm_bf16_row_split && nb >= 1 && nb + ns <= MAX_PROBS && !fp8 &&
+    if (g_gemm_bf16_row_split && nb >= 1 && nb + ns <= MAX_PROBS &&
         (epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_BIAS_SILU || epi == EPI_QKV_NORM)) {
         const Prob& q = big.p[nb - 1];
-        long long before = 0;  // tiles of the many-row problems in front of the one that is split
-        for (int i = 0; i + 1 < nb; i++) before += tiles(big.p[i], 256);
+        long long before = 0, all = 0;  // 256x256 tiles of the many-row problems in front of the one that is split, and of all of them
+        for (int i = 0; i < nb; i++) {
+            if (i + 1 < nb) before += tiles_of(big.p[i], TILE_256);
+            all += tiles_of(big.p[i], TILE_256);
+        }
         const int tn = (q.N + 255) / 256, tm = (q.M + 255) / 256;
-        const long long R = big256 / cus, avail = R * cus - before;
-        const int m1 = (R > 0 && avail > 0) ? (int)(avail / tn) : 0;  // row tiles of q that fit the R full rounds
+        const long long avail = all / cus * cus - before;
+        const int m1 = avail > 0 ? (int)(avail / tn) : 0;  // row tiles of q that fit the full rounds
         if (m1 > 0 && m1 < tm) {
             Prob head = q, tail = q;
             head.M = m1 * 256;
             tail.M = q.M - head.M;
             tail.A = q.A + (long long)head.M * q.K;
             tail.out = (char*)q.out + (long long)head.M * q.ldc * (out_is_f32 ? 4 : 2);
-            const double split = rounds(before + tiles(head, 256), cus) + ROUND128 * rounds(tiles(tail, 128) + small128, 2 * cus);
-            if (split < best) {
-                ProbSet first{}, second{};
-                for (int i = 0; i + 1 < nb; i++) first.p[i] = big.p[i];
-                first.p[nb - 1] = head;
-                second.p[0] = tail;
-                for (int i = 0; i < ns; i++) second.p[1 + i] = small.p[i];
-                SD3_TRY(launch(first, nb, 4));
-                return launch(second, 1 + ns, 0);
+            ProbSet first{}, second{};
+            for (int i = 0; i + 1 < nb; i++) first.p[i] = big.p[i];
+            first.p[nb - 1] = head;
+            second.p[0] = tail;
+            for (int i = 0; i < ns; i++) second.p[1 + i] = small.p[i];
+            double c2;
+            const int s2 = cheapest_shape(second, 1 + ns, cus, c2);
+            if (launch_cost(first, nb, TILE_256, cus) + c2 + LAUNCH < best) {
+                SD3_TRY(launch(first, nb, TILE_256));
+                return launch(second, 1 + ns, s2);
             }
         }
     }
-    if (plan >= 2) {
-        SD3_TRY(launch(small, ns, v_small));
-        return launch(big, nb, plan == 2 ? 4 : 0);
+    if (apart_big >= 0) {
+        SD3_TRY(launch(small, ns, apart_small));
+        return launch(big, nb, apart_big);
     }
-    return launch(args, m, plan == 0 ? 4 : 0);
+    return launch(args, m, together);
 }
 
 int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st) { return grouped_impl(probs, n, out_is_f32, epi, false, st); }
@@ -693,8 +1026,8 @@ int gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* out, int out_is_f32, int 
 }  // namespace sd3
 
 extern "C" int sd3_gemm_bf16_force_tile(int tile) {
-    if (tile != 0 && tile != 128 && tile != 192 && tile != 256)
-        return sd3::fail(SD3_ERR_INVALID_ARG, "sd3_gemm_bf16_force_tile: tile must be 0, 128, 192 or 256 (got %d)", tile);
-    sd3::g_gemm_bf16_variant = tile == 0 ? -1 : (tile == 256 ? 4 : tile == 192 ? 5 : 0);
+    if (tile != 0 && tile != 192 && sd3::forced_shape(tile) < 0)
+        return sd3::fail(SD3_ERR_INVALID_ARG, "sd3_gemm_bf16_force_tile: tile must be 0, 128, 192, 256, 64064, 64128, 128064 or 256128 (got %d)", tile);
+    sd3::g_gemm_bf16_tile = tile;
     return SD3_OK;
 }
