@@ -44,9 +44,6 @@ constexpr int smem_bytes(bool norm) {
     return ((prefetch_tiles(norm) + 2) * STAGE_BYTES > NW * QW * O_PITCH * 2) ? (prefetch_tiles(norm) + 2) * STAGE_BYTES : NW * QW * O_PITCH * 2;
 }
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef const __attribute__((address_space(1))) void* glb_ptr_t;
-
 struct SegDev {
     const bf16_t* q[2];
     const bf16_t* k[2];
@@ -740,6 +737,251 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     }
 }
 
+// ---- short sequences ----
+// Used up to SHORT_KEYS keys, whatever the batch (a batch element's result stays what it is alone): 24 heads, 333 tokens, batch 1 / 2 / 4 / 8:
+// 13.9 / 14.3 / 14.8 / 20.8 -> 8.1 / 11.2 / 17.0 / 26.4 us (every workgroup reads all keys for 32 queries, so many of them are bound by
+// the loads); 730 tokens, batch 1 / 4: 19.3 / 30.5 -> 16.4 / 41 us.
+// The kernel above gives a workgroup 256 queries and runs through all keys tile by tile behind a barrier each: at 333 tokens that is 48
+// workgroups with a serial chain of six tiles, at 1178 tokens 240 with nineteen. Here a workgroup has 32 queries and its KS wavefronts
+// split the KEYS (tile t of 32 keys goes to wavefront t % KS), each with its own K rows in registers (straight from memory: a K row chunk
+// of 8 values is the matrix operand as it lies) and its own V tile in LDS, so that there is no barrier before the merge at the end.
+// v_mfma_f32_16x16x32_bf16 throughout. S^T = K Q^T leaves lane l with query l%16 and keys 4g + r of a 16-key block, g = l/16: the two
+// blocks of a tile are, packed, the P^T operand with k slots {4g .. 4g+3, 16+4g .. 16+4g+3}; the transposing LDS reads fetch V^T in the
+// same slots. Softmax as above: a reference that is subtracted on the matrix unit and moved only when a row sum says so.
+constexpr int SHORT_KEYS = 416;
+template <int QB, int KS>
+__global__ void __launch_bounds__(KS * 64, 2) flash_attn_bf16_split_kernel(const AttnSets sets, float q_scale) {
+    constexpr int TKEYS = 32, V_TILE = TKEYS * 128;
+    constexpr int PITCH = 16 * QB + 2 * QB;  // floats per lane in the merge buffer
+    constexpr int V_SPACE = KS * 2 * V_TILE, MERGE = (KS / 2) * 64 * PITCH * 4;
+    __shared__ __attribute__((aligned(1024))) char smem[V_SPACE > MERGE ? V_SPACE : MERGE];
+    const int which = (blockIdx.x >= (unsigned)sets.end[0]) + (blockIdx.x >= (unsigned)sets.end[1]);
+    const SegDev& s = sets.set[which];
+    const int wg_first = which ? sets.end[which - 1] : 0;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int b, h, q0;
+    {
+        const int total = sets.end[which] - wg_first, wg = blockIdx.x - wg_first, xcd = wg % 8, local = wg / 8;
+        const int per = (total + 7) / 8, tall = (total % 8) ? (total % 8) : 8;
+        const int item = (xcd < tall) ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+        const int bh = item / s.nqb;
+        q0 = (item % s.nqb) * (16 * QB);
+        b = bh / s.NH;
+        h = bh % s.NH;
+    }
+    const int T0 = s.T[0], T1 = s.T[1], Tq0 = s.Tq[0], TQ = s.Tq[0] + s.Tq[1];
+    Frag q[QB][2];
+#pragma unroll
+    for (int i = 0; i < QB; i++) {
+        const int qt = min(q0 + 16 * i + lr, TQ - 1), seg = qt < Tq0 ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
+        const bf16_t* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_qkv[seg] + h * HS + 8 * lg;
+#pragma unroll
+        for (int st = 0; st < 2; st++) q[i][st].u = *reinterpret_cast<const uint4*>(p + 32 * st);
+    }
+    f32x4_t o[4][QB];
+    float m_run[QB], l_run[QB];  // l_run: over the keys of this lane
+#pragma unroll
+    for (int i = 0; i < QB; i++) {
+        m_run[i] = 0.f;
+        l_run[i] = 0.f;
+#pragma unroll
+        for (int d = 0; d < 4; d++) o[d][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    constexpr float L_BOUND = 1073741824.0f;  // 2^30
+
+    // key tiles are counted segment by segment, so that a tile's rows have one scalar base and 32-bit offsets
+    const int nt0 = (T0 + TKEYS - 1) / TKEYS, n_t = nt0 + (T1 + TKEYS - 1) / TKEYS;
+    const int ld0 = s.ld_qkv[0], ld1 = s.ld_qkv[1];
+    const bf16_t* k0 = s.k[0] + (long long)b * T0 * ld0 + h * HS;
+    const bf16_t* k1 = s.k[1] + (long long)b * T1 * ld1 + h * HS;
+    const bf16_t* v0 = s.v[0] + (long long)b * T0 * ld0 + h * HS;
+    const bf16_t* v1 = s.v[1] + (long long)b * T1 * ld1 + h * HS;
+    char* const v_lds = smem + wave * 2 * V_TILE;
+    Frag k[2][2];  // [16-key block][32-wide step of d]
+    unsigned k_at[2], v_at[4];  // offsets of this lane's rows in a tile: they change with the segment and in a segment's last tile
+    int at_seg = -1, at_last = -1;
+    // V first, then K: loads return in order, so whoever has waited for a tile's K rows finds its V tile in LDS
+    auto load_tile = [&](int t, int stage) {
+        const int seg = t < nt0 ? 0 : 1, t0 = (seg ? t - nt0 : t) * TKEYS, last = min((seg ? T1 : T0) - t0, TKEYS) - 1, ld = seg ? ld1 : ld0;
+        if (seg != at_seg || last != at_last) {
+            at_seg = seg;
+            at_last = last;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {  // rows 8i .. 8i+7; chunk pairs of rows of one parity land in different bank groups
+                const int row = 8 * i + (lane >> 3), chunk = (lane & 7) ^ (2 * ((row >> 1) & 3));
+                v_at[i] = __umul24(min(row, last), ld) + chunk * 8;
+            }
+#pragma unroll
+            for (int kb16 = 0; kb16 < 2; kb16++) k_at[kb16] = __umul24(min(16 * kb16 + lr, last), ld) + 8 * lg;
+        }
+        const bf16_t* vb = (seg ? v1 : v0) + (long long)t0 * ld;
+        const bf16_t* kb = (seg ? k1 : k0) + (long long)t0 * ld;
+#pragma unroll
+        for (int i = 0; i < 4; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(vb + v_at[i]), (lds_ptr_t)(v_lds + stage * V_TILE + i * 1024), 16, 0, 0);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+            for (int st = 0; st < 2; st++) k[kb16][st].u = *reinterpret_cast<const uint4*>(kb + k_at[kb16] + 32 * st);
+        return last + 1;
+    };
+    const uint32_t v_addr = (uint32_t)(uintptr_t)(lds_ptr_t)v_lds;
+    uint32_t v_off[2];  // transposing reads: key half hb, d block 0 (d block db: the chunk pair 2 db, xor-ed in)
+    int v_key[2];
+#pragma unroll
+    for (int hb = 0; hb < 2; hb++) {
+        const int row = 16 * hb + 4 * lg + (lr >> 2);
+        v_key[hb] = 2 * ((row >> 1) & 3);
+        v_off[hb] = row * 128 + 8 * (lr & 1);
+    }
+    const int v_chunk = (lr & 3) >> 1;
+
+    int t = wave, left = 0;
+    bool first = true;
+    if (t < n_t) left = load_tile(t, 0);
+    __builtin_amdgcn_sched_barrier(0);  // (the first tile is on its way before the wait for the queries)
+#pragma unroll
+    for (int i = 0; i < QB; i++)
+#pragma unroll
+        for (int st = 0; st < 2; st++) {
+            float f[8];
+            unpack8(q[i][st].u, f);
+#pragma unroll
+            for (int e = 0; e < 8; e++) f[e] *= q_scale;
+            q[i][st].u = pack8(f);
+        }
+    for (int stage = 0; t < n_t; t += KS, stage ^= 1) {
+        // scores relative to the reference m_run (the accumulators start from its negative)
+        f32x4_t sc[2][QB];
+#pragma unroll
+        for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+            for (int i = 0; i < QB; i++)
+                sc[kb16][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kb16][0].v, q[i][0].v, f32x4_t{-m_run[i], -m_run[i], -m_run[i], -m_run[i]}, 0, 0, 0);
+#pragma unroll
+        for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+            for (int i = 0; i < QB; i++) sc[kb16][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kb16][1].v, q[i][1].v, sc[kb16][i], 0, 0, 0);
+        // V^T of this tile (its loads came before the K rows just used), then the requests for the next tile
+        __builtin_amdgcn_sched_barrier(0);
+        uint2 vf[4][2];
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+#pragma unroll
+            for (int hb = 0; hb < 2; hb++)
+                vf[d][hb] = lds_read_tr16_b64(v_addr + stage * V_TILE + v_off[hb] + (((2 * d + v_chunk) ^ v_key[hb]) * 16), 0);
+        const int cur = left;
+        if (t + KS < n_t) left = load_tile(t + KS, stage ^ 1);
+        if (cur < TKEYS) {
+#pragma unroll
+            for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (16 * kb16 + 4 * lg + r >= cur)
+#pragma unroll
+                        for (int i = 0; i < QB; i++) sc[kb16][i][r] = -1e30f;
+        }
+        Frag p[QB];
+        float inc[QB];
+        bool move = first;
+        auto probs = [&](int i) {
+            float f[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) f[e] = __builtin_amdgcn_exp2f(sc[e >> 2][i][e & 3]);
+            inc[i] = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+            p[i].u = pack8(f);
+        };
+#pragma unroll
+        for (int i = 0; i < QB; i++) {
+            probs(i);
+            move = move || !(inc[i] <= L_BOUND);
+        }
+        // The reference goes to the running maximum with the first tile and whenever a lane's sum over a tile exceeds L_BOUND
+        if (__any(move)) {
+#pragma unroll
+            for (int i = 0; i < QB; i++) {
+                float mx = fmaxf(fmaxf(fmaxf(sc[0][i][0], sc[0][i][1]), fmaxf(sc[0][i][2], sc[0][i][3])),
+                                 fmaxf(fmaxf(sc[1][i][0], sc[1][i][1]), fmaxf(sc[1][i][2], sc[1][i][3])));
+                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+                if (!first) mx = fmaxf(mx, 0.f);
+                const float alpha = first ? 0.f : __builtin_amdgcn_exp2f(-mx);
+                m_run[i] += mx;
+                l_run[i] *= alpha;
+#pragma unroll
+                for (int d = 0; d < 4; d++) o[d][i] *= alpha;
+#pragma unroll
+                for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) sc[kb16][i][r] -= mx;
+                probs(i);
+            }
+            first = false;
+        }
+#pragma unroll
+        for (int i = 0; i < QB; i++) l_run[i] += inc[i];
+        asm volatile("s_waitcnt lgkmcnt(0)"
+                     : "+v"(vf[0][0]), "+v"(vf[0][1]), "+v"(vf[1][0]), "+v"(vf[1][1]), "+v"(vf[2][0]), "+v"(vf[2][1]), "+v"(vf[3][0]), "+v"(vf[3][1]));
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            Frag vv;
+            vv.u = make_uint4(vf[d][0].x, vf[d][0].y, vf[d][1].x, vf[d][1].y);
+#pragma unroll
+            for (int i = 0; i < QB; i++) o[d][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv.v, p[i].v, o[d][i], 0, 0, 0);
+        }
+    }
+
+    if (first)  // no tile came to this wavefront: weight zero in the merge
+#pragma unroll
+        for (int i = 0; i < QB; i++) m_run[i] = -1e30f;
+    // merge in a fixed tree: in each step the upper half of the wavefronts hands its state to the lower half (V tiles are free by then)
+    float* const merge = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int half = KS / 2; half >= 1; half /= 2) {
+        float* mine = merge + (wave < half ? wave : wave - half) * 64 * PITCH + lane;  // value v of a lane at 64 v: no bank conflicts
+        __syncthreads();
+        if (wave >= half && wave < 2 * half) {
+#pragma unroll
+            for (int i = 0; i < QB; i++) {
+                mine[64 * (2 * i)] = m_run[i];
+                mine[64 * (2 * i + 1)] = l_run[i];
+#pragma unroll
+                for (int d = 0; d < 4; d++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) mine[64 * (2 * QB + (i * 4 + d) * 4 + r)] = o[d][i][r];
+            }
+        }
+        __syncthreads();
+        if (wave < half) {
+#pragma unroll
+            for (int i = 0; i < QB; i++) {
+                const float om = mine[64 * (2 * i)], mx = fmaxf(m_run[i], om);
+                const float wa = __builtin_amdgcn_exp2f(m_run[i] - mx), wb = __builtin_amdgcn_exp2f(om - mx);
+                m_run[i] = mx;
+                l_run[i] = l_run[i] * wa + mine[64 * (2 * i + 1)] * wb;
+#pragma unroll
+                for (int d = 0; d < 4; d++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) o[d][i][r] = o[d][i][r] * wa + mine[64 * (2 * QB + (i * 4 + d) * 4 + r)] * wb;
+            }
+        }
+    }
+    if (wave) return;
+#pragma unroll
+    for (int i = 0; i < QB; i++) {
+        const int qt = q0 + 16 * i + lr, seg = qt < Tq0 ? 0 : 1;
+        float l = l_run[i] + __shfl_xor(l_run[i], 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        if (qt >= TQ || !s.out[seg]) continue;
+        const float inv = 1.0f / l;
+        bf16_t* op = s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_out[seg] + h * HS + 4 * lg;
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+            *reinterpret_cast<uint2*>(op + 16 * d) = make_uint2(pack_bf16x2(o[d][i][0] * inv, o[d][i][1] * inv), pack_bf16x2(o[d][i][2] * inv, o[d][i][3] * inv));
+    }
+}
+
 // Merges the kv_splits partial results of every query of a split set, in split order: with M = max_s m_s,
 // out = sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M). 16 lanes per query row, 4 of the 64 output values each.
 __global__ void __launch_bounds__(256) attn_combine_kernel(const SegDev s, int B) {
@@ -824,11 +1066,12 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     if (B <= 0 || NH <= 0) return SD3_OK;
     AttnSets sets{};
     bool norm = false;
-    int m = 0, total = 0;
+    int m = 0, total = 0, longest = 0;
     for (int i = 0; i < n; i++) {
         const AttnSegments& a = jobs[i];
         const int T = a.T[0] + a.T[1], TQ = a.Tq[0] + a.Tq[1];
         if (TQ <= 0) continue;
+        longest = T > longest ? T : longest;
         if (T <= 0) return fail(SD3_ERR_INVALID_ARG, "attention: no keys");
         SegDev& s = sets.set[m];
         SD3_TRY(fill_set(a, NH, s, norm));
@@ -847,6 +1090,19 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     if (m == 0) return SD3_OK;
     for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
     const float q_scale = 1.4426950408889634f / sqrtf((float)HS);
+    if (!norm && longest <= SHORT_KEYS) {
+        constexpr int QB = 2, KS = 4;
+        total = 0;
+        for (int i = 0; i < m; i++) {  // (a split along the keys happens inside the workgroups: kv_splits does not apply)
+            SegDev& s = sets.set[i];
+            s.nqb = (s.Tq[0] + s.Tq[1] + 16 * QB - 1) / (16 * QB);
+            total += s.nqb * NH * B;
+            sets.end[i] = total;
+        }
+        for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
+        hipLaunchKernelGGL((flash_attn_bf16_split_kernel<QB, KS>), dim3((unsigned)total), dim3(KS * 64), 0, st, sets, q_scale);
+        return launch_status("flash_attention_bf16");
+    }
     dim3 grid((unsigned)total), block(NW * 64);
     if (norm) hipLaunchKernelGGL(flash_attn_bf16_kernel<true>, grid, block, 0, st, sets, q_scale, 1e-6f);
     else hipLaunchKernelGGL(flash_attn_bf16_kernel<false>, grid, block, 0, st, sets, q_scale, 1e-6f);
