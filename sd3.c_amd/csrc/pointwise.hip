@@ -43,7 +43,10 @@ template <typename OutT>
 struct LnSegPair {
     LnSegDev<OutT> s[2];  // rows [0, s[0].rows) belong to the first tensor, the rest to the second (the two streams of a block)
 };
-template <typename OutT, int NV>
+// EARLY: the modulation vectors are requested together with the row instead of behind the statistics. That is another 24 registers per
+// vector at C = 1536, which costs occupancy where many rows are in flight and one memory latency less where a launch is nothing but
+// latency (336 rows in the block: 6.9 -> 6.6 us).
+template <typename OutT, int NV, bool EARLY>
 __global__ void __launch_bounds__(256) ln_mod_vec_kernel(const LnSegPair<OutT> segs, float eps, int C) {
     const int lane = threadIdx.x & (WAVE - 1);
     // (the wavefront's index as a scalar: the row, the segment it belongs to and every pointer derived from them then live in scalar
@@ -59,24 +62,11 @@ __global__ void __launch_bounds__(256) ln_mod_vec_kernel(const LnSegPair<OutT> s
     const int nvec = C >> 2;
     const float4* xr = reinterpret_cast<const float4*>(g.x + row * C);
     float4 v[NV];
-    float s = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         int j = lane + i * WAVE;
         v[i] = (j < nvec) ? xr[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-        s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
     }
-    const float mu = wave_sum(s) / C;
-    float q = 0.f;
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-        int j = lane + i * WAVE;
-        if (j < nvec) {
-            float a = v[i].x - mu, b = v[i].y - mu, c = v[i].z - mu, d = v[i].w - mu;
-            q += (a * a + b * b) + (c * c + d * d);
-        }
-    }
-    const float rstd = 1.0f / sqrtf(wave_sum(q) / C + eps);
     long long b = 0;  // batch element of the row: with at most 8 of them a few comparisons instead of a 64-bit division
     if (g.rows <= 8LL * T) {
 #pragma unroll
@@ -88,19 +78,48 @@ __global__ void __launch_bounds__(256) ln_mod_vec_kernel(const LnSegPair<OutT> s
     const float4* sc = g.scale ? reinterpret_cast<const float4*>(g.scale + b * mod_ld) : nullptr;
     const float4* sh2 = g.shift2 ? reinterpret_cast<const float4*>(g.shift2 + b * mod_ld) : nullptr;
     const float4* sc2 = g.scale2 ? reinterpret_cast<const float4*>(g.scale2 + b * mod_ld) : nullptr;
+    float4 msc[EARLY ? NV : 1], msh[EARLY ? NV : 1], msc2[EARLY ? NV : 1], msh2[EARLY ? NV : 1];
+    if (EARLY) {
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int j = min(lane + i * WAVE, nvec - 1);
+            if (sc) {
+                msc[i] = sc[j];
+                msh[i] = sh[j];
+            }
+            if (out2) {
+                msc2[i] = sc2[j];
+                msh2[i] = sh2[j];
+            }
+        }
+    }
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+    const float mu = wave_sum(s) / C;
+    float q = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        int j = lane + i * WAVE;
+        if (j < nvec) {
+            float a = v[i].x - mu, b = v[i].y - mu, c = v[i].z - mu, d = v[i].w - mu;
+            q += (a * a + b * b) + (c * c + d * d);
+        }
+    }
+    const float rstd = 1.0f / sqrtf(wave_sum(q) / C + eps);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         int j = lane + i * WAVE;
         if (j < nvec) {
             float n0 = rstd * (v[i].x - mu), n1 = rstd * (v[i].y - mu), n2 = rstd * (v[i].z - mu), n3 = rstd * (v[i].w - mu);
             if (sc) {
-                float4 a = sc[j], c = sh[j];
+                const float4 a = EARLY ? msc[i] : sc[j], c = EARLY ? msh[i] : sh[j];
                 store4<OutT>(out + row * C + 4 * j, n0 * (1.0f + a.x) + c.x, n1 * (1.0f + a.y) + c.y, n2 * (1.0f + a.z) + c.z, n3 * (1.0f + a.w) + c.w);
             } else {
                 store4<OutT>(out + row * C + 4 * j, n0, n1, n2, n3);
             }
             if (out2) {
-                float4 a = sc2[j], c = sh2[j];
+                const float4 a = EARLY ? msc2[i] : sc2[j], c = EARLY ? msh2[i] : sh2[j];
                 store4<OutT>(out2 + row * C + 4 * j, n0 * (1.0f + a.x) + c.x, n1 * (1.0f + a.y) + c.y, n2 * (1.0f + a.z) + c.z, n3 * (1.0f + a.w) + c.w);
             }
         }
@@ -156,9 +175,12 @@ static int ln_mod_launch_vec(const LnSegPair<OutT>& segs, float eps, int C, hipS
     const long long rows = segs.s[0].rows + segs.s[1].rows;
     dim3 grid((unsigned)((rows + wpb - 1) / wpb)), block(wpb * WAVE);
     const int nv = (C / 4 + WAVE - 1) / WAVE;
-#define SD3_LN_CASE(N)                                                                       \
-    case N:                                                                                  \
-        hipLaunchKernelGGL((ln_mod_vec_kernel<OutT, N>), grid, block, 0, st, segs, eps, C); \
+    // (2048 rows: two wavefronts per SIMD)
+    const bool early = rows <= 2048;
+#define SD3_LN_CASE(N)                                                                                        \
+    case N:                                                                                                   \
+        if (early) hipLaunchKernelGGL((ln_mod_vec_kernel<OutT, N, true>), grid, block, 0, st, segs, eps, C);  \
+        else hipLaunchKernelGGL((ln_mod_vec_kernel<OutT, N, false>), grid, block, 0, st, segs, eps, C);       \
         break;
     switch (nv) { SD3_LN_CASE(1) SD3_LN_CASE(2) SD3_LN_CASE(3) SD3_LN_CASE(4) SD3_LN_CASE(5) SD3_LN_CASE(6) SD3_LN_CASE(7) SD3_LN_CASE(8)
                   SD3_LN_CASE(9) SD3_LN_CASE(10) SD3_LN_CASE(11) SD3_LN_CASE(12) }
