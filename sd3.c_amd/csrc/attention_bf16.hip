@@ -1040,15 +1040,33 @@ int fill_set(const AttnSegments& a, int NH, SegDev& s, bool& norm) {
 
 }  // namespace
 
-// Key splits for the context queries of a joint attention, or 0 when the one-set launch is the better choice. The joint sequence
-// of the headline shape has 17 query blocks of 256 per (batch, head), the last one holding the 154 leftover rows: 816 workgroups,
-// which run as long as 1024 would (two per compute unit: 512 at a time). With the latent queries alone the count is 768, whose
-// last 256 have a compute unit to themselves and finish early; the context queries then go, split four ways along the keys into
-// short work items, into the slots those leave free, and a small kernel merges their partial results.
+// Key splits for the context queries of a joint attention, or 0 when the one-set launch is the better choice. The few context queries
+// make one more query block per (batch, head): 17 instead of 16 at 4096 + 154 tokens, 792 workgroups instead of 768 with the extra
+// self-attention of a dual block beside it. Whether that costs anything depends on the compute units' rounds. A unit works on two workgroups
+// at a time, a pair taking 1.65 times as long as one alone, so 768 = 3 per unit take 2.65 and 792 = some units with 4 take 3.3 times a
+// workgroup's time. Where the context queries would start such a round they go, split four ways along the keys into short
+// work items, into the slots the last round leaves free, and a small kernel (5 us) merges their partial results. Forwards with and without:
+// 4096 + 154 tokens, batch 1 / 2 / 4 / 8: 12.7 / 22.4 / 43.9 / 86.0 and 13.0 / 23.1 / 44.1 / 85.7 ms; 16384 + 154: 79.0 and 82.5 ms;
+// everything else tried between 1024 and 9216 latent tokens is 0.3 to 3.4 % faster without (1024 + 154, batch 1: 4.89 and 4.75 ms).
+// The choice looks at batches of one and two (a guidance pair) whatever the batch is: results of the context rows differ in the last
+// bf16 bit with the split, and a batch element's result stays what it is alone.
 int g_attention_context_splits = -1;  // -1: chosen from the sizes; 0: never split; n >= 2: n splits wherever splitting applies (sd3_tune)
-int attention_bf16_context_splits(int Tc, int Tx) {
+int attention_bf16_context_splits(int Tc, int Tx, int NH, bool dual) {
     const int nt_all = (Tc + Tx + BKV - 1) / BKV;
     if (Tc <= 0 || Tc > BQ || Tx < 4 * BQ || nt_all < 16 || g_attention_context_splits == 0) return 0;
+    if (g_attention_context_splits < 0) {
+        const int cus = compute_units();
+        const double tile_us = 1.0, merge_us = 5.0;
+        auto rounds = [&](long long items) {
+            const long long k = (items + cus - 1) / cus;
+            return (double)(k / 2) * 1.65 + (double)(k % 2);
+        };
+        const long long latent = (Tx + BQ - 1) / BQ, joint = (Tc + Tx + BQ - 1) / BQ;
+        double gain = 0;
+        for (int b = 1; b <= 2; b++)
+            gain += (rounds((joint + (dual ? latent : 0)) * NH * b) - rounds((dual ? 2 : 1) * latent * NH * b)) * nt_all * tile_us - merge_us;
+        if (cus <= 0 || gain <= 0) return 0;
+    }
     int S = g_attention_context_splits > 0 ? g_attention_context_splits : 4;
     S = S < 2 ? 2 : (S > 8 ? 8 : S);
     // every split must own at least one key tile: with ceil(nt_all / S) tiles each, the last one starts at (S-1) * that

@@ -285,7 +285,7 @@ int attention_bf16(const AttnSegments& s, int B, int NH, int HS, hipStream_t st)
 // second, small kernel. attention_bf16_context_splits: the number of splits that pays for the Tc context queries of a joint
 // attention next to Tx latent ones, or 0 when the plain one-set launch is the better choice.
 int attention_bf16_multi(const AttnSegments* sets, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int HS, hipStream_t st);
-int attention_bf16_context_splits(int Tc, int Tx);
+int attention_bf16_context_splits(int Tc, int Tx, int NH, bool dual);
 size_t attention_bf16_split_workspace_floats(int B, int NH, int Tc, int splits);
 
 }  // namespace sd3

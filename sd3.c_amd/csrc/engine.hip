@@ -1,6 +1,7 @@
 // Host side of the library: context (bound weights, bf16 copies, workspace), the block schedule
 // (dit_block, modules.cpp:1340-1505) and the full forward (DiT_forward, modules.cpp:1605-1780) expressed as
 // launches of the fused kernels. No arithmetic happens on the host.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -279,7 +280,8 @@ size_t block_workspace_bytes(const Dims& d, int prec) {
     act(mc * d.C); act(mx * d.C);                          // c_att, x_att
     if (is_bf(prec)) {
         if (d.dual) act(mx * d.C);                         // x_att2: both attentions of a dual block run in one launch
-        const int S = attention_bf16_context_splits(d.Tc, d.Tx);
+        // (a forward's blocks share one layout: room for the split of either kind of block)
+        const int S = std::max(attention_bf16_context_splits(d.Tc, d.Tx, d.NH, false), attention_bf16_context_splits(d.Tc, d.Tx, d.NH, true));
         if (S) b.take<float>(attention_bf16_split_workspace_floats(d.B, d.NH, d.Tc, S));
     }
     act(mc * d.E * d.C); act(mx * d.E * d.C);              // c_mlp, x_mlp
@@ -417,7 +419,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     void* x_att = act((size_t)mx * C);
     void* x_att2 = x_att;  // output of the extra self-attention (bf16 path: a buffer of its own, the two attentions share a launch)
     float* split_ws = nullptr;
-    const int ctx_splits = is_bf(prec) ? attention_bf16_context_splits(Tc, Tx) : 0;
+    const int ctx_splits = is_bf(prec) ? attention_bf16_context_splits(Tc, Tx, d.NH, d.dual) : 0;
     if (is_bf(prec)) {
         if (d.dual) x_att2 = act((size_t)mx * C);
         if (ctx_splits) split_ws = ws.take<float>(attention_bf16_split_workspace_floats(B, d.NH, Tc, ctx_splits));
@@ -504,13 +506,11 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         int n = 0;
         double flop = 0;
         const double Tj = (double)Tc + Tx;
-        if (ctx_splits) {
-            sets[n] = joint;
-            sets[n].Tq[0] = 0; sets[n].out[0] = nullptr;
-            n++;
-        } else {
-            sets[n++] = joint;
+        sets[n] = joint;
+        if (ctx_splits || d.discard) {
+            sets[n].Tq[0] = 0; sets[n].out[0] = nullptr;  // (a discard_context block needs no context queries)
         }
+        n++;
         flop += 4.0 * B * d.NH * (d.discard ? (double)Tx : Tj) * Tj * d.HS;  // (a discard_context block computes no context queries)
         if (d.dual) {
             sets[n++] = dual_set;
