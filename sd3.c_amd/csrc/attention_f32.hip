@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(SegDev s, int HS, float s
 // and split the KEYS (tile t goes to wavefront t % KS); K and V rows come straight from memory (L2: all workgroups of a head run on one
 // XCD) into registers, half a tile of matrix work ahead of their use; the KS partial results are merged in a fixed tree at the end.
 // This gives every SIMD work also where there are few queries: 1178 tokens and 2 heads are 20 workgroups of 128 queries with the keys in
-// one run (290 us), 1184 wavefronts this way (35 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 157 us, 70 -> 109 TFLOP/s of 155.
+// one run (290 us), 592 wavefronts this way (32 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 157 us, 70 -> 109 TFLOP/s of 155.
 //
 // Contraction order: K and Q are read as float4 along d, so step s of 16-wide chunk c contracts d = 16c + 4g + s over the lane groups
 // g = l/16. S^T registers r of a 16x16 block are keys 4g + r of query l%16: as they are, the operand of step r of O^T += V^T P^T, whose
@@ -437,11 +437,13 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     const float scale = (float)(1.0 / sqrtf((float)HS));
     const float scale2 = (float)(1.4426950408889634 / sqrt((double)HS));  // scores in powers of two: the exponentials are one instruction
     if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 24) && a.ld_qkv[1] < (1 << 24)) {
-        // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16 and twice as many key runs.
-        // (Not by the batch: a batch element's result stays what it is alone.)
+        // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. (Not by the batch: a batch
+        // element's result stays what it is alone.) Four key runs in both: eight, or the keys over several workgroups and a second
+        // kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four
+        // runs 32).
         const bool few = (long long)NH * ((TQ + 31) / 32) < 192;
-        if (HS == 64) return few ? launch_split<64, 1, 2, 8>(s, B, NH, scale2, st) : launch_split<64, 2, 1, 4>(s, B, NH, scale2, st);
-        return few ? launch_split<128, 1, 1, 8>(s, B, NH, scale2, st) : launch_split<128, 2, 1, 4>(s, B, NH, scale2, st);
+        if (HS == 64) return few ? launch_split<64, 1, 2, 4>(s, B, NH, scale2, st) : launch_split<64, 2, 1, 4>(s, B, NH, scale2, st);
+        return few ? launch_split<128, 1, 1, 4>(s, B, NH, scale2, st) : launch_split<128, 2, 1, 4>(s, B, NH, scale2, st);
     }
     dim3 grid((TQ + BQ - 1) / BQ, NH, B), block(256);
     const int hsp = HS <= 32 ? 32 : (HS <= 64 ? 64 : 128);
