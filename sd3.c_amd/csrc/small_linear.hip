@@ -28,18 +28,21 @@ struct WLoad<bf16_t> {
     static __device__ __forceinline__ float load1(const bf16_t* p) { return bf16_to_f32(*p); }
 };
 
-// Block = 256 threads = 32 column groups (4 columns each, 128 columns per block) x 8 slices of K.
+// Block = 256 threads = CG column groups (4 columns each) x 256 / CG slices of K. A launch is bound by the weights it streams once enough
+// rows of them are requested at a time: 128 columns and 8 slices (CG = 32) per workgroup do where thousands of workgroups are resident.
+// With fewer workgroups a thread's run of K is a chain of memory latencies, so the columns are cut finer and K into more slices.
 // x is staged transposed in LDS (xs[k][m]) so that a thread reads its M inputs for one k with wide LDS loads.
 // Jobs travel as a kernel argument (no device-side table to keep coherent with the host).
 struct SmallLinearJobPack {
     SmallLinearJob j[SMALL_LINEAR_JOBS_PER_LAUNCH];  // 52 x 56 bytes of kernel arguments: the 49 projections of a 24-block forward in one launch
 };
 
-template <int M, typename WT, bool VEC>
+template <int M, typename WT, bool VEC, int CG>
 __global__ void __launch_bounds__(256) small_linear_kernel(const float* __restrict__ x_all, int m_real, int K_all, const SmallLinearJobPack jobs, int act) {
     extern __shared__ float smem[];
     const SmallLinearJob job = jobs.j[blockIdx.y];
-    const int col_base = blockIdx.x * 128;
+    constexpr int COLS = CG * 4, SLICES = 256 / CG;
+    const int col_base = blockIdx.x * COLS;
     if (col_base >= job.N) return;
     const float* __restrict__ x = job.x ? job.x : x_all;  // (uniform over the workgroup)
     const int K = job.x ? job.K : K_all;
@@ -49,10 +52,10 @@ __global__ void __launch_bounds__(256) small_linear_kernel(const float* __restri
         for (int k = tid; k < K; k += 256) smem[k * M + m] = (m < m_real) ? x[(long long)m * K + k] : 0.f;
     __syncthreads();
 
-    const int cl = tid & 31, ks = tid >> 5;
+    const int cl = tid % CG, ks = tid / CG;
     const int c0 = col_base + cl * 4;
-    const int kper = (K + 7) / 8;
-    const int kbeg = ks * kper, kend = min(K, kbeg + kper);
+    const int kper = (K + SLICES - 1) / SLICES;
+    const int kbeg = ks * kper, kend = min(K, kbeg + kper);  // (with few rows the last slices may be empty)
     const WT* W = reinterpret_cast<const WT*>(job.W) + job.n0 + c0;
     float acc[M][4];
 #pragma unroll
@@ -80,19 +83,19 @@ __global__ void __launch_bounds__(256) small_linear_kernel(const float* __restri
             }
         }
     }
-    __syncthreads();  // everyone is done with xs; reuse it for the cross-slice reduction: red[ks][m][128]
+    __syncthreads();  // everyone is done with xs; reuse it for the cross-slice reduction: red[ks][m][COLS]
 #pragma unroll
     for (int m = 0; m < M; m++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) smem[(ks * M + m) * 128 + cl * 4 + j] = acc[m][j];
+        for (int j = 0; j < 4; j++) smem[(ks * M + m) * COLS + cl * 4 + j] = acc[m][j];
     __syncthreads();
-    for (int e = tid; e < M * 128; e += 256) {
-        const int m = e >> 7, c = e & 127;
+    for (int e = tid; e < M * COLS; e += 256) {
+        const int m = e / COLS, c = e % COLS;
         const int col = col_base + c;
         if (m < m_real && col < job.N) {
             float s = 0.f;
 #pragma unroll
-            for (int s8 = 0; s8 < 8; s8++) s += smem[(s8 * M + m) * 128 + c];
+            for (int sl = 0; sl < SLICES; sl++) s += smem[(sl * M + m) * COLS + c];
             if (job.bias) s += job.bias[job.n0 + col];
             if (act == SD3_ACT_SILU) s = silu_precise(s);
             else if (act == SD3_ACT_GELU_TANH) s = gelu_tanh_precise(s);
@@ -101,19 +104,34 @@ __global__ void __launch_bounds__(256) small_linear_kernel(const float* __restri
     }
 }
 
-template <int M>
-static void launch_small(const float* x, int m_real, int K, int K_max, const SmallLinearJobPack& jobs, int n_jobs, int max_N, int w_is_bf16, bool vec, int act,
-                         hipStream_t st) {
-    dim3 grid((max_N + 127) / 128, n_jobs), block(256);
+template <int M, int CG>
+static void launch_groups(const float* x, int m_real, int K, int K_max, const SmallLinearJobPack& jobs, int n_jobs, int max_N, int w_is_bf16, bool vec, int act,
+                          hipStream_t st) {
+    dim3 grid((max_N + 4 * CG - 1) / (4 * CG), n_jobs), block(256);
     const int kk = K_max > 1024 ? K_max : 1024;
     const size_t smem = (size_t)kk * M * sizeof(float);
     if (w_is_bf16) {
-        if (vec) hipLaunchKernelGGL((small_linear_kernel<M, bf16_t, true>), grid, block, smem, st, x, m_real, K, jobs, act);
-        else hipLaunchKernelGGL((small_linear_kernel<M, bf16_t, false>), grid, block, smem, st, x, m_real, K, jobs, act);
+        if (vec) hipLaunchKernelGGL((small_linear_kernel<M, bf16_t, true, CG>), grid, block, smem, st, x, m_real, K, jobs, act);
+        else hipLaunchKernelGGL((small_linear_kernel<M, bf16_t, false, CG>), grid, block, smem, st, x, m_real, K, jobs, act);
     } else {
-        if (vec) hipLaunchKernelGGL((small_linear_kernel<M, float, true>), grid, block, smem, st, x, m_real, K, jobs, act);
-        else hipLaunchKernelGGL((small_linear_kernel<M, float, false>), grid, block, smem, st, x, m_real, K, jobs, act);
+        if (vec) hipLaunchKernelGGL((small_linear_kernel<M, float, true, CG>), grid, block, smem, st, x, m_real, K, jobs, act);
+        else hipLaunchKernelGGL((small_linear_kernel<M, float, false, CG>), grid, block, smem, st, x, m_real, K, jobs, act);
     }
+}
+
+// The split is chosen from the weights of the launch alone, so that a row's result does not depend on how many rows there are: up to two
+// wide workgroups per compute unit, runs of one cache line (32 fp32 or 64 bf16 columns, 32 or 16 slices). Wide and narrow, us: the
+// timestep and text MLPs (2 x 12 wide workgroups, K up to 2048) 24.0 and 11.8 with one row, 45 and 20 with four; the modulation
+// vectors of one block, 1536 columns a chunk, bf16 (180): 16.3 and 13.4; 768, fp32, eight rows (90): 38 and 21; those of a 24-block forward
+// (5242): 260 and 288 -- shorter runs than a line lose everywhere from 16 workgroups on.
+template <int M>
+static void launch_small(const float* x, int m_real, int K, int K_max, const SmallLinearJobPack& jobs, int n_jobs, int max_N, int w_is_bf16, bool vec, int act,
+                         hipStream_t st) {
+    long long wide = 0;  // workgroups of 128 columns
+    for (int i = 0; i < n_jobs; i++) wide += (jobs.j[i].N + 127) / 128;
+    if (wide > 512) launch_groups<M, 32>(x, m_real, K, K_max, jobs, n_jobs, max_N, w_is_bf16, vec, act, st);
+    else if (w_is_bf16) launch_groups<M, 16>(x, m_real, K, K_max, jobs, n_jobs, max_N, w_is_bf16, vec, act, st);
+    else launch_groups<M, 8>(x, m_real, K, K_max, jobs, n_jobs, max_N, w_is_bf16, vec, act, st);
 }
 
 int small_linear_batched(const float* x, int M, int K, const SmallLinearJob* jobs_host, int n_jobs, int w_is_bf16, int act, hipStream_t st) {
