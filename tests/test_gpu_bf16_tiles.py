@@ -26,7 +26,7 @@ def test_bf16_tile_shapes(m, n, k, epi, f32):
     rows = (m, 40)
     A = [torch.randn((r, k), device="cuda", generator=g).bfloat16() for r in rows]
     W = [(0.1 * torch.randn((n, k), device="cuda", generator=g)).bfloat16() for _ in rows]
-    bias, gate, rms = (torch.randn(s, device="cuda", generator=g) for s in ((n,), (m, n), (64,)))
+    bias, gate, rms = (torch.randn(s, device="cuda", generator=g) for s in ((n,), (max(rows), n), (64,)))  # (a gate row for every row of either problem)
     resid = [torch.randn((r, n), device="cuda", generator=g) for r in rows]
     per = max(1, m // 3)
     first = None
