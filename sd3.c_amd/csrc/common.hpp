@@ -182,6 +182,7 @@ struct GemmBf16Problem {
     void* out;
     int ldc, M, N, K;
     GemmEpilogueArgs ea;
+    const GemmBf16Problem* then = nullptr;  // EPI_GATE_RESID: a second layer of the same M, N, K and out whose residual is this one's result
 };
 extern std::atomic<long long> g_gemm_bf16_launches;  // kernels launched by the bf16 GEMM so far (for per-launch profile figures)
 int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st);

@@ -306,6 +306,7 @@ int linear_layer(sd3_ctx* ctx, int prec, const void* A, const float* W, const fl
 
 // The same layer of the latent stream and of the context stream (different weights and rows, same kind): both
 // go into one launch, so that the few context rows ride along instead of paying a launch of their own.
+// then (bf16 only, gated epilogue): a layer that adds to the result of the first one, whose rows must not be empty.
 struct LayerCall {
     const void* A;
     const float* W;
@@ -314,7 +315,7 @@ struct LayerCall {
     int ldc, M, N, K;
     GemmEpilogueArgs ea;
 };
-int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f32, int epi) {
+int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f32, int epi, const LayerCall* then = nullptr) {
     if (n > 3) return fail(SD3_ERR_INVALID_ARG, "linear_pair: at most three layers per group");
     if (!is_bf(prec)) {
         GemmF32Problem probs[3];
@@ -346,6 +347,16 @@ int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f
         probs[m].ea.bias = c.bias;
         flop += 2.0 * c.M * c.N * c.K;
         m++;
+    }
+    GemmBf16Problem second;
+    if (then) {
+        if (!then->W) return fail(SD3_ERR_MISSING_PARAM, "a weight needed by this configuration is not bound (N=%d K=%d)", then->N, then->K);
+        const void* wp = nullptr;
+        SD3_TRY(get_packed(ctx, then->W, then->K, then->N, 0, &wp));
+        second = GemmBf16Problem{(const bf16_t*)then->A, (const bf16_t*)wp, then->out, then->ldc, then->M, then->N, then->K, then->ea};
+        second.ea.bias = then->bias;
+        probs[0].then = &second;
+        flop += 2.0 * then->M * then->N * then->K;
     }
     if (m == 0) return SD3_OK;
     ProfScope ps(ctx, SD3_PROF_GEMM, flop);
@@ -534,12 +545,16 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     gx.rows_per_batch = Tx; gx.gate = xchunk(2); gx.gate_ld = ldx_ada; gx.resid = x;
     {
         LayerCall proj[2] = {{x_att, w.x_out_w, w.x_out_b, x, C, mx, C, C, gx}, {c_att, w.c_out_w, w.c_out_b, c, C, d.discard ? 0 : mc, C, C, gc}};
-        SD3_TRY(linear_pair(ctx, prec, proj, 2, 1, EPI_GATE_RESID));
+        // with dual attention, bf16: the second projection of the latent rows (modules.cpp:1450-1453, 1486) rides behind the first, in its launch
+        GemmEpilogueArgs g2;
+        g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;
+        const LayerCall proj2{x_att2, w.x2_out_w, w.x2_out_b, x, C, mx, C, C, g2};
+        SD3_TRY(linear_pair(ctx, prec, proj, 2, 1, EPI_GATE_RESID, d.dual && bf ? &proj2 : nullptr));
     }
 
-    // ---- extra self-attention over the latent tokens (modules.cpp:1440-1453, 1486)
-    if (d.dual) {
-        if (!bf) SD3_TRY(attention(ctx, dual_set, B, d.NH, d.HS, bf));
+    // ---- fp32: extra self-attention over the latent tokens (modules.cpp:1440-1453, 1486)
+    if (d.dual && !bf) {
+        SD3_TRY(attention(ctx, dual_set, B, d.NH, d.HS, bf));
         GemmEpilogueArgs g2;
         g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;
         SD3_TRY(linear_layer(ctx, prec, x_att2, w.x2_out_w, w.x2_out_b, x, 1, C, mx, C, C, EPI_GATE_RESID, g2));
