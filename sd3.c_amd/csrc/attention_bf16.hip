@@ -17,6 +17,8 @@
 // barrier per tile.
 #include <type_traits>
 
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace sd3 {
@@ -68,7 +70,30 @@ constexpr int MAX_SETS = 3;
 struct AttnSets {
     SegDev set[MAX_SETS];
     int end[MAX_SETS];
+    Ahead ahead;  // read by the workgroups from end[MAX_SETS - 1] on
 };
+
+// One load per 128-byte line of every run, the value dropped: workgroup `wg` of `wgs`, NT threads each.
+// Attention leaves HBM idle and the layers behind it wait for their weights (a launch of 333 / 1178 / 2356 / 4250 rows of mlp-1 and mlp-2
+// takes 51 / 74 / 108 / 173 us with weights from HBM, 36 / 60 / 94 / 156 from the last-level cache), so the workgroup slots that its
+// last round leaves free stream the block's remaining weights: forwards of 256px 2976 -> 2957 us, 512px 4681 -> 4617, its guided pair 6514 ->
+// 6454, 1024px 12726 -> 12594. (The same in the LayerNorm launches or on the compute units that a layer's tiles leave idle: slower on most.)
+template <int NT>
+__device__ __forceinline__ void read_ahead(const Ahead& a, unsigned wg, unsigned wgs) {
+    constexpr uint32_t LINE = 128, UNROLL = 4;
+    const uint32_t stride = wgs * NT;
+#pragma unroll
+    for (int s = 0; s < MAX_AHEAD; s++) {
+        const uint32_t lines = a.bytes[s] / LINE;  // (runs are whole lines, or their last few bytes are left out)
+        for (uint32_t l = wg * NT + threadIdx.x; l < lines; l += stride * UNROLL) {
+            uint32_t v[UNROLL];
+#pragma unroll
+            for (uint32_t i = 0; i < UNROLL; i++) v[i] = *reinterpret_cast<const uint32_t*>(a.p[s] + (size_t)min(l + i * stride, lines - 1) * LINE);
+#pragma unroll
+            for (uint32_t i = 0; i < UNROLL; i++) asm volatile("" ::"v"(v[i]));
+        }
+    }
+}
 
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
@@ -134,6 +159,10 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    if (blockIdx.x >= (unsigned)sets.end[MAX_SETS - 1]) {
+        read_ahead<NW * 64>(sets.ahead, blockIdx.x - sets.end[MAX_SETS - 1], gridDim.x - sets.end[MAX_SETS - 1]);
+        return;
+    }
     const int which = (blockIdx.x >= (unsigned)sets.end[0]) + (blockIdx.x >= (unsigned)sets.end[1]);  // uniform
     const SegDev& s = sets.set[which];
     const int wg_first = which ? sets.end[which - 1] : 0;
@@ -755,6 +784,10 @@ __global__ void __launch_bounds__(KS * 64, 2) flash_attn_bf16_split_kernel(const
     constexpr int PITCH = 16 * QB + 2 * QB;  // floats per lane in the merge buffer
     constexpr int V_SPACE = KS * 2 * V_TILE, MERGE = (KS / 2) * 64 * PITCH * 4;
     __shared__ __attribute__((aligned(1024))) char smem[V_SPACE > MERGE ? V_SPACE : MERGE];
+    if (blockIdx.x >= (unsigned)sets.end[MAX_SETS - 1]) {
+        read_ahead<KS * 64>(sets.ahead, blockIdx.x - sets.end[MAX_SETS - 1], gridDim.x - sets.end[MAX_SETS - 1]);
+        return;
+    }
     const int which = (blockIdx.x >= (unsigned)sets.end[0]) + (blockIdx.x >= (unsigned)sets.end[1]);
     const SegDev& s = sets.set[which];
     const int wg_first = which ? sets.end[which - 1] : 0;
@@ -1078,7 +1111,8 @@ size_t attention_bf16_split_workspace_floats(int B, int NH, int Tc, int splits) 
     return items * BQ * (HS + 2);
 }
 
-int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int hs, hipStream_t st) {
+int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int hs, hipStream_t st,
+                         const Ahead* ahead) {
     if (n < 1 || n > MAX_SETS) return fail(SD3_ERR_INVALID_ARG, "attention: 1 to %d sets per launch (got %d)", MAX_SETS, n);
     if (hs != HS) return fail(SD3_ERR_UNSUPPORTED, "attention (bf16): head_dim must be 64 (got %d)", hs);
     if (B <= 0 || NH <= 0) return SD3_OK;
@@ -1108,6 +1142,24 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     if (m == 0) return SD3_OK;
     for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
     const float q_scale = 1.4426950408889634f / sqrtf((float)HS);
+    // Workgroups that read ahead: the slots (two per compute unit) that the last round of `items` leaves free, for about as long as that
+    // round lasts (a key tile is about 1 us), at a rate well below what HBM gives the same number of workgroups.
+    auto readers = [&](int items) -> int {
+        const int slots = 2 * compute_units();
+        if (!ahead || slots <= 0) return 0;
+        const int idle = (slots - items % slots) % slots;
+        const size_t per_wg = (size_t)6144 * (3 + (longest + BKV - 1) / BKV);
+        size_t left = per_wg * idle, taken = 0;
+        for (int i = 0; i < MAX_AHEAD; i++) {
+            const uint32_t b = (uint32_t)std::min<size_t>(ahead->bytes[i], left);
+            sets.ahead.p[i] = ahead->p[i];
+            sets.ahead.bytes[i] = b;
+            left -= b;
+            taken += b;
+        }
+        constexpr size_t LEAST = 32768;  // one line per thread
+        return (int)std::min<size_t>(idle, (taken + LEAST - 1) / LEAST);
+    };
     if (!norm && longest <= SHORT_KEYS) {
         constexpr int QB = 2, KS = 4;
         total = 0;
@@ -1118,10 +1170,10 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
             sets.end[i] = total;
         }
         for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
-        hipLaunchKernelGGL((flash_attn_bf16_split_kernel<QB, KS>), dim3((unsigned)total), dim3(KS * 64), 0, st, sets, q_scale);
+        hipLaunchKernelGGL((flash_attn_bf16_split_kernel<QB, KS>), dim3((unsigned)(total + readers(total))), dim3(KS * 64), 0, st, sets, q_scale);
         return launch_status("flash_attention_bf16");
     }
-    dim3 grid((unsigned)total), block(NW * 64);
+    dim3 grid((unsigned)(total + readers(total))), block(NW * 64);
     if (norm) hipLaunchKernelGGL(flash_attn_bf16_kernel<true>, grid, block, 0, st, sets, q_scale, 1e-6f);
     else hipLaunchKernelGGL(flash_attn_bf16_kernel<false>, grid, block, 0, st, sets, q_scale, 1e-6f);
     SD3_TRY(launch_status("flash_attention_bf16"));

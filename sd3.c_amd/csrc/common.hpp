@@ -285,7 +285,15 @@ int attention_bf16(const AttnSegments& s, int B, int NH, int HS, hipStream_t st)
 // work item each, whose partial results go through split_ws[i] (attention_bf16_split_workspace_floats floats) and are merged by a
 // second, small kernel. attention_bf16_context_splits: the number of splits that pays for the Tc context queries of a joint
 // attention next to Tx latent ones, or 0 when the plain one-set launch is the better choice.
-int attention_bf16_multi(const AttnSegments* sets, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int HS, hipStream_t st);
+// ahead (or null): memory that the launches behind this one are about to stream (weights); as much of it as fits the launch's idle
+// workgroup slots is read once, in order, so that it lies in the last-level cache (256 MB, shared by the XCDs) when they ask for it.
+constexpr int MAX_AHEAD = 7;
+struct Ahead {
+    const char* p[MAX_AHEAD];
+    uint32_t bytes[MAX_AHEAD];
+};
+int attention_bf16_multi(const AttnSegments* sets, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int HS, hipStream_t st,
+                         const Ahead* ahead = nullptr);
 int attention_bf16_context_splits(int Tc, int Tx, int NH, bool dual);
 size_t attention_bf16_split_workspace_floats(int B, int NH, int Tc, int splits);
 
