@@ -8,7 +8,7 @@
 // LDS buffers with one workgroup barrier per 64-deep K tile; LDS rows are 128 bytes with the 16-byte chunk index
 // XOR-swizzled by a key of the row, which makes both the linear LDS fill and the 16-byte MFMA operand reads conflict-free.
 // Two kernels: gemm_bf16_kernel (256x256 tiles by persistent workgroups; also the fp8 form) for launches that fill the device with
-// them, gemm_bf16_ring_kernel (64x64 to 256x128 tiles) for the others; tile_shapes says where the line is.
+// them, gemm_bf16_ring_kernel (64x64 to 256x128 tiles; 192x256 ones are the first kernel's) for the others; tile_shapes says where the line is.
 #include "common.hpp"
 
 #include <type_traits>
@@ -758,7 +758,8 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
 
     fill_ring();
     k_loop();
-    if (EPI == EPI_GATE_RESID && pr.then) {
+    constexpr bool PAIR = EPI == EPI_GATE_RESID && TM * TN <= 64 * 128;  // (see grouped_impl)
+    if (PAIR && pr.then) {
         // The second layer of the same rows and columns (the two out-projections of a block with dual attention): its ring is filled behind
         // the last LDS reads of the first and lands while the first one's results are on their way out; a thread reads back what it wrote.
         const Prob& next = args.second;
@@ -800,14 +801,17 @@ int launch_ring(ProbSet& args, int n, hipStream_t st) {
 // The tile shapes of the bf16 GEMM, smallest first, and what an output tile costs its compute unit in microseconds: `fixed` + `per_k` for
 // each K tile of 64. Fitted to launches with cold weights at K = 1536 and 6144, 333 to 4250 rows, N = 1536 .. 6144 (a constant for the
 // first round, the same for all shapes, left out); what they stand for is the traffic of (tm + tn) * 128 bytes per K tile through one
-// compute unit's load path and, from 128x128 on, the matrix instructions.
+// compute unit's load path and, from 128x128 on, the matrix instructions. 192x256 tiles (the persistent kernel's, like 256x256) save little
+// per tile but are there for what is left of a round: q|k|v of 2 x 1024 + 154 rows, 162 or 234 tiles, 50.2 -> 46.0 us; 128x256 beside 256x128
+// for rows that are not multiples of 256: mlp-1 of 1581 + 999 rows, 504 tiles instead of 528 in two rounds of 256, 73 -> 60 us.
 struct TileShape {
     int tm, tn;
     double fixed, per_k;
 };
-enum { TILE_64, TILE_128_64, TILE_64_128, TILE_128, TILE_256_128, TILE_256, TILE_SHAPES };
+enum { TILE_64, TILE_128_64, TILE_64_128, TILE_128, TILE_256_128, TILE_128_256, TILE_192_256, TILE_256, TILE_SHAPES };
 constexpr TileShape tile_shapes[TILE_SHAPES] = {{64, 64, 1.3, 0.19},    {128, 64, 2.3, 0.285},  {64, 128, 2.3, 0.285},
-                                                {128, 128, 7.3, 0.403}, {256, 128, 11.3, 0.59}, {256, 256, 11.3, 1.28}};
+                                                {128, 128, 7.3, 0.403}, {256, 128, 11.3, 0.59}, {128, 256, 11.5, 0.615},
+                                                {192, 256, 6.0, 1.315}, {256, 256, 11.3, 1.28}};
 
 long long tiles_of(const Prob& q, int shape) {
     const TileShape& t = tile_shapes[shape];
@@ -821,7 +825,12 @@ double launch_cost(const ProbSet& set, int n, int shape, int cus) {
         depth += c * (set.p[i].K / BK);
     }
     const TileShape& t = tile_shapes[shape];
-    return (double)((tiles + cus - 1) / cus) * (t.fixed + t.per_k * ((double)depth / tiles));
+    const long long rounds = (tiles + cus - 1) / cus;
+    // 128x256 tiles in two rounds cost more than the table says: mlp-1 of 1581 + 999 rows, 504 tiles, 60 us and not 53, the out-projection of
+    // 9996 rows, 504 tiles, 81 and not 53, its mlp-2 207 and not 141 (256x256 tiles in one round: 74 and 191).
+    // (192x256 tiles in two rounds where 256x256 ones take two as well: 12255 + 770 rows, forward 0.8 % slower)
+    const double again = rounds == 1 ? 1.0 : shape == TILE_128_256 ? 1.25 : shape == TILE_192_256 ? 1.06 : 1.0;
+    return again * (double)rounds * (t.fixed + t.per_k * ((double)depth / tiles));
 }
 int cheapest_shape(const ProbSet& set, int n, int cus, double& cost) {
     int best = TILE_256;
@@ -854,6 +863,8 @@ int launch_shape(int shape, ProbSet& args, int n, int cus, hipStream_t st) {
             return launch_ring<64, 128, 4, 2, 3, 4, EPI, OUT_F32>(args, n, st);
         case TILE_128: return launch_ring<128, 128, 4, 2, 4, 2, EPI, OUT_F32>(args, n, st);
         case TILE_256_128: return launch_ring<256, 128, 4, 2, 3, 2, EPI, OUT_F32>(args, n, st);
+        case TILE_128_256: return launch_ring<128, 256, 2, 4, 3, 2, EPI, OUT_F32>(args, n, st);
+        case TILE_192_256: return launch_cfg<192, 256, 2, 4, 2, EPI, OUT_F32>(args, n, st);
         default: return launch_cfg<256, 256, 2, 4, 2, EPI, OUT_F32>(args, n, st);
     }
 }
@@ -1004,7 +1015,7 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         int pair = -1;
         if (g_gemm_bf16_tile) {
             pair = can ? forced_shape(g_gemm_bf16_tile) : -1;
-            if (pair == TILE_256) pair = -1;
+            if (pair > TILE_64_128) pair = -1;
         } else if (can) {
             ProbSet second{};
             second.p[0] = args.second;
@@ -1108,7 +1119,7 @@ int gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* out, int out_is_f32, int 
 
 extern "C" int sd3_gemm_bf16_force_tile(int tile) {
     if (tile != 0 && tile != 192 && sd3::forced_shape(tile) < 0)
-        return sd3::fail(SD3_ERR_INVALID_ARG, "sd3_gemm_bf16_force_tile: tile must be 0, 128, 192, 256, 64064, 64128, 128064 or 256128 (got %d)", tile);
+        return sd3::fail(SD3_ERR_INVALID_ARG, "sd3_gemm_bf16_force_tile: tile must be 0, 128, 192, 256, 64064, 64128, 128064, 256128, 128256 or 192256 (got %d)", tile);
     sd3::g_gemm_bf16_tile = tile;
     return SD3_OK;
 }

@@ -19,7 +19,7 @@ def test_block_does_not_depend_on_the_tile_of_its_projections(B, Tc, Tx, C, disc
     y, c, x = (torch.randn(s, device="cuda", generator=g) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
     first = None
     try:
-        for tile in (256, 64064, 128064, 64128, 128, 256128, 0, 0):
+        for tile in (256, 64064, 128064, 64128, 128, 256128, 128256, 192256, 0, 0):
             L.call("sd3_gemm_bf16_force_tile", tile)
             got = M.Dit_block(y, c.clone(), x.clone(), P, B, Tc, Tx, C, C // 64, 2, True, True, discard, precision="bf16")
             torch.cuda.synchronize()

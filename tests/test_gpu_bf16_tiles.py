@@ -6,7 +6,7 @@ from gpu_util import M  # noqa: F401  (loads the package)
 from sd3_c_amd import lib as L
 
 pytestmark = pytest.mark.gpu
-SHAPES = (64064, 128064, 64128, 128, 256128, 256, 0)
+SHAPES = (64064, 128064, 64128, 128, 256128, 128256, 192256, 256, 0)
 
 
 def _grouped(problems, epi, f32):
