@@ -375,7 +375,8 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
         // (rings no deeper than that two or three workgroups fit a compute unit: they hide each other's waits better than a deeper ring)
         case 0: return launch_tile<128, 128, 2, 2, 2, EPI>(set, n, st);
         case 1: return launch_tile<128, 64, 4, 1, 3, EPI>(set, n, st);
-        case 2: return launch_tile<64, 64, 2, 2, 3, EPI>(set, n, st);
+        // (64 columns per wavefront: W in 16-byte LDS reads; as 2x2 wavefronts of 32x32 2202 x 4608 x 1536 took 260 us instead of 255)
+        case 2: return launch_tile<64, 64, 4, 1, 3, EPI>(set, n, st);
         case 3: return launch_tile<32, 64, 2, 2, 4, EPI>(set, n, st);
         default: return launch_tile<32, 32, 2, 2, 5, EPI>(set, n, st);
     }
