@@ -258,7 +258,7 @@ int sd3_gemm_bf16_force_tile(int tile);
  * sd3_gemm_bf16_force_tile; "attention_context_splits": -1 chosen from the sizes (default), 0 never, 2..8 that many key splits for
  * the context queries of a block's joint attention wherever splitting applies (results of those rows change in the last bf16 bit
  * with the number of splits); "gemm_bf16_row_split": 0 / 1 (default), whether a many-row problem that leaves a partial round of
- * 256x256 tiles may send its last rows to a second launch of 128x128 tiles; "gemm_f32_tile": -1 chosen from the sizes (default), 0..4 a
+ * 256x256 tiles may send its last rows to a second launch of smaller tiles; "gemm_f32_tile": -1 chosen from the sizes (default), 0..4 a
  * fixed tile shape of the fp32 GEMM (128x128, 128x64, 64x64, 32x64, 32x32). Unknown names return SD3_ERR_INVALID_ARG. */
 int sd3_tune(const char* name, int value);
 /* Measurement aid with no counterpart in the reference: the rate (in TFLOP/s) at which the device's matrix cores run the
