@@ -991,20 +991,6 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
     // the ring kernel stores four columns at a time; rows that are not made of such chunks take the 256x256 tiles
     bool whole_chunks = true;
     for (int i = 0; i < m; i++) whole_chunks = whole_chunks && ring_can(args.p[i], epi);
-    if (g_gemm_bf16_tile == 192) {
-        if (epi == EPI_QKV_NORM) return fail(SD3_ERR_UNSUPPORTED, "gemm_bf16: this tile shape cannot fuse the qk-norm");
-#define SD3_GEMM_BF16_192(E) \
-    case E: return out_is_f32 ? launch_cfg<256, 192, 2, 4, 2, E, true>(args, m, st) : launch_cfg<256, 192, 2, 4, 2, E, false>(args, m, st)
-        switch (epi) {
-            SD3_GEMM_BF16_192(EPI_BIAS);
-            SD3_GEMM_BF16_192(EPI_BIAS_GELU);
-            SD3_GEMM_BF16_192(EPI_BIAS_SILU);
-            SD3_GEMM_BF16_192(EPI_GATE_RESID);
-            SD3_GEMM_BF16_192(EPI_BIAS_ROWADD);
-            default: return fail(SD3_ERR_INVALID_ARG, "gemm_bf16: unknown epilogue %d", epi);
-        }
-#undef SD3_GEMM_BF16_192
-    }
     if (then) {
         // Both layers in one launch where they are one round of small tiles, i.e. a launch's start and end are a good part of it: dual blocks
         // of 256 + 77, 1024 + 154 tokens 106.7 -> 105.3 us, forwards 2972 -> 2951, 4708 -> 4681 us. From 128x128 tiles on the second layer
@@ -1014,7 +1000,7 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         const bool can = whole_chunks && ring_can(args.second, epi);
         int pair = -1;
         if (g_gemm_bf16_tile) {
-            pair = can ? forced_shape(g_gemm_bf16_tile) : -1;
+            pair = can ? forced_shape(g_gemm_bf16_tile) : -1;  // (256x192 tiles, 192, have no shape of the table: two launches)
             if (pair > TILE_64_128) pair = -1;
         } else if (can) {
             ProbSet second{};
@@ -1044,6 +1030,20 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         }
         SD3_TRY(grouped_impl(rest, n, out_is_f32, epi, false, st));
         return grouped_impl(then, 1, out_is_f32, epi, false, st);
+    }
+    if (g_gemm_bf16_tile == 192) {
+        if (epi == EPI_QKV_NORM) return fail(SD3_ERR_UNSUPPORTED, "gemm_bf16: this tile shape cannot fuse the qk-norm");
+#define SD3_GEMM_BF16_192(E) \
+    case E: return out_is_f32 ? launch_cfg<256, 192, 2, 4, 2, E, true>(args, m, st) : launch_cfg<256, 192, 2, 4, 2, E, false>(args, m, st)
+        switch (epi) {
+            SD3_GEMM_BF16_192(EPI_BIAS);
+            SD3_GEMM_BF16_192(EPI_BIAS_GELU);
+            SD3_GEMM_BF16_192(EPI_BIAS_SILU);
+            SD3_GEMM_BF16_192(EPI_GATE_RESID);
+            SD3_GEMM_BF16_192(EPI_BIAS_ROWADD);
+            default: return fail(SD3_ERR_INVALID_ARG, "gemm_bf16: unknown epilogue %d", epi);
+        }
+#undef SD3_GEMM_BF16_192
     }
     if (!whole_chunks) return launch(args, m, TILE_256);
     if (g_gemm_bf16_tile) return launch(args, m, forced_shape(g_gemm_bf16_tile));

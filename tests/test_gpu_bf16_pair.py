@@ -1,4 +1,4 @@
-"""The two out-projections of a block with dual attention: one launch on the small tiles, one after the other on the 256x256 ones."""
+"""The two out-projections of a block with dual attention: one launch on the small tiles, one after the other on the others."""
 import pytest
 import torch
 
@@ -24,6 +24,25 @@ def test_block_does_not_depend_on_the_tile_of_its_projections(B, Tc, Tx, C, disc
             got = M.Dit_block(y, c.clone(), x.clone(), P, B, Tc, Tx, C, C // 64, 2, True, True, discard, precision="bf16")
             torch.cuda.synchronize()
             assert torch.isfinite(got[1]).all()
+            first = got if first is None else first
+            assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), tile
+    finally:
+        L.call("sd3_gemm_bf16_force_tile", 0)
+
+
+@pytest.mark.parametrize("B,Tc,Tx,C", [(1, 3, 63, 320), (2, 0, 65, 384), (1, 77, 257, 512)])
+@pytest.mark.parametrize("discard", [False, True])
+def test_block_without_qk_norm_on_every_tile(B, Tc, Tx, C, discard):
+    """The same without the qk-norm, which 256x192 tiles (192) cannot fuse: every tile that a caller can force takes the whole block."""
+    g = torch.Generator(device="cuda").manual_seed(B * 100 + Tx + 1)
+    P = {k: 0.1 * torch.randn(s, device="cuda", generator=g) for k, s in block_param_shapes(C, 2, True, False, discard, 64).items()}
+    y, c, x = (torch.randn(s, device="cuda", generator=g) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
+    first = None
+    try:
+        for tile in (256, 192, 64064, 128064, 64128, 128, 256128, 128256, 192256, 0):
+            L.call("sd3_gemm_bf16_force_tile", tile)
+            got = M.Dit_block(y, c.clone(), x.clone(), P, B, Tc, Tx, C, C // 64, 2, True, False, discard, precision="bf16")
+            torch.cuda.synchronize()
             first = got if first is None else first
             assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), tile
     finally:
