@@ -9,6 +9,7 @@
 #include <cstdio>
 
 #include "../../include/sd3_hip.h"
+#include "device.hpp"
 
 namespace sd3 {
 
@@ -35,20 +36,6 @@ inline int launch_status(const char* what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(SD3_ERR_HIP, "launch of %s failed: %s", what, hipGetErrorString(e));
     return SD3_OK;
-}
-
-// compute units of the current device (0 after a failed query, which has set the error message)
-inline int compute_units() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-            fail(SD3_ERR_HIP, "cannot query the number of compute units");
-            return 0;
-        }
-        cus = n;
-    }
-    return cus;
 }
 
 // ---- bf16 as raw 16-bit storage ----

@@ -513,11 +513,8 @@ template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, boo
 int launch_cfg(ProbSet& args, int n, hipStream_t st) {
     auto kern = gemm_bf16_kernel<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8>;
     constexpr int smem = smem_bytes<BM, BN, WM, WN, STAGES>();
-    static bool attr_done = false;  // raising the dynamic LDS limit is a per-function, per-process setting
-    if (smem > 65536 && !attr_done) {
-        SD3_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-        attr_done = true;
-    }
+    static DynamicLds lds;
+    SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
     if (EPI == EPI_QKV_NORM && (BN / WN) % 64 != 0) return fail(SD3_ERR_UNSUPPORTED, "gemm_bf16: this tile shape cannot fuse the qk-norm");
     int total = 0;
     for (int i = 0; i < MAX_PROBS; i++) {
@@ -783,11 +780,8 @@ template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_
 int launch_ring(ProbSet& args, int n, hipStream_t st) {
     auto kern = gemm_bf16_ring_kernel<TM, TN, WM, WN, STAGES, MW, EPI, OUT_F32>;
     constexpr int smem = STAGES * (TM + TN) * 128;
-    static bool attr_done = false;  // raising the dynamic LDS limit is a per-function, per-process setting
-    if (smem > 65536 && !attr_done) {
-        SD3_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-        attr_done = true;
-    }
+    static DynamicLds lds;
+    SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
     int total = 0;
     for (int i = 0; i < MAX_PROBS; i++) {
         if (i < n) total += ((args.p[i].N + TN - 1) / TN) * ((args.p[i].M + TM - 1) / TM);

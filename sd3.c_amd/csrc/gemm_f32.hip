@@ -347,11 +347,8 @@ template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
 int launch_tile(TileProbSet& set, int n, hipStream_t st) {
     auto kern = gemm_f32_tile_kernel<TM, TN, WM, WN, STAGES, EPI>;
     constexpr int smem = STAGES * (TM * 128 + TK * TN * 4);
-    static bool attr_done = false;  // raising the dynamic LDS limit is a per-function, per-process setting
-    if (smem > 65536 && !attr_done) {
-        SD3_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem));
-        attr_done = true;
-    }
+    static DynamicLds lds;
+    SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
     int total = 0;
     for (int i = 0; i < MAX_PROBS; i++) {
         if (i < n) total += ((set.p[i].M + TM - 1) / TM) * ((set.p[i].N + TN - 1) / TN);
