@@ -4,6 +4,7 @@ import torch
 
 from gpu_util import M
 from sd3_c_amd import lib as L
+from sd3_c_amd.params import block_param_shapes
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24  # unit roundoff of fp32
@@ -40,6 +41,68 @@ def test_gemm_f32_column_window_and_unaligned_rows():
         y = M.partial_linear(x, W, b, n0, n)
         xd, Wd, bd = x.double(), W[:, n0:n0 + n].double(), b[n0:n0 + n].double()
         assert ((y.double() - (xd @ Wd + bd)).abs() <= (k + 2) * U * (xd.abs() @ Wd.abs() + bd.abs())).all()
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 36, 68), (154, 96, 132)])
+def test_gemm_f32_output_at_any_float(m, k, n):
+    """The output may begin at any float: the same kernel, hence the same bits, for every tile shape, and nothing beside it is written."""
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, n), (n,)))
+    want = M.linear(x, W, b)
+    for tile in (-1, 0, 1, 2, 3, 4):
+        L.call("sd3_tune", b"gemm_f32_tile", tile)
+        for off in (1, 2, 3):
+            buf = torch.full((m * n + 8,), 7.0, device="cuda")
+            L.call("sd3_linear", x.data_ptr(), W.data_ptr(), b.data_ptr(), buf.data_ptr() + 4 * off, m, k, n, None)
+            torch.cuda.synchronize()
+            assert torch.equal(buf[off:off + m * n].view(m, n), want) and bool((buf[:off] == 7).all()) and bool((buf[off + m * n:] == 7).all()), (tile, off)
+
+
+@pytest.mark.parametrize("B,Tc,Tx,C,discard", [(2, 5, 33, 192, False), (3, 77, 70, 128, False), (1, 0, 65, 64, True)])
+def test_block_f32_every_tile_shape_and_streams_at_any_float(B, Tc, Tx, C, discard):
+    """The gated epilogue (a gate row per batch element, residual in place) in a block with dual attention: every tile shape gives equal bits,
+    also on streams that begin one float after a 16-byte boundary. Those go through another LayerNorm, whose sums have another order: a
+    few u sqrt(K) of relative difference (K <= 384 terms, 1e-6) in each of the six layers behind one another."""
+    g = torch.Generator(device="cuda").manual_seed(Tx)
+    P = {k: 0.1 * torch.randn(s, device="cuda", generator=g) for k, s in block_param_shapes(C, 2, True, True, discard, 64).items()}
+    y, c, x = (torch.randn(s, device="cuda", generator=g) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
+
+    def at(t, off):
+        buf = torch.empty(t.numel() + 4, device="cuda")
+        return buf[off:off + t.numel()].view(t.shape).copy_(t)
+
+    results = []
+    for off in (0, 1):
+        first = None
+        for tile in (-1, 0, 1, 2, 3, 4):
+            L.call("sd3_tune", b"gemm_f32_tile", tile)
+            got = M.Dit_block(y, at(c, off), at(x, off), P, B, Tc, Tx, C, C // 64, 2, True, True, discard)
+            torch.cuda.synchronize()
+            assert torch.isfinite(got[1]).all()
+            first = got if first is None else first
+            assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), (tile, off)
+        results.append(first)
+    for a, b in zip(*results):
+        assert float((a - b).norm()) <= 1e-5 * float(b.norm())
+
+
+def test_forward_f32_every_tile_shape():
+    """The row-table epilogue (patch embedding, 63 positions per batch element) in a forward: every tile shape gives equal bits."""
+    from sd3_c_amd.config import reference_dit_test
+    from sd3_c_amd.params import dit_param_shapes
+
+    cfg = reference_dit_test()
+    g = torch.Generator(device="cuda").manual_seed(3)
+    P = {k: 0.05 * torch.randn(s, device="cuda", generator=g) for k, s in dit_param_shapes(cfg).items()}
+    inputs = [torch.randn(s, device="cuda", generator=g) for s in ((2, cfg.pooled_dim), (2, 5, cfg.captions_dim), (2, cfg.in_channels, 14, 18))]
+    first = None
+    for tile in (-1, 0, 1, 2, 3, 4):
+        L.call("sd3_tune", b"gemm_f32_tile", tile)
+        out = M.DiT(*inputs, torch.tensor([3.0, 700.0], device="cuda"), P, cfg.num_layers, cfg.dual_attention_layers, cfg.pooled_dim, cfg.captions_dim, cfg.in_channels,
+                    cfg.emb_dim, cfg.attn_heads, cfg.mlp_expand, cfg.patch_size, cfg.pos_embed_max_size, cfg.base_height, True)
+        assert torch.isfinite(out).all()
+        first = out if first is None else first
+        assert torch.equal(out, first), tile
 
 
 @pytest.mark.parametrize("B,NH,hs,Tq,Tk", [(1, 1, 64, 1, 1), (2, 3, 64, 15, 17), (1, 2, 64, 33, 65), (1, 24, 64, 300, 129), (1, 2, 128, 17, 16),
