@@ -73,7 +73,8 @@ struct Prob {
     void* out;
     int ldc, M, N, K;
     EpiDev epi;
-    bool then;  // ring kernel, EPI_GATE_RESID: the same tile of ProbSet::second follows in the same workgroup
+    bool then;   // ring kernel, EPI_GATE_RESID: the same tile of ProbSet::second follows in the same workgroup
+    bool whole;  // rows are made of aligned groups of four columns, in the output and in what the epilogue reads (whole_rows)
 };
 constexpr int MAX_PROBS = 3;
 struct ProbSet {
@@ -558,7 +559,8 @@ __device__ __forceinline__ void wait_tiles(int ahead) {
     else if (ahead >= MAX) wait_vmcnt<MAX * PER>();
     else wait_tiles<MAX - 1, PER>(ahead);
 }
-template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_F32>
+// WHOLE_ROWS: the epilogue stores (and reads back) four columns at a time, as every problem of the launch allows; else element by element
+template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_F32, bool WHOLE_ROWS>
 __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const ProbSet args) {
     constexpr int NT = WM * WN * 64, TI = TM / WM / 16, WC = TN / WN, NJ = WC / 16;
     constexpr int A_BYTES = TM * 128, STAGE_BYTES = (TM + TN) * 128;
@@ -712,13 +714,19 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     };
     auto epilogue = [&](const Prob& pr) {
         const int n0 = n_blk + wn * WC + NJ * lr;
-        if (n0 >= N) return;  // (N is a multiple of 4)
+        if (n0 >= N) return;
         const EpiDev& epi = pr.epi;
         const int rpb = epi.rows_per_batch;
+        const int valid = N - n0;  // (element by element: columns of this lane's four that exist, if fewer than four)
+        auto four = [&](const float* p) {
+            if (WHOLE_ROWS) return *reinterpret_cast<const float4*>(p);
+            return make_float4(p[0], valid > 1 ? p[1] : 0.f, valid > 2 ? p[2] : 0.f, valid > 3 ? p[3] : 0.f);
+        };
         float bias4[4] = {0.f, 0.f, 0.f, 0.f};
         if (epi.bias)
 #pragma unroll
-            for (int c = 0; c < 4; c++) bias4[c] = epi.bias[n0 + c];
+            for (int c = 0; c < 4; c++)
+                if (WHOLE_ROWS || c < valid) bias4[c] = epi.bias[n0 + c];
         float4 norm_w = make_float4(1.f, 1.f, 1.f, 1.f);
         const int third = EPI == EPI_QKV_NORM ? n0 / epi.gate_ld : 0;
         if (EPI == EPI_QKV_NORM && third < 2) norm_w = *reinterpret_cast<const float4*>((third == 0 ? epi.gate : epi.resid) + (n0 & 63));
@@ -739,23 +747,34 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
 #pragma unroll
                     for (int c = 0; c < 4; c++) v[c] = v[c] / (1.0f + __expf(-v[c]));
                 } else if (EPI == EPI_GATE_RESID) {
-                    const float4 g4 = *reinterpret_cast<const float4*>(epi.gate + (long long)(m / rpb) * epi.gate_ld + n0);
-                    const float4 r4 = *reinterpret_cast<const float4*>(epi.resid + idx);
+                    const float4 g4 = four(epi.gate + (long long)(m / rpb) * epi.gate_ld + n0);
+                    const float4 r4 = four(epi.resid + idx);
                     v[0] = fmaf(g4.x, v[0], r4.x); v[1] = fmaf(g4.y, v[1], r4.y); v[2] = fmaf(g4.z, v[2], r4.z); v[3] = fmaf(g4.w, v[3], r4.w);
                 } else if (EPI == EPI_BIAS_ROWADD) {
-                    const float4 t4 = *reinterpret_cast<const float4*>(epi.table + (long long)(m % rpb) * epi.gate_ld + n0);
+                    const float4 t4 = four(epi.table + (long long)(m % rpb) * epi.gate_ld + n0);
                     v[0] += t4.x; v[1] += t4.y; v[2] += t4.z; v[3] += t4.w;
                 } else if (EPI == EPI_QKV_NORM && third < 2) {
                     qk_norm4(v, norm_w);
                 }
-                if (OUT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(pr.out) + idx) = make_float4(v[0], v[1], v[2], v[3]);
-                else *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(pr.out) + idx) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                float* const of = reinterpret_cast<float*>(pr.out) + idx;
+                bf16_t* const oh = reinterpret_cast<bf16_t*>(pr.out) + idx;
+                if (WHOLE_ROWS) {
+                    if (OUT_F32) *reinterpret_cast<float4*>(of) = make_float4(v[0], v[1], v[2], v[3]);
+                    else *reinterpret_cast<uint2*>(oh) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        if (c < valid) {
+                            if (OUT_F32) of[c] = v[c];
+                            else oh[c] = f32_to_bf16(v[c]);
+                        }
+                }
             }
     };
 
     fill_ring();
     k_loop();
-    constexpr bool PAIR = EPI == EPI_GATE_RESID && TM * TN <= 64 * 128;  // (see grouped_impl)
+    constexpr bool PAIR = WHOLE_ROWS && EPI == EPI_GATE_RESID && TM * TN <= 64 * 128;  // (see grouped_impl)
     if (PAIR && pr.then) {
         // The second layer of the same rows and columns (the two out-projections of a block with dual attention): its ring is filled behind
         // the last LDS reads of the first and lands while the first one's results are on their way out; a thread reads back what it wrote.
@@ -776,9 +795,9 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     epilogue(pr);
 }
 
-template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_F32>
+template <int TM, int TN, int WM, int WN, int STAGES, int MW, int EPI, bool OUT_F32, bool WHOLE_ROWS = true>
 int launch_ring(ProbSet& args, int n, hipStream_t st) {
-    auto kern = gemm_bf16_ring_kernel<TM, TN, WM, WN, STAGES, MW, EPI, OUT_F32>;
+    auto kern = gemm_bf16_ring_kernel<TM, TN, WM, WN, STAGES, MW, EPI, OUT_F32, WHOLE_ROWS>;
     constexpr int smem = STAGES * (TM + TN) * 128;
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
@@ -826,10 +845,24 @@ double launch_cost(const ProbSet& set, int n, int shape, int cus) {
     const double again = rounds == 1 ? 1.0 : shape == TILE_128_256 ? 1.25 : shape == TILE_192_256 ? 1.06 : 1.0;
     return again * (double)rounds * (t.fixed + t.per_k * ((double)depth / tiles));
 }
+// Rows that are not made of aligned groups of four columns go element by element. Of the ring kernel three shapes are built for them: with
+// 256x256 tiles alone 333 x 1541 x 1536 took, gated, 69.7 us instead of 9.5 (1536 columns: 7.7), 4250 rows, plain, 41.9 instead of 28.3,
+// and as a run-time branch in every shape the form cost the other rows 0.3 us a launch (the compiler merges parts of the two).
+bool all_whole(const ProbSet& set, int n) {
+    for (int i = 0; i < n; i++)
+        if (!set.p[i].whole) return false;
+    return true;
+}
+bool shape_takes(int shape, bool whole) {
+    return whole || shape == TILE_64 || shape == TILE_128 || shape == TILE_256_128 || shape == TILE_192_256 || shape == TILE_256;
+}
+
 int cheapest_shape(const ProbSet& set, int n, int cus, double& cost) {
+    const bool whole = all_whole(set, n);
     int best = TILE_256;
     cost = launch_cost(set, n, TILE_256, cus);
     for (int s = TILE_256 - 1; s >= 0; s--) {
+        if (!shape_takes(s, whole)) continue;
         const double c = launch_cost(set, n, s, cus);
         if (c < cost) {
             best = s;
@@ -847,6 +880,12 @@ int launch_shape(int shape, ProbSet& args, int n, int cus, hipStream_t st) {
     long long tiles = 0;
     for (int i = 0; i < n; i++) tiles += tiles_of(args.p[i], shape);
     const bool one_round = tiles <= cus;
+    if (!all_whole(args, n)) {
+        if (shape == TILE_64) return launch_ring<64, 64, 4, 1, 5, 2, EPI, OUT_F32, false>(args, n, st);
+        if (shape == TILE_128) return launch_ring<128, 128, 4, 2, 4, 2, EPI, OUT_F32, false>(args, n, st);
+        if (shape == TILE_256_128) return launch_ring<256, 128, 4, 2, 3, 2, EPI, OUT_F32, false>(args, n, st);
+        if (!shape_takes(shape, false)) shape = TILE_256;
+    }
     switch (shape) {
         case TILE_64: return launch_ring<64, 64, 4, 1, 5, 2, EPI, OUT_F32>(args, n, st);
         case TILE_128_64:
@@ -876,7 +915,8 @@ static int forced_shape(int tile) {
         if (tile == tile_shapes[s].tm * 1000 + tile_shapes[s].tn) return s;
     return -1;
 }
-static bool ring_can(const Prob& q, int epi) {
+// whether rows are made of aligned groups of four columns, in the output and in what the epilogue reads
+static bool whole_rows(const Prob& q, int epi) {
     auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     if (q.N % 4 || q.ldc % 4 || !al(q.out)) return false;
     if (epi == EPI_GATE_RESID) return al(q.epi.gate) && al(q.epi.resid) && q.epi.gate_ld % 4 == 0;
@@ -952,6 +992,7 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
                 return fail(SD3_ERR_INVALID_ARG, "gemm_bf16: the fused qk-norm needs N = 3C with C a multiple of 64 and two aligned weight vectors");
             d.epi.gate_ld = q.N / 3;
         }
+        d.whole = whole_rows(d, epi);
         return SD3_OK;
     };
     for (int i = 0; i < n; i++) {
@@ -982,21 +1023,18 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         }
 #undef SD3_GEMM_BF16_LAUNCH
     };
-    // the ring kernel stores four columns at a time; rows that are not made of such chunks take the 256x256 tiles
-    bool whole_chunks = true;
-    for (int i = 0; i < m; i++) whole_chunks = whole_chunks && ring_can(args.p[i], epi);
     if (then) {
         // Both layers in one launch where they are one round of small tiles, i.e. a launch's start and end are a good part of it: dual blocks
         // of 256 + 77, 1024 + 154 tokens 106.7 -> 105.3 us, forwards 2972 -> 2951, 4708 -> 4681 us. From 128x128 tiles on the second layer
         // does better in a launch (and tiles) of its own: 2048 + 308, 1581 + 999, 8192 + 308 rows, forwards 0.1, 0.6, 1 % slower together.
         constexpr double GAP = 2.0;  // between two launches, us
         SD3_TRY(fill(*then, args.second));
-        const bool can = whole_chunks && ring_can(args.second, epi);
+        const bool whole = all_whole(args, m) && args.second.whole;
         int pair = -1;
         if (g_gemm_bf16_tile) {
-            pair = can ? forced_shape(g_gemm_bf16_tile) : -1;  // (256x192 tiles, 192, have no shape of the table: two launches)
+            if (whole) pair = forced_shape(g_gemm_bf16_tile);  // (256x192 tiles, 192, have no shape of the table: two launches)
             if (pair > TILE_64_128) pair = -1;
-        } else if (can) {
+        } else if (whole) {
             ProbSet second{};
             second.p[0] = args.second;
             double best, after;
@@ -1039,7 +1077,6 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         }
 #undef SD3_GEMM_BF16_192
     }
-    if (!whole_chunks) return launch(args, m, TILE_256);
     if (g_gemm_bf16_tile) return launch(args, m, forced_shape(g_gemm_bf16_tile));
     // One launch with the cheapest shape, or two: the many-row problems apart from the few-row ones (a launch of its own costs LAUNCH), or
     // full rounds of 256x256 tiles first and the last rows of the last many-row problem with the few-row problems behind them. The

@@ -47,3 +47,33 @@ def test_block_without_qk_norm_on_every_tile(B, Tc, Tx, C, discard):
             assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), tile
     finally:
         L.call("sd3_gemm_bf16_force_tile", 0)
+
+
+@pytest.mark.parametrize("B,Tc,Tx,C", [(1, 3, 63, 320), (2, 5, 129, 128)])
+def test_streams_that_are_not_16_byte_aligned(B, Tc, Tx, C):
+    """Streams that begin one float after a 16-byte boundary: outputs and residuals go element by element, on every tile with equal bits, and
+    differ from the aligned ones by no more than bf16 rounding (their LayerNorm sums in another order)."""
+    g = torch.Generator(device="cuda").manual_seed(Tx)
+    P = {k: 0.1 * torch.randn(s, device="cuda", generator=g) for k, s in block_param_shapes(C, 2, True, True, False, 64).items()}
+    y, c, x = (torch.randn(s, device="cuda", generator=g) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
+
+    def at(t, off):
+        buf = torch.empty(t.numel() + 4, device="cuda")
+        return buf[off:off + t.numel()].view(t.shape).copy_(t)
+
+    def block(off):
+        got = M.Dit_block(y, at(c, off), at(x, off), P, B, Tc, Tx, C, C // 64, 2, True, True, False, precision="bf16")
+        torch.cuda.synchronize()
+        return got
+
+    aligned, first = block(0), None
+    try:
+        for tile in (256, 64064, 128064, 64128, 128, 256128, 128256, 192256, 0):
+            L.call("sd3_gemm_bf16_force_tile", tile)
+            got = block(1)
+            first = got if first is None else first
+            assert torch.equal(got[0], first[0]) and torch.equal(got[1], first[1]), tile
+    finally:
+        L.call("sd3_gemm_bf16_force_tile", 0)
+    for a, b in zip(first, aligned):
+        assert float((a - b).norm()) <= 2.0 ** -8 * float(b.norm())
