@@ -767,64 +767,247 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
 }
 
 // ---- short sequences ----
-// Used up to SHORT_KEYS keys, whatever the batch (a batch element's result stays what it is alone): 24 heads, 333 tokens, batch 1 / 2 / 4 / 8:
-// 13.9 / 14.3 / 14.8 / 20.8 -> 8.1 / 11.2 / 17.0 / 26.4 us (every workgroup reads all keys for 32 queries, so many of them are bound by
-// the loads); 730 tokens, batch 1 / 4: 19.3 / 30.5 -> 16.4 / 41 us.
-// The kernel above gives a workgroup 256 queries and runs through all keys tile by tile behind a barrier each: at 333 tokens that is 48
-// workgroups with a serial chain of six tiles, at 1178 tokens 240 with nineteen. Here a workgroup has 32 queries and its KS wavefronts
-// split the KEYS (tile t of 32 keys goes to wavefront t % KS), each with its own K rows in registers (straight from memory: a K row chunk
-// of 8 values is the matrix operand as it lies) and its own V tile in LDS, so that there is no barrier before the merge at the end.
+// Up to SHORT_KEYS keys, whatever the batch (a batch element's result stays what it is alone). The kernel above gives a workgroup 256 queries
+// and runs through all keys tile by tile behind a barrier each: at 333 tokens and 24 heads that is 48 workgroups with a serial chain of
+// six tiles. Here a wavefront has 32 queries and the tiles of 32 keys are RUNS runs (run r has the tiles r, r + RUNS, ...), each with a softmax
+// state of its own, merged in their order. What is left is a choice of who takes the runs:
+//  * few queries: the wavefronts of a workgroup share 32 queries and take a run each (flash_attn_bf16_split_kernel);
+//  * many: a wavefront takes all runs of 32 queries of its own, one behind the other, and the workgroup shares the tiles
+//    (flash_attn_bf16_runs_kernel): a quarter of the loads, and the queries scaled, the states merged and the results stored once.
+// Both round alike, so the results do not depend on the choice. It is the first kernel as long as its workgroups are resident at once, three
+// per compute unit. 24 heads, us, kernel above | split | runs:
+//   141 tokens, batch  4, 6, 8, 16:            10.6 10.7 10.9 14.6           |  7.2  8.7 12.5 18.3           |  8.7 10.7 10.8 13.4
+//   333 tokens, batch  1, 2, 3, 4, 8, 16, 32:  14.1 14.2 14.3 14.5 20.1 32 58 | 7.6 10.1 13.7 15.9 25.8 47 88 | 11.9 12.0 12.2 14.6 18.1 29 47
+//   410 tokens, batch  1, 2, 3, 4, 8, 16, 24:  14.7 15.1 15.1 15.5 22.2 35 54 | 9.0 11.8 15.7 18.2 33.7 60 88 | 12.8 13.1 15.9 16.2 20.6 37 51
+//   730 tokens, batch  1, 4:                   19.3 30.5                     | 16.4 41
+// (the split alone for every batch was the first form of this: 8.2, 10.6, 14.4, 16.6, 26.2, 48 us for 333 tokens, batch 1, 2, 3, 4, 8, 16). Both
+// are bound by the issue of instructions (333 tokens, batch 16, runs: the vector unit of a SIMD works 14.6 of 27 us, the matrix unit 5.3;
+// twice the queries per workgroup in the split kernel, i.e. half its loads, changed nothing).
 // v_mfma_f32_16x16x32_bf16 throughout. S^T = K Q^T leaves lane l with query l%16 and keys 4g + r of a 16-key block, g = l/16: the two
 // blocks of a tile are, packed, the P^T operand with k slots {4g .. 4g+3, 16+4g .. 16+4g+3}; the transposing LDS reads fetch V^T in the
 // same slots. Softmax as above: a reference that is subtracted on the matrix unit and moved only when a row sum says so.
 constexpr int SHORT_KEYS = 416;
-template <int QB, int KS>
-__global__ void __launch_bounds__(KS * 64, 2) flash_attn_bf16_split_kernel(const AttnSets sets, float q_scale) {
-    constexpr int TKEYS = 32, V_TILE = TKEYS * 128;
-    constexpr int PITCH = 16 * QB + 2 * QB;  // floats per lane in the merge buffer
-    constexpr int V_SPACE = KS * 2 * V_TILE, MERGE = (KS / 2) * 64 * PITCH * 4;
-    __shared__ __attribute__((aligned(1024))) char smem[V_SPACE > MERGE ? V_SPACE : MERGE];
-    if (blockIdx.x >= (unsigned)sets.end[MAX_SETS - 1]) {
-        read_ahead<KS * 64>(sets.ahead, blockIdx.x - sets.end[MAX_SETS - 1], gridDim.x - sets.end[MAX_SETS - 1]);
-        return;
-    }
-    const int which = (blockIdx.x >= (unsigned)sets.end[0]) + (blockIdx.x >= (unsigned)sets.end[1]);
-    const SegDev& s = sets.set[which];
-    const int wg_first = which ? sets.end[which - 1] : 0;
-    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int b, h, q0;
-    {
-        const int total = sets.end[which] - wg_first, wg = blockIdx.x - wg_first, xcd = wg % 8, local = wg / 8;
-        const int per = (total + 7) / 8, tall = (total % 8) ? (total % 8) : 8;
-        const int item = (xcd < tall) ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
-        const int bh = item / s.nqb;
-        q0 = (item % s.nqb) * (16 * QB);
-        b = bh / s.NH;
-        h = bh % s.NH;
-    }
-    const int T0 = s.T[0], T1 = s.T[1], Tq0 = s.Tq[0], TQ = s.Tq[0] + s.Tq[1];
-    Frag q[QB][2];
+constexpr int RUNS = 4;               // runs of key tiles: run r has the tiles r, r + RUNS, ...
+constexpr int SQB = 2, SQ = 16 * SQB;  // 16-query blocks and queries of a wavefront
+constexpr int STK = 32;               // keys of a tile
+
+struct ShortState {  // what a wavefront has accumulated over one or several runs
+    f32x4_t o[4][SQB];
+    f32x4_t nm[SQB];       // the negative of the reference, four times (what the scores' accumulators start from)
+    float l[SQB];          // the sum over the keys of this lane
+    __device__ __forceinline__ void refer(int i, float m) { nm[i] = f32x4_t{-m, -m, -m, -m}; }
+    __device__ __forceinline__ float m(int i) const { return -nm[i][0]; }
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int i = 0; i < QB; i++) {
-        const int qt = min(q0 + 16 * i + lr, TQ - 1), seg = qt < Tq0 ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
-        const bf16_t* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_qkv[seg] + h * HS + 8 * lg;
+        for (int i = 0; i < SQB; i++) {
+            refer(i, 0.f);
+            l[i] = 0.f;
+#pragma unroll
+            for (int d = 0; d < 4; d++) o[d][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    __device__ __forceinline__ void weightless() {  // (no tile in the run)
+#pragma unroll
+        for (int i = 0; i < SQB; i++) refer(i, -1e30f);
+    }
+};
+// The state over the keys of two runs, (m, l, o) and (m2, l2, o2), taking the place of the first: which is which is part of the result, and runs
+// are merged in their order. Explicit fused multiply-adds, so that both kernels below round alike.
+__device__ __forceinline__ void short_weights(float& m, float m2, float& w, float& w2) {
+    const float mx = fmaxf(m, m2);
+    w = __builtin_amdgcn_exp2f(m - mx);
+    w2 = __builtin_amdgcn_exp2f(m2 - mx);
+    m = mx;
+}
+__device__ __forceinline__ float short_add(float a, float w, float b, float w2) { return fmaf(a, w, b * w2); }
+
+// queries q0 .. of one (batch, head) as matrix operands: requested, then scaled
+__device__ __forceinline__ void short_request_queries(const SegDev& s, int b, int h, int q0, Frag (&q)[SQB][2]) {
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4, TQ = s.Tq[0] + s.Tq[1];
+#pragma unroll
+    for (int i = 0; i < SQB; i++) {
+        const int qt = min(q0 + 16 * i + lr, TQ - 1), seg = qt < s.Tq[0] ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
+        const bf16_t* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - s.Tq[0] : qt)) * s.ld_qkv[seg] + h * HS + 8 * lg;
 #pragma unroll
         for (int st = 0; st < 2; st++) q[i][st].u = *reinterpret_cast<const uint4*>(p + 32 * st);
     }
-    f32x4_t o[4][QB];
-    float m_run[QB], l_run[QB];  // l_run: over the keys of this lane
+}
+__device__ __forceinline__ void short_scale_queries(float q_scale, Frag (&q)[SQB][2]) {
 #pragma unroll
-    for (int i = 0; i < QB; i++) {
-        m_run[i] = 0.f;
-        l_run[i] = 0.f;
+    for (int i = 0; i < SQB; i++)
 #pragma unroll
-        for (int d = 0; d < 4; d++) o[d][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
+        for (int st = 0; st < 2; st++) {
+            float f[8];
+            unpack8(q[i][st].u, f);
+#pragma unroll
+            for (int e = 0; e < 8; e++) f[e] *= q_scale;
+            q[i][st].u = pack8(f);
+        }
+}
+// scores of a tile relative to the references
+__device__ __forceinline__ void short_scores(const Frag (&k)[2][2], const Frag (&q)[SQB][2], const ShortState& z, f32x4_t (&sc)[2][SQB]) {
+#pragma unroll
+    for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+        for (int i = 0; i < SQB; i++)
+            sc[kb16][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kb16][0].v, q[i][0].v, z.nm[i], 0, 0, 0);
+#pragma unroll
+    for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+        for (int i = 0; i < SQB; i++) sc[kb16][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kb16][1].v, q[i][1].v, sc[kb16][i], 0, 0, 0);
+}
+// the largest of the four values of lanes l, l ^ 16, l ^ 32, l ^ 48 (row and half swaps, no trip through LDS)
+__device__ __forceinline__ float max_of_rows(float v) {
+    const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
+    const auto r32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r32[0]), __uint_as_float(r32[1]));
+}
+// Probabilities of a tile with `keys` keys from its scores. The first tile of a run sets the reference to the maximum of its scores (a
+// reference of 0 would do for scores of ordinary size and save 6 % of the time, but a largest probability of 1 needs no rounding: error
+// against 64 bits, 333 tokens, 2.78e-3, with 0 2.87e-3); later the reference of 16 queries goes to their running maximum whenever a lane's sum over a
+// tile exceeds L_BOUND (decided for each 16 queries: their results do not depend on the wavefront's others).
+__device__ __forceinline__ void short_probs(f32x4_t (&sc)[2][SQB], int keys, bool first, ShortState& z, Frag (&p)[SQB]) {
     constexpr float L_BOUND = 1073741824.0f;  // 2^30
+    const int lg = (threadIdx.x & 63) >> 4;
+    if (keys < STK) {
+#pragma unroll
+        for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (16 * kb16 + 4 * lg + r >= keys)
+#pragma unroll
+                    for (int i = 0; i < SQB; i++) sc[kb16][i][r] = -1e30f;
+    }
+    auto largest = [&](int i) {
+        return max_of_rows(fmaxf(fmaxf(fmaxf(sc[0][i][0], sc[0][i][1]), fmaxf(sc[0][i][2], sc[0][i][3])),
+                                 fmaxf(fmaxf(sc[1][i][0], sc[1][i][1]), fmaxf(sc[1][i][2], sc[1][i][3]))));
+    };
+    auto raise = [&](int i, float by) {
+        z.refer(i, z.m(i) + by);
+#pragma unroll
+        for (int kb16 = 0; kb16 < 2; kb16++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) sc[kb16][i][r] -= by;
+    };
+    if (first) {
+        float mx[SQB];
+#pragma unroll
+        for (int i = 0; i < SQB; i++) mx[i] = largest(i);
+#pragma unroll
+        for (int i = 0; i < SQB; i++) raise(i, mx[i]);
+    }
+    float inc[SQB];
+    uint64_t move[SQB], any = 0;  // one bit per lane
+    auto probs = [&](int i) {
+        float f[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] = __builtin_amdgcn_exp2f(sc[e >> 2][i][e & 3]);
+        inc[i] = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
+        p[i].u = pack8(f);
+    };
+#pragma unroll
+    for (int i = 0; i < SQB; i++) {
+        probs(i);
+        move[i] = __builtin_amdgcn_ballot_w64(!(inc[i] <= L_BOUND));
+        any |= move[i];
+    }
+    if (any) {
+#pragma unroll
+        for (int i = 0; i < SQB; i++) {
+            if (!move[i]) continue;
+            const float mx = fmaxf(largest(i), 0.f), alpha = __builtin_amdgcn_exp2f(-mx);
+            z.l[i] *= alpha;
+#pragma unroll
+            for (int d = 0; d < 4; d++) z.o[d][i] *= alpha;
+            raise(i, mx);
+            probs(i);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < SQB; i++) z.l[i] += inc[i];
+}
+__device__ __forceinline__ void short_add_values(uint2 (&vf)[4][2], const Frag (&p)[SQB], ShortState& z) {
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(vf[0][0]), "+v"(vf[0][1]), "+v"(vf[1][0]), "+v"(vf[1][1]), "+v"(vf[2][0]), "+v"(vf[2][1]), "+v"(vf[3][0]), "+v"(vf[3][1]));
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        Frag vv;
+        vv.u = make_uint4(vf[d][0].x, vf[d][0].y, vf[d][1].x, vf[d][1].y);
+#pragma unroll
+        for (int i = 0; i < SQB; i++) z.o[d][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv.v, p[i].v, z.o[d][i], 0, 0, 0);
+    }
+}
+// V tiles in LDS: rows of 128 bytes, chunk c of row r at position c ^ v_chunk_key(r) (chunk pairs of rows of one parity land in different
+// bank groups). The transposing reads of d block d: at[d] for the first 16 keys, 2048 bytes on for the others (the key is the same there).
+__device__ __forceinline__ int v_chunk_key(int row) { return 2 * ((row >> 1) & 3); }
+struct ShortVReads {
+    uint32_t at[4];
+    __device__ __forceinline__ explicit ShortVReads(uint32_t base) {
+        const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4, row = 4 * lg + (lr >> 2);
+#pragma unroll
+        for (int d = 0; d < 4; d++) at[d] = base + row * 128 + 8 * (lr & 1) + (((2 * d + ((lr & 3) >> 1)) ^ v_chunk_key(row)) * 16);
+    }
+    __device__ __forceinline__ void read(uint32_t offset, uint2 (&vf)[4][2]) const {
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            const uint32_t a = at[d] + offset;
+            vf[d][0] = lds_read_tr16_b64(a, 0);
+            vf[d][1] = lds_read_tr16_b64(a, 16 * 128);
+        }
+    }
+};
+// the sum over all keys of a query from the lanes' shares
+__device__ __forceinline__ float short_total(float l) {
+    l += __shfl_xor(l, 16, 64);
+    return l + __shfl_xor(l, 32, 64);
+}
+// where query 16 i + lane % 16 of the block goes, this lane's four values of d block 0 (null: nowhere)
+__device__ __forceinline__ bf16_t* short_out(const SegDev& s, int b, int h, int q0, int i) {
+    const int lane = threadIdx.x & 63, qt = q0 + 16 * i + (lane & 15), seg = qt < s.Tq[0] ? 0 : 1;
+    if (qt >= s.Tq[0] + s.Tq[1] || !s.out[seg]) return nullptr;
+    return s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - s.Tq[0] : qt)) * s.ld_out[seg] + h * HS + 4 * (lane >> 4);
+}
+__device__ __forceinline__ void short_store4(bf16_t* p, const f32x4_t& o, float inv) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(o[0] * inv, o[1] * inv), pack_bf16x2(o[2] * inv, o[3] * inv));
+}
+// work item of a workgroup: (batch, head, query block) in an order that keeps the query blocks of a head on one XCD
+__device__ __forceinline__ const SegDev& short_item(const AttnSets& sets, int& b, int& h, int& block) {
+    const int which = (blockIdx.x >= (unsigned)sets.end[0]) + (blockIdx.x >= (unsigned)sets.end[1]);
+    const SegDev& s = sets.set[which];
+    const int wg_first = which ? sets.end[which - 1] : 0;
+    const int total = sets.end[which] - wg_first, wg = blockIdx.x - wg_first, xcd = wg % 8, local = wg / 8;
+    const int per = (total + 7) / 8, tall = (total % 8) ? (total % 8) : 8;
+    const int item = (xcd < tall) ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+    const int bh = item / s.nqb;
+    block = item % s.nqb;
+    b = bh / s.NH;
+    h = bh % s.NH;
+    return s;
+}
+
+// The wavefronts of a workgroup share its 32 queries and take a run each, with its K rows in registers (straight from memory: a K row chunk
+// of 8 values is the matrix operand as it lies) and V tiles in LDS of their own, so that there is no barrier before the merge.
+__global__ void __launch_bounds__(RUNS * 64, 2) flash_attn_bf16_split_kernel(const AttnSets sets, float q_scale) {
+    constexpr int V_TILE = STK * 128;
+    constexpr int VALUES = 18 * SQB;  // of a lane's state
+    constexpr int V_SPACE = RUNS * 2 * V_TILE, MERGE = RUNS * 64 * VALUES * 4;
+    __shared__ __attribute__((aligned(1024))) char smem[V_SPACE > MERGE ? V_SPACE : MERGE];
+    if (blockIdx.x >= (unsigned)sets.end[MAX_SETS - 1]) {
+        read_ahead<RUNS * 64>(sets.ahead, blockIdx.x - sets.end[MAX_SETS - 1], gridDim.x - sets.end[MAX_SETS - 1]);
+        return;
+    }
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int b, h, q0;
+    const SegDev& s = short_item(sets, b, h, q0);
+    q0 *= SQ;
+    const int T0 = s.T[0], T1 = s.T[1];
+    Frag q[SQB][2];
+    short_request_queries(s, b, h, q0, q);
 
     // key tiles are counted segment by segment, so that a tile's rows have one scalar base and 32-bit offsets
-    const int nt0 = (T0 + TKEYS - 1) / TKEYS, n_t = nt0 + (T1 + TKEYS - 1) / TKEYS;
+    const int nt0 = (T0 + STK - 1) / STK, n_t = nt0 + (T1 + STK - 1) / STK;
     const int ld0 = s.ld_qkv[0], ld1 = s.ld_qkv[1];
     const bf16_t* k0 = s.k[0] + (long long)b * T0 * ld0 + h * HS;
     const bf16_t* k1 = s.k[1] + (long long)b * T1 * ld1 + h * HS;
@@ -836,13 +1019,13 @@ __global__ void __launch_bounds__(KS * 64, 2) flash_attn_bf16_split_kernel(const
     int at_seg = -1, at_last = -1;
     // V first, then K: loads return in order, so whoever has waited for a tile's K rows finds its V tile in LDS
     auto load_tile = [&](int t, int stage) {
-        const int seg = t < nt0 ? 0 : 1, t0 = (seg ? t - nt0 : t) * TKEYS, last = min((seg ? T1 : T0) - t0, TKEYS) - 1, ld = seg ? ld1 : ld0;
+        const int seg = t < nt0 ? 0 : 1, t0 = (seg ? t - nt0 : t) * STK, last = min((seg ? T1 : T0) - t0, STK) - 1, ld = seg ? ld1 : ld0;
         if (seg != at_seg || last != at_last) {
             at_seg = seg;
             at_last = last;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {  // rows 8i .. 8i+7; chunk pairs of rows of one parity land in different bank groups
-                const int row = 8 * i + (lane >> 3), chunk = (lane & 7) ^ (2 * ((row >> 1) & 3));
+            for (int i = 0; i < 4; i++) {  // rows 8i .. 8i+7
+                const int row = 8 * i + (lane >> 3), chunk = (lane & 7) ^ v_chunk_key(row);
                 v_at[i] = __umul24(min(row, last), ld) + chunk * 8;
             }
 #pragma unroll
@@ -859,159 +1042,197 @@ __global__ void __launch_bounds__(KS * 64, 2) flash_attn_bf16_split_kernel(const
             for (int st = 0; st < 2; st++) k[kb16][st].u = *reinterpret_cast<const uint4*>(kb + k_at[kb16] + 32 * st);
         return last + 1;
     };
-    const uint32_t v_addr = (uint32_t)(uintptr_t)(lds_ptr_t)v_lds;
-    uint32_t v_off[2];  // transposing reads: key half hb, d block 0 (d block db: the chunk pair 2 db, xor-ed in)
-    int v_key[2];
-#pragma unroll
-    for (int hb = 0; hb < 2; hb++) {
-        const int row = 16 * hb + 4 * lg + (lr >> 2);
-        v_key[hb] = 2 * ((row >> 1) & 3);
-        v_off[hb] = row * 128 + 8 * (lr & 1);
-    }
-    const int v_chunk = (lr & 3) >> 1;
+    const ShortVReads v_reads((uint32_t)(uintptr_t)(lds_ptr_t)v_lds);
 
+    ShortState z;
+    z.clear();
     int t = wave, left = 0;
-    bool first = true;
     if (t < n_t) left = load_tile(t, 0);
     __builtin_amdgcn_sched_barrier(0);  // (the first tile is on its way before the wait for the queries)
-#pragma unroll
-    for (int i = 0; i < QB; i++)
-#pragma unroll
-        for (int st = 0; st < 2; st++) {
-            float f[8];
-            unpack8(q[i][st].u, f);
-#pragma unroll
-            for (int e = 0; e < 8; e++) f[e] *= q_scale;
-            q[i][st].u = pack8(f);
-        }
-    for (int stage = 0; t < n_t; t += KS, stage ^= 1) {
-        // scores relative to the reference m_run (the accumulators start from its negative)
-        f32x4_t sc[2][QB];
-#pragma unroll
-        for (int kb16 = 0; kb16 < 2; kb16++)
-#pragma unroll
-            for (int i = 0; i < QB; i++)
-                sc[kb16][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kb16][0].v, q[i][0].v, f32x4_t{-m_run[i], -m_run[i], -m_run[i], -m_run[i]}, 0, 0, 0);
-#pragma unroll
-        for (int kb16 = 0; kb16 < 2; kb16++)
-#pragma unroll
-            for (int i = 0; i < QB; i++) sc[kb16][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[kb16][1].v, q[i][1].v, sc[kb16][i], 0, 0, 0);
+    short_scale_queries(q_scale, q);
+    for (int stage = 0; t < n_t; t += RUNS, stage ^= 1) {
+        f32x4_t sc[2][SQB];
+        short_scores(k, q, z, sc);
         // V^T of this tile (its loads came before the K rows just used), then the requests for the next tile
         __builtin_amdgcn_sched_barrier(0);
         uint2 vf[4][2];
+        v_reads.read(stage * V_TILE, vf);
+        const int keys = left;
+        if (t + RUNS < n_t) left = load_tile(t + RUNS, stage ^ 1);
+        Frag p[SQB];
+        short_probs(sc, keys, t < RUNS, z, p);
+        short_add_values(vf, p, z);
+    }
+    if (wave >= n_t) z.weightless();
+    // All states go to LDS (the V tiles are free behind the barrier), and wavefront w merges d block w of them, in the order of the runs.
+    float* const states = reinterpret_cast<float*>(smem);
+    auto at = [&](int run, int v) -> float& { return states[(run * VALUES + v) * 64 + lane]; };
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < SQB; i++) {
+        at(wave, 2 * i) = z.m(i);
+        at(wave, 2 * i + 1) = z.l[i];
 #pragma unroll
         for (int d = 0; d < 4; d++)
 #pragma unroll
-            for (int hb = 0; hb < 2; hb++)
-                vf[d][hb] = lds_read_tr16_b64(v_addr + stage * V_TILE + v_off[hb] + (((2 * d + v_chunk) ^ v_key[hb]) * 16), 0);
-        const int cur = left;
-        if (t + KS < n_t) left = load_tile(t + KS, stage ^ 1);
-        if (cur < TKEYS) {
+            for (int r = 0; r < 4; r++) at(wave, 2 * SQB + (d * SQB + i) * 4 + r) = z.o[d][i][r];
+    }
+    __syncthreads();
+    static_assert(RUNS == 4, "a d block of 16 values for each wavefront");
+#pragma unroll
+    for (int i = 0; i < SQB; i++) {
+        float m = at(0, 2 * i), l = at(0, 2 * i + 1);
+        f32x4_t o;
+#pragma unroll
+        for (int r = 0; r < 4; r++) o[r] = at(0, 2 * SQB + (wave * SQB + i) * 4 + r);
+#pragma unroll
+        for (int run = 1; run < RUNS; run++) {
+            float w, w2;
+            short_weights(m, at(run, 2 * i), w, w2);
+            l = short_add(l, w, at(run, 2 * i + 1), w2);
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[r] = short_add(o[r], w, at(run, 2 * SQB + (wave * SQB + i) * 4 + r), w2);
+        }
+        const float inv = 1.0f / short_total(l);
+        bf16_t* const to = short_out(s, b, h, q0, i);
+        if (to) short_store4(to + 16 * wave, o, inv);
+    }
+}
+
+// Every wavefront has 32 queries of its own and takes all runs. A tile is loaded once for the workgroup, straight into a ring of LDS stages,
+// RING - 1 tiles ahead, by one wavefront in turn (each a quarter of every tile: 333 tokens, batch 8, 3 % slower), with one barrier per tile.
+// Not better: three wavefronts per workgroup; wavefronts without queries that end at once and leave the loads to the others.
+constexpr int RING = 4;
+constexpr int WAVES = 4;
+__global__ void __launch_bounds__(WAVES * 64, 3) flash_attn_bf16_runs_kernel(const AttnSets sets, float q_scale) {
+    constexpr int TILE = STK * 128, STAGE = 2 * TILE;  // K rows, then V rows
+    __shared__ __attribute__((aligned(1024))) char smem[RING * STAGE];
+    if (blockIdx.x >= (unsigned)sets.end[MAX_SETS - 1]) {
+        read_ahead<WAVES * 64>(sets.ahead, blockIdx.x - sets.end[MAX_SETS - 1], gridDim.x - sets.end[MAX_SETS - 1]);
+        return;
+    }
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int b, h, q0;
+    const SegDev& s = short_item(sets, b, h, q0);
+    q0 = (q0 * WAVES + wave) * SQ;
+    const int T0 = s.T[0], T1 = s.T[1];
+    const int nt0 = (T0 + STK - 1) / STK, n_t = nt0 + (T1 + STK - 1) / STK;
+    const int ld0 = s.ld_qkv[0], ld1 = s.ld_qkv[1];
+    const bf16_t* k0 = s.k[0] + (long long)b * T0 * ld0 + h * HS;
+    const bf16_t* k1 = s.k[1] + (long long)b * T1 * ld1 + h * HS;
+    const bf16_t* v0 = s.v[0] + (long long)b * T0 * ld0 + h * HS;
+    const bf16_t* v1 = s.v[1] + (long long)b * T1 * ld1 + h * HS;
+    auto keys_of = [&](int t) { return t < nt0 ? T0 - t * STK : T1 - (t - nt0) * STK; };  // (STK or more: a whole tile)
+    // Wavefront w requests the tiles at the positions w, w + WAVES, ... of their order, whole. A lane has row 8i + lane / 8, and there a chunk of
+    // 16 bytes; the chunks are exchanged in K as the GEMM's 16x16x32 operands are, which is the exchange of V here too.
+    static_assert(RING == WAVES, "a stage for each wavefront's tile");
+    int next = 0, next_run = 0;  // the next tile to request (by one of them), in the order of the runs
+    const unsigned chunk = ((lane & 7) ^ v_chunk_key(lane >> 3)) * 16;
+    char* const to = smem + wave * STAGE;
+    auto request = [&](bool mine) {
+        if (mine) {
+            const bool seg = next >= nt0;
+            const int t0 = (seg ? next - nt0 : next) * STK, ld = seg ? ld1 : ld0, last = keys_of(next) - 1;
+            const long long first_row = (long long)t0 * ld * 2;
+            const char* const kb = reinterpret_cast<const char*>(seg ? k1 : k0) + first_row;
+            const char* const vb = reinterpret_cast<const char*>(seg ? v1 : v0) + first_row;
+            unsigned at[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) at[i] = __umul24(min(8 * i + (lane >> 3), last), ld) * 2u + chunk;
+#pragma unroll
+            for (int i = 0; i < 4; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(kb + at[i]), (lds_ptr_t)(to + i * 1024), 16, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(vb + at[i]), (lds_ptr_t)(to + TILE + i * 1024), 16, 0, 0);
+        }
+        next += RUNS;
+        if (next >= n_t) next = ++next_run;
+    };
+    Frag q[SQB][2];
+    short_request_queries(s, b, h, q0, q);
+#pragma unroll
+    for (int i = 0; i < RING - 1; i++)
+        if (i < n_t) request(i == wave);
+    short_scale_queries(q_scale, q);
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+    const uint32_t k_at[2] = {lds + lr * 128u + ((unsigned)lg ^ (lr & 6)) * 16u, lds + lr * 128u + ((4u + lg) ^ (lr & 6)) * 16u};  // steps of d
+    const ShortVReads v_reads(lds + TILE);
+    unsigned done = 0;  // tiles
+    auto await = [&]() {
+        // the tile has landed where its wavefront says so; behind the barrier that holds for everyone, and everyone has done with the tile
+        // before, whose stage the next request fills
+        if (done % WAVES == (unsigned)wave) wait_vmcnt<0>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto proceed = [&]() {
+        if (done + RING - 1 < (unsigned)n_t) request((done + RING - 1) % WAVES == (unsigned)wave);
+        done++;
+    };
+    if (q0 >= s.Tq[0] + s.Tq[1]) {  // no queries for this wavefront: it loads its share of the tiles
+        while (done < (unsigned)n_t) {
+            await();
+            proceed();
+        }
+        return;
+    }
+    ShortState sum;
+#pragma unroll 1
+    for (int r = 0; r < RUNS; r++) {
+        ShortState z;
+        z.clear();
+#pragma unroll 1
+        for (int t = r; t < n_t; t += RUNS) {
+            await();
+            const uint32_t tile = done % RING * STAGE;
+            Frag k[2][2];
 #pragma unroll
             for (int kb16 = 0; kb16 < 2; kb16++)
 #pragma unroll
-                for (int r = 0; r < 4; r++)
-                    if (16 * kb16 + 4 * lg + r >= cur)
-#pragma unroll
-                        for (int i = 0; i < QB; i++) sc[kb16][i][r] = -1e30f;
+                for (int st = 0; st < 2; st++) k[kb16][st].v = lds_read_b128(k_at[st] + tile, kb16 * 16 * 128);
+            proceed();
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(k[0][0].v), "+v"(k[0][1].v), "+v"(k[1][0].v), "+v"(k[1][1].v));
+            f32x4_t sc[2][SQB];
+            short_scores(k, q, z, sc);
+            __builtin_amdgcn_sched_barrier(0);
+            uint2 vf[4][2];
+            v_reads.read(tile, vf);
+            Frag p[SQB];
+            short_probs(sc, keys_of(t), t < RUNS, z, p);
+            short_add_values(vf, p, z);
         }
-        Frag p[QB];
-        float inc[QB];
-        bool move = first;
-        auto probs = [&](int i) {
-            float f[8];
+        if (r >= n_t) z.weightless();
+        if (r == 0) {
+            sum = z;
+        } else {
 #pragma unroll
-            for (int e = 0; e < 8; e++) f[e] = __builtin_amdgcn_exp2f(sc[e >> 2][i][e & 3]);
-            inc[i] = ((f[0] + f[1]) + (f[2] + f[3])) + ((f[4] + f[5]) + (f[6] + f[7]));
-            p[i].u = pack8(f);
-        };
+            for (int i = 0; i < SQB; i++) {
+                float w, w2;
+                if (!__builtin_amdgcn_ballot_w64(sum.m(i) != z.m(i))) {  // both weights 1: the products below are the values themselves
+                    sum.l[i] += z.l[i];
 #pragma unroll
-        for (int i = 0; i < QB; i++) {
-            probs(i);
-            move = move || !(inc[i] <= L_BOUND);
-        }
-        // The reference goes to the running maximum with the first tile and whenever a lane's sum over a tile exceeds L_BOUND
-        if (__any(move)) {
-#pragma unroll
-            for (int i = 0; i < QB; i++) {
-                float mx = fmaxf(fmaxf(fmaxf(sc[0][i][0], sc[0][i][1]), fmaxf(sc[0][i][2], sc[0][i][3])),
-                                 fmaxf(fmaxf(sc[1][i][0], sc[1][i][1]), fmaxf(sc[1][i][2], sc[1][i][3])));
-                mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-                if (!first) mx = fmaxf(mx, 0.f);
-                const float alpha = first ? 0.f : __builtin_amdgcn_exp2f(-mx);
-                m_run[i] += mx;
-                l_run[i] *= alpha;
-#pragma unroll
-                for (int d = 0; d < 4; d++) o[d][i] *= alpha;
-#pragma unroll
-                for (int kb16 = 0; kb16 < 2; kb16++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) sc[kb16][i][r] -= mx;
-                probs(i);
-            }
-            first = false;
-        }
-#pragma unroll
-        for (int i = 0; i < QB; i++) l_run[i] += inc[i];
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(vf[0][0]), "+v"(vf[0][1]), "+v"(vf[1][0]), "+v"(vf[1][1]), "+v"(vf[2][0]), "+v"(vf[2][1]), "+v"(vf[3][0]), "+v"(vf[3][1]));
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-            Frag vv;
-            vv.u = make_uint4(vf[d][0].x, vf[d][0].y, vf[d][1].x, vf[d][1].y);
-#pragma unroll
-            for (int i = 0; i < QB; i++) o[d][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv.v, p[i].v, o[d][i], 0, 0, 0);
-        }
-    }
-
-    if (first)  // no tile came to this wavefront: weight zero in the merge
-#pragma unroll
-        for (int i = 0; i < QB; i++) m_run[i] = -1e30f;
-    // merge in a fixed tree: in each step the upper half of the wavefronts hands its state to the lower half (V tiles are free by then)
-    float* const merge = reinterpret_cast<float*>(smem);
-#pragma unroll
-    for (int half = KS / 2; half >= 1; half /= 2) {
-        float* mine = merge + (wave < half ? wave : wave - half) * 64 * PITCH + lane;  // value v of a lane at 64 v: no bank conflicts
-        __syncthreads();
-        if (wave >= half && wave < 2 * half) {
-#pragma unroll
-            for (int i = 0; i < QB; i++) {
-                mine[64 * (2 * i)] = m_run[i];
-                mine[64 * (2 * i + 1)] = l_run[i];
+                    for (int d = 0; d < 4; d++) sum.o[d][i] += z.o[d][i];
+                    continue;
+                }
+                float m = sum.m(i);
+                short_weights(m, z.m(i), w, w2);
+                sum.refer(i, m);
+                sum.l[i] = short_add(sum.l[i], w, z.l[i], w2);
 #pragma unroll
                 for (int d = 0; d < 4; d++)
 #pragma unroll
-                    for (int r = 0; r < 4; r++) mine[64 * (2 * QB + (i * 4 + d) * 4 + r)] = o[d][i][r];
-            }
-        }
-        __syncthreads();
-        if (wave < half) {
-#pragma unroll
-            for (int i = 0; i < QB; i++) {
-                const float om = mine[64 * (2 * i)], mx = fmaxf(m_run[i], om);
-                const float wa = __builtin_amdgcn_exp2f(m_run[i] - mx), wb = __builtin_amdgcn_exp2f(om - mx);
-                m_run[i] = mx;
-                l_run[i] = l_run[i] * wa + mine[64 * (2 * i + 1)] * wb;
-#pragma unroll
-                for (int d = 0; d < 4; d++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) o[d][i][r] = o[d][i][r] * wa + mine[64 * (2 * QB + (i * 4 + d) * 4 + r)] * wb;
+                    for (int e = 0; e < 4; e++) sum.o[d][i][e] = short_add(sum.o[d][i][e], w, z.o[d][i][e], w2);
             }
         }
     }
-    if (wave) return;
 #pragma unroll
-    for (int i = 0; i < QB; i++) {
-        const int qt = q0 + 16 * i + lr, seg = qt < Tq0 ? 0 : 1;
-        float l = l_run[i] + __shfl_xor(l_run[i], 16, 64);
-        l += __shfl_xor(l, 32, 64);
-        if (qt >= TQ || !s.out[seg]) continue;
-        const float inv = 1.0f / l;
-        bf16_t* op = s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_out[seg] + h * HS + 4 * lg;
+    for (int i = 0; i < SQB; i++) {
+        const float inv = 1.0f / short_total(sum.l[i]);
+        bf16_t* const to = short_out(s, b, h, q0, i);
+        if (to)
 #pragma unroll
-        for (int d = 0; d < 4; d++)
-            *reinterpret_cast<uint2*>(op + 16 * d) = make_uint2(pack_bf16x2(o[d][i][0] * inv, o[d][i][1] * inv), pack_bf16x2(o[d][i][2] * inv, o[d][i][3] * inv));
+            for (int d = 0; d < 4; d++) short_store4(to + 16 * d, sum.o[d][i], inv);
     }
 }
 
@@ -1161,16 +1382,25 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
         return (int)std::min<size_t>(idle, (taken + LEAST - 1) / LEAST);
     };
     if (!norm && longest <= SHORT_KEYS) {
-        constexpr int QB = 2, KS = 4;
-        total = 0;
-        for (int i = 0; i < m; i++) {  // (a split along the keys happens inside the workgroups: kv_splits does not apply)
-            SegDev& s = sets.set[i];
-            s.nqb = (s.Tq[0] + s.Tq[1] + 16 * QB - 1) / (16 * QB);
-            total += s.nqb * NH * B;
-            sets.end[i] = total;
-        }
-        for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
-        hipLaunchKernelGGL((flash_attn_bf16_split_kernel<QB, KS>), dim3((unsigned)(total + readers(total))), dim3(KS * 64), 0, st, sets, q_scale);
+        auto items = [&](int queries) {  // (a split along the keys happens inside the kernels: kv_splits does not apply)
+            total = 0;
+            for (int i = 0; i < MAX_SETS; i++) {
+                SegDev& s = sets.set[i];
+                if (i < m) {
+                    s.nqb = (s.Tq[0] + s.Tq[1] + queries - 1) / queries;
+                    total += s.nqb * NH * B;
+                }
+                sets.end[i] = total;
+            }
+            return total;
+        };
+        const int cus = compute_units();
+        if (cus <= 0) return SD3_ERR_HIP;
+        const bool split = items(SQ) <= 3 * cus;  // three of its workgroups fit a compute unit
+        if (!split) items(WAVES * SQ);
+        const dim3 grid((unsigned)(total + readers(total)));
+        if (split) hipLaunchKernelGGL(flash_attn_bf16_split_kernel, grid, dim3(RUNS * 64), 0, st, sets, q_scale);
+        else hipLaunchKernelGGL(flash_attn_bf16_runs_kernel, grid, dim3(WAVES * 64), 0, st, sets, q_scale);
         return launch_status("flash_attention_bf16");
     }
     dim3 grid((unsigned)(total + readers(total))), block(NW * 64);
