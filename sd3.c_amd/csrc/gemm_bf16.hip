@@ -756,17 +756,15 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
                 } else if (EPI == EPI_QKV_NORM && third < 2) {
                     qk_norm4(v, norm_w);
                 }
-                float* const of = reinterpret_cast<float*>(pr.out) + idx;
-                bf16_t* const oh = reinterpret_cast<bf16_t*>(pr.out) + idx;
                 if (WHOLE_ROWS) {
-                    if (OUT_F32) *reinterpret_cast<float4*>(of) = make_float4(v[0], v[1], v[2], v[3]);
-                    else *reinterpret_cast<uint2*>(oh) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                    if (OUT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(pr.out) + idx) = make_float4(v[0], v[1], v[2], v[3]);
+                    else *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(pr.out) + idx) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
                 } else {
 #pragma unroll
                     for (int c = 0; c < 4; c++)
                         if (c < valid) {
-                            if (OUT_F32) of[c] = v[c];
-                            else oh[c] = f32_to_bf16(v[c]);
+                            if (OUT_F32) reinterpret_cast<float*>(pr.out)[idx + c] = v[c];
+                            else reinterpret_cast<bf16_t*>(pr.out)[idx + c] = f32_to_bf16(v[c]);
                         }
                 }
             }
@@ -839,9 +837,14 @@ double launch_cost(const ProbSet& set, int n, int shape, int cus) {
     }
     const TileShape& t = tile_shapes[shape];
     const long long rounds = (tiles + cus - 1) / cus;
-    // 128x256 tiles in two rounds cost more than the table says: mlp-1 of 1581 + 999 rows, 504 tiles, 60 us and not 53, the out-projection of
-    // 9996 rows, 504 tiles, 81 and not 53, its mlp-2 207 and not 141 (256x256 tiles in one round: 74 and 191).
-    // (192x256 tiles in two rounds where 256x256 ones take two as well: 12255 + 770 rows, forward 0.8 % slower)
+    // The table is a first round's. A further round costs more the fuller it is, since its tiles share what feeds the compute units. 128x256
+    // tiles in two rounds, measured over the table's figure (cold weights, K = 1536 and 6144, N = 1536 .. 6144, 512 .. 12288 rows): 0.89 .. 1.07 with the
+    // second round 12 % full, 0.94 .. 1.16 with 48 to 69 %, 1.17 .. 1.23 with 85 to 97 % (504 tiles, mlp-1 of 2580 rows: 64.7 us, the table 52.5).
+    // The factor is that of a nearly full round, so that beyond one round the shape is taken where it saves a round (504 tiles instead of 528 of
+    // 256x128) and not for a few percent of the model. From three rounds on it measured 0.94 .. 1.14 and is overrated; there another shape was
+    // always within 1 % of it (up to 12288 rows). 192x256 tiles: 1.02 .. 1.13 in two rounds at K = 1536 where there are more than 270 (0.94 at 336 of
+    // mlp-1), 0.87 .. 0.91 at K = 6144, 0.95 .. 1.05 from three rounds on. Their factor matters only where 256x256 tiles take two rounds as
+    // well: with 1, 12255 + 770 rows take them and the forward is 0.8 % slower.
     const double again = rounds == 1 ? 1.0 : shape == TILE_128_256 ? 1.25 : shape == TILE_192_256 ? 1.06 : 1.0;
     return again * (double)rounds * (t.fixed + t.per_k * ((double)depth / tiles));
 }
@@ -1027,7 +1030,10 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         // Both layers in one launch where they are one round of small tiles, i.e. a launch's start and end are a good part of it: dual blocks
         // of 256 + 77, 1024 + 154 tokens 106.7 -> 105.3 us, forwards 2972 -> 2951, 4708 -> 4681 us. From 128x128 tiles on the second layer
         // does better in a launch (and tiles) of its own: 2048 + 308, 1581 + 999, 8192 + 308 rows, forwards 0.1, 0.6, 1 % slower together.
-        constexpr double GAP = 2.0;  // between two launches, us
+        // GAP: what a launch less saves, us. A launch of one tile behind another launch takes 2.7 to 3.5; the chained layer keeps some of that
+        // (between its K loops lie a barrier and a filling of the ring). With 5 instead of 2, blocks with 308 to 999 context rows beside 512 to
+        // 1344 latent ones were up to 1.1 % faster at widths 768 and 1536 and 0.8 % slower at 2432, the forwards the same.
+        constexpr double GAP = 2.0;
         SD3_TRY(fill(*then, args.second));
         const bool whole = all_whole(args, m) && args.second.whole;
         int pair = -1;
@@ -1081,6 +1087,8 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
     // One launch with the cheapest shape, or two: the many-row problems apart from the few-row ones (a launch of its own costs LAUNCH), or
     // full rounds of 256x256 tiles first and the last rows of the last many-row problem with the few-row problems behind them. The
     // latter only for epilogues that do not look at the row index (a row split would shift the batch boundaries).
+    // LAUNCH, us: the 2.7 to 3.5 of a launch behind another and the part of a first round that the table leaves out. (With 3.5 the batch-1
+    // forward of 1024 x 1024 pixels takes 12.80 instead of 12.72 ms, the others the same.)
     constexpr double LAUNCH = 5.0;
     double best;
     const int together = cheapest_shape(args, m, cus, best);
