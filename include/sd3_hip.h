@@ -252,7 +252,9 @@ int sd3_gemm_fp8(const void* aq, const float* a_scale, const void* wq, const flo
 int sd3_cast_f32_to_bf16(const float* in, void* out, long long n, void* stream);
 /* Tuning hook with no counterpart in the reference: forces the output tile of the bf16 GEMM for every later call in this
  * process. tile = 0: chosen per call from the problem sizes (the default); 128, 256: 128x128, 256x256 tiles; 192: 256x192 tiles (not with
- * the fused qk-norm epilogue); 64064, 64128, 128064, 256128, 128256, 192256: 64x64, 64x128, 128x64, 256x128, 128x256, 192x256 tiles. Results do not depend on the choice. */
+ * the fused qk-norm epilogue); 64064, 64128, 128064, 256128, 128256, 192256: 64x64, 64x128, 128x64, 256x128, 128x256, 192x256 tiles (problems
+ * whose rows are not aligned groups of four columns have 64x64, 128x128, 256x128, 256x192, 192x256 and 256x256 ones; the others run as
+ * 256x256). Results do not depend on the choice. */
 int sd3_gemm_bf16_force_tile(int tile);
 /* Process-wide tuning switches by name (no counterpart in the reference); results never depend on them. "gemm_bf16_tile": as
  * sd3_gemm_bf16_force_tile; "attention_context_splits": -1 chosen from the sizes (default), 0 never, 2..8 that many key splits for

@@ -76,8 +76,8 @@ struct AttnSets {
 // One load per 128-byte line of every run, the value dropped: workgroup `wg` of `wgs`, NT threads each.
 // Attention leaves HBM idle and the layers behind it wait for their weights (a launch of 333 / 1178 / 2356 / 4250 rows of mlp-1 and mlp-2
 // takes 51 / 74 / 108 / 173 us with weights from HBM, 36 / 60 / 94 / 156 from the last-level cache), so the workgroup slots that its
-// last round leaves free stream the block's remaining weights: forwards of 256px 2976 -> 2957 us, 512px 4681 -> 4617, its guided pair 6514 ->
-// 6454, 1024px 12726 -> 12594. (The same in the LayerNorm launches or on the compute units that a layer's tiles leave idle: slower on most.)
+// last round leaves free stream the block's remaining weights: forwards of 256px 2967 -> 2947 us, 512px 4631 -> 4548, its guided pair 6519 ->
+// 6442, 1024px 12610 -> 12505. (The same in the LayerNorm launches, 16 MB each: 256px 0.9 % slower, 1024px 0.5 % faster.)
 template <int NT>
 __device__ __forceinline__ void read_ahead(const Ahead& a, unsigned wg, unsigned wgs) {
     constexpr uint32_t LINE = 128, UNROLL = 4;
