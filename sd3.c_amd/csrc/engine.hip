@@ -64,7 +64,7 @@ static int static_scratch_of(int device, void** out) {
 struct PackedWeight {
     void* ptr = nullptr;
     long long K = 0, N = 0;
-    int kind = 0;  // 0: bf16 (N,K) transposed for the MFMA GEMM; 1: bf16 (K,N) plain cast for small_linear; 2: fp32 (K,N) transpose of an (N,K) tensor;
+    int kind = 0;  // 0: bf16 K tiles (K/64, N, 64) for the MFMA GEMM; 1: bf16 (K,N) plain cast for small_linear; 2: fp32 (K,N) transpose of an (N,K) tensor;
                    // 3 / 4: fp8 e4m3 (N,K) followed (at the next 256-byte boundary) by N fp32 factors, one per output column (3) or all equal (4)
 };
 static inline size_t fp8_scale_offset(long long K, long long N) { return ((size_t)K * N + 255) & ~(size_t)255; }
@@ -193,7 +193,7 @@ int get_packed(sd3_ctx* ctx, const float* w, long long K, long long N, int kind,
         return fail(SD3_ERR_OOM, "bf16 weight copy of %zu bytes: %s", bytes, hipGetErrorString(e));
     }
     int rc;
-    if (kind == 0) rc = pack_weight_bf16(w, (bf16_t*)p.ptr, (int)K, (int)N, ctx->stream);
+    if (kind == 0) rc = pack_weight_bf16(w, (bf16_t*)p.ptr, (int)K, (int)N, true, ctx->stream);
     else if (kind == 1) rc = cast_f32_to_bf16(w, (bf16_t*)p.ptr, K * N, ctx->stream);
     else if (kind >= 3) rc = quantize_weight_fp8(w, (uint8_t*)p.ptr, (float*)((char*)p.ptr + fp8_scale_offset(K, N)), (int)K, (int)N, kind == 4, ctx->stream);
     else rc = transpose_f32(w, (float*)p.ptr, (int)N, (int)K, ctx->stream);  // input is (N,K): transpose to (K,N)
@@ -301,7 +301,7 @@ int linear_layer(sd3_ctx* ctx, int prec, const void* A, const float* W, const fl
     const void* wp = nullptr;
     SD3_TRY(get_packed(ctx, W, K, N, 0, &wp));
     ProfScope ps(ctx, SD3_PROF_GEMM, 2.0 * M * N * K);
-    return gemm_bf16((const bf16_t*)A, (const bf16_t*)wp, out, out_f32, ldc, M, N, K, epi, ea, ctx->stream);
+    return gemm_bf16((const bf16_t*)A, (const bf16_t*)wp, true, out, out_f32, ldc, M, N, K, epi, ea, ctx->stream);
 }
 
 // The same layer of the latent stream and of the context stream (different weights and rows, same kind): both
@@ -343,7 +343,7 @@ int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f
         if (!c.W) return fail(SD3_ERR_MISSING_PARAM, "a weight needed by this configuration is not bound (N=%d K=%d)", c.N, c.K);
         const void* wp = nullptr;
         SD3_TRY(get_packed(ctx, c.W, c.K, c.N, 0, &wp));
-        probs[m] = GemmBf16Problem{(const bf16_t*)c.A, (const bf16_t*)wp, c.out, c.ldc, c.M, c.N, c.K, c.ea};
+        probs[m] = GemmBf16Problem{(const bf16_t*)c.A, (const bf16_t*)wp, c.out, c.ldc, c.M, c.N, c.K, c.ea, true};
         probs[m].ea.bias = c.bias;
         flop += 2.0 * c.M * c.N * c.K;
         m++;
@@ -353,7 +353,7 @@ int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f
         if (!then->W) return fail(SD3_ERR_MISSING_PARAM, "a weight needed by this configuration is not bound (N=%d K=%d)", then->N, then->K);
         const void* wp = nullptr;
         SD3_TRY(get_packed(ctx, then->W, then->K, then->N, 0, &wp));
-        second = GemmBf16Problem{(const bf16_t*)then->A, (const bf16_t*)wp, then->out, then->ldc, then->M, then->N, then->K, then->ea};
+        second = GemmBf16Problem{(const bf16_t*)then->A, (const bf16_t*)wp, then->out, then->ldc, then->M, then->N, then->K, then->ea, true};
         second.ea.bias = then->bias;
         probs[0].then = &second;
         flop += 2.0 * then->M * then->N * then->K;
@@ -1221,7 +1221,7 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
             const void* wp = nullptr;
             SD3_TRY(get_packed(ctx, patch_w, C, Kp, 1, &wp));
             ProfScope ps(ctx, SD3_PROF_GEMM, 2.0 * B * Tx * C * Kp);
-            SD3_TRY(gemm_bf16((const bf16_t*)patches, (const bf16_t*)wp, x, 1, C, B * Tx, C, Kp, EPI_BIAS_ROWADD, ea, st));
+            SD3_TRY(gemm_bf16((const bf16_t*)patches, (const bf16_t*)wp, false, x, 1, C, B * Tx, C, Kp, EPI_BIAS_ROWADD, ea, st));
         } else {
             const void* wt = nullptr;
             SD3_TRY(get_packed(ctx, patch_w, Kp, C, 2, &wt));
@@ -1334,7 +1334,7 @@ int sd3_flash_attention_bf16_split(const void* qkv0, const void* qkv1, void* out
 int sd3_pack_weight_bf16(const float* W, void* wpacked, int K, int N, void* stream) {
     SD3_REQUIRE(K > 0 && N > 0, "pack_weight_bf16: bad sizes");
     NOTNULL(W); NOTNULL(wpacked);
-    return pack_weight_bf16(W, (bf16_t*)wpacked, K, N, ST(stream));
+    return pack_weight_bf16(W, (bf16_t*)wpacked, K, N, false, ST(stream));
 }
 int sd3_gemm_bf16(const void* A, const void* wpacked, const float* bias, void* out, int M, int N, int K, int epilogue, void* stream) {
     SD3_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_bf16: bad sizes");
@@ -1343,7 +1343,7 @@ int sd3_gemm_bf16(const void* A, const void* wpacked, const float* bias, void* o
     NOTNULL(A); NOTNULL(wpacked); NOTNULL(out);
     GemmEpilogueArgs ea;
     ea.bias = bias;
-    return gemm_bf16((const bf16_t*)A, (const bf16_t*)wpacked, out, 0, N, M, N, K, epilogue, ea, ST(stream));
+    return gemm_bf16((const bf16_t*)A, (const bf16_t*)wpacked, false, out, 0, N, M, N, K, epilogue, ea, ST(stream));
 }
 int sd3_gemm_bf16_grouped(const sd3_gemm_bf16_problem* problems, int n_problems, int epilogue, int out_is_f32, void* stream) {
     NOTNULL(problems);

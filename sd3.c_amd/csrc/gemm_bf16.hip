@@ -1,6 +1,6 @@
 // bf16 GEMM on the gfx950 matrix cores (v_mfma_f32_16x16x32_bf16), fp32 accumulation:
-//   out(M,N) = A(M,K) @ Wp^T + epilogue,  A bf16 row-major, Wp bf16 (N,K) row-major (the reference's (K,N) fp32
-//   weight transposed and rounded once by pack_weight_bf16), so that both operands are K-contiguous.
+//   out(M,N) = A(M,K) @ Wp^T + epilogue,  A bf16 row-major, Wp bf16 (N,K) row-major or as K tiles (K/64, N, 64) (the reference's (K,N)
+//   fp32 weight transposed and rounded once by pack_weight_bf16), so that both operands are K-contiguous.
 // It replaces linear / partial_linear of the reference (modules.cpp:475-511) for the QKV, out-projection and MLP
 // layers. Epilogues: bias | bias+GELU-tanh | bias+SiLU | gate*(.)+residual (fp32, in place) | bias + row table.
 //
@@ -72,6 +72,7 @@ struct Prob {
     const bf16_t* Wp;
     void* out;
     int ldc, M, N, K;
+    bool tiled;  // layout of Wp (GemmBf16Problem::w_tiled)
     EpiDev epi;
     bool then;   // ring kernel, EPI_GATE_RESID: the same tile of ProbSet::second follows in the same workgroup
     bool whole;  // rows are made of aligned groups of four columns, in the output and in what the epilogue reads (whole_rows)
@@ -117,6 +118,8 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
     const char* ga[LA];
     const char* gb[LB];
     const long long row_bytes = (long long)K * ESZ;
+    // bytes from one row of Wp to the next, and from one K tile to the next
+    const long long w_row = !FP8 && pr.tiled ? 128 : row_bytes, w_tile = !FP8 && pr.tiled ? 128LL * N : 128;
 #pragma unroll
     for (int i = 0; i < LA; i++) {
         const int q = i * NT + tid, row = q >> 3, lc = (q & 7) ^ key(row);
@@ -127,7 +130,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
     for (int i = 0; i < LB; i++) {
         const int q = i * NT + tid, row = q >> 3, lc = (q & 7) ^ key(row);
         const int n = min(n_blk + row, N - 1);
-        gb[i] = Wp + (long long)n * row_bytes + lc * 16;
+        gb[i] = Wp + n * w_row + lc * 16;
     }
     auto issue_tile = [&](int kt, int stage) {
         char* sa = smem + stage * STAGE_BYTES + wave * 1024;
@@ -135,7 +138,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
 #pragma unroll
         for (int i = 0; i < LA; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(ga[i] + kt * 128), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
 #pragma unroll
-        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + kt * 128), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + kt * w_tile), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
     };
 
     // bf16 uses v_mfma_f32_16x16x32_bf16: on this device the clock under matrix load is set by the power limit, and measured on
@@ -581,7 +584,10 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
 
     const char* ga[LA];
     const char* gb[LB];
-    auto operands = [&](const bf16_t* A, const bf16_t* Wp) {
+    long long w_tile;  // bytes from one K tile of the weight to the next
+    auto operands = [&](const bf16_t* A, const bf16_t* Wp, bool tiled) {
+        const long long w_row = tiled ? 128 : 2LL * K;
+        w_tile = tiled ? 128LL * N : 128;
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int q = i * NT + tid, row = q >> 3;
@@ -591,19 +597,20 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
         for (int i = 0; i < LB; i++) {
             const int q = i * NT + tid, row = q >> 3;
             const int n = n_blk + row / WC * WC + NJ * (row % 16) + row % WC / 16;
-            gb[i] = reinterpret_cast<const char*>(Wp + (long long)min(n, N - 1) * K) + ((q & 7) ^ swz16(row)) * 16;
+            gb[i] = reinterpret_cast<const char*>(Wp) + min(n, N - 1) * w_row + ((q & 7) ^ swz16(row)) * 16;
         }
     };
-    operands(pr.A, pr.Wp);
+    operands(pr.A, pr.Wp, pr.tiled);
     const int nkt = K / BK;
     auto issue_tile = [&](int kt, int stage) {
         char* sa = smem + stage * STAGE_BYTES + wave * 1024;
         char* sb = sa + A_BYTES;
         const int off = kt * 128;
+        const long long w_off = kt * w_tile;
 #pragma unroll
         for (int i = 0; i < LA; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(ga[i] + off), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
 #pragma unroll
-        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + off), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + w_off), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
     };
     f32x4_t acc[TI][NJ];
     // Fragments are fetched ahead of their matrix instructions: a whole K tile ahead where it fits the registers, else one 32-deep half
@@ -781,7 +788,7 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        operands(next.A, next.Wp);
+        operands(next.A, next.Wp, next.tiled);
         fill_ring();
         epilogue(pr);
         k_loop();
@@ -986,7 +993,7 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
         if (q.K <= 0 || (q.K % kmult) != 0) return fail(SD3_ERR_UNSUPPORTED, "gemm_%s: K=%d must be a positive multiple of %d", fp8 ? "fp8" : "bf16", q.K, kmult);
         if ((reinterpret_cast<uintptr_t>(q.A) & 15) || (reinterpret_cast<uintptr_t>(q.Wp) & 15))
             return fail(SD3_ERR_INVALID_ARG, "gemm_bf16: operands must be 16-byte aligned");
-        d.A = q.A; d.Wp = q.Wp; d.out = q.out; d.ldc = q.ldc; d.M = q.M; d.N = q.N; d.K = q.K;
+        d.A = q.A; d.Wp = q.Wp; d.out = q.out; d.ldc = q.ldc; d.M = q.M; d.N = q.N; d.K = q.K; d.tiled = q.w_tiled && !fp8;
         d.epi = EpiDev{fp8 ? q.ea.a_scale : nullptr, fp8 ? q.ea.w_scale : nullptr, q.ea.bias, q.ea.gate, q.ea.resid, q.ea.table, q.ea.gate_ld,
                        q.ea.rows_per_batch > 0 ? q.ea.rows_per_batch : 1};
         if (epi == EPI_BIAS_ROWADD) d.epi.gate_ld = q.N;
@@ -1148,9 +1155,9 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
 int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st) { return grouped_impl(probs, n, out_is_f32, epi, false, st); }
 int gemm_fp8_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st) { return grouped_impl(probs, n, out_is_f32, epi, true, st); }
 
-int gemm_bf16(const bf16_t* A, const bf16_t* Wp, void* out, int out_is_f32, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
+int gemm_bf16(const bf16_t* A, const bf16_t* Wp, bool w_tiled, void* out, int out_is_f32, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
               hipStream_t st) {
-    GemmBf16Problem q{A, Wp, out, ldc, M, N, K, ea};
+    GemmBf16Problem q{A, Wp, out, ldc, M, N, K, ea, w_tiled};
     return gemm_bf16_grouped(&q, 1, out_is_f32, epi, st);
 }
 
