@@ -427,9 +427,9 @@ int cast_f32_to_bf16(const float* in, bf16_t* out, long long n, hipStream_t st) 
     return launch_status("cast_f32_to_bf16");
 }
 
-// (K,N) fp32 -> (N,K) or (K/64, N, 64) bf16 or fp32 through a 32x33 LDS tile so that both sides are coalesced.
+// (K,N) fp32 -> (N,K) bf16 or fp32 through a 32x33 LDS tile so that both sides are coalesced.
 template <typename OutT>
-__global__ void __launch_bounds__(256) pack_weight_kernel(const float* __restrict__ W, OutT* __restrict__ out, int K, int N, bool tiled) {
+__global__ void __launch_bounds__(256) pack_weight_kernel(const float* __restrict__ W, OutT* __restrict__ out, int K, int N) {
     __shared__ float tile[32][33];
     const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
     const int n0 = blockIdx.x * 32, k0 = blockIdx.y * 32;
@@ -440,17 +440,34 @@ __global__ void __launch_bounds__(256) pack_weight_kernel(const float* __restric
     __syncthreads();
     for (int r = ty; r < 32; r += 8) {
         int n = n0 + r, k = k0 + tx;
-        if (n < N && k < K) store1<OutT>(out + (tiled ? ((long long)(k >> 6) * N + n) * 64 + (k & 63) : (long long)n * K + k), tile[tx][r]);
+        if (n < N && k < K) store1<OutT>(out + (long long)n * K + k, tile[tx][r]);
     }
+}
+// The same as K tiles, 64 x 32 at a time: a tile's rows are 128 bytes, 32 of them in a row
+__global__ void __launch_bounds__(256) pack_weight_tiles_kernel(const float* __restrict__ W, bf16_t* __restrict__ out, int K, int N) {
+    __shared__ float tile[64][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
+    const int n0 = blockIdx.x * 32, k0 = blockIdx.y * 64;
+#pragma unroll
+    for (int r = ty; r < 64; r += 8) tile[r][tx] = n0 + tx < N ? W[(long long)(k0 + r) * N + n0 + tx] : 0.f;
+    __syncthreads();
+#pragma unroll
+    for (int r = ty; r < 32; r += 8)
+        if (n0 + r < N) *reinterpret_cast<uint32_t*>(out + ((long long)blockIdx.y * N + n0 + r) * 64 + 2 * tx) = pack_bf16x2(tile[2 * tx][r], tile[2 * tx + 1][r]);
 }
 int pack_weight_bf16(const float* W, bf16_t* out, int K, int N, bool tiled, hipStream_t st) {
     if (K == 0 || N == 0) return SD3_OK;
-    hipLaunchKernelGGL((pack_weight_kernel<bf16_t>), dim3((N + 31) / 32, (K + 31) / 32), dim3(256), 0, st, W, out, K, N, tiled);
+    if (tiled) {
+        if (K % 64) return fail(SD3_ERR_UNSUPPORTED, "pack_weight_bf16: K=%d is not made of whole K tiles", K);
+        hipLaunchKernelGGL(pack_weight_tiles_kernel, dim3((N + 31) / 32, K / 64), dim3(256), 0, st, W, out, K, N);
+        return launch_status("pack_weight_bf16");
+    }
+    hipLaunchKernelGGL((pack_weight_kernel<bf16_t>), dim3((N + 31) / 32, (K + 31) / 32), dim3(256), 0, st, W, out, K, N);
     return launch_status("pack_weight_bf16");
 }
 int transpose_f32(const float* W, float* out, int K, int N, hipStream_t st) {
     if (K == 0 || N == 0) return SD3_OK;
-    hipLaunchKernelGGL((pack_weight_kernel<float>), dim3((N + 31) / 32, (K + 31) / 32), dim3(256), 0, st, W, out, K, N, false);
+    hipLaunchKernelGGL((pack_weight_kernel<float>), dim3((N + 31) / 32, (K + 31) / 32), dim3(256), 0, st, W, out, K, N);
     return launch_status("transpose_f32");
 }
 
