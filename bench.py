@@ -46,7 +46,7 @@ def measured_traffic(kernel_class):
     """HBM bytes per launch of the class's kernel from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary (both scaled by
     what the same counters read for a 1 GiB copy kernel in the same run); None if the summary is not there."""
     name = {"gemm": "gemm_bf16_kernel", "attention": "flash_attn_bf16_kernel", "layernorm_modulate": "ln_mod_vec_kernel",
-            "adaln_linear": "small_linear_kernel"}.get(kernel_class)
+            "adaln_linear": "ada_panel_kernel"}.get(kernel_class)
     path = os.path.join(ROOT, "profiles", "dit_forward_1024px_b2_bf16_hbm_traffic.txt")
     if not name or not os.path.exists(path):
         return None

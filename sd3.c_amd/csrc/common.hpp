@@ -124,6 +124,123 @@ __device__ __forceinline__ void tile_of_workgroup(int wg, int tiles_m, int tiles
     tile_n = (t % in_group) / gsize;
 }
 
+// ---- modulation projections of the bf16 path ----
+// out (B, N) = y (B, K) @ W + bias, W bf16 as panels of 64 columns (N/64, K, 64). A panel is K * 128 bytes that one workgroup streams from
+// end to end; the launches' own kernel is in small_linear.hip, and a GEMM launch that leaves compute units idle takes panels of the NEXT
+// block along (AdaCarry), in workgroups behind those of its tiles.
+struct AdaJob {
+    const bf16_t* W;
+    const float* bias;
+    float* out;
+    int N, ld;  // columns (whole panels) and the row stride of out
+};
+constexpr int ADA_CARRY_JOBS = 3, ADA_CARRY_ROWS = 4;  // what a GEMM launch takes along at most: the two streams of a block and the output layer; batch elements
+constexpr int ADA_SLICES = 32;
+struct AdaWork {
+    AdaJob job[ADA_CARRY_JOBS];
+    const float* y;
+    int B, K;
+    int first, count;  // panels of this launch, counted over the jobs
+};
+constexpr int ada_lds_bytes(int rows, int K) { return (rows * K + ADA_SLICES * rows * 64) * 4; }
+// y transposed into LDS, xs[k][m]
+template <int NT, int M>
+__device__ __forceinline__ void ada_stage_rows(const float* __restrict__ y, int B, int K, float* xs) {
+#pragma unroll
+    for (int m = 0; m < M; m++)
+        for (int k = threadIdx.x; k < K; k += NT) xs[k * M + m] = m < B ? y[(long long)m * K + k] : 0.f;
+    __syncthreads();
+}
+// One panel. A thread has 4 columns and one (NT = 512) or two of the 32 slices of K, 16 rows of weights in flight; the order of the sums does
+// not depend on NT or M (explicit multiply-adds), so that a row has the same bits in either kernel and in any batch.
+// ONCE: nobody reads these weights again in a forward, so they are not to push the blocks' activations and the weights that attention reads
+// ahead out of the last-level cache (non-temporal loads; forwards of 256px, 512px, its pair, 1024px 0.6, 0.7, 0.6, 0.9 % less). A block that
+// is called over and over finds them there (106.3 -> 104 us without).
+template <int NT, int M, bool ONCE>
+__device__ __forceinline__ void ada_panel(const bf16_t* __restrict__ W, const float* __restrict__ bias, float* __restrict__ out, int ld, int B, int K,
+                                          const float* xs, float* red) {
+    const int cg = threadIdx.x % 16, kper = K / ADA_SLICES;
+    for (int sl = threadIdx.x / 16; sl < ADA_SLICES; sl += NT / 16) {
+        const bf16_t* p = W + ((long long)sl * kper) * 64 + cg * 4;
+        const float* xk = xs + sl * kper * M;
+        float acc[M][4];
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[m][j] = 0.f;
+        auto add = [&](int k, const uint2 v) {
+            const float w[4] = {__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const float xv = xk[k * M + m];
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc[m][j] = fmaf(xv, w[j], acc[m][j]);
+            }
+        };
+        auto row = [](const bf16_t* q) {
+            const unsigned long long* p8 = reinterpret_cast<const unsigned long long*>(q);
+            return __builtin_bit_cast(uint2, ONCE ? __builtin_nontemporal_load(p8) : *p8);
+        };
+        constexpr int U = 16;  // rows of weights in flight (and as many again while they are used)
+        uint2 v[U], n[U];
+        const int whole = kper / U * U;
+        if (whole) {
+#pragma unroll
+            for (int i = 0; i < U; i++) v[i] = row(p + i * 64);
+            for (int k = 0; k < whole; k += U) {
+                const bf16_t* q = p + (k + U < whole ? k + U : k) * 64;
+#pragma unroll
+                for (int i = 0; i < U; i++) n[i] = row(q + i * 64);
+#pragma unroll
+                for (int i = 0; i < U; i++) add(k + i, v[i]);
+#pragma unroll
+                for (int i = 0; i < U; i++) v[i] = n[i];
+            }
+        }
+        for (int k = whole; k < kper; k++) add(k, row(p + k * 64));
+#pragma unroll
+        for (int m = 0; m < M; m++) *reinterpret_cast<float4*>(red + (sl * M + m) * 64 + cg * 4) = make_float4(acc[m][0], acc[m][1], acc[m][2], acc[m][3]);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < M * 64; e += NT) {
+        const int m = e / 64, c = e % 64;
+        if (m < B) {
+            float s = 0.f;
+#pragma unroll
+            for (int sl = 0; sl < ADA_SLICES; sl++) s += red[(sl * M + m) * 64 + c];
+            out[(long long)m * ld + c] = s + bias[c];
+        }
+    }
+    __syncthreads();
+}
+// Workgroup `wg` of `wgs` that a GEMM launch has added to its own
+template <int NT, int M>
+__device__ __forceinline__ void ada_carried_rows(const AdaWork& a, int wg, int wgs, char* smem) {
+    float* xs = reinterpret_cast<float*>(smem);
+    ada_stage_rows<NT, M>(a.y, a.B, a.K, xs);
+    for (int i = wg; i < a.count; i += wgs) {
+        int t = a.first + i, j = 0;
+        while (j + 1 < ADA_CARRY_JOBS && t >= a.job[j].N / 64) t -= a.job[j++].N / 64;
+        const AdaJob& q = a.job[j];
+        ada_panel<NT, M, true>(q.W + (long long)t * 64 * a.K, q.bias + t * 64, q.out + t * 64, q.ld, a.B, a.K, xs, xs + M * a.K);
+    }
+}
+template <int NT>
+__device__ __forceinline__ void ada_carried(const AdaWork& a, int wg, int wgs, char* smem) {
+    if (a.B == 1) ada_carried_rows<NT, 1>(a, wg, wgs, smem);
+    else if (a.B == 2) ada_carried_rows<NT, 2>(a, wg, wgs, smem);
+    else ada_carried_rows<NT, ADA_CARRY_ROWS>(a, wg, wgs, smem);
+}
+// What is left of a block's panels; a GEMM launch takes `first` onwards as many as it has room for and moves `first` on.
+struct AdaCarry {
+    AdaWork work{};
+    int total = 0;
+    bool last = false;  // the block's last launch
+    int left() const { return total - work.first; }
+};
+int ada_panels(const float* y, int B, int K, const AdaJob* jobs, int n, hipStream_t st);
+int pack_ada_panels(const float* W, bf16_t* out, int K, int N, hipStream_t st);
+
 // ---- epilogues of the GEMM kernels ----
 enum Epilogue : int {
     EPI_BIAS = 0,         // out = acc + bias
@@ -176,7 +293,7 @@ struct GemmBf16Problem {
     const GemmBf16Problem* then = nullptr;  // EPI_GATE_RESID: a second layer of the same M, N, K and out whose residual is this one's result
 };
 extern std::atomic<long long> g_gemm_bf16_launches;  // kernels launched by the bf16 GEMM so far (for per-launch profile figures)
-int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st);
+int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st, AdaCarry* carry = nullptr);
 // The same with OCP fp8 (e4m3) operands: A (M,K) and Wp (N,K) are bytes, K % 128 == 0, and the accumulators are multiplied by
 // ea.a_scale[m] * ea.w_scale[n] before the epilogue (epilogues: bias, bias+GELU, gate+residual, q|k|v with qk-norm).
 int gemm_fp8_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st);
@@ -242,9 +359,9 @@ int unpatchify(const float* tokens, float* out, int B, int Cin, int H, int W, in
 int unpatchify_cfg_euler(const float* tokens, const float* latent, float* out, int n_samples, int Cin, int H, int W, int p, float guidance, float dsigma,
                          hipStream_t st);
 
-// Small-M linear (M <= 8): out(M, N) = act(x(M,K) @ W[:, n0:n0+N] + b[n0:n0+N]); W fp32 (K, ldw) or bf16 (K, ldw), both N-contiguous.
+// Small-M linear (M <= 8): out(M, N) = act(x(M,K) @ W[:, n0:n0+N] + b[n0:n0+N]); W fp32 (K, ldw), N-contiguous.
 struct SmallLinearJob {
-    const void* W;
+    const float* W;
     const float* bias;
     float* out;
     int N;    // columns of this job
@@ -254,7 +371,7 @@ struct SmallLinearJob {
     int K = 0;                 // its depth (with x)
 };
 constexpr int SMALL_LINEAR_JOBS_PER_LAUNCH = 52;
-int small_linear_batched(const float* x, int M, int K, const SmallLinearJob* jobs_host, int n_jobs, int w_is_bf16, int act /* -1 none */,
+int small_linear_batched(const float* x, int M, int K, const SmallLinearJob* jobs_host, int n_jobs, int act /* -1 none */,
                          hipStream_t st);
 
 // Attention. Two token segments (segment 0 first in the joint sequence); each has its own q/k/v/out pointers and row strides.

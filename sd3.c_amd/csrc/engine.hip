@@ -64,8 +64,9 @@ static int static_scratch_of(int device, void** out) {
 struct PackedWeight {
     void* ptr = nullptr;
     long long K = 0, N = 0;
-    int kind = 0;  // 0: bf16 K tiles (K/64, N, 64) for the MFMA GEMM; 1: bf16 (K,N) plain cast for small_linear; 2: fp32 (K,N) transpose of an (N,K) tensor;
-                   // 3 / 4: fp8 e4m3 (N,K) followed (at the next 256-byte boundary) by N fp32 factors, one per output column (3) or all equal (4)
+    int kind = 0;  // 0: bf16 K tiles (K/64, N, 64) for the MFMA GEMM; 1: bf16 plain cast (the patch convolution's weight); 2: fp32 (K,N) transpose of an (N,K) tensor;
+                   // 3 / 4: fp8 e4m3 (N,K) followed (at the next 256-byte boundary) by N fp32 factors, one per output column (3) or all equal (4);
+                   // 5: bf16 panels (N/64, K, 64) for the modulation projections
 };
 static inline size_t fp8_scale_offset(long long K, long long N) { return ((size_t)K * N + 255) & ~(size_t)255; }
 static inline bool is_bf(int prec) { return prec != SD3_PREC_F32; }
@@ -186,7 +187,7 @@ int get_packed(sd3_ctx* ctx, const float* w, long long K, long long N, int kind,
     }
     PackedWeight p;
     p.K = K; p.N = N; p.kind = kind;
-    const size_t bytes = kind >= 3 ? fp8_scale_offset(K, N) + (size_t)N * sizeof(float) : (size_t)K * N * (kind == 2 ? 4 : 2);
+    const size_t bytes = kind == 3 || kind == 4 ? fp8_scale_offset(K, N) + (size_t)N * sizeof(float) : (size_t)K * N * (kind == 2 ? 4 : 2);
     hipError_t e = hipMalloc(&p.ptr, bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
@@ -195,6 +196,7 @@ int get_packed(sd3_ctx* ctx, const float* w, long long K, long long N, int kind,
     int rc;
     if (kind == 0) rc = pack_weight_bf16(w, (bf16_t*)p.ptr, (int)K, (int)N, true, ctx->stream);
     else if (kind == 1) rc = cast_f32_to_bf16(w, (bf16_t*)p.ptr, K * N, ctx->stream);
+    else if (kind == 5) rc = pack_ada_panels(w, (bf16_t*)p.ptr, (int)K, (int)N, ctx->stream);
     else if (kind >= 3) rc = quantize_weight_fp8(w, (uint8_t*)p.ptr, (float*)((char*)p.ptr + fp8_scale_offset(K, N)), (int)K, (int)N, kind == 4, ctx->stream);
     else rc = transpose_f32(w, (float*)p.ptr, (int)N, (int)K, ctx->stream);  // input is (N,K): transpose to (K,N)
     if (rc != SD3_OK) {
@@ -210,7 +212,7 @@ int get_packed(sd3_ctx* ctx, const float* w, long long K, long long N, int kind,
 // Frees every derived copy made from the tensor at `w` (after the work that may still read them has finished).
 int drop_packed_of(sd3_ctx* ctx, const float* w) {
     bool synced = false;
-    for (int kind = 0; kind < 5; kind++) {
+    for (int kind = 0; kind < 6; kind++) {
         auto it = ctx->packed.find(std::make_pair(w, kind));
         if (it == ctx->packed.end()) continue;
         if (!synced) {
@@ -315,7 +317,7 @@ struct LayerCall {
     int ldc, M, N, K;
     GemmEpilogueArgs ea;
 };
-int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f32, int epi, const LayerCall* then = nullptr) {
+int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f32, int epi, const LayerCall* then = nullptr, AdaCarry* carry = nullptr) {
     if (n > 3) return fail(SD3_ERR_INVALID_ARG, "linear_pair: at most three layers per group");
     if (!is_bf(prec)) {
         GemmF32Problem probs[3];
@@ -360,21 +362,35 @@ int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f
     }
     if (m == 0) return SD3_OK;
     ProfScope ps(ctx, SD3_PROF_GEMM, flop);
-    return gemm_bf16_grouped(probs, m, out_f32, epi, ctx->stream);
+    return gemm_bf16_grouped(probs, m, out_f32, epi, ctx->stream, carry);
 }
 
-int ada_jobs_run(sd3_ctx* ctx, int prec, const float* y, int B, int C, std::vector<SmallLinearJob>& jobs) {
-    if (is_bf(prec)) {
-        for (auto& j : jobs) {
-            const void* wp = nullptr;
-            SD3_TRY(get_packed(ctx, (const float*)j.W, C, j.ldw, 1, &wp));
-            j.W = wp;
-        }
-    }
+// One modulation projection: a whole weight (C, N) and its bias, out (B, N)
+struct AdaCall {
+    const float* W;
+    const float* bias;
+    float* out;
+    int N;
+};
+int ada_panel_job(sd3_ctx* ctx, const AdaCall& c, int C, AdaJob* job) {
+    const void* wp = nullptr;
+    SD3_TRY(get_packed(ctx, c.W, C, c.N, 5, &wp));
+    *job = AdaJob{(const bf16_t*)wp, c.bias, c.out, c.N, c.N};
+    return SD3_OK;
+}
+int ada_jobs_run(sd3_ctx* ctx, int prec, const float* y, int B, int C, const std::vector<AdaCall>& calls) {
     double bytes = 0;
-    for (auto& j : jobs) bytes += (double)C * j.N * (is_bf(prec) ? 2 : 4) + (double)B * j.N * 4;
+    for (auto& c : calls) bytes += (double)C * c.N * (is_bf(prec) ? 2 : 4) + (double)B * c.N * 4;
+    if (is_bf(prec)) {
+        std::vector<AdaJob> jobs(calls.size());
+        for (size_t i = 0; i < calls.size(); i++) SD3_TRY(ada_panel_job(ctx, calls[i], C, &jobs[i]));
+        ProfScope ps(ctx, SD3_PROF_ADALN, bytes, ((long long)jobs.size() + SMALL_LINEAR_JOBS_PER_LAUNCH - 1) / SMALL_LINEAR_JOBS_PER_LAUNCH);
+        return ada_panels(y, B, C, jobs.data(), (int)jobs.size(), ctx->stream);
+    }
+    std::vector<SmallLinearJob> jobs;
+    for (auto& c : calls) jobs.push_back({c.W, c.bias, c.out, c.N, c.N, 0});
     ProfScope ps(ctx, SD3_PROF_ADALN, bytes, ((long long)jobs.size() + SMALL_LINEAR_JOBS_PER_LAUNCH - 1) / SMALL_LINEAR_JOBS_PER_LAUNCH);
-    return small_linear_batched(y, B, C, jobs.data(), (int)jobs.size(), is_bf(prec), -1, ctx->stream);
+    return small_linear_batched(y, B, C, jobs.data(), (int)jobs.size(), -1, ctx->stream);
 }
 
 // LayerNorm + modulation, timed as a memory-bound launch: reads x once (fp32), writes one or two outputs.
@@ -405,7 +421,7 @@ int attention(sd3_ctx* ctx, const AttnSegments& a, int B, int NH, int HS, bool b
 
 // The block. ada_c / ada_x: modulation vectors (B, chunks*C) already computed, or null to compute them here.
 int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const sd3_block_weights& w, const Dims& d, const float* ada_c,
-              const float* ada_x, Bump& ws) {
+              const float* ada_x, Bump& ws, AdaCarry* carry = nullptr) {
     hipStream_t st = ctx->stream;
     const int B = d.B, Tc = d.Tc, Tx = d.Tx, C = d.C;
     const int mc = B * Tc, mx = B * Tx;
@@ -453,11 +469,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
 
     // modulation vectors: every chunk of both streams in one launch (the reference issues 12-20 partial_linear calls)
     if (!ada_c || !ada_x) {
-        std::vector<SmallLinearJob> jobs = {
-            {w.c_ada_w, w.c_ada_b, ada_c_buf, cch * C, cch * C, 0},
-            {w.x_ada_w, w.x_ada_b, ada_x_buf, xch * C, xch * C, 0},
-        };
-        SD3_TRY(ada_jobs_run(ctx, prec, y, B, C, jobs));
+        SD3_TRY(ada_jobs_run(ctx, prec, y, B, C, {{w.c_ada_w, w.c_ada_b, ada_c_buf, cch * C}, {w.x_ada_w, w.x_ada_b, ada_x_buf, xch * C}}));
         ada_c = ada_c_buf;
         ada_x = ada_x_buf;
     }
@@ -489,7 +501,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         LayerCall qkv[3] = {{x_hid, w.x_qkv_w, w.x_qkv_b, x_qkv, 3 * C, mx, 3 * C, C, fused_norm ? nx : none},
                             {x_hid2, w.x2_qkv_w, w.x2_qkv_b, x_qkv2, 3 * C, d.dual ? mx : 0, 3 * C, C, fused_norm ? n2 : none},
                             {c_hid, w.c_qkv_w, w.c_qkv_b, c_qkv, 3 * C, mc, 3 * C, C, fused_norm ? nc : none}};
-        SD3_TRY(linear_pair(ctx, prec, qkv, 3, !bf, fused_norm ? EPI_QKV_NORM : EPI_BIAS));
+        SD3_TRY(linear_pair(ctx, prec, qkv, 3, !bf, fused_norm ? EPI_QKV_NORM : EPI_BIAS, nullptr, carry));
     }
 
     // ---- joint attention over [context ; latent] (modules.cpp:1427-1432); fp32 path: qk-norm in place first
@@ -571,7 +583,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         GemmEpilogueArgs g2;
         g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;
         const LayerCall proj2{x_att2, w.x2_out_w, w.x2_out_b, x, C, mx, C, C, g2};
-        SD3_TRY(linear_pair(ctx, prec, proj, 2, 1, EPI_GATE_RESID, d.dual && bf ? &proj2 : nullptr));
+        SD3_TRY(linear_pair(ctx, prec, proj, 2, 1, EPI_GATE_RESID, d.dual && bf ? &proj2 : nullptr, carry));
     }
 
     // ---- fp32: extra self-attention over the latent tokens (modules.cpp:1440-1453, 1486)
@@ -630,11 +642,12 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     {
         LayerCall up[2] = {{x_hid, w.x_mlp_w1, w.x_mlp_b1, x_mlp, d.E * C, mx, d.E * C, C, none},
                            {c_hid, w.c_mlp_w1, w.c_mlp_b1, c_mlp, d.E * C, mcm, d.E * C, C, none}};
-        SD3_TRY(linear_pair(ctx, prec, up, 2, !bf, EPI_BIAS_GELU));
+        SD3_TRY(linear_pair(ctx, prec, up, 2, !bf, EPI_BIAS_GELU, nullptr, carry));
         gc.gate = cchunk(5);
         gx.gate = xchunk(5);
         LayerCall down[2] = {{x_mlp, w.x_mlp_w2, w.x_mlp_b2, x, C, mx, C, d.E * C, gx}, {c_mlp, w.c_mlp_w2, w.c_mlp_b2, c, C, mcm, C, d.E * C, gc}};
-        SD3_TRY(linear_pair(ctx, prec, down, 2, 1, EPI_GATE_RESID));
+        if (carry) carry->last = true;
+        SD3_TRY(linear_pair(ctx, prec, down, 2, 1, EPI_GATE_RESID, nullptr, carry));
     }
     return SD3_OK;
 }
@@ -997,7 +1010,7 @@ int sd3_weights_prepare(sd3_ctx* ctx, int precision) {
         const bool adaln = ends_with(name, "ada_lnorm.linear.weight") || name == "ada_ln_out.linear.weight";
         const bool gemm = ends_with(name, "_to_qkv.weight") || ends_with(name, "_attn_Wout.weight") || ends_with(name, "_mlp.lin1.weight") ||
                           ends_with(name, "_mlp.lin2.weight") || name == "captions_linear.weight" || name == "linear_out.weight";
-        if (adaln) SD3_TRY(get_packed(ctx, kv.second.first, K, N, 1, &unused));
+        if (adaln && N % 64 == 0) SD3_TRY(get_packed(ctx, kv.second.first, K, N, 5, &unused));
         else if (gemm && K % 64 == 0) SD3_TRY(get_packed(ctx, kv.second.first, K, N, 0, &unused));
     }
     return SD3_OK;
@@ -1178,9 +1191,9 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     {
         // the two MLPs side by side: both first layers in one launch (each job brings its own input), then both second layers
         const SmallLinearJob first[2] = {{t_w0, t_b0, h1, C, C, 0, temb, 256}, {p_w0, p_b0, h2, C, C, 0, pooled, pooled_dim}};
-        SD3_TRY(small_linear_batched(nullptr, B, 0, first, 2, 0, SD3_ACT_SILU, st));
+        SD3_TRY(small_linear_batched(nullptr, B, 0, first, 2, SD3_ACT_SILU, st));
         const SmallLinearJob second[2] = {{t_w2, t_b2, yt, C, C, 0, h1, C}, {p_w2, p_b2, yp, C, C, 0, h2, C}};
-        SD3_TRY(small_linear_batched(nullptr, B, 0, second, 2, 0, -1, st));
+        SD3_TRY(small_linear_batched(nullptr, B, 0, second, 2, -1, st));
         SD3_TRY(add_silu_op(yt, yp, y, (long long)B * C, st));
     }
     // ---- c = captions @ W + b (modules.cpp:1678)
@@ -1229,25 +1242,53 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
             SD3_TRY(gemm_f32((const float*)patches, Kp, (const float*)wt, C, 0, x, C, B * Tx, C, Kp, EPI_BIAS_ROWADD, ea, st));
         }
     }
-    // ---- modulation vectors of every block and of the output layer: y does not change across blocks, so all
-    //      adaLN projections (0.77 G parameters) are streamed once, up front
+    // ---- modulation vectors of every block and of the output layer (0.77 G parameters, streamed once): y does not change across blocks.
+    //      bf16, few rows: only the first block's up front; a block's GEMM launches take those of the next block along on the compute
+    //      units that their tiles leave idle.
+    auto ada_calls = [&](int l) {
+        const int cch = bd[l].discard ? 2 : 6, xch = bd[l].dual ? 9 : 6;
+        float* base = ada_all + (size_t)l * B * 15 * C;
+        std::vector<AdaCall> calls = {{bw[l].c_ada_w, bw[l].c_ada_b, base, cch * C}, {bw[l].x_ada_w, bw[l].x_ada_b, base + (size_t)B * 6 * C, xch * C}};
+        if (l == num_layers - 1) calls.push_back({ao_w, ao_b, ada_out, 2 * C});
+        return calls;
+    };
+    //      Up to 4096 rows: beyond them the device is at its power limit, where what streams beside the matrix kernels costs them clock (4250 rows,
+    //      forward against all projections up front: -1.0, 0 and +1.3 % on three devices; 2048px 0).
+    const bool carried = bf && !fp8_kind(precision) && B <= ADA_CARRY_ROWS && (long long)B * (Tx + Tc) <= 4096;
     {
-        std::vector<SmallLinearJob> jobs;
-        for (int l = 0; l < num_layers; l++) {
-            const int cch = bd[l].discard ? 2 : 6, xch = bd[l].dual ? 9 : 6;
-            float* base = ada_all + (size_t)l * B * 15 * C;
-            jobs.push_back({bw[l].c_ada_w, bw[l].c_ada_b, base, cch * C, cch * C, 0});
-            jobs.push_back({bw[l].x_ada_w, bw[l].x_ada_b, base + (size_t)B * 6 * C, xch * C, xch * C, 0});
-        }
-        jobs.push_back({ao_w, ao_b, ada_out, 2 * C, 2 * C, 0});
-        SD3_TRY(ada_jobs_run(ctx, precision, y, B, C, jobs));
+        std::vector<AdaCall> calls;
+        for (int l = 0; l < (carried ? 1 : num_layers); l++)
+            for (const AdaCall& c : ada_calls(l)) calls.push_back(c);
+        SD3_TRY(ada_jobs_run(ctx, precision, y, B, C, calls));
     }
     // ---- blocks (modules.cpp:1687-1718)
     for (int l = 0; l < num_layers; l++) {
         Bump bws(ctx->ws, ctx->ws_bytes);
         bws.off = block_ws_off;
         const float* base = ada_all + (size_t)l * B * 15 * C;
-        SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], base, base + (size_t)B * 6 * C, bws));
+        AdaCarry carry;
+        if (carried && l + 1 < num_layers) {
+            carry.work.y = y;
+            carry.work.B = B;
+            carry.work.K = C;
+            int i = 0;
+            for (const AdaCall& q : ada_calls(l + 1)) {
+                SD3_TRY(ada_panel_job(ctx, q, C, &carry.work.job[i++]));
+                carry.total += q.N / 64;
+            }
+        }
+        SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], base, base + (size_t)B * 6 * C, bws, &carry));
+        if (carry.left() > 0) {  // what no launch had room for
+            AdaJob rest[ADA_CARRY_JOBS];
+            int n = 0, skip = carry.work.first;
+            for (const AdaJob& j : carry.work.job) {
+                const int done = std::min(skip, j.N / 64);
+                skip -= done;
+                if (done * 64 < j.N) rest[n++] = AdaJob{j.W + (size_t)done * 64 * C, j.bias + done * 64, j.out + done * 64, j.N - done * 64, j.ld};
+            }
+            ProfScope ps(ctx, SD3_PROF_ADALN, (2.0 * C + 4.0 * B) * 64 * carry.left());
+            SD3_TRY(ada_panels(y, B, C, rest, n, st));
+        }
     }
     // ---- output layer: LN(eps 1e-5), chunk 0 = scale, chunk 1 = shift, projection, tokens -> pixels (modules.cpp:1721-1752)
     {

@@ -82,7 +82,13 @@ struct ProbSet {
     Prob p[MAX_PROBS];
     int end[MAX_PROBS];  // running totals of tiles
     Prob second;         // (see Prob::then)
+    int tiles_wgs;       // workgroups from here on work on `ada`
+    AdaWork ada;
+    float us;            // (host) about how long the launch takes
+    bool ada_last;       // (host) no launch behind this one can take any
 };
+// the epilogues of the layers whose launches take modulation projections along
+constexpr bool carries(int epi) { return epi == EPI_BIAS_GELU || epi == EPI_GATE_RESID || epi == EPI_QKV_NORM; }
 
 // One output tile: K loop + epilogue. `wg` is the tile's position in the XCD-aware order of its problem.
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8_t;
@@ -506,11 +512,35 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
 template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet args) {
     extern __shared__ __attribute__((aligned(1024))) char smem[];
-    for (int w = blockIdx.x; w < args.end[MAX_PROBS - 1]; w += gridDim.x) {
+    if (carries(EPI) && !FP8 && (int)blockIdx.x >= args.tiles_wgs) {
+        ada_carried<WM * WN * 64>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
+        return;
+    }
+    for (int w = blockIdx.x; w < args.end[MAX_PROBS - 1]; w += args.tiles_wgs) {
         const int which = (w >= args.end[0]) + (w >= args.end[1]);
         gemm_tile<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8>(args.p[which], w - (which ? args.end[which - 1] : 0), smem);
         __syncthreads();  // the staging slabs of this tile's epilogue alias the ring the next tile fills
     }
+}
+
+// How many workgroups a launch of `wgs` adds for the modulation projections (args.ada.count panels at most; what it takes is left there): one
+// for every compute unit that it leaves idle, each as many panels as it has time for. A panel of 1536 x 64 takes such a workgroup 6 to 7 us; with
+// 5.5 / 5 instead of 6.5 / 6 forwards of 512px and its guided pair are 0.8 % slower, of 1024px 0.5 % faster. The last launch of a block may take up
+// to five panels a workgroup more than that (the cost table is a quarter below what a launch with 96 K tiles takes beside the others): a
+// launch of their own costs the 512px forward 2.8 %. A share per launch (a third of the block's panels) instead of as many as there is room:
+// 256px 0, 496x272 +3.3 %.
+template <int EPI>
+int carried_wgs(ProbSet& args, int wgs, int cus, int smem) {
+    constexpr double FIRST = 6.0, PANEL = 6.5;  // us
+    constexpr int OVER = 5;
+    const int idle = cus - wgs, want = args.ada.count;
+    args.ada.count = 0;
+    if (!carries(EPI) || want <= 0 || idle <= 0 || smem < ada_lds_bytes(ADA_CARRY_ROWS, args.ada.K)) return 0;
+    const int room = (int)((args.us - FIRST) / PANEL), rest = (want + idle - 1) / idle;
+    const int per = args.ada_last && rest <= room + OVER ? rest : room;
+    if (per <= 0) return 0;
+    args.ada.count = want < (long long)per * idle ? want : per * idle;
+    return (args.ada.count + per - 1) / per;
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false>
@@ -531,7 +561,8 @@ int launch_cfg(ProbSet& args, int n, hipStream_t st) {
     if (cus <= 0) return SD3_ERR_HIP;
     constexpr int per_cu = (160 * 1024) / smem > 1 ? 2 : 1;
     const int resident = (cus * per_cu / 8 * 8) > 8 ? (cus * per_cu / 8 * 8) : 8;
-    dim3 grid(total < resident ? total : resident), block(WM * WN * 64);
+    args.tiles_wgs = total < resident ? total : resident;
+    const dim3 grid(args.tiles_wgs + carried_wgs<EPI>(args, args.tiles_wgs, cus, smem)), block(WM * WN * 64);
     hipLaunchKernelGGL(kern, grid, block, smem, st, args);
     g_gemm_bf16_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_status("gemm_bf16");
@@ -571,6 +602,10 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     static_assert(NJ == 4 && TI >= 1 && TM * 8 % NT == 0 && TN * 8 % NT == 0, "tile shape");
     static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "the loads in flight must fit the 6-bit counter");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
+    if (carries(EPI) && (int)blockIdx.x >= args.tiles_wgs) {
+        ada_carried<NT>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
+        return;
+    }
     const int w = blockIdx.x;
     const int which = (w >= args.end[0]) + (w >= args.end[1]);
     const Prob& pr = args.p[which];
@@ -811,7 +846,10 @@ int launch_ring(ProbSet& args, int n, hipStream_t st) {
         if (i < n) total += ((args.p[i].N + TN - 1) / TN) * ((args.p[i].M + TM - 1) / TM);
         args.end[i] = total;
     }
-    hipLaunchKernelGGL(kern, dim3(total), dim3(WM * WN * 64), smem, st, args);
+    const int cus = compute_units();
+    if (cus <= 0) return SD3_ERR_HIP;
+    args.tiles_wgs = total;
+    hipLaunchKernelGGL(kern, dim3(total + carried_wgs<EPI>(args, total, cus, smem)), dim3(WM * WN * 64), smem, st, args);
     g_gemm_bf16_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_status("gemm_bf16");
 }
@@ -982,7 +1020,7 @@ static int fp8_launches(ProbSet& args, int m, int out_is_f32, int epi, int cus, 
     return launch(args, m, plan == 0 ? 4 : 0);
 }
 
-static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, bool fp8, hipStream_t st) {
+static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, bool fp8, hipStream_t st, AdaCarry* carry) {
     if (n < 1 || n > MAX_PROBS) return fail(SD3_ERR_INVALID_ARG, "gemm_bf16_grouped: 1 to %d problems (got %d)", MAX_PROBS, n);
     ProbSet args{};
     int m = 0;
@@ -1020,7 +1058,7 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
     const int cus = compute_units();
     if (cus <= 0) return SD3_ERR_HIP;
     if (fp8) return fp8_launches(args, m, out_is_f32, epi, cus, st);
-    auto launch = [&](ProbSet& pp, int count, int shape) -> int {
+    auto launch_tiles = [&](ProbSet& pp, int count, int shape) -> int {
 #define SD3_GEMM_BF16_LAUNCH(E) return out_is_f32 ? launch_shape<E, true>(shape, pp, count, cus, st) : launch_shape<E, false>(shape, pp, count, cus, st)
         switch (epi) {
             case EPI_BIAS: SD3_GEMM_BF16_LAUNCH(EPI_BIAS);
@@ -1032,6 +1070,17 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
             default: return fail(SD3_ERR_INVALID_ARG, "gemm_bf16: unknown epilogue %d", epi);
         }
 #undef SD3_GEMM_BF16_LAUNCH
+    };
+    auto launch = [&](ProbSet& pp, int count, int shape) -> int {
+        if (!carry || carry->left() <= 0) return launch_tiles(pp, count, shape);
+        constexpr double START = 3.0;  // the constant of a first round that the cost table leaves out
+        pp.ada = carry->work;
+        pp.ada.count = carry->left();
+        pp.ada_last = carry->last;
+        pp.us = (float)(START + launch_cost(pp, count, shape, cus) * (pp.p[0].then ? 2 : 1));
+        SD3_TRY(launch_tiles(pp, count, shape));
+        carry->work.first += pp.ada.count;
+        return SD3_OK;
     };
     if (then) {
         // Both layers in one launch where they are one round of small tiles, i.e. a launch's start and end are a good part of it: dual blocks
@@ -1073,8 +1122,8 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
             rest[i] = probs[i];
             rest[i].then = nullptr;
         }
-        SD3_TRY(grouped_impl(rest, n, out_is_f32, epi, false, st));
-        return grouped_impl(then, 1, out_is_f32, epi, false, st);
+        SD3_TRY(grouped_impl(rest, n, out_is_f32, epi, false, st, carry));
+        return grouped_impl(then, 1, out_is_f32, epi, false, st, carry);
     }
     if (g_gemm_bf16_tile == 192) {
         if (epi == EPI_QKV_NORM) return fail(SD3_ERR_UNSUPPORTED, "gemm_bf16: this tile shape cannot fuse the qk-norm");
@@ -1152,8 +1201,10 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
     return launch(args, m, together);
 }
 
-int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st) { return grouped_impl(probs, n, out_is_f32, epi, false, st); }
-int gemm_fp8_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st) { return grouped_impl(probs, n, out_is_f32, epi, true, st); }
+int gemm_bf16_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st, AdaCarry* carry) {
+    return grouped_impl(probs, n, out_is_f32, epi, false, st, carry);
+}
+int gemm_fp8_grouped(const GemmBf16Problem* probs, int n, int out_is_f32, int epi, hipStream_t st) { return grouped_impl(probs, n, out_is_f32, epi, true, st, nullptr); }
 
 int gemm_bf16(const bf16_t* A, const bf16_t* Wp, bool w_tiled, void* out, int out_is_f32, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
               hipStream_t st) {
