@@ -73,28 +73,6 @@ struct AttnSets {
     Ahead ahead;  // read by the workgroups from end[MAX_SETS - 1] on
 };
 
-// One load per 128-byte line of every run, the value dropped: workgroup `wg` of `wgs`, NT threads each.
-// Attention leaves HBM idle and the layers behind it wait for their weights (a launch of 333 / 1178 / 2356 / 4250 rows of mlp-1 and mlp-2
-// takes 51 / 74 / 108 / 173 us with weights from HBM, 36 / 60 / 94 / 156 from the last-level cache), so the workgroup slots that its
-// last round leaves free stream the block's remaining weights: forwards of 256px 2967 -> 2947 us, 512px 4631 -> 4548, its guided pair 6519 ->
-// 6442, 1024px 12610 -> 12505. (The same in the LayerNorm launches, 16 MB each: 256px 0.9 % slower, 1024px 0.5 % faster.)
-template <int NT>
-__device__ __forceinline__ void read_ahead(const Ahead& a, unsigned wg, unsigned wgs) {
-    constexpr uint32_t LINE = 128, UNROLL = 4;
-    const uint32_t stride = wgs * NT;
-#pragma unroll
-    for (int s = 0; s < MAX_AHEAD; s++) {
-        const uint32_t lines = a.bytes[s] / LINE;  // (runs are whole lines, or their last few bytes are left out)
-        for (uint32_t l = wg * NT + threadIdx.x; l < lines; l += stride * UNROLL) {
-            uint32_t v[UNROLL];
-#pragma unroll
-            for (uint32_t i = 0; i < UNROLL; i++) v[i] = *reinterpret_cast<const uint32_t*>(a.p[s] + (size_t)min(l + i * stride, lines - 1) * LINE);
-#pragma unroll
-            for (uint32_t i = 0; i < UNROLL; i++) asm volatile("" ::"v"(v[i]));
-        }
-    }
-}
-
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 __device__ __forceinline__ void unpack8(const uint4& u, float (&f)[8]) {

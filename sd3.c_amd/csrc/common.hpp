@@ -124,6 +124,45 @@ __device__ __forceinline__ void tile_of_workgroup(int wg, int tiles_m, int tiles
     tile_n = (t % in_group) / gsize;
 }
 
+// ---- reading ahead ----
+// Memory that launches to come are about to stream (weights); as much of it as fits a launch's idle workgroup slots is read once, in order,
+// so that it lies in the last-level cache (256 MB, shared by the XCDs) when they ask for it.
+constexpr int MAX_AHEAD = 7;
+struct Ahead {
+    const char* p[MAX_AHEAD];
+    uint32_t bytes[MAX_AHEAD];
+    // keeps the first `budget` bytes and says how many there are
+    size_t trim(size_t budget) {
+        size_t taken = 0;
+        for (int i = 0; i < MAX_AHEAD; i++) {
+            if (bytes[i] > budget - taken) bytes[i] = (uint32_t)(budget - taken);
+            taken += bytes[i];
+        }
+        return taken;
+    }
+};
+// One load per 128-byte line of every run, the value dropped: workgroup `wg` of `wgs`, NT threads each.
+// Attention leaves HBM idle and the layers behind it wait for their weights (a launch of 333 / 1178 / 2356 / 4250 rows of mlp-1 and mlp-2
+// takes 51 / 74 / 108 / 173 us with weights from HBM, 36 / 60 / 94 / 156 from the last-level cache), so the workgroup slots that its
+// last round leaves free stream the block's remaining weights: forwards of 256px 2967 -> 2947 us, 512px 4631 -> 4548, its guided pair 6519 ->
+// 6442, 1024px 12610 -> 12505. (The same in the LayerNorm launches, 16 MB each: 256px 0.9 % slower, 1024px 0.5 % faster.)
+template <int NT>
+__device__ __forceinline__ void read_ahead(const Ahead& a, unsigned wg, unsigned wgs) {
+    constexpr uint32_t LINE = 128, UNROLL = 4;
+    const uint32_t stride = wgs * NT;
+#pragma unroll
+    for (int s = 0; s < MAX_AHEAD; s++) {
+        const uint32_t lines = a.bytes[s] / LINE;  // (runs are whole lines, or their last few bytes are left out)
+        for (uint32_t l = wg * NT + threadIdx.x; l < lines; l += stride * UNROLL) {
+            uint32_t v[UNROLL];
+#pragma unroll
+            for (uint32_t i = 0; i < UNROLL; i++) v[i] = *reinterpret_cast<const uint32_t*>(a.p[s] + (size_t)min(l + i * stride, lines - 1) * LINE);
+#pragma unroll
+            for (uint32_t i = 0; i < UNROLL; i++) asm volatile("" ::"v"(v[i]));
+        }
+    }
+}
+
 // ---- modulation projections of the bf16 path ----
 // out (B, N) = y (B, K) @ W + bias, W bf16 as panels of 64 columns (N/64, K, 64). A panel is K * 128 bytes that one workgroup streams from
 // end to end; the launches' own kernel is in small_linear.hip, and a GEMM launch that leaves compute units idle takes panels of the NEXT
@@ -236,6 +275,7 @@ struct AdaCarry {
     AdaWork work{};
     int total = 0;
     bool last = false;  // the block's last launch
+    Ahead ahead{};      // what the launch may read ahead once it has taken its panels
     int left() const { return total - work.first; }
 };
 int ada_panels(const float* y, int B, int K, const AdaJob* jobs, int n, hipStream_t st);
@@ -393,13 +433,7 @@ int attention_bf16(const AttnSegments& s, int B, int NH, int HS, hipStream_t st)
 // work item each, whose partial results go through split_ws[i] (attention_bf16_split_workspace_floats floats) and are merged by a
 // second, small kernel. attention_bf16_context_splits: the number of splits that pays for the Tc context queries of a joint
 // attention next to Tx latent ones, or 0 when the plain one-set launch is the better choice.
-// ahead (or null): memory that the launches behind this one are about to stream (weights); as much of it as fits the launch's idle
-// workgroup slots is read once, in order, so that it lies in the last-level cache (256 MB, shared by the XCDs) when they ask for it.
-constexpr int MAX_AHEAD = 7;
-struct Ahead {
-    const char* p[MAX_AHEAD];
-    uint32_t bytes[MAX_AHEAD];
-};
+// ahead (or null): what the launch's idle workgroup slots read ahead.
 int attention_bf16_multi(const AttnSegments* sets, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int HS, hipStream_t st,
                          const Ahead* ahead = nullptr);
 int attention_bf16_context_splits(int Tc, int Tx, int NH, bool dual);

@@ -419,9 +419,14 @@ int attention(sd3_ctx* ctx, const AttnSegments& a, int B, int NH, int HS, bool b
     return bf ? attention_bf16(a, B, NH, HS, ctx->stream) : attention_f32(a, B, NH, HS, ctx->stream);
 }
 
-// The block. ada_c / ada_x: modulation vectors (B, chunks*C) already computed, or null to compute them here.
+struct AheadWeight {
+    const float* w;
+    int K, N;
+};
+// The block. ada_c / ada_x: modulation vectors (B, chunks*C) already computed, or null to compute them here. carry, next (the block behind
+// this one): what its GEMM launches take along, see carried_wgs.
 int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const sd3_block_weights& w, const Dims& d, const float* ada_c,
-              const float* ada_x, Bump& ws, AdaCarry* carry = nullptr) {
+              const float* ada_x, Bump& ws, AdaCarry* carry = nullptr, const sd3_block_weights* next = nullptr, bool next_dual = false) {
     hipStream_t st = ctx->stream;
     const int B = d.B, Tc = d.Tc, Tx = d.Tx, C = d.C;
     const int mc = B * Tc, mx = B * Tx;
@@ -477,6 +482,20 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     auto cchunk = [&](int k) { return ada_c + (size_t)k * C; };
     auto xchunk = [&](int k) { return ada_x + (size_t)k * C; };
     GemmEpilogueArgs none;
+    constexpr double LAST_LEVEL = 256e6;
+    bool ahead_fits = false;
+    auto read_ahead_of = [&](std::initializer_list<AheadWeight> list) -> int {
+        if (!carry || !ahead_fits) return SD3_OK;
+        int n = 0;
+        for (const AheadWeight& a : list) {
+            if (!a.w) continue;
+            const void* wp = nullptr;
+            SD3_TRY(get_packed(ctx, a.w, a.K, a.N, 0, &wp));
+            carry->ahead.p[n] = (const char*)wp;
+            carry->ahead.bytes[n++] = (uint32_t)std::min<size_t>((size_t)a.K * a.N * 2, UINT32_MAX);
+        }
+        return SD3_OK;
+    };
 
     // ---- both streams up to q,k,v (modules.cpp:1381-1423); with discard_context chunk 0 is the scale, chunk 1 the shift;
     //      the dual branch's input comes from the same normalised latent rows
@@ -551,9 +570,9 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         // hidden rows) fit the last-level cache together: with 8500 rows (1024px pair) they push each other out, the forward takes 0.4 % more.
         // (A block called alone finds its weights where its last call left them.)
         Ahead ahead{};
-        constexpr double LAST_LEVEL = 256e6;
         const double weights = 2.0 * C * C * ((1 + 2 * d.E) * (d.discard ? 1 : 2) + (d.dual ? 1 : 0)), rows = (double)(mx + mc) * C * (2 + 4 + 2 + 2 * d.E);
-        if (in_forward && !f8 && weights + rows <= LAST_LEVEL) {
+        ahead_fits = in_forward && !f8 && weights + rows <= LAST_LEVEL;
+        if (ahead_fits) {
             struct {
                 const float* w;
                 int K, N;
@@ -583,6 +602,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         GemmEpilogueArgs g2;
         g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;
         const LayerCall proj2{x_att2, w.x2_out_w, w.x2_out_b, x, C, mx, C, C, g2};
+        SD3_TRY(read_ahead_of({{w.x_mlp_w1, C, d.E * C}, {d.discard || !mc ? nullptr : w.c_mlp_w1, C, d.E * C}}));
         SD3_TRY(linear_pair(ctx, prec, proj, 2, 1, EPI_GATE_RESID, d.dual && bf ? &proj2 : nullptr, carry));
     }
 
@@ -642,11 +662,13 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     {
         LayerCall up[2] = {{x_hid, w.x_mlp_w1, w.x_mlp_b1, x_mlp, d.E * C, mx, d.E * C, C, none},
                            {c_hid, w.c_mlp_w1, w.c_mlp_b1, c_mlp, d.E * C, mcm, d.E * C, C, none}};
+        SD3_TRY(read_ahead_of({{w.x_mlp_w2, d.E * C, C}, {mcm ? w.c_mlp_w2 : nullptr, d.E * C, C}}));
         SD3_TRY(linear_pair(ctx, prec, up, 2, !bf, EPI_BIAS_GELU, nullptr, carry));
         gc.gate = cchunk(5);
         gx.gate = xchunk(5);
         LayerCall down[2] = {{x_mlp, w.x_mlp_w2, w.x_mlp_b2, x, C, mx, C, d.E * C, gx}, {c_mlp, w.c_mlp_w2, w.c_mlp_b2, c, C, mcm, C, d.E * C, gc}};
         if (carry) carry->last = true;
+        if (next) SD3_TRY(read_ahead_of({{next->x_qkv_w, C, 3 * C}, {mc ? next->c_qkv_w : nullptr, C, 3 * C}, {next_dual ? next->x2_qkv_w : nullptr, C, 3 * C}}));
         SD3_TRY(linear_pair(ctx, prec, down, 2, 1, EPI_GATE_RESID, nullptr, carry));
     }
     return SD3_OK;
@@ -1254,7 +1276,8 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     };
     //      Up to 4096 rows: beyond them the device is at its power limit, where what streams beside the matrix kernels costs them clock (4250 rows,
     //      forward against all projections up front: -1.0, 0 and +1.3 % on three devices; 2048px 0).
-    const bool carried = bf && !fp8_kind(precision) && B <= ADA_CARRY_ROWS && (long long)B * (Tx + Tc) <= 4096;
+    //      The same holds for reading weights ahead in those workgroups.
+    const bool few_rows = bf && !fp8_kind(precision) && (long long)B * (Tx + Tc) <= 4096, carried = few_rows && B <= ADA_CARRY_ROWS;
     {
         std::vector<AdaCall> calls;
         for (int l = 0; l < (carried ? 1 : num_layers); l++)
@@ -1277,7 +1300,7 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
                 carry.total += q.N / 64;
             }
         }
-        SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], base, base + (size_t)B * 6 * C, bws, &carry));
+        SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], base, base + (size_t)B * 6 * C, bws, few_rows ? &carry : nullptr, l + 1 < num_layers ? &bw[l + 1] : nullptr, l + 1 < num_layers && bd[l + 1].dual));
         if (carry.left() > 0) {  // what no launch had room for
             AdaJob rest[ADA_CARRY_JOBS];
             int n = 0, skip = carry.work.first;

@@ -84,6 +84,7 @@ struct ProbSet {
     Prob second;         // (see Prob::then)
     int tiles_wgs;       // workgroups from here on work on `ada`
     AdaWork ada;
+    Ahead ahead;
     float us;            // (host) about how long the launch takes
     bool ada_last;       // (host) no launch behind this one can take any
 };
@@ -514,6 +515,7 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet ar
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     if (carries(EPI) && !FP8 && (int)blockIdx.x >= args.tiles_wgs) {
         ada_carried<WM * WN * 64>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
+        read_ahead<WM * WN * 64>(args.ahead, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs);
         return;
     }
     for (int w = blockIdx.x; w < args.end[MAX_PROBS - 1]; w += args.tiles_wgs) {
@@ -529,18 +531,31 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet ar
 // to five panels a workgroup more than that (the cost table is a quarter below what a launch with 96 K tiles takes beside the others): a
 // launch of their own costs the 512px forward 2.8 %. A share per launch (a third of the block's panels) instead of as many as there is room:
 // 256px 0, 496x272 +3.3 %.
+// In the time that is left they read the weights ahead that the next launches ask for (args.ahead; what is read is left there). At 12, 24, 40, 60,
+// 100 KB per us and workgroup: forwards of 256px -0.9, -2.4, -3.0, -3.1, -3.3 %, its pair -6.0 from 40 on, of the 512px pair +0.1, -0.7, -1.25, -1.25,
+// -1.0, 496x272 batch 3 -0.1, -0.2, 0, +0.9, +13 (the launch is then longer for it), 512px 0 (16 to 28 idle units).
 template <int EPI>
 int carried_wgs(ProbSet& args, int wgs, int cus, int smem) {
     constexpr double FIRST = 6.0, PANEL = 6.5;  // us
+    constexpr double RATE = 40960;              // bytes per us and workgroup that reads ahead
     constexpr int OVER = 5;
     const int idle = cus - wgs, want = args.ada.count;
     args.ada.count = 0;
-    if (!carries(EPI) || want <= 0 || idle <= 0 || smem < ada_lds_bytes(ADA_CARRY_ROWS, args.ada.K)) return 0;
-    const int room = (int)((args.us - FIRST) / PANEL), rest = (want + idle - 1) / idle;
-    const int per = args.ada_last && rest <= room + OVER ? rest : room;
-    if (per <= 0) return 0;
-    args.ada.count = want < (long long)per * idle ? want : per * idle;
-    return (args.ada.count + per - 1) / per;
+    if (!carries(EPI) || idle <= 0) {
+        args.ahead = Ahead{};
+        return 0;
+    }
+    int panels = 0;  // a workgroup's
+    if (want > 0 && smem >= ada_lds_bytes(ADA_CARRY_ROWS, args.ada.K)) {
+        const int room = (int)((args.us - FIRST) / PANEL), rest = (want + idle - 1) / idle;
+        panels = args.ada_last && rest <= room + OVER ? rest : room;
+        panels = panels < 0 ? 0 : panels > rest ? rest : panels;
+        args.ada.count = want < panels * idle ? want : panels * idle;
+    }
+    const double us = args.us - (panels ? FIRST + panels * PANEL : FIRST / 2);
+    const size_t ahead = args.ahead.trim(us > 0 ? (size_t)(us * RATE * idle) : 0);
+    const int readers = (int)(ahead / 32768 < (size_t)idle ? ahead / 32768 : idle), takers = panels ? (args.ada.count + panels - 1) / panels : 0;
+    return readers > takers ? readers : takers;
 }
 
 template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false>
@@ -604,6 +619,7 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     if (carries(EPI) && (int)blockIdx.x >= args.tiles_wgs) {
         ada_carried<NT>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
+        read_ahead<NT>(args.ahead, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs);
         return;
     }
     const int w = blockIdx.x;
@@ -1072,14 +1088,16 @@ static int grouped_impl(const GemmBf16Problem* probs, int n, int out_is_f32, int
 #undef SD3_GEMM_BF16_LAUNCH
     };
     auto launch = [&](ProbSet& pp, int count, int shape) -> int {
-        if (!carry || carry->left() <= 0) return launch_tiles(pp, count, shape);
+        if (!carry) return launch_tiles(pp, count, shape);
         constexpr double START = 3.0;  // the constant of a first round that the cost table leaves out
         pp.ada = carry->work;
         pp.ada.count = carry->left();
         pp.ada_last = carry->last;
+        pp.ahead = carry->ahead;
         pp.us = (float)(START + launch_cost(pp, count, shape, cus) * (pp.p[0].then ? 2 : 1));
         SD3_TRY(launch_tiles(pp, count, shape));
         carry->work.first += pp.ada.count;
+        carry->ahead = Ahead{};  // (of the launches of a layer the first one reads)
         return SD3_OK;
     };
     if (then) {
