@@ -876,12 +876,14 @@ int launch_ring(ProbSet& args, int n, hipStream_t st) {
 // compute unit's load path and, from 128x128 on, the matrix instructions. 192x256 tiles (the persistent kernel's, like 256x256) save little
 // per tile but are there for what is left of a round: q|k|v of 2 x 1024 + 154 rows, 162 or 234 tiles, 50.2 -> 46.0 us; 128x256 beside 256x128
 // for rows that are not multiples of 256: mlp-1 of 1581 + 999 rows, 504 tiles instead of 528 in two rounds of 256, 73 -> 60 us.
+// Where 128x64 and 64x128 are the same number of rounds the former is taken: out-projection and mlp-2 of 1024 + 154 rows 16.7 -> 15.8 and 44.4 ->
+// 42.4 us; forwards of 24 x 40 patches -3.4 %, two of 256px -1.6 %, 512px +0.3 %.
 struct TileShape {
     int tm, tn;
     double fixed, per_k;
 };
 enum { TILE_64, TILE_128_64, TILE_64_128, TILE_128, TILE_256_128, TILE_128_256, TILE_192_256, TILE_256, TILE_SHAPES };
-constexpr TileShape tile_shapes[TILE_SHAPES] = {{64, 64, 1.3, 0.19},    {128, 64, 2.3, 0.285},  {64, 128, 2.3, 0.285},
+constexpr TileShape tile_shapes[TILE_SHAPES] = {{64, 64, 1.3, 0.19},    {128, 64, 2.25, 0.285}, {64, 128, 2.3, 0.285},
                                                 {128, 128, 7.3, 0.403}, {256, 128, 11.3, 0.59}, {128, 256, 11.5, 0.615},
                                                 {192, 256, 6.0, 1.315}, {256, 256, 11.3, 1.28}};
 
