@@ -181,7 +181,8 @@ __device__ __forceinline__ void store_cols(float* p, const float (&v)[NJ]) {
     *reinterpret_cast<typename Cols<NJ>::mem*>(p) = t;
 }
 
-template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
+// WHOLE_K: K is made of whole tiles in every problem
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI, bool WHOLE_K>
 __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const TileProbSet set) {
     constexpr int NT = WM * WN * 64, TI = TM / WM / 16, NJ = TN / WN / 16;
     constexpr int A_BYTES = TM * 128, STAGE_BYTES = A_BYTES + TK * TN * 4;
@@ -203,12 +204,14 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const Til
 
     const float* ga[LA];
     const float* gb[LB];
-    int ka[LA], kb[LB];  // k of the chunk within its tile
+    int ka[LA], kb[LB];            // k of the chunk within its tile
+    unsigned a_off[LA], b_off[LB];  // WHOLE_K: bytes of the chunk behind the tile's first one
 #pragma unroll
     for (int i = 0; i < LA; i++) {
         const int q = i * NT + tid, row = q >> 3;
         ka[i] = ((q & 7) ^ (row & 6)) * 4;
         ga[i] = pr.A + (long long)min(m_blk + row, M - 1) * pr.lda + ka[i];  // rows beyond M re-read the last one and are never stored
+        a_off[i] = ((unsigned)min(row, M - 1 - m_blk) * pr.lda + ka[i]) * 4;
     }
 #pragma unroll
     for (int i = 0; i < LB; i++) {
@@ -216,17 +219,40 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const Til
         kb[i] = q / CPR;
         const int c = (q % CPR) ^ ((((kb[i] >> 2) & WXM) * WX) & (CPR - 1));
         gb[i] = pr.W + (long long)kb[i] * pr.ldw + pr.n0 + min(n_blk + c * 4, N - 4);
+        b_off[i] = ((unsigned)kb[i] * pr.ldw + min(n_blk + c * 4, N - 4)) * 4;
     }
+    const char* a_tile = reinterpret_cast<const char*>(pr.A + (long long)m_blk * pr.lda);
+    const char* b_tile = reinterpret_cast<const char*>(pr.W + pr.n0);
     const long long b_step = (long long)TK * pr.ldw;
     const int nkt = (K + TK - 1) / TK;
     const float* zeros = zero_chunk;
     asm volatile("" : "+s"(zeros));  // (kept in registers: the compiler would fetch the address anew inside the loop)
     // requests the next tile (the pointers advance with every call); past the last one zeros, into a stage that nobody reads again.
     // No branches, so that the requests can be spread over the matrix instructions.
+    // WHOLE_K: one scalar address per operand that moves on and a 32-bit offset per thread that does not, which the load takes as they are: a
+    // 64-bit address per load costs the vector unit two or three operations between the matrix instructions and the load more cycles to issue. Past
+    // the end the last tile once more. 1178 x 1536 x 6144 (128x64 tiles) 207 -> 180 us, 1178 x 4608 x 1536 150 -> 135, 10656 x 3072 x 768 375 -> 352,
+    // 4096 x 6144 x 1536 557 -> 520 (149 of 157 TFLOP/s).
     auto issue_tile = [&](int kt, int stage) {
         const int left = K - kt * TK;
         char* sa = smem + stage * STAGE_BYTES + wave * 1024;
         char* sb = sa + A_BYTES;
+        if constexpr (WHOLE_K) {
+#pragma unroll
+            for (int i = 0; i < LA; i++) {
+                asm volatile("" : "+v"(a_off[i]));  // (or the compiler widens the offset outside the loop and adds it to the address inside)
+                __builtin_amdgcn_global_load_lds((glb_ptr_t)(a_tile + a_off[i]), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < LB; i++) {
+                asm volatile("" : "+v"(b_off[i]));
+                __builtin_amdgcn_global_load_lds((glb_ptr_t)(b_tile + b_off[i]), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+            }
+            const bool more = left > TK;
+            a_tile += more ? TK * 4 : 0;
+            b_tile += more ? b_step * 4 : 0;
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             __builtin_amdgcn_global_load_lds((glb_ptr_t)(ka[i] < left ? ga[i] : zeros), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
@@ -270,7 +296,7 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const Til
                 for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][i][s], b[h][s][j], acc[i][j], 0, 0, 0);
     };
     // Schedule of a half: an LDS read behind each of the first matrix instructions, then one direct load behind every second. Issued in
-    // one go the four wavefronts queue up for the LDS and the address unit while the matrix units stand still (4096 x 6144 x 1536: 618 -> 559 us, 125 -> 138 TFLOP/s).
+    // one go the four wavefronts queue up for the LDS and the address unit while the matrix units stand still (4096 x 6144 x 1536: 618 -> 559 us).
     auto spread = [&](auto loads_tag) {
         constexpr int NM = TI * NJ * 4, R = TI + 4, LOADS = decltype(loads_tag)::value ? LA + LB : 0;
         constexpr int PER_READ = NM / 2 >= R * 2 ? 2 : 1;                    // matrix instructions in front of a read
@@ -347,9 +373,9 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const Til
         }
 }
 
-template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
-int launch_tile(TileProbSet& set, int n, hipStream_t st) {
-    auto kern = gemm_f32_tile_kernel<TM, TN, WM, WN, STAGES, EPI>;
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI, bool WHOLE_K>
+int launch_tile_k(TileProbSet& set, int n, hipStream_t st) {
+    auto kern = gemm_f32_tile_kernel<TM, TN, WM, WN, STAGES, EPI, WHOLE_K>;
     constexpr int smem = STAGES * (TM * 128 + TK * TN * 4);
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
@@ -362,13 +388,20 @@ int launch_tile(TileProbSet& set, int n, hipStream_t st) {
     return launch_status("gemm_f32");
 }
 
+template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
+int launch_tile(TileProbSet& set, int n, hipStream_t st) {
+    bool whole = true;  // (and offsets within a tile of 32 bits)
+    for (int i = 0; i < n; i++) whole = whole && set.p[i].K % TK == 0 && set.p[i].lda <= (1 << 22) && set.p[i].ldw <= (1 << 22);
+    return whole ? launch_tile_k<TM, TN, WM, WN, STAGES, EPI, true>(set, n, st) : launch_tile_k<TM, TN, WM, WN, STAGES, EPI, false>(set, n, st);
+}
+
 // The tile shapes, largest first, and what one K tile (32 k values) of one output tile costs in cycles, measured over N = 1536 .. 6144
 // and K = 1536, 6144: alone on its compute unit, and with two or three workgroups sharing one (the matrix instructions alone: TM*TN/4).
 struct TileShape {
     int tm, tn;
     double alone, shared;
 };
-constexpr TileShape TILE_SHAPES[] = {{128, 128, 4690, 4660}, {128, 64, 2560, 2430}, {64, 64, 1480, 1300}, {32, 64, 890, 720}, {32, 32, 580, 410}};
+constexpr TileShape TILE_SHAPES[] = {{128, 128, 4270, 4250}, {128, 64, 2150, 2155}, {64, 64, 1150, 1100}, {32, 64, 670, 590}, {32, 32, 440, 325}};
 
 template <int EPI>
 int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
@@ -384,7 +417,6 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 }
 
 // The shape whose busiest compute unit is done first: with r output tiles on it, r * shared cycles per K tile (alone for r = 1).
-// 1024 x 1536 x 6144 (96 / 192 / 384 / 768 / 1536 tiles): 378 / 211 / 211 / 186 / 202 us.
 int pick_tile(const TileProbSet& set, int n, int cus) {
     int best = 0;
     double best_cost = 0;

@@ -120,3 +120,19 @@ def test_attention_f32(B, NH, hs, Tq, Tk):
     score_err = (hs + 3) * U * float((heads[0].abs() @ kt.abs()).max()) / hs ** 0.5
     bound = (2 * score_err + (Tk + 8) * U) * float(v.abs().max())
     assert float((out.double() - want.transpose(1, 2).reshape(B, Tq, -1)).abs().max()) <= bound
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 32, 4), (31, 96, 36), (130, 160, 132), (65, 192, 68)])
+def test_gemm_f32_depths_of_whole_k_tiles(m, k, n):
+    """Depths of one to six whole K tiles of 32 (fewer than, as many as and more than the rings hold), whose operands are addressed by one scalar and a
+    32-bit offset: for every tile shape the bound of a sum of k products in any order, and the bits of the same product 4 deeper with zeros behind it
+    (the path of all other depths)."""
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, n), (n,)))
+    want = x.double() @ W.double() + b.double()
+    bound = (k + 2) * U * (x.double().abs() @ W.double().abs() + b.double().abs())
+    deeper = M.linear(torch.cat([x, torch.zeros(m, 4, device="cuda")], 1).contiguous(), torch.cat([W, torch.zeros(4, n, device="cuda")]).contiguous(), b)
+    for tile in (-1, 0, 1, 2, 3, 4):
+        L.call("sd3_tune", b"gemm_f32_tile", tile)
+        y = M.linear(x, W, b)
+        assert ((y.double() - want).abs() <= bound).all() and torch.equal(y, deeper), tile
