@@ -97,7 +97,9 @@ typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4_t;
 
 // FP8: the operands are OCP e4m3 bytes (A (M,K) and Wp (N,K), both K-contiguous); a 128-byte LDS row then holds 128 k values and
 // the matrix instruction is v_mfma_f32_32x32x64_f8f6f4; the accumulators are multiplied by a_scale[m] * w_scale[n] in the epilogue.
-template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8>
+// WIDE: operand rows so long (more than LONG_K values) that offsets inside a tile do not fit 32 bits.
+constexpr int LONG_K = 1 << 22;
+template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8, bool WIDE>
 __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* smem) {
     constexpr int ESZ = FP8 ? 1 : 2;                  // bytes per operand element
     const char* __restrict__ A = reinterpret_cast<const char*>(pr.A);
@@ -122,30 +124,40 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
     const int m_blk = tile_m * BM, n_blk = tile_n * BN;
 
     // ---- loader: chunk q = i*NT + tid lands at LDS byte q*16 of its tile, i.e. row q/8, physical chunk q%8 ----
-    const char* ga[LA];
-    const char* gb[LB];
+    // Direct loads take one scalar address per operand, which moves on with the K tiles, and a 32-bit offset per thread, which does not: a 64-bit
+    // address per load costs the vector unit an addition between the matrix instructions. 8192 + 308 rows, 256x256 tiles, warm: q|k|v 140 -> 132 us,
+    // mlp-1 175 -> 168; the smaller tiles of the ring kernel gain 0 to 1 %; forwards 0.9 (2048px) to 1.8 % (guided 512px pair), 256px 0.
+    typedef typename std::conditional<WIDE, long long, unsigned>::type offset_t;
+    offset_t a_off[LA], b_off[LB];
     const long long row_bytes = (long long)K * ESZ;
     // bytes from one row of Wp to the next, and from one K tile to the next
     const long long w_row = !FP8 && pr.tiled ? 128 : row_bytes, w_tile = !FP8 && pr.tiled ? 128LL * N : 128;
 #pragma unroll
     for (int i = 0; i < LA; i++) {
         const int q = i * NT + tid, row = q >> 3, lc = (q & 7) ^ key(row);
-        const int m = min(m_blk + row, M - 1);  // rows beyond M re-read the last row; their results are never stored
-        ga[i] = A + (long long)m * row_bytes + lc * 16;
+        const int m = min(row, M - 1 - m_blk);  // rows beyond M re-read the last row; their results are never stored
+        a_off[i] = (offset_t)m * (offset_t)row_bytes + lc * 16;
     }
 #pragma unroll
     for (int i = 0; i < LB; i++) {
         const int q = i * NT + tid, row = q >> 3, lc = (q & 7) ^ key(row);
-        const int n = min(n_blk + row, N - 1);
-        gb[i] = Wp + n * w_row + lc * 16;
+        const int n = min(row, N - 1 - n_blk);
+        b_off[i] = (offset_t)n * (offset_t)w_row + lc * 16;
     }
+    const char *a_base = A + (long long)m_blk * row_bytes, *b_base = Wp + (long long)n_blk * w_row;
     auto issue_tile = [&](int kt, int stage) {
         char* sa = smem + stage * STAGE_BYTES + wave * 1024;
         char* sb = sa + A_BYTES;
 #pragma unroll
-        for (int i = 0; i < LA; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(ga[i] + kt * 128), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+        for (int i = 0; i < LA; i++) {
+            if (!WIDE) asm volatile("" : "+v"(a_off[i]));  // (or the compiler widens the offset outside the loop and adds it to the address inside)
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(a_base + kt * 128LL + a_off[i]), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+        }
 #pragma unroll
-        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + kt * w_tile), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+        for (int i = 0; i < LB; i++) {
+            if (!WIDE) asm volatile("" : "+v"(b_off[i]));
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(b_base + kt * w_tile + b_off[i]), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+        }
     };
 
     // bf16 uses v_mfma_f32_16x16x32_bf16: on this device the clock under matrix load is set by the power limit, and measured on
@@ -510,7 +522,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
 // Persistent kernel: one workgroup per compute unit walks over the tiles of up to three problems. The stores of a finished
 // tile drain while the next tile's K loop is already running, instead of holding the compute unit until they retire.
 // Workgroup g takes work items g, g + G, g + 2G ... (G = grid size, a multiple of 8), so it stays on its XCD's run of tiles.
-template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false>
+template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false, bool WIDE = false>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet args) {
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     if (carries(EPI) && !FP8 && (int)blockIdx.x >= args.tiles_wgs) {
@@ -520,7 +532,7 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet ar
     }
     for (int w = blockIdx.x; w < args.end[MAX_PROBS - 1]; w += args.tiles_wgs) {
         const int which = (w >= args.end[0]) + (w >= args.end[1]);
-        gemm_tile<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8>(args.p[which], w - (which ? args.end[which - 1] : 0), smem);
+        gemm_tile<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8, WIDE>(args.p[which], w - (which ? args.end[which - 1] : 0), smem);
         __syncthreads();  // the staging slabs of this tile's epilogue alias the ring the next tile fills
     }
 }
@@ -558,9 +570,9 @@ int carried_wgs(ProbSet& args, int wgs, int cus, int smem) {
     return readers > takers ? readers : takers;
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false>
+template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false, bool WIDE = false>
 int launch_cfg(ProbSet& args, int n, hipStream_t st) {
-    auto kern = gemm_bf16_kernel<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8>;
+    auto kern = gemm_bf16_kernel<BM, BN, WM, WN, STAGES, EPI, OUT_F32, FP8, WIDE>;
     constexpr int smem = smem_bytes<BM, BN, WM, WN, STAGES>();
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
@@ -583,9 +595,16 @@ int launch_cfg(ProbSet& args, int n, hipStream_t st) {
     return launch_status("gemm_bf16");
 }
 
+bool any_long(const ProbSet& set, int n) {
+    for (int i = 0; i < n; i++)
+        if (set.p[i].K > LONG_K) return true;
+    return false;
+}
+
 // fp8 operands: 256x256 tiles (variant 4) or 128x128 tiles with a ring of two stages (anything else)
 template <int EPI, bool OUT_F32>
 int launch_epi_fp8(int variant, ProbSet& args, int n, hipStream_t st) {
+    if (any_long(args, n)) return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32, true, true>(args, n, st);
     if (variant == 4) return launch_cfg<256, 256, 2, 4, 2, EPI, OUT_F32, true>(args, n, st);
     return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32, true>(args, n, st);
 }
@@ -633,22 +652,25 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     tile_of_workgroup(w - (which ? args.end[which - 1] : 0), (M + TM - 1) / TM, (N + TN - 1) / TN, tile_m, tile_n);
     const int m_blk = tile_m * TM, n_blk = tile_n * TN;
 
-    const char* ga[LA];
-    const char* gb[LB];
+    // Direct loads take one scalar address per operand, which moves on with the K tiles, and a 32-bit offset per thread, which does not
+    unsigned a_off[LA], b_off[LB];
+    const char *a_base, *b_base;
     long long w_tile;  // bytes from one K tile of the weight to the next
     auto operands = [&](const bf16_t* A, const bf16_t* Wp, bool tiled) {
-        const long long w_row = tiled ? 128 : 2LL * K;
+        const int w_row = tiled ? 128 : 2 * K;
         w_tile = tiled ? 128LL * N : 128;
+        a_base = reinterpret_cast<const char*>(A + (long long)m_blk * K);
+        b_base = reinterpret_cast<const char*>(Wp) + (long long)n_blk * w_row;
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             const int q = i * NT + tid, row = q >> 3;
-            ga[i] = reinterpret_cast<const char*>(A + (long long)min(m_blk + row, M - 1) * K) + ((q & 7) ^ swz16(row)) * 16;
+            a_off[i] = (unsigned)min(row, M - 1 - m_blk) * (2 * K) + ((q & 7) ^ swz16(row)) * 16;
         }
 #pragma unroll
         for (int i = 0; i < LB; i++) {
             const int q = i * NT + tid, row = q >> 3;
-            const int n = n_blk + row / WC * WC + NJ * (row % 16) + row % WC / 16;
-            gb[i] = reinterpret_cast<const char*>(Wp) + min(n, N - 1) * w_row + ((q & 7) ^ swz16(row)) * 16;
+            const int n = row / WC * WC + NJ * (row % 16) + row % WC / 16;
+            b_off[i] = (unsigned)min(n, N - 1 - n_blk) * w_row + ((q & 7) ^ swz16(row)) * 16;
         }
     };
     operands(pr.A, pr.Wp, pr.tiled);
@@ -656,12 +678,17 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     auto issue_tile = [&](int kt, int stage) {
         char* sa = smem + stage * STAGE_BYTES + wave * 1024;
         char* sb = sa + A_BYTES;
-        const int off = kt * 128;
-        const long long w_off = kt * w_tile;
+        const char *a = a_base + kt * 128, *b = b_base + kt * w_tile;
 #pragma unroll
-        for (int i = 0; i < LA; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(ga[i] + off), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+        for (int i = 0; i < LA; i++) {
+            asm volatile("" : "+v"(a_off[i]));  // (or the compiler widens the offset outside the loop and adds it to the address inside)
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(a + a_off[i]), (lds_ptr_t)(sa + i * NT * 16), 16, 0, 0);
+        }
 #pragma unroll
-        for (int i = 0; i < LB; i++) __builtin_amdgcn_global_load_lds((glb_ptr_t)(gb[i] + w_off), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+        for (int i = 0; i < LB; i++) {
+            asm volatile("" : "+v"(b_off[i]));
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(b + b_off[i]), (lds_ptr_t)(sb + i * NT * 16), 16, 0, 0);
+        }
     };
     f32x4_t acc[TI][NJ];
     // Fragments are fetched ahead of their matrix instructions: a whole K tile ahead where it fits the registers, else one 32-deep half
@@ -946,6 +973,7 @@ int launch_shape(int shape, ProbSet& args, int n, int cus, hipStream_t st) {
     long long tiles = 0;
     for (int i = 0; i < n; i++) tiles += tiles_of(args.p[i], shape);
     const bool one_round = tiles <= cus;
+    if (any_long(args, n)) return launch_cfg<128, 256, 1, 4, 2, EPI, OUT_F32, false, true>(args, n, st);
     if (!all_whole(args, n)) {
         if (shape == TILE_64) return launch_ring<64, 64, 4, 1, 5, 2, EPI, OUT_F32, false>(args, n, st);
         if (shape == TILE_128) return launch_ring<128, 128, 4, 2, 4, 2, EPI, OUT_F32, false>(args, n, st);
