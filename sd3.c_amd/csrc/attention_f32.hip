@@ -176,7 +176,8 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(SegDev s, int HS, float s
 // and split the KEYS (tile t goes to wavefront t % KS); K and V rows come straight from memory (L2: all workgroups of a head run on one
 // XCD) into registers, half a tile of matrix work ahead of their use; the KS partial results are merged in a fixed tree at the end.
 // This gives every SIMD work also where there are few queries: 1178 tokens and 2 heads are 20 workgroups of 128 queries with the keys in
-// one run (290 us), 592 wavefronts this way (32 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 157 us, 70 -> 109 TFLOP/s of 155.
+// one run (290 us), 592 wavefronts this way (30 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 152 us, 70 -> 112 TFLOP/s of 155 (the matrix
+// instructions alone 130, the softmax 12, the loads 9).
 //
 // Contraction order: K and Q are read as float4 along d, so step s of 16-wide chunk c contracts d = 16c + 4g + s over the lane groups
 // g = l/16. S^T registers r of a 16x16 block are keys 4g + r of query l%16: as they are, the operand of step r of O^T += V^T P^T, whose
@@ -228,33 +229,35 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
         t0 = (seg ? t - nt0 : t) * TKEYS;
         return (seg ? T1 : T0) - t0;  // keys from here to the end of the segment
     };
-    // Where a lane's chunks of a tile's rows are: scalar base and row offsets. The chunks are requested one by one, each right behind the
-    // last use of the register it goes to, so that the requests are spread over the matrix work of a whole tile.
+    // Where a lane's chunks of a tile's rows are: a scalar base and 32-bit row offsets in bytes, which the loads take as they are (as 64-bit addresses:
+    // 24 heads of 64, 1178 tokens, batch 2 160 us instead of 152, 4250 tokens 967 instead of 916; 2 heads of 128, batch 8 138 instead of 127). The
+    // chunks are requested one by one, each right behind the last use of the register it goes to, so that the requests are spread over the matrix
+    // work of a whole tile.
     struct Rows {
-        const float* base;
-        unsigned off[4 * KB];
+        const char* base;
+        unsigned off[4 * KB];  // bytes
     };
     auto k_rows = [&](int t, Rows& w) {
         int seg, t0;
         const int left = keys_of(t, seg, t0), ld = seg ? ld1 : ld0;
-        w.base = (seg ? k1 : k0) + (long long)t0 * ld;
+        w.base = reinterpret_cast<const char*>((seg ? k1 : k0) + (long long)t0 * ld);
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++) w.off[kb] = __umul24(min(16 * kb + lr, left - 1), ld) + 4 * lg;
+        for (int kb = 0; kb < KB; kb++) w.off[kb] = __umul24(min(16 * kb + lr, left - 1), 4 * ld) + 16 * lg;
     };
     auto v_rows = [&](int t, Rows& w) {
         int seg, t0;
         const int left = keys_of(t, seg, t0), ld = seg ? ld1 : ld0;
-        w.base = (seg ? v1 : v0) + (long long)t0 * ld;
+        w.base = reinterpret_cast<const char*>((seg ? v1 : v0) + (long long)t0 * ld);
 #pragma unroll
-        for (int x = 0; x < 4 * KB; x++) w.off[x] = __umul24(min(16 * (x / 4) + 4 * lg + x % 4, left - 1), ld) + 4 * lr;
+        for (int x = 0; x < 4 * KB; x++) w.off[x] = __umul24(min(16 * (x / 4) + 4 * lg + x % 4, left - 1), 4 * ld) + 16 * lr;
     };
     auto load_k = [&](const Rows& w, int c) {
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++) k[kb][c] = *reinterpret_cast<const f32x4_t*>(w.base + w.off[kb] + 16 * c);
+        for (int kb = 0; kb < KB; kb++) k[kb][c] = *reinterpret_cast<const f32x4_t*>(w.base + w.off[kb] + 64 * c);
     };
     auto load_v = [&](const Rows& w, int x) {
 #pragma unroll
-        for (int u = 0; u < NU; u++) v[x / 4][x % 4][u] = *reinterpret_cast<const f32x4_t*>(w.base + w.off[x] + 64 * u);
+        for (int u = 0; u < NU; u++) v[x / 4][x % 4][u] = *reinterpret_cast<const f32x4_t*>(w.base + w.off[x] + 256 * u);
     };
     constexpr int VECTOR_ONLY = 0x486;  // what may cross: vector, scalar and transcendental instructions and LDS exchanges
 
@@ -436,7 +439,7 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     }
     const float scale = (float)(1.0 / sqrtf((float)HS));
     const float scale2 = (float)(1.4426950408889634 / sqrt((double)HS));  // scores in powers of two: the exponentials are one instruction
-    if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 24) && a.ld_qkv[1] < (1 << 24)) {
+    if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 22) && a.ld_qkv[1] < (1 << 22)) {
         // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. (Not by the batch: a batch
         // element's result stays what it is alone.) Four key runs in both: eight, or the keys over several workgroups and a second
         // kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four
