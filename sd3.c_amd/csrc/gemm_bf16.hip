@@ -88,8 +88,8 @@ struct ProbSet {
     float us;            // (host) about how long the launch takes
     bool ada_last;       // (host) no launch behind this one can take any
 };
-// the epilogues of the layers whose launches take modulation projections along
-constexpr bool carries(int epi) { return epi == EPI_BIAS_GELU || epi == EPI_GATE_RESID || epi == EPI_QKV_NORM; }
+// the layers of a block, whose launches take modulation projections along and read ahead
+constexpr bool carries(int epi, bool out_f32) { return epi == EPI_GATE_RESID ? out_f32 : (epi == EPI_BIAS_GELU || epi == EPI_QKV_NORM) && !out_f32; }
 
 // One output tile: K loop + epilogue. `wg` is the tile's position in the XCD-aware order of its problem.
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8_t;
@@ -525,7 +525,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
 template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8 = false, bool WIDE = false>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet args) {
     extern __shared__ __attribute__((aligned(1024))) char smem[];
-    if (carries(EPI) && !FP8 && (int)blockIdx.x >= args.tiles_wgs) {
+    if (carries(EPI, OUT_F32) && !FP8 && !WIDE && (int)blockIdx.x >= args.tiles_wgs) {
         ada_carried<WM * WN * 64>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
         read_ahead<WM * WN * 64>(args.ahead, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs);
         return;
@@ -546,14 +546,14 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet ar
 // In the time that is left they read the weights ahead that the next launches ask for (args.ahead; what is read is left there). At 12, 24, 40, 60,
 // 100 KB per us and workgroup: forwards of 256px -0.9, -2.4, -3.0, -3.1, -3.3 %, its pair -6.0 from 40 on, of the 512px pair +0.1, -0.7, -1.25, -1.25,
 // -1.0, 496x272 batch 3 -0.1, -0.2, 0, +0.9, +13 (the launch is then longer for it), 512px 0 (16 to 28 idle units).
-template <int EPI>
+template <bool CARRIES>
 int carried_wgs(ProbSet& args, int wgs, int cus, int smem) {
     constexpr double FIRST = 6.0, PANEL = 6.5;  // us
     constexpr double RATE = 40960;              // bytes per us and workgroup that reads ahead
     constexpr int OVER = 5;
     const int idle = cus - wgs, want = args.ada.count;
     args.ada.count = 0;
-    if (!carries(EPI) || idle <= 0) {
+    if (!CARRIES || idle <= 0) {
         args.ahead = Ahead{};
         return 0;
     }
@@ -589,7 +589,7 @@ int launch_cfg(ProbSet& args, int n, hipStream_t st) {
     constexpr int per_cu = (160 * 1024) / smem > 1 ? 2 : 1;
     const int resident = (cus * per_cu / 8 * 8) > 8 ? (cus * per_cu / 8 * 8) : 8;
     args.tiles_wgs = total < resident ? total : resident;
-    const dim3 grid(args.tiles_wgs + carried_wgs<EPI>(args, args.tiles_wgs, cus, smem)), block(WM * WN * 64);
+    const dim3 grid(args.tiles_wgs + carried_wgs<carries(EPI, OUT_F32) && !FP8 && !WIDE>(args, args.tiles_wgs, cus, smem)), block(WM * WN * 64);
     hipLaunchKernelGGL(kern, grid, block, smem, st, args);
     g_gemm_bf16_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_status("gemm_bf16");
@@ -636,7 +636,7 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     static_assert(NJ == 4 && TI >= 1 && TM * 8 % NT == 0 && TN * 8 % NT == 0, "tile shape");
     static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "the loads in flight must fit the 6-bit counter");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
-    if (carries(EPI) && (int)blockIdx.x >= args.tiles_wgs) {
+    if (carries(EPI, OUT_F32) && WHOLE_ROWS && (int)blockIdx.x >= args.tiles_wgs) {
         ada_carried<NT>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
         read_ahead<NT>(args.ahead, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs);
         return;
@@ -679,6 +679,7 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
         char* sa = smem + stage * STAGE_BYTES + wave * 1024;
         char* sb = sa + A_BYTES;
         const char *a = a_base + kt * 128, *b = b_base + kt * w_tile;
+        asm volatile("" : "+s"(a), "+s"(b));  // (or of two tiles that are unrolled together one gets 64-bit addresses per thread again)
 #pragma unroll
         for (int i = 0; i < LA; i++) {
             asm volatile("" : "+v"(a_off[i]));  // (or the compiler widens the offset outside the loop and adds it to the address inside)
@@ -892,7 +893,7 @@ int launch_ring(ProbSet& args, int n, hipStream_t st) {
     const int cus = compute_units();
     if (cus <= 0) return SD3_ERR_HIP;
     args.tiles_wgs = total;
-    hipLaunchKernelGGL(kern, dim3(total + carried_wgs<EPI>(args, total, cus, smem)), dim3(WM * WN * 64), smem, st, args);
+    hipLaunchKernelGGL(kern, dim3(total + carried_wgs<carries(EPI, OUT_F32) && WHOLE_ROWS>(args, total, cus, smem)), dim3(WM * WN * 64), smem, st, args);
     g_gemm_bf16_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_status("gemm_bf16");
 }
