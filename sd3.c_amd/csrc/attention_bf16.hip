@@ -12,7 +12,8 @@
 //   O^T (d x queries)   += V^T . P^T   : the lane's S^T registers 8j..8j+7 are, unchanged, the P^T operand of step j
 // which needs V^T (d-major) in LDS; V rows are transposed while being staged (two keys packed per 32-bit store).
 // A wavefront owns 64 queries (two 32-query blocks), so every K / V^T fragment read from LDS feeds two matrix
-// instructions; a workgroup of 4 wavefronts shares each 64-key tile. K tiles go global -> LDS directly
+// instructions; a workgroup of 4 wavefronts shares each 64-key tile. (Launches that leave the device half empty have wavefronts of
+// 32 queries, four or eight of them in a workgroup: the rule stands at the launch.) K tiles go global -> LDS directly
 // (global_load_lds_dwordx4) into 128-byte rows with XOR-swizzled 16-byte chunks; tiles are double-buffered with one
 // barrier per tile.
 #include <type_traits>
@@ -25,9 +26,7 @@ namespace sd3 {
 namespace {
 
 constexpr int HS = 64;
-constexpr int NW = 4;            // wavefronts per workgroup
-constexpr int QW = 64;           // queries per wavefront
-constexpr int BQ = NW * QW;      // queries per workgroup
+constexpr int BQ = 256;      // queries per workgroup where a wavefront has 64 (half as many where it has 32)
 constexpr int BKV = 64;          // keys per tile
 constexpr int K_BYTES = BKV * 128, V_BYTES = BKV * 128, STAGE_BYTES = K_BYTES + V_BYTES;
 constexpr int O_PITCH = 72;      // bf16 per staged output row
@@ -43,7 +42,7 @@ constexpr int prefetch_tiles(bool norm) {
 #endif
 }
 constexpr int smem_bytes(bool norm) {
-    return ((prefetch_tiles(norm) + 2) * STAGE_BYTES > NW * QW * O_PITCH * 2) ? (prefetch_tiles(norm) + 2) * STAGE_BYTES : NW * QW * O_PITCH * 2;
+    return ((prefetch_tiles(norm) + 2) * STAGE_BYTES > BQ * O_PITCH * 2) ? (prefetch_tiles(norm) + 2) * STAGE_BYTES : BQ * O_PITCH * 2;
 }
 
 struct SegDev {
@@ -105,6 +104,15 @@ __device__ __forceinline__ bf16x8_t lds_read_b128(uint32_t lds_byte_addr, int im
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(r) : "v"(lds_byte_addr), "i"(imm_offset));
     return r;
 }
+__device__ __forceinline__ void lds_wait_k_v(bf16x8_t (&k)[4], uint2 (&v)[8]) {  // everything
+    asm volatile("s_waitcnt lgkmcnt(0)"
+                 : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3]), "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+}
+template <int HALF>
+__device__ __forceinline__ void lds_wait_v8(uint2 (&v)[8]) {  // one group of four of the transposing reads, eight newer reads on their way
+    constexpr int I = 4 * HALF;
+    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(v[I]), "+v"(v[I + 1]), "+v"(v[I + 2]), "+v"(v[I + 3]));
+}
 template <int N>
 __device__ __forceinline__ void lds_wait_k(bf16x8_t (&k)[4]) {
     static_assert(N == 0 || N == 4 || N == 8, "outstanding LDS reads behind the four K fragments");
@@ -123,16 +131,18 @@ __device__ __forceinline__ void lds_wait_last4(uint2 (&a)[8]) {
 
 // NORM: apply the per-head RMSNorm to q and k while loading them (K then goes through registers instead of the
 // direct global->LDS path). Without it q and k are taken as they are (already normalised by the QKV GEMM epilogue).
-template <bool NORM>
+// NQ: 32-query blocks of a wavefront; NW: wavefronts of a workgroup. A query's result does not depend on them.
+template <bool NORM, int NQ, int NW>
 __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnSets sets, float q_scale /* log2(e)/sqrt(64) */, float eps) {
-    constexpr int PF = prefetch_tiles(NORM);
+    constexpr int PF = prefetch_tiles(NORM), QW = 32 * NQ, CHUNKS = 512 / (NW * 64);  // 16-byte chunks of a K (V) tile per thread
+    static_assert(NQ == 2 || (NQ == 1 && !NORM), "32-query blocks of a wavefront");
     __shared__ __attribute__((aligned(1024))) char smem[smem_bytes(NORM)];
     // The barrier in the middle of a tile, which publishes tile t+1 and retires the stage of tile t-1. In front of it a thread's own
     // requests for tile t+1 must have landed -- every thread requests four 16-byte chunks per tile, so that is "all but the newest
     // 4 (PF - 1)" -- and its LDS accesses must be done. A bare barrier between compiler fences: __syncthreads() would wait for
     // every load in flight, the tiles requested further ahead included.
     auto tile_barrier = [&]() {
-        __builtin_amdgcn_s_waitcnt(((4 * (PF - 1)) & 15) | (7 << 4) | (0 << 8));  // vmcnt(4 (PF - 1)), lgkmcnt(0)
+        __builtin_amdgcn_s_waitcnt(((2 * CHUNKS * (PF - 1)) & 15) | (7 << 4) | (0 << 8));  // lgkmcnt(0)
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
@@ -170,10 +180,10 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     const int nt = min(nt_per, nt_all - split * nt_per);  // >= 1: the host chooses kv_splits so that no item is empty
 
     // ---- Q^T operands: for block qb the lane is query (q0 + 32 qb + l32); k-step ks covers d = 16 ks + 8 lk + (0..7) ----
-    const int q0 = qblk * BQ + wave * QW;
-    Frag qf[2][4];
+    const int q0 = qblk * (NW * QW) + wave * QW;
+    Frag qf[NQ][4];
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < NQ; qb++) {
         const int qt = q0 + qb * 32 + l32;
         const int seg = (qt < Tq0) ? 0 : 1;
         float f[4][8];
@@ -208,16 +218,16 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         }
     }
 
-    f32x16_t oacc[2][2];  // [d block][query block]
+    f32x16_t oacc[2][NQ];  // [d block][query block]
     // Softmax reference point m_run per query (any value works as long as numerator and denominator use the same one) and
     // this lane's share l_run of the row sum. The matrix unit subtracts the reference and masks keys beyond the sequence:
     // a score block starts from AUX . NEGM, where AUX[key][k=0] = 1, AUX[key][k=1] = (key beyond the sequence),
     // NEGM[k=0][query] = -m_run (kept representable in bf16), NEGM[k=1][query] = -1e30 and everything else is zero.
     // While the reference is zero and no key of a block is masked that product is zero, and the loop over such tiles
     // ("fast" tiles below) leaves it out.
-    float m_run[2], l_run[2];
+    float m_run[NQ], l_run[NQ];
     const uint32_t NEG_BIG_HI = pack_bf16x2(0.f, -1e30f);  // bf16(-1e30) in the upper half
-    Frag negm_f[2];
+    Frag negm_f[NQ];
     // a partial row sum of 16 probabilities above this bound (or infinite) moves the reference
     constexpr float L_BOUND = 1073741824.0f;  // 2^30
 
@@ -230,11 +240,11 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         const int seg = (t < T0) ? 0 : 1;
         return base[seg] + ((long long)b * s.T[seg] + (seg ? t - T0 : t)) * s.ld_qkv[seg] + h * HS;
     };
-    uint4 rk[2];
+    uint4 rk[CHUNKS];
     // Row pointers of this thread's two K chunks and two V chunks. Inside a segment they advance by a constant per tile;
     // they are recomputed from scratch only for the first tile, the tiles around the segment boundary and the last tile.
-    const bf16_t* kp[2];
-    const bf16_t* vp[2];
+    const bf16_t* kp[CHUNKS];
+    const bf16_t* vp[CHUNKS];
     // advance() moves the four row pointers to the tile that starts at key t0 (branches; kept out of the pipeline steps),
     // fetch_tile() issues the loads through them (straight-line; interleaved with a step's matrix instructions)
     // (the two strides are read once, here: inside advance() the set's row stride, a kernel argument selected by `which`, was a
@@ -245,14 +255,14 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         if (in0 || in1) {
             const long long step = in1 ? tile_step1 : tile_step0;
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
+            for (int i = 0; i < CHUNKS; i++) {
                 kp[i] += step;
                 vp[i] += step;
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const int q = i * 256 + tid, row = q >> 3;
+            for (int i = 0; i < CHUNKS; i++) {
+                const int q = i * (NW * 64) + tid, row = q >> 3;
                 kp[i] = kv_row_ptr(s.k, t0 + row) + ((q & 7) ^ swz(row)) * 8;
                 vp[i] = kv_row_ptr(s.v, t0 + row) + ((q & 7) ^ (2 * (row & 3))) * 8;
             }
@@ -261,17 +271,17 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     auto fetch_tile = [&](int stage_byte) {
         char* ks_ = smem + stage_byte;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < CHUNKS; i++) {
             if (NORM) rk[i] = *reinterpret_cast<const uint4*>(kp[i]);
-            else __builtin_amdgcn_global_load_lds((glb_ptr_t)kp[i], (lds_ptr_t)(ks_ + (i * 256 + wave * 64) * 16), 16, 0, 0);
-            __builtin_amdgcn_global_load_lds((glb_ptr_t)vp[i], (lds_ptr_t)(ks_ + K_BYTES + (i * 256 + wave * 64) * 16), 16, 0, 0);
+            else __builtin_amdgcn_global_load_lds((glb_ptr_t)kp[i], (lds_ptr_t)(ks_ + (i * (NW * 64) + wave * 64) * 16), 16, 0, 0);
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)vp[i], (lds_ptr_t)(ks_ + K_BYTES + (i * (NW * 64) + wave * 64) * 16), 16, 0, 0);
         }
     };
     auto store_k_normed = [&](int t0, int stage_byte) {  // NORM only: K rows pass through registers to be normalised
         char* ks_ = smem + stage_byte;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int q = i * 256 + tid, row = q >> 3, lc = (q & 7) ^ swz(row);
+        for (int i = 0; i < CHUNKS; i++) {
+            const int q = i * (NW * 64) + tid, row = q >> 3, lc = (q & 7) ^ swz(row);
             const float* w = s.rms_k[(min(t0 + row, T - 1) < T0) ? 0 : 1];
             uint4 u = rk[i];
             if (w) {
@@ -318,8 +328,9 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     //      so that neither unit waits for the other inside a wavefront. Tiles live in a ring of three LDS stages: the
     //      loads of tile t+2 are issued right after the barrier that publishes tile t+1, at which point every wavefront
     //      has finished its reads of tile t-1, whose stage they overwrite. ----
-    f32x16_t sacc[2];   // sacc[qb]: scores of the unit of query block qb that is in the pipeline
-    Frag pf[2][2];      // pf[qb][j]: its probabilities as P^T operands
+    // (One query block, NQ = 1: a unit is a key half of a tile, and "slot" below is the key half instead of the query block.)
+    f32x16_t sacc[2];   // sacc[slot]: scores of the unit of query block qb that is in the pipeline
+    Frag pf[2][2];      // pf[slot][j]: its probabilities as P^T operands
     bf16x8_t kf[4];     // K fragments of the key half whose scores are being issued
     uint2 vfr[8];       // V^T fragments of the key half whose PV products are being issued: [j][d block][keys 0-3 | 8-11 of the step]
     // AUX rows for keys key_base + l32: one persistent operand whose first register alone changes from unit to unit
@@ -329,15 +340,15 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < NQ; j++)
 #pragma unroll
                 for (int r = 0; r < 16; r++) oacc[i][j][r] = 0.f;
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
-            l_run[qb] = 0.f;
+        for (int qb = 0; qb < NQ; qb++) l_run[qb] = 0.f;
 #pragma unroll
-            for (int j = 0; j < 2; j++) pf[qb][j].u = make_uint4(0u, 0u, 0u, 0u);
-        }
+        for (int slot = 0; slot < 2; slot++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) pf[slot][j].u = make_uint4(0u, 0u, 0u, 0u);
 #pragma unroll
         for (int i = 0; i < 8; i++) vfr[i] = make_uint2(0u, 0u);
     };
@@ -349,18 +360,19 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         asm volatile("" : "+v"(lane_o));
         first_masked = T - (lane_o & 31);
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < NQ; qb++) {
             m_run[qb] = 0.f;
             negm_f[qb].u = make_uint4((lane_o >> 5) == 0 ? NEG_BIG_HI : 0u, 0u, 0u, 0u);
         }
         aux.u = make_uint4(0u, 0u, 0u, 0u);
     };
-    auto scores = [&](int qb, int key_base) {
+    auto scores = [&](int slot, int key_base) {
+        const int qb = NQ == 2 ? slot : 0;
         aux.u.x = (key_base >= first_masked) ? 0x3f803f80u : 0x00003f80u;
-        sacc[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aux.v, negm_f[qb].v, zero, 0, 0, 0);
-        sacc[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[qb][0].v, sacc[qb], 0, 0, 0);
+        sacc[slot] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aux.v, negm_f[qb].v, zero, 0, 0, 0);
+        sacc[slot] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[0], qf[qb][0].v, sacc[slot], 0, 0, 0);
 #pragma unroll
-        for (int ks = 1; ks < 4; ks++) sacc[qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[qb][ks].v, sacc[qb], 0, 0, 0);
+        for (int ks = 1; ks < 4; ks++) sacc[slot] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qf[qb][ks].v, sacc[slot], 0, 0, 0);
     };
     auto load_k = [&](int stage_byte, int kb) {
 #pragma unroll
@@ -384,13 +396,14 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         }
         return ls0 + ls1;
     };
-    // O^T += V^T . P^T for query block qb, half j of it: contracts keys 16j + {4lk..4lk+3, 8+4lk..8+4lk+3} of the key half in vfr
-    auto pv = [&](int qb, int j) {
+    // O^T += V^T . P^T for the unit of a slot, half j of it: contracts keys 16j + {4lk..4lk+3, 8+4lk..8+4lk+3} of the key half in vfr
+    auto pv = [&](int slot, int j) {
+        const int qb = NQ == 2 ? slot : 0;
 #pragma unroll
         for (int db = 0; db < 2; db++) {
             Frag vf;
             vf.u = make_uint4(vfr[(j * 2 + db) * 2].x, vfr[(j * 2 + db) * 2].y, vfr[(j * 2 + db) * 2 + 1].x, vfr[(j * 2 + db) * 2 + 1].y);
-            oacc[db][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[qb][j].v, oacc[db][qb], 0, 0, 0);
+            oacc[db][qb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[slot][j].v, oacc[db][qb], 0, 0, 0);
         }
     };
     // the V^T fragments of half j of key half kb: issued as soon as the products that used the previous contents are issued
@@ -401,22 +414,28 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
             for (int hi = 0; hi < 2; hi++)
                 vfr[(j * 2 + db) * 2 + hi] = lds_read_tr16_b64(smem_addr + stage_byte + voff[db], (kb * 32 + 16 * j + 8 * hi) * 128);
     };
-    // probabilities of the unit in sacc[qb] -> pf[qb]; returns this lane's row-sum increment
-    auto probs = [&](int qb) -> float {
+    // probabilities of the unit in sacc[slot] -> pf[slot]; returns this lane's row-sum increment
+    auto probs = [&](int slot) -> float {
         f32x16_t pr;
 #pragma unroll
-        for (int r = 0; r < 16; r++) pr[r] = __builtin_amdgcn_exp2f(sacc[qb][r]);
-        return pack_probs(pr, pf[qb]);
+        for (int r = 0; r < 16; r++) pr[r] = __builtin_amdgcn_exp2f(sacc[slot][r]);
+        return pack_probs(pr, pf[slot]);
     };
     // When the reference has to move (forced for the first units: they run with reference 0), the raw scores are
     // recovered from the matrix unit's result, the reference goes to the running maximum, what was accumulated for this
-    // query block is rescaled and the probabilities are redone.
-    auto settle = [&](int qb, float inc, bool force) {
-        if (__any(inc > L_BOUND) || force) {
+    // query block is rescaled and the probabilities are redone. Which query blocks do so depends on nothing but their own 32 queries:
+    // where an item starts again without fast tiles (below), a block that was fine with them (`safe`) keeps the reference of zero in
+    // their place (the first `n_keep` tiles), so that its bits do not depend on the queries beside it in the workgroup.
+    bool safe[NQ] = {};
+    int n_keep = 0;
+    auto settle = [&](int slot, float inc, int t, bool first) {
+        const int qb = NQ == 2 ? slot : 0;
+        const bool keep = safe[qb] && t < n_keep, force = first && t == 0;
+        if (!keep && (__any(inc > L_BOUND) || force)) {
             const float m_old = m_run[qb];
-            float tmax = fmaxf(sacc[qb][0], sacc[qb][1]);
+            float tmax = fmaxf(sacc[slot][0], sacc[slot][1]);
 #pragma unroll
-            for (int r = 2; r < 16; r += 2) tmax = fmaxf(tmax, fmaxf(sacc[qb][r], sacc[qb][r + 1]));
+            for (int r = 2; r < 16; r += 2) tmax = fmaxf(tmax, fmaxf(sacc[slot][r], sacc[slot][r + 1]));
             // lanes l and l^32 hold the two key halves of the same query and feed the same accumulators: same reference
             // (forced = the first unit of a query block: nothing has been accumulated, the reference is still zero and goes to that unit's
             // maximum wherever that lies, also far below zero, where a reference of zero would turn every probability into nothing)
@@ -434,8 +453,8 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
                 for (int r = 0; r < 16; r++) oacc[db][qb][r] *= alpha;
             f32x16_t pr;
 #pragma unroll
-            for (int r = 0; r < 16; r++) pr[r] = __builtin_amdgcn_exp2f(sacc[qb][r] + (m_old - m_ref));
-            inc = pack_probs(pr, pf[qb]);
+            for (int r = 0; r < 16; r++) pr[r] = __builtin_amdgcn_exp2f(sacc[slot][r] + (m_old - m_ref));
+            inc = pack_probs(pr, pf[slot]);
         }
         l_run[qb] += inc;
     };
@@ -464,6 +483,31 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     // One tile of the pipeline on the general path (any key may be masked, the reference may move): four steps.
     auto tile = [&](int t) {
         float inc;
+        if (NQ == 1) {
+            // One query block: the scores of a unit start from the reference that the unit before may have moved, so a step's matrix
+            // and vector work follow one another here.
+            auto step = [&](auto kb_tag) {
+                constexpr int KB = decltype(kb_tag)::value;
+                inc = probs(KB);
+                lds_wait_k_v(kf, vfr);
+                pv(KB ^ 1, 0);
+                load_v(st_cur, KB, 0);
+                pv(KB ^ 1, 1);
+                load_v(st_cur, KB, 1);
+                settle(KB, inc, t, KB == 0);
+                scores(KB ^ 1, kv0 + t * BKV + 32 * (KB + 1));
+                if (KB == 0) {
+                    tile_barrier();
+                    if (t + PF + 1 < nt) advance(kv0 + (t + PF + 1) * BKV);
+                    fetch_tile(st_ld);
+                }
+                load_k(st_nxt, KB);
+            };
+            step(std::integral_constant<int, 0>());
+            step(std::integral_constant<int, 1>());
+            rotate_stages();
+            return;
+        }
         // ---- step (t, 0, 0): PV of (t-1,1,1), each half followed by the fetch of V of key half 0 into the registers it
         //      frees; scores of (t,0,1); then fetch K of half 1 ----
         pv(1, 0);
@@ -474,7 +518,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         pv(1, 1);
         load_v(st_cur, 0, 1);
         interleave();
-        settle(0, inc, t == 0);
+        settle(0, inc, t, true);
         // ---- step (t, 0, 1): PV of (t,0,0); scores of (t,1,0) ----
         lds_wait_first4(vfr);
         pv(0, 0);
@@ -483,7 +527,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         lds_wait_last4(vfr);
         pv(0, 1);
         interleave();
-        settle(1, inc, t == 0);
+        settle(1, inc, t, true);
         // ---- step (t, 1, 0): tile t+1 becomes visible and the loads of tile t+2 set off (past the end: the last tile once
         //      more, into a stage nobody reads again); PV of (t,0,1) and fetch of V of key half 1; scores of (t,1,1); then
         //      fetch K of half 0 of tile t+1 (past the last tile: stale LDS, feeding scores that are never used) ----
@@ -499,7 +543,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         pv(1, 1);
         load_v(st_cur, 1, 1);
         interleave();
-        settle(0, inc, false);
+        settle(0, inc, t, false);
         // ---- step (t, 1, 1): PV of (t,1,0); scores of (t+1,0,0) ----
         lds_wait_first4(vfr);
         pv(0, 0);
@@ -508,7 +552,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         lds_wait_last4(vfr);
         pv(0, 1);
         interleave();
-        settle(1, inc, false);
+        settle(1, inc, t, false);
         rotate_stages();
     };
 
@@ -523,8 +567,11 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     //      operands, 1.7 % with N(0,1) operands, where the power limit and not the instruction stream sets the pace. (Also tried
     //      on this basis: the row sums as two more matrix instructions per unit, ONES . P^T, instead of 16 additions: 7.5 % faster
     //      on zeros, 3 % slower on N(0,1) operands; the requests for the next tile spread over a step: slower.) ----
-    auto fast_step = [&](auto qb_tag, auto loads_tag, auto vkb_tag, int v_stage, auto kkb_tag, int k_stage) {
-        constexpr int QB = decltype(qb_tag)::value, PQ = QB ^ 1;     // probabilities of query block QB; scores and PV of the other one
+    //      One query block (NQ = 1): the same slices; every step fetches its successor's fragments, and the barrier of a tile stands behind
+    //      the four score products of its first step, where the reads of the step before have long landed.
+    auto fast_step = [&](auto qb_tag, auto loads_tag, auto vkb_tag, int v_stage, auto kkb_tag, int k_stage, auto publish) {
+        constexpr int QB = decltype(qb_tag)::value, PQ = QB ^ 1;     // probabilities of slot QB; scores and PV of the other one
+        constexpr int SQ_ = NQ == 2 ? PQ : 0, LQ_ = NQ == 2 ? QB : 0;  // their query blocks
         constexpr bool LOADS = decltype(loads_tag)::value;          // even steps fetch K of the next key half and V of this one
         constexpr int VKB = decltype(vkb_tag)::value, KKB = decltype(kkb_tag)::value;
         // The vector instructions are written as assembly statements, which the compiler keeps in the order given (as plain
@@ -549,20 +596,23 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         auto join = [&](int c) {
             if (c >= 2) asm volatile("v_add_f32 %0, %0, %1" : "+v"(ls[c & 1]) : "v"(pair[c & 1]));
         };
-        if (!LOADS) lds_wait_k<8>(kf);  // the K fragments fetched in the step before (eight V reads may still be on their way)
+        if (!LOADS || NQ == 1) lds_wait_k<8>(kf);  // the K fragments fetched in the step before (eight V reads may still be on their way)
         // matrix instructions of the step: 0-3 scores; 4, 5 PV of key quarter 0; 6, 7 PV of quarter 1
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             if (i < 4) {
-                sacc[PQ] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[PQ][i].v, i == 0 ? zero : sacc[PQ], 0, 0, 0);
+                sacc[PQ] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[SQ_][i].v, i == 0 ? zero : sacc[PQ], 0, 0, 0);
             } else {
                 const int j = (i - 4) >> 1, db = (i - 4) & 1;
                 if (!LOADS && i == 4) lds_wait_first4(vfr);
                 if (!LOADS && i == 6) lds_wait_last4(vfr);
+                if (NQ == 1 && i == 4) lds_wait_v8<0>(vfr);
+                if (NQ == 1 && i == 6) lds_wait_v8<1>(vfr);
                 Frag vf;
                 vf.u = make_uint4(vfr[(j * 2 + db) * 2].x, vfr[(j * 2 + db) * 2].y, vfr[(j * 2 + db) * 2 + 1].x, vfr[(j * 2 + db) * 2 + 1].y);
-                oacc[db][PQ] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[PQ][j].v, oacc[db][PQ], 0, 0, 0);
+                oacc[db][SQ_] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[PQ][j].v, oacc[db][SQ_], 0, 0, 0);
             }
+            if (i == 3) publish();
             if (LOADS && i == 3) {
 #pragma unroll
                 for (int ks = 0; ks < 4; ks++) kf[ks] = lds_read_b128(smem_addr + k_stage + koff[ks], KKB * 32 * 128);
@@ -589,7 +639,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
                 float both;
                 asm volatile("v_add_f32 %0, %1, %2" : "=v"(both) : "v"(ls[0]), "v"(ls[1]));
                 asm volatile("v_nop");
-                asm volatile("v_add_f32 %0, %0, %1" : "+v"(l_run[QB]) : "v"(both));
+                asm volatile("v_add_f32 %0, %0, %1" : "+v"(l_run[LQ_]) : "v"(both));
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -601,14 +651,23 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         const std::integral_constant<int, 1> I1;
         const std::integral_constant<bool, true> YES;
         const std::integral_constant<bool, false> NO;
-        fast_step(I0, YES, I0, st_cur, I1, st_cur);  // (t,0,0): V of key half 0, K of key half 1
-        fast_step(I1, NO, I0, 0, I0, 0);             // (t,0,1)
-        tile_barrier();
-        if (t + PF + 1 < nt) advance(kv0 + (t + PF + 1) * BKV);
-        fetch_tile(st_ld);
-        __builtin_amdgcn_sched_barrier(0);
-        fast_step(I0, YES, I1, st_cur, I0, st_nxt);  // (t,1,0): V of key half 1, K of key half 0 of tile t+1
-        fast_step(I1, NO, I0, 0, I0, 0);             // (t,1,1)
+        auto nothing = [] {};
+        auto publish = [&]() {
+            tile_barrier();
+            if (t + PF + 1 < nt) advance(kv0 + (t + PF + 1) * BKV);
+            fetch_tile(st_ld);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if constexpr (NQ == 1) {
+            fast_step(I0, YES, I0, st_cur, I0, st_nxt, publish);  // (t,0): V of key half 0, K of key half 0 of tile t+1
+            fast_step(I1, YES, I1, st_cur, I1, st_nxt, nothing);  // (t,1): V of key half 1, K of key half 1 of tile t+1
+        } else {
+            fast_step(I0, YES, I0, st_cur, I1, st_cur, nothing);  // (t,0,0): V of key half 0, K of key half 1
+            fast_step(I1, NO, I0, 0, I0, 0, nothing);             // (t,0,1)
+            publish();
+            fast_step(I0, YES, I1, st_cur, I0, st_nxt, nothing);  // (t,1,0): V of key half 1, K of key half 0 of tile t+1
+            fast_step(I1, NO, I0, 0, I0, 0, nothing);             // (t,1,1)
+        }
         rotate_stages();
     };
 
@@ -642,7 +701,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
             if (nt > 1) {
                 advance(first_key + BKV);
                 fetch_tile(STAGE_BYTES);
-                __builtin_amdgcn_s_waitcnt((7 << 4) | (0 << 8) | 4);  // vmcnt(4): all but the four loads of tile 1; lgkmcnt(0)
+                __builtin_amdgcn_s_waitcnt((7 << 4) | (0 << 8) | (2 * CHUNKS));  // all but the loads of tile 1; lgkmcnt(0)
             } else {
                 __builtin_amdgcn_s_waitcnt((7 << 4) | (0 << 8));
             }
@@ -654,7 +713,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
             fetch_tile(STAGE_BYTES);
             if (nt > 2) advance(first_key + 2 * BKV);
             fetch_tile(2 * STAGE_BYTES);
-            __builtin_amdgcn_s_waitcnt((7 << 4) | (0 << 8) | 8);  // vmcnt(8): all but the eight loads of tiles 1 and 2; lgkmcnt(0)
+            __builtin_amdgcn_s_waitcnt((7 << 4) | (0 << 8) | (4 * CHUNKS));  // all but the loads of tiles 1 and 2; lgkmcnt(0)
             st_cur = 0, st_nxt = STAGE_BYTES, st_nx2 = 2 * STAGE_BYTES, st_ld = 3 * STAGE_BYTES;
         }
         asm volatile("" ::: "memory");  // (a bare barrier: __syncthreads() would wait for the tiles requested ahead as well)
@@ -662,16 +721,21 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         asm volatile("" ::: "memory");
         load_k(0, 0);
         scores(0, kv0);
+        if (NQ == 1) load_k(0, 1);
 
         // verdict on the fast tiles so far, the same for every wavefront of the workgroup: flags raised in front of a barrier, read behind it
         auto unsafe = [&]() -> bool {
-            const bool bad = !(l_run[0] <= L_HUGE && l_run[1] <= L_HUGE) || l_run[0] < L_TINY || l_run[1] < L_TINY;
             volatile int* flag = &unsafe_flag;
-            if (__any(bad)) *flag = 1;
+#pragma unroll
+            for (int qb = 0; qb < NQ; qb++) {
+                safe[qb] = !__any(!(l_run[qb] <= L_HUGE) || l_run[qb] < L_TINY);
+                if (!safe[qb]) *flag = 1;
+            }
             __syncthreads();
             return __builtin_amdgcn_readfirstlane(*flag) != 0;
         };
         for (int t = 0; t < n_fast; t++) fast_tile(t);
+        if (NQ == 1 && n_fast > 0) lds_wait_k_v(kf, vfr);  // the last fast step's fetches
         const bool redo = n_fast > 0 && unsafe();
         if (!redo) {
             if (n_fast > 0) zero_reference();
@@ -681,8 +745,10 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         // start again without fast tiles, once every wavefront is done with the LDS stages and no load into them is in flight
         __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
         __syncthreads();
+        n_keep = n_fast;
         n_fast = 0;
     }
+    if (NQ == 1) lds_wait_k_v(kf, vfr);
     pv(1, 0);  // PV of the last unit
     pv(1, 1);
     __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // the redundant loads issued past the last tile have landed before LDS is reused
@@ -693,9 +759,9 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     asm volatile("" : "+v"(lane_e));
     const int l32e = lane_e & 31, lke = lane_e >> 5;
     // ---- an item of a split: leave the unnormalised accumulators, the reference and the row sum for the combining kernel ----
-    if (s.kv_splits > 1) {
+    if (NQ == 2 && s.kv_splits > 1) {
 #pragma unroll
-        for (int qb = 0; qb < 2; qb++) {
+        for (int qb = 0; qb < NQ; qb++) {
             const long long prow = (long long)item * BQ + wave * QW + qb * 32 + l32e;
             const float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 32, 64);
             if (lke == 0) *reinterpret_cast<float2*>(s.part_ml + prow * 2) = make_float2(m_run[qb], l_tot);
@@ -712,7 +778,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     __syncthreads();
     bf16_t* Ow = reinterpret_cast<bf16_t*>(smem) + wave * QW * O_PITCH;
 #pragma unroll
-    for (int qb = 0; qb < 2; qb++) {
+    for (int qb = 0; qb < NQ; qb++) {
         const float l_tot = l_run[qb] + __shfl_xor(l_run[qb], 32, 64);
         const float inv = 1.0f / l_tot;
 #pragma unroll
@@ -728,9 +794,9 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // 64 rows x 8 chunks per wavefront = 512 chunks, 8 per lane_e
+    // QW rows x 8 chunks per wavefront
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
+    for (int i = 0; i < 4 * NQ; i++) {
         const int c = lane_e + i * 64;
         const int row = c >> 3, ch = c & 7;
         const int t = q0 + row;
@@ -1316,7 +1382,7 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     if (hs != HS) return fail(SD3_ERR_UNSUPPORTED, "attention (bf16): head_dim must be 64 (got %d)", hs);
     if (B <= 0 || NH <= 0) return SD3_OK;
     AttnSets sets{};
-    bool norm = false;
+    bool norm = false, any_split = false;
     int m = 0, total = 0, longest = 0;
     for (int i = 0; i < n; i++) {
         const AttnSegments& a = jobs[i];
@@ -1332,6 +1398,7 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
             if (per * (S - 1) >= nt_all) return fail(SD3_ERR_INVALID_ARG, "attention: %d key splits leave an empty one for %d keys", S, T);
             if (!split_ws || !split_ws[i]) return fail(SD3_ERR_INVALID_ARG, "attention: a split set needs its workspace");
             s.kv_splits = S;
+            any_split = true;
             s.part_o = split_ws[i];
             s.part_ml = split_ws[i] + (size_t)B * NH * s.nqb * S * BQ * HS;
         }
@@ -1341,10 +1408,10 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     if (m == 0) return SD3_OK;
     for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
     const float q_scale = 1.4426950408889634f / sqrtf((float)HS);
-    // Workgroups that read ahead: the slots (two per compute unit) that the last round of `items` leaves free, for about as long as that
+    // Workgroups that read ahead: the slots (`per_cu` per compute unit) that the last round of `items` leaves free, for about as long as that
     // round lasts (a key tile is about 1 us), at a rate well below what HBM gives the same number of workgroups.
-    auto readers = [&](int items) -> int {
-        const int slots = 2 * compute_units();
+    auto readers = [&](int items, int per_cu) -> int {
+        const int slots = per_cu * compute_units();
         if (!ahead || slots <= 0) return 0;
         const int idle = (slots - items % slots) % slots;
         const size_t per_wg = (size_t)6144 * (3 + (longest + BKV - 1) / BKV);
@@ -1359,31 +1426,55 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
         constexpr size_t LEAST = 32768;  // one line per thread
         return (int)std::min<size_t>(idle, (taken + LEAST - 1) / LEAST);
     };
-    if (!norm && longest <= SHORT_KEYS) {
-        auto items = [&](int queries) {  // (a split along the keys happens inside the kernels: kv_splits does not apply)
-            total = 0;
-            for (int i = 0; i < MAX_SETS; i++) {
-                SegDev& s = sets.set[i];
-                if (i < m) {
-                    s.nqb = (s.Tq[0] + s.Tq[1] + queries - 1) / queries;
-                    total += s.nqb * NH * B;
-                }
-                sets.end[i] = total;
+    auto items = [&](int queries) {  // the sets cut into blocks of that many queries
+        total = 0;
+        for (int i = 0; i < MAX_SETS; i++) {
+            SegDev& s = sets.set[i];
+            if (i < m) {
+                s.nqb = (s.Tq[0] + s.Tq[1] + queries - 1) / queries;
+                total += s.nqb * NH * B;
             }
-            return total;
-        };
-        const int cus = compute_units();
-        if (cus <= 0) return SD3_ERR_HIP;
+            sets.end[i] = total;
+        }
+        return total;
+    };
+    const int cus = compute_units();
+    if (cus <= 0) return SD3_ERR_HIP;
+    if (!norm && longest <= SHORT_KEYS) {  // (a split along the keys happens inside the kernels: kv_splits does not apply)
         const bool split = items(SQ) <= 3 * cus;  // three of its workgroups fit a compute unit
         if (!split) items(WAVES * SQ);
-        const dim3 grid((unsigned)(total + readers(total)));
+        const dim3 grid((unsigned)(total + readers(total, 2)));
         if (split) hipLaunchKernelGGL(flash_attn_bf16_split_kernel, grid, dim3(RUNS * 64), 0, st, sets, q_scale);
         else hipLaunchKernelGGL(flash_attn_bf16_runs_kernel, grid, dim3(WAVES * 64), 0, st, sets, q_scale);
         return launch_status("flash_attention_bf16");
     }
-    dim3 grid((unsigned)(total + readers(total))), block(NW * 64);
-    if (norm) hipLaunchKernelGGL(flash_attn_bf16_kernel<true>, grid, block, 0, st, sets, q_scale, 1e-6f);
-    else hipLaunchKernelGGL(flash_attn_bf16_kernel<false>, grid, block, 0, st, sets, q_scale, 1e-6f);
+    // A wavefront of 64 queries feeds two matrix instructions with every fragment it reads, which is what many workgroups want; but where
+    // there are fewer workgroups than compute units it is one serial chain per SIMD (1.0 us per key tile), and half the queries are
+    // done in 0.65 us. So: workgroups of 128 queries, four wavefronts of 32, as long as each has a compute unit of its own, or where they
+    // are resident at once, two on a unit, while those of 256 queries need a second round; else, below one workgroup of 256 queries per unit,
+    // eight wavefronts of 32 queries in it. us, random operands, 4 wavefronts of 64 | 4 of 32 | 8 of 32 queries:
+    //   1178 tokens, 24 heads, batch 1, 2, 4:      26.9 27.5 43.9 | 19.4 27.2 50.9 | 24.2 25.8 49.0
+    //   621 tokens, 24 heads, batch 1, 2, 3, 4:    18.0 18.5 19.0 25.8 | 13.0 13.6 18.0 19.3 | 16.0 16.2 16.8 30.6
+    //   420 tokens, 24 heads, batch 1, 3:          15.1 16.2 | 10.6 14.8 | 12.9 14.0
+    //   2458 tokens, 24 heads, batch 1:            45.8 | 47.4 | 44.6
+    //   4096 tokens, 8, 12, 15 heads:              64.1 65.1 69.1 | 46.3 66.2 71.8 | 61.4 62.4 68.3
+    //   8192 tokens, 8 heads (a unit each):        132.4 | 140.9 | 134.6
+    // All three round alike.
+    if (!norm && !any_split) {
+        const int wide = total, narrow = items(BQ / 2);
+        if (narrow <= (wide > cus ? 2 * cus : cus)) {
+            hipLaunchKernelGGL((flash_attn_bf16_kernel<false, 1, 4>), dim3((unsigned)(total + readers(total, 2))), dim3(256), 0, st, sets, q_scale, 1e-6f);
+            return launch_status("flash_attention_bf16");
+        }
+        items(BQ);
+        if (wide < cus) {  // (a unit's registers hold one such workgroup)
+            hipLaunchKernelGGL((flash_attn_bf16_kernel<false, 1, 8>), dim3((unsigned)(total + readers(total, 1))), dim3(512), 0, st, sets, q_scale, 1e-6f);
+            return launch_status("flash_attention_bf16");
+        }
+    }
+    dim3 grid((unsigned)(total + readers(total, 2))), block(BQ);
+    if (norm) hipLaunchKernelGGL((flash_attn_bf16_kernel<true, 2, 4>), grid, block, 0, st, sets, q_scale, 1e-6f);
+    else hipLaunchKernelGGL((flash_attn_bf16_kernel<false, 2, 4>), grid, block, 0, st, sets, q_scale, 1e-6f);
     SD3_TRY(launch_status("flash_attention_bf16"));
     for (int i = 0; i < m; i++) {
         const SegDev& s = sets.set[i];
