@@ -70,6 +70,8 @@ struct AttnSets {
     SegDev set[MAX_SETS];
     int end[MAX_SETS];
     Ahead ahead;  // read by the workgroups from end[MAX_SETS - 1] on
+    AdaWork ada;  // modulation panels: done by the first `ada_wgs` of those before they read
+    int ada_wgs;
 };
 
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
@@ -148,7 +150,12 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         asm volatile("" ::: "memory");
     };
     if (blockIdx.x >= (unsigned)sets.end[MAX_SETS - 1]) {
-        read_ahead<NW * 64>(sets.ahead, blockIdx.x - sets.end[MAX_SETS - 1], gridDim.x - sets.end[MAX_SETS - 1]);
+        const int extra = blockIdx.x - sets.end[MAX_SETS - 1];
+        if (NQ == 1 && extra < sets.ada_wgs) {
+            if (sets.ada.B == 1) ada_carried_rows<NW * 64, 1>(sets.ada, extra, sets.ada_wgs, smem);
+            else ada_carried_rows<NW * 64, 2>(sets.ada, extra, sets.ada_wgs, smem);
+        }
+        read_ahead<NW * 64>(sets.ahead, extra, gridDim.x - sets.end[MAX_SETS - 1]);
         return;
     }
     const int which = (blockIdx.x >= (unsigned)sets.end[0]) + (blockIdx.x >= (unsigned)sets.end[1]);  // uniform
@@ -819,7 +826,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
 //  * many: a wavefront takes all runs of 32 queries of its own, one behind the other, and the workgroup shares the tiles
 //    (flash_attn_bf16_runs_kernel): a quarter of the loads, and the queries scaled, the states merged and the results stored once.
 // Both round alike, so the results do not depend on the choice. It is the first kernel as long as its workgroups are resident at once, three
-// per compute unit. 24 heads, us, kernel above | split | runs:
+// per compute unit. 24 heads, us, kernel above (64 queries per wavefront) | split | runs:
 //   141 tokens, batch  4, 6, 8, 16:            10.6 10.7 10.9 14.6           |  7.2  8.7 12.5 18.3           |  8.7 10.7 10.8 13.4
 //   333 tokens, batch  1, 2, 3, 4, 8, 16, 32:  14.1 14.2 14.3 14.5 20.1 32 58 | 7.6 10.1 13.7 15.9 25.8 47 88 | 11.9 12.0 12.2 14.6 18.1 29 47
 //   410 tokens, batch  1, 2, 3, 4, 8, 16, 24:  14.7 15.1 15.1 15.5 22.2 35 54 | 9.0 11.8 15.7 18.2 33.7 60 88 | 12.8 13.1 15.9 16.2 20.6 37 51
@@ -1377,7 +1384,7 @@ size_t attention_bf16_split_workspace_floats(int B, int NH, int Tc, int splits) 
 }
 
 int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int hs, hipStream_t st,
-                         const Ahead* ahead) {
+                         const Ahead* ahead, AdaCarry* carry) {
     if (n < 1 || n > MAX_SETS) return fail(SD3_ERR_INVALID_ARG, "attention: 1 to %d sets per launch (got %d)", MAX_SETS, n);
     if (hs != HS) return fail(SD3_ERR_UNSUPPORTED, "attention (bf16): head_dim must be 64 (got %d)", hs);
     if (B <= 0 || NH <= 0) return SD3_OK;
@@ -1460,17 +1467,31 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     //   4096 tokens, 8, 12, 15 heads:              64.1 65.1 69.1 | 46.3 66.2 71.8 | 61.4 62.4 68.3
     //   8192 tokens, 8 heads (a unit each):        132.4 | 140.9 | 134.6
     // All three round alike.
+    // Modulation panels of the next block in workgroups on the compute units that have none of the launch's own, as many as fit the launch (the
+    // times of a panel and of a workgroup's start as in the GEMM launches). Dual blocks of 512px leave their GEMM launches, 240 of 256
+    // tiles, room for 254 of 360 panels: the rest, a launch of 11 us, fits the 40 units free here.
+    auto take_panels = [&](double tile_us) {
+        constexpr double START = 6.0, FIRST = 6.0, PANEL = 6.5;
+        const int idle = cus - total;
+        if (!carry || carry->left() <= 0 || idle <= 0 || B > 2 || ada_lds_bytes(B, carry->work.K) > smem_bytes(false)) return;
+        const int room = (int)((START + tile_us * ((longest + BKV - 1) / BKV) - FIRST) / PANEL), panels = std::min(room, (carry->left() + idle - 1) / idle);
+        if (panels <= 0) return;
+        sets.ada = carry->work;
+        sets.ada.count = std::min(carry->left(), panels * idle);
+        sets.ada_wgs = (sets.ada.count + panels - 1) / panels;
+    };
+    auto launch_32 = [&](auto kern, int threads, int per_cu, double tile_us) -> int {
+        take_panels(tile_us);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(total + std::max(readers(total, per_cu), sets.ada_wgs))), dim3(threads), 0, st, sets, q_scale, 1e-6f);
+        SD3_TRY(launch_status("flash_attention_bf16"));
+        if (carry) carry->work.first += sets.ada.count;
+        return SD3_OK;
+    };
     if (!norm && !any_split) {
         const int wide = total, narrow = items(BQ / 2);
-        if (narrow <= (wide > cus ? 2 * cus : cus)) {
-            hipLaunchKernelGGL((flash_attn_bf16_kernel<false, 1, 4>), dim3((unsigned)(total + readers(total, 2))), dim3(256), 0, st, sets, q_scale, 1e-6f);
-            return launch_status("flash_attention_bf16");
-        }
+        if (narrow <= (wide > cus ? 2 * cus : cus)) return launch_32(flash_attn_bf16_kernel<false, 1, 4>, 256, 2, 0.65);
         items(BQ);
-        if (wide < cus) {  // (a unit's registers hold one such workgroup)
-            hipLaunchKernelGGL((flash_attn_bf16_kernel<false, 1, 8>), dim3((unsigned)(total + readers(total, 1))), dim3(512), 0, st, sets, q_scale, 1e-6f);
-            return launch_status("flash_attention_bf16");
-        }
+        if (wide < cus) return launch_32(flash_attn_bf16_kernel<false, 1, 8>, 512, 1, 0.95);  // (a unit's registers hold one such workgroup)
     }
     dim3 grid((unsigned)(total + readers(total, 2))), block(BQ);
     if (norm) hipLaunchKernelGGL((flash_attn_bf16_kernel<true, 2, 4>), grid, block, 0, st, sets, q_scale, 1e-6f);

@@ -435,7 +435,7 @@ int attention_bf16(const AttnSegments& s, int B, int NH, int HS, hipStream_t st)
 // attention next to Tx latent ones, or 0 when the plain one-set launch is the better choice.
 // ahead (or null): what the launch's idle workgroup slots read ahead.
 int attention_bf16_multi(const AttnSegments* sets, const int* kv_splits, float* const* split_ws, int n, int B, int NH, int HS, hipStream_t st,
-                         const Ahead* ahead = nullptr);
+                         const Ahead* ahead = nullptr, AdaCarry* carry = nullptr);
 int attention_bf16_context_splits(int Tc, int Tx, int NH, bool dual);
 size_t attention_bf16_split_workspace_floats(int B, int NH, int Tc, int splits);
 

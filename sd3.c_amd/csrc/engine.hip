@@ -588,7 +588,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
             }
         }
         ProfScope ps(ctx, SD3_PROF_ATTENTION, flop, 1 + ((ctx_splits && !d.discard) ? 1 : 0));  // (+ the kernel that merges the key splits)
-        SD3_TRY(attention_bf16_multi(sets, splits, wsp, n, B, d.NH, d.HS, st, &ahead));  // q and k arrive normalised
+        SD3_TRY(attention_bf16_multi(sets, splits, wsp, n, B, d.NH, d.HS, st, &ahead, carry));  // q and k arrive normalised
     } else {
         SD3_TRY(attention(ctx, joint, B, d.NH, d.HS, bf));
     }

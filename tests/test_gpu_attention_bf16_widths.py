@@ -2,8 +2,10 @@
 import pytest
 import torch
 
-from gpu_util import M  # noqa: F401  (loads the package)
+from gpu_util import M
 from sd3_c_amd import lib as L
+from sd3_c_amd.config import DiTConfig
+from sd3_c_amd.params import dit_param_shapes
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +49,22 @@ def test_attention_bf16_of_a_batch_element_alone(B, T0, T1, NH, kind):
     want = (torch.softmax(q @ k.transpose(2, 3).contiguous() / 8, -1) @ v).transpose(1, 2).reshape(B, T0 + T1, NH * 64)
     assert torch.isfinite(got).all()
     assert float((got.float() - want).norm() / want.norm()) <= (1e-2 if kind == "plain" else 3e-2)
+
+
+@pytest.mark.parametrize("C,Tc,h,w", [(64, 1, 20, 21), (192, 9, 32, 33), (320, 77, 20, 18), (1536, 154, 32, 34)])
+def test_modulation_taken_along_by_attention(C, Tc, h, w):
+    """One or two batch elements have modulation vectors of the next block computed in the attention launch's free compute units, six by a
+    launch of their own: every element has the same bits either way."""
+    cfg = DiTConfig(num_layers=3, dual_attention_layers=(0, 2), emb_dim=C, attn_heads=C // 64, pooled_dim=64, captions_dim=64, pos_embed_max_size=64, base_height=32)
+    g = torch.Generator(device="cuda").manual_seed(C + Tc)
+    P = {n: (1 if "rmsnorm" in n else 0) + 0.05 * torch.randn(s, device="cuda", generator=g) for n, s in dit_param_shapes(cfg).items()}
+    a = [torch.randn(s, device="cuda", generator=g) for s in ((6, 64), (6, Tc, 64), (6, 16, 2 * h, 2 * w))] + [1000 * torch.rand(6, device="cuda", generator=g)]
+    den = M.Denoiser(P, cfg, "bf16")
+    try:
+        whole = den(*a).clone()
+        for first, n in ((0, 1), (5, 1), (2, 2)):
+            part = [t[first:first + n].contiguous() for t in a]
+            got = [den(*part).clone() for _ in range(2)]
+            assert torch.equal(got[0], whole[first:first + n]) and torch.equal(got[1], got[0]), (first, n)
+    finally:
+        den.ctx.close()
