@@ -1415,13 +1415,13 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     if (m == 0) return SD3_OK;
     for (int i = m; i < MAX_SETS; i++) sets.end[i] = total;
     const float q_scale = 1.4426950408889634f / sqrtf((float)HS);
-    // Workgroups that read ahead: the slots (`per_cu` per compute unit) that the last round of `items` leaves free, for about as long as that
-    // round lasts (a key tile is about 1 us), at a rate well below what HBM gives the same number of workgroups.
-    auto readers = [&](int items, int per_cu) -> int {
-        const int slots = per_cu * compute_units();
-        if (!ahead || slots <= 0) return 0;
+    const int cus = compute_units();
+    if (cus <= 0) return SD3_ERR_HIP;
+    // Workgroups that read ahead: the slots (`per_cu` per compute unit) that the last round of `items` leaves free, `per_wg` bytes each.
+    auto readers = [&](int items, int per_cu, size_t per_wg) -> int {
+        const int slots = per_cu * cus;
+        if (!ahead) return 0;
         const int idle = (slots - items % slots) % slots;
-        const size_t per_wg = (size_t)6144 * (3 + (longest + BKV - 1) / BKV);
         size_t left = per_wg * idle, taken = 0;
         for (int i = 0; i < MAX_AHEAD; i++) {
             const uint32_t b = (uint32_t)std::min<size_t>(ahead->bytes[i], left);
@@ -1445,12 +1445,13 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
         }
         return total;
     };
-    const int cus = compute_units();
-    if (cus <= 0) return SD3_ERR_HIP;
+    // Beside other workgroups of the launch they read for about as long as the last round lasts (a key tile is about 1 us), at a rate well below
+    // what HBM gives the same number of workgroups.
+    const size_t beside = (size_t)6144 * (3 + (longest + BKV - 1) / BKV);
     if (!norm && longest <= SHORT_KEYS) {  // (a split along the keys happens inside the kernels: kv_splits does not apply)
         const bool split = items(SQ) <= 3 * cus;  // three of its workgroups fit a compute unit
         if (!split) items(WAVES * SQ);
-        const dim3 grid((unsigned)(total + readers(total, 2)));
+        const dim3 grid((unsigned)(total + readers(total, 2, beside)));
         if (split) hipLaunchKernelGGL(flash_attn_bf16_split_kernel, grid, dim3(RUNS * 64), 0, st, sets, q_scale);
         else hipLaunchKernelGGL(flash_attn_bf16_runs_kernel, grid, dim3(WAVES * 64), 0, st, sets, q_scale);
         return launch_status("flash_attention_bf16");
@@ -1470,30 +1471,35 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     // Modulation panels of the next block in workgroups on the compute units that have none of the launch's own, as many as fit the launch (the
     // times of a panel and of a workgroup's start as in the GEMM launches). Dual blocks of 512px leave their GEMM launches, 240 of 256
     // tiles, room for 254 of 360 panels: the rest, a launch of 11 us, fits the 40 units free here.
+    int panels = 0;  // a workgroup's
     auto take_panels = [&](double tile_us) {
         constexpr double START = 6.0, FIRST = 6.0, PANEL = 6.5;
         const int idle = cus - total;
         if (!carry || carry->left() <= 0 || idle <= 0 || B > 2 || ada_lds_bytes(B, carry->work.K) > smem_bytes(false)) return;
-        const int room = (int)((START + tile_us * ((longest + BKV - 1) / BKV) - FIRST) / PANEL), panels = std::min(room, (carry->left() + idle - 1) / idle);
+        const int room = (int)((START + tile_us * ((longest + BKV - 1) / BKV) - FIRST) / PANEL);
+        panels = std::min(room, (carry->left() + idle - 1) / idle);
         if (panels <= 0) return;
         sets.ada = carry->work;
         sets.ada.count = std::min(carry->left(), panels * idle);
         sets.ada_wgs = (sets.ada.count + panels - 1) / panels;
     };
-    auto launch_32 = [&](auto kern, int threads, int per_cu, double tile_us) -> int {
+    auto launch_32 = [&](auto kern, int threads, double tile_us) -> int {
         take_panels(tile_us);
-        hipLaunchKernelGGL(kern, dim3((unsigned)(total + std::max(readers(total, per_cu), sets.ada_wgs))), dim3(threads), 0, st, sets, q_scale, 1e-6f);
+        // These workgroups read on compute units of their own, so they may take more: with 6, 12, 15, 20, 30 and 40 KB per key tile (and with 6, also in the free
+        // slots beside the launch's own workgroups) forwards of 512px 4127, 4095, 4055, 4042, 4082, 4186 us, 24 x 40 patches 4088, 4060, 4031, 4019, 4075, 4175.
+        const size_t per_wg = (size_t)16384 * (3 + (longest + BKV - 1) / BKV);
+        hipLaunchKernelGGL(kern, dim3((unsigned)(total + std::max(readers(total, 1, per_wg), sets.ada_wgs))), dim3(threads), 0, st, sets, q_scale, 1e-6f);
         SD3_TRY(launch_status("flash_attention_bf16"));
         if (carry) carry->work.first += sets.ada.count;
         return SD3_OK;
     };
     if (!norm && !any_split) {
         const int wide = total, narrow = items(BQ / 2);
-        if (narrow <= (wide > cus ? 2 * cus : cus)) return launch_32(flash_attn_bf16_kernel<false, 1, 4>, 256, 2, 0.65);
+        if (narrow <= (wide > cus ? 2 * cus : cus)) return launch_32(flash_attn_bf16_kernel<false, 1, 4>, 256, 0.65);
         items(BQ);
-        if (wide < cus) return launch_32(flash_attn_bf16_kernel<false, 1, 8>, 512, 1, 0.95);  // (a unit's registers hold one such workgroup)
+        if (wide < cus) return launch_32(flash_attn_bf16_kernel<false, 1, 8>, 512, 0.95);  // (a unit's registers hold one such workgroup)
     }
-    dim3 grid((unsigned)(total + readers(total, 2))), block(BQ);
+    dim3 grid((unsigned)(total + readers(total, 2, beside))), block(BQ);
     if (norm) hipLaunchKernelGGL((flash_attn_bf16_kernel<true, 2, 4>), grid, block, 0, st, sets, q_scale, 1e-6f);
     else hipLaunchKernelGGL((flash_attn_bf16_kernel<false, 2, 4>), grid, block, 0, st, sets, q_scale, 1e-6f);
     SD3_TRY(launch_status("flash_attention_bf16"));
