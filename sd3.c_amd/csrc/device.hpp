@@ -4,7 +4,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <atomic>
-#include <cstdint>
+#include <mutex>
 
 #include "../../include/sd3_hip.h"
 
@@ -32,20 +32,25 @@ inline int compute_units() {
 }
 
 // One per kernel (a static of its launcher): allows it `bytes` of dynamic LDS on the current device, where a launch may otherwise have
-// no more than 64 KiB. The setting belongs to the function on one device; two threads that get here together both set it.
+// no more than 64 KiB. The setting belongs to the function on one device and replaces the one before, so what is set is the most that the
+// kernel was ever asked to have, one thread at a time: a size that was allowed stays allowed.
 class DynamicLds {
-    std::atomic<uint64_t> done_{0};  // one bit per device
+    std::atomic<int> allowed_[KNOWN_DEVICES] = {};  // bytes
+    std::mutex setting_;
+    int most_ = 0;
 
   public:
     int allow(const void* kernel, int bytes) {
         if (bytes <= 65536) return SD3_OK;
         int dev = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0) return fail(SD3_ERR_HIP, "cannot query the current device");
-        const uint64_t bit = dev < KNOWN_DEVICES ? 1ull << dev : 0;
-        if (done_.load(std::memory_order_relaxed) & bit) return SD3_OK;
-        const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-        if (e != hipSuccess) return fail(SD3_ERR_HIP, "cannot allow a kernel %d bytes of LDS: %s", bytes, hipGetErrorString(e));
-        done_.fetch_or(bit, std::memory_order_relaxed);
+        if (dev < KNOWN_DEVICES && allowed_[dev].load(std::memory_order_acquire) >= bytes) return SD3_OK;
+        std::lock_guard<std::mutex> one(setting_);
+        const int size = most_ > bytes ? most_ : bytes;
+        const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, size);
+        if (e != hipSuccess) return fail(SD3_ERR_HIP, "cannot allow a kernel %d bytes of LDS: %s", size, hipGetErrorString(e));
+        most_ = size;
+        if (dev < KNOWN_DEVICES) allowed_[dev].store(size, std::memory_order_release);
         return SD3_OK;
     }
 };
