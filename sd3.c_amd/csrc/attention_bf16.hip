@@ -1468,16 +1468,15 @@ int attention_bf16_multi(const AttnSegments* jobs, const int* kv_splits, float* 
     //   4096 tokens, 8, 12, 15 heads:              64.1 65.1 69.1 | 46.3 66.2 71.8 | 61.4 62.4 68.3
     //   8192 tokens, 8 heads (a unit each):        132.4 | 140.9 | 134.6
     // All three round alike.
-    // Modulation panels of the next block in workgroups on the compute units that have none of the launch's own, as many as fit the launch (the
-    // times of a panel and of a workgroup's start as in the GEMM launches). Dual blocks of 512px leave their GEMM launches, 240 of 256
+    // Modulation panels of the next block in workgroups on the compute units that have none of the launch's own, as many as fit the launch
+    // (passenger_panels; rows of y beyond two do not fit these kernels' 48 KB of LDS at width 1536). Dual blocks of 512px leave their GEMM launches, 240 of 256
     // tiles, room for 254 of 360 panels: the rest, a launch of 11 us, fits the 40 units free here.
     int panels = 0;  // a workgroup's
     auto take_panels = [&](double tile_us) {
-        constexpr double START = 6.0, FIRST = 6.0, PANEL = 6.5;
+        constexpr double START = 6.0;  // us of the launch's own workgroups in front of their first tile and behind the last
         const int idle = cus - total;
         if (!carry || carry->left() <= 0 || idle <= 0 || B > 2 || ada_lds_bytes(B, carry->work.K) > smem_bytes(false)) return;
-        const int room = (int)((START + tile_us * ((longest + BKV - 1) / BKV) - FIRST) / PANEL);
-        panels = std::min(room, (carry->left() + idle - 1) / idle);
+        panels = passenger_panels(START + tile_us * ((longest + BKV - 1) / BKV), carry->work.K, carry->left(), idle, false);
         if (panels <= 0) return;
         sets.ada = carry->work;
         sets.ada.count = std::min(carry->left(), panels * idle);

@@ -538,19 +538,15 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_bf16_kernel(const ProbSet ar
 }
 
 // How many workgroups a launch of `wgs` adds for the modulation projections (args.ada.count panels at most; what it takes is left there): one
-// for every compute unit that it leaves idle, each as many panels as it has time for. A panel of 1536 x 64 takes such a workgroup 6 to 7 us; with
-// 5.5 / 5 instead of 6.5 / 6 forwards of 512px and its guided pair are 0.8 % slower, of 1024px 0.5 % faster. The last launch of a block may take up
-// to five panels a workgroup more than that (the cost table is a quarter below what a launch with 96 K tiles takes beside the others): a
-// launch of their own costs the 512px forward 2.8 %. A share per launch (a third of the block's panels) instead of as many as there is room:
-// 256px 0, 496x272 +3.3 %.
+// for every compute unit that it leaves idle, each as many panels as it has time for (passenger_panels). At width 1536, with 5.5 us for a panel and
+// 5 for the start instead of 6.5 and 6, forwards of 512px and its guided pair are 0.8 % slower. A share per launch (a third of the block's panels)
+// instead of as many as there is room: 256px 0, 496x272 +3.3 %.
 // In the time that is left they read the weights ahead that the next launches ask for (args.ahead; what is read is left there). At 12, 24, 40, 60,
 // 100 KB per us and workgroup: forwards of 256px -0.9, -2.4, -3.0, -3.1, -3.3 %, its pair -6.0 from 40 on, of the 512px pair +0.1, -0.7, -1.25, -1.25,
 // -1.0, 496x272 batch 3 -0.1, -0.2, 0, +0.9, +13 (the launch is then longer for it), 512px 0 (16 to 28 idle units).
 template <bool CARRIES>
 int carried_wgs(ProbSet& args, int wgs, int cus, int smem) {
-    constexpr double FIRST = 6.0, PANEL = 6.5;  // us
-    constexpr double RATE = 40960;              // bytes per us and workgroup that reads ahead
-    constexpr int OVER = 5;
+    constexpr double RATE = 40960;  // bytes per us and workgroup that reads ahead
     const int idle = cus - wgs, want = args.ada.count;
     args.ada.count = 0;
     if (!CARRIES || idle <= 0) {
@@ -559,12 +555,10 @@ int carried_wgs(ProbSet& args, int wgs, int cus, int smem) {
     }
     int panels = 0;  // a workgroup's
     if (want > 0 && smem >= ada_lds_bytes(ADA_CARRY_ROWS, args.ada.K)) {
-        const int room = (int)((args.us - FIRST) / PANEL), rest = (want + idle - 1) / idle;
-        panels = args.ada_last && rest <= room + OVER ? rest : room;
-        panels = panels < 0 ? 0 : panels > rest ? rest : panels;
+        panels = passenger_panels(args.us, args.ada.K, want, idle, args.ada_last);
         args.ada.count = want < panels * idle ? want : panels * idle;
     }
-    const double us = args.us - (panels ? FIRST + panels * PANEL : FIRST / 2);
+    const double us = args.us - (panels ? PASSENGER_START + panels * passenger_panel_us(args.ada.K) : PASSENGER_START / 2);
     const size_t ahead = args.ahead.trim(us > 0 ? (size_t)(us * RATE * idle) : 0);
     const int readers = (int)(ahead / 32768 < (size_t)idle ? ahead / 32768 : idle), takers = panels ? (args.ada.count + panels - 1) / panels : 0;
     return readers > takers ? readers : takers;
