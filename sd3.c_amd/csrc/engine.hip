@@ -1277,7 +1277,8 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     //      Up to 4096 rows: beyond them the device is at its power limit, where what streams beside the matrix kernels costs them clock (4250 rows,
     //      forward against all projections up front: -1.0, 0 and +1.3 % on three devices; 2048px 0).
     //      The same holds for reading weights ahead in those workgroups.
-    const bool few_rows = bf && !fp8_kind(precision) && (long long)B * (Tx + Tc) <= 4096, carried = few_rows && B <= ADA_CARRY_ROWS;
+    const bool few_rows = bf && !fp8_kind(precision) && (long long)B * (Tx + Tc) <= 4096;
+    bool carried = few_rows && B <= ADA_CARRY_ROWS;
     {
         std::vector<AdaCall> calls;
         for (int l = 0; l < (carried ? 1 : num_layers); l++)
@@ -1302,15 +1303,25 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
         }
         SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], base, base + (size_t)B * 6 * C, bws, few_rows ? &carry : nullptr, l + 1 < num_layers ? &bw[l + 1] : nullptr, l + 1 < num_layers && bd[l + 1].dual));
         if (carry.left() > 0) {  // what no launch had room for
-            AdaJob rest[ADA_CARRY_JOBS];
-            int n = 0, skip = carry.work.first;
+            std::vector<AdaJob> rest;
+            int skip = carry.work.first;
             for (const AdaJob& j : carry.work.job) {
                 const int done = std::min(skip, j.N / 64);
                 skip -= done;
-                if (done * 64 < j.N) rest[n++] = AdaJob{j.W + (size_t)done * 64 * C, j.bias + done * 64, j.out + done * 64, j.N - done * 64, j.ld};
+                if (done * 64 < j.N) rest.push_back({j.W + (size_t)done * 64 * C, j.bias + done * 64, j.out + done * 64, j.N - done * 64, j.ld});
             }
-            ProfScope ps(ctx, SD3_PROF_ADALN, (2.0 * C + 4.0 * B) * 64 * carry.left());
-            SD3_TRY(ada_panels(y, B, C, rest, n, st));
+            if (!passengers_pay(carry.work.first, C)) {  // neither will the blocks behind: theirs in the same launch
+                carried = false;
+                for (int k = l + 2; k < num_layers; k++)
+                    for (const AdaCall& q : ada_calls(k)) {
+                        rest.emplace_back();
+                        SD3_TRY(ada_panel_job(ctx, q, C, &rest.back()));
+                    }
+            }
+            double bytes = 0;
+            for (const AdaJob& j : rest) bytes += (2.0 * C + 4.0 * B) * j.N;
+            ProfScope ps(ctx, SD3_PROF_ADALN, bytes, ((long long)rest.size() + SMALL_LINEAR_JOBS_PER_LAUNCH - 1) / SMALL_LINEAR_JOBS_PER_LAUNCH);
+            SD3_TRY(ada_panels(y, B, C, rest.data(), (int)rest.size(), st));
         }
     }
     // ---- output layer: LN(eps 1e-5), chunk 0 = scale, chunk 1 = shift, projection, tokens -> pixels (modules.cpp:1721-1752)

@@ -4,7 +4,8 @@ import pytest
 import torch
 
 from gpu_util import M
-from sd3_c_amd.params import block_param_shapes
+from sd3_c_amd.config import DiTConfig
+from sd3_c_amd.params import block_param_shapes, dit_param_shapes
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +35,21 @@ def test_gates_of_any_depth(C, B):
             w, bias = W[s][:, chunk * C:(chunk + 1) * C].bfloat16().double(), b[s][chunk * C:(chunk + 1) * C].double()
             bound = (C + 2) * 2.0 ** -24 * (y.double().abs() @ w.abs() + bias.abs())
             assert ((out[s].double() - (y.double() @ w + bias)[:, None]).abs() <= bound[:, None]).all(), (s, chunk)
+
+
+@pytest.mark.parametrize("C,B,Tc,h,w", [(768, 4, 77, 16, 16), (768, 3, 5, 18, 18), (256, 2, 20, 24, 25), (1536, 4, 154, 16, 16)])
+def test_forwards_whose_launches_leave_little_room(C, B, Tc, h, w):
+    """Launches that fill the device take few panels along; the blocks' remaining modulation vectors are then computed together. Batch elements have the
+    bits that they have in a batch too large to take any along."""
+    cfg = DiTConfig(num_layers=5, dual_attention_layers=(0, 3), emb_dim=C, attn_heads=C // 64, pooled_dim=64, captions_dim=64, pos_embed_max_size=64, base_height=32)
+    g = torch.Generator(device="cuda").manual_seed(C + Tc)
+    P = {n: (1 if "rmsnorm" in n else 0) + 0.05 * torch.randn(s, device="cuda", generator=g) for n, s in dit_param_shapes(cfg).items()}
+    a = [torch.randn(s, device="cuda", generator=g) for s in ((B + 5, 64), (B + 5, Tc, 64), (B + 5, 16, 2 * h, 2 * w))] + [1000 * torch.rand(B + 5, device="cuda", generator=g)]
+    den = M.Denoiser(P, cfg, "bf16")
+    try:
+        whole = den(*a).clone()
+        part = [t[2:2 + B].contiguous() for t in a]
+        for _ in range(2):
+            assert torch.equal(den(*part), whole[2:2 + B])
+    finally:
+        den.ctx.close()

@@ -29,6 +29,8 @@ int main() {
                     }
     // width 1536 in the launches of a 512px forward: 16 idle units, a launch of 41 us and the block's last
     assert(passenger_panels(41.0, 1536, 360, 16, false) == 5 && passenger_panels(41.0, 1536, 160, 16, true) == 10 && passenger_panels(41.0, 1536, 176, 16, true) == 5);
+    // what was taken is worth a launch for the rest from 6 us of streaming at 5.4 TB/s on
+    assert(!passengers_pay(0, 1536) && !passengers_pay(164, 1536) && passengers_pay(165, 1536) && !passengers_pay(180, 768) && passengers_pay(83, 3072));
     return 0;
 }
 """
