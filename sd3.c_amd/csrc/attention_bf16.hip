@@ -498,10 +498,10 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
                 inc = probs(KB);
                 lds_wait_k_v(kf, vfr);
                 pv(KB ^ 1, 0);
-                load_v(st_cur, KB, 0);
                 pv(KB ^ 1, 1);
-                load_v(st_cur, KB, 1);
                 settle(KB, inc, t, KB == 0);
+                load_v(st_cur, KB, 0);
+                load_v(st_cur, KB, 1);
                 scores(KB ^ 1, kv0 + t * BKV + 32 * (KB + 1));
                 if (KB == 0) {
                     tile_barrier();
@@ -512,6 +512,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
             };
             step(std::integral_constant<int, 0>());
             step(std::integral_constant<int, 1>());
+            lds_wait_k_v(kf, vfr);  // (see fast_tile)
             rotate_stages();
             return;
         }
@@ -575,7 +576,8 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     //      on this basis: the row sums as two more matrix instructions per unit, ONES . P^T, instead of 16 additions: 7.5 % faster
     //      on zeros, 3 % slower on N(0,1) operands; the requests for the next tile spread over a step: slower.) ----
     //      One query block (NQ = 1): the same slices; every step fetches its successor's fragments, and the barrier of a tile stands behind
-    //      the four score products of its first step, where the reads of the step before have long landed.
+    //      the four score products of its first step, where the reads of the step before have long landed. Those of its second step are waited
+    //      for at its end: the compiler takes their registers for written and may move them about between one round of the loop and the next.
     auto fast_step = [&](auto qb_tag, auto loads_tag, auto vkb_tag, int v_stage, auto kkb_tag, int k_stage, auto publish) {
         constexpr int QB = decltype(qb_tag)::value, PQ = QB ^ 1;     // probabilities of slot QB; scores and PV of the other one
         constexpr int SQ_ = NQ == 2 ? PQ : 0, LQ_ = NQ == 2 ? QB : 0;  // their query blocks
@@ -668,6 +670,7 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         if constexpr (NQ == 1) {
             fast_step(I0, YES, I0, st_cur, I0, st_nxt, publish);  // (t,0): V of key half 0, K of key half 0 of tile t+1
             fast_step(I1, YES, I1, st_cur, I1, st_nxt, nothing);  // (t,1): V of key half 1, K of key half 1 of tile t+1
+            lds_wait_k_v(kf, vfr);
         } else {
             fast_step(I0, YES, I0, st_cur, I1, st_cur, nothing);  // (t,0,0): V of key half 0, K of key half 1
             fast_step(I1, NO, I0, 0, I0, 0, nothing);             // (t,0,1)
@@ -742,7 +745,6 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
             return __builtin_amdgcn_readfirstlane(*flag) != 0;
         };
         for (int t = 0; t < n_fast; t++) fast_tile(t);
-        if (NQ == 1 && n_fast > 0) lds_wait_k_v(kf, vfr);  // the last fast step's fetches
         const bool redo = n_fast > 0 && unsafe();
         if (!redo) {
             if (n_fast > 0) zero_reference();
@@ -755,7 +757,6 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
         n_keep = n_fast;
         n_fast = 0;
     }
-    if (NQ == 1) lds_wait_k_v(kf, vfr);
     pv(1, 0);  // PV of the last unit
     pv(1, 1);
     __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // the redundant loads issued past the last tile have landed before LDS is reused
