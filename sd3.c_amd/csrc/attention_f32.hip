@@ -182,7 +182,10 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(SegDev s, int HS, float s
 // Contraction order: K and Q are read as float4 along d, so step s of 16-wide chunk c contracts d = 16c + 4g + s over the lane groups
 // g = l/16. S^T registers r of a 16x16 block are keys 4g + r of query l%16: as they are, the operand of step r of O^T += V^T P^T, whose
 // V rows 4g + r are read as float4 along d: block j of the four takes d = 4(l%16) + j, so a lane ends with 16 consecutive d of its query.
-template <int HS, int QB, int KB, int KS>
+// LONG_ROWS: rows are 2^22 floats or more apart (and less than 2^24): four times the stride does not fit the 24-bit product of the row offsets. An
+// instantiation of its own, since the shift behind the product, done in every case, costs the others up to 2 %. 65536 heads of 64, 2 queries, 40 keys:
+// 691 us, with attn_f32_kernel 2204.
+template <int HS, int QB, int KB, int KS, bool LONG_ROWS>
 __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, int NH, int n_q, int total, float scale) {
     constexpr int NC = HS / 16, NU = HS / 64, TKEYS = 16 * KB, QW = 16 * QB;
     constexpr int PITCH = NU * 16 * QB + 2 * QB;  // floats per lane in the merge buffer
@@ -233,6 +236,7 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
     // 24 heads of 64, 1178 tokens, batch 2 160 us instead of 152, 4250 tokens 967 instead of 916; 2 heads of 128, batch 8 138 instead of 127). The
     // chunks are requested one by one, each right behind the last use of the register it goes to, so that the requests are spread over the matrix
     // work of a whole tile.
+    auto row_at = [](int row, int ld) { return LONG_ROWS ? __umul24(row, ld) * 4u : (unsigned)__umul24(row, 4 * ld); };
     struct Rows {
         const char* base;
         unsigned off[4 * KB];  // bytes
@@ -242,14 +246,14 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
         const int left = keys_of(t, seg, t0), ld = seg ? ld1 : ld0;
         w.base = reinterpret_cast<const char*>((seg ? k1 : k0) + (long long)t0 * ld);
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++) w.off[kb] = __umul24(min(16 * kb + lr, left - 1), 4 * ld) + 16 * lg;
+        for (int kb = 0; kb < KB; kb++) w.off[kb] = row_at(min(16 * kb + lr, left - 1), ld) + 16 * lg;
     };
     auto v_rows = [&](int t, Rows& w) {
         int seg, t0;
         const int left = keys_of(t, seg, t0), ld = seg ? ld1 : ld0;
         w.base = reinterpret_cast<const char*>((seg ? v1 : v0) + (long long)t0 * ld);
 #pragma unroll
-        for (int x = 0; x < 4 * KB; x++) w.off[x] = __umul24(min(16 * (x / 4) + 4 * lg + x % 4, left - 1), 4 * ld) + 16 * lr;
+        for (int x = 0; x < 4 * KB; x++) w.off[x] = row_at(min(16 * (x / 4) + 4 * lg + x % 4, left - 1), ld) + 16 * lr;
     };
     auto load_k = [&](const Rows& w, int c) {
 #pragma unroll
@@ -409,12 +413,12 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
     }
 }
 
-template <int HS, int QB, int KB, int KS>
+template <int HS, int QB, int KB, int KS, bool LONG_ROWS = false>
 int launch_split(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
     const int TQ = s.Tq[0] + s.Tq[1], n_q = (TQ + 16 * QB - 1) / (16 * QB);
     const long long total = (long long)B * NH * n_q;
     if (total > 0x7fffffff) return fail(SD3_ERR_UNSUPPORTED, "attention (fp32): too many work items");
-    hipLaunchKernelGGL((attn_f32_split_kernel<HS, QB, KB, KS>), dim3((unsigned)total), dim3(KS * 64), 0, st, s, NH, n_q, (int)total, scale);
+    hipLaunchKernelGGL((attn_f32_split_kernel<HS, QB, KB, KS, LONG_ROWS>), dim3((unsigned)total), dim3(KS * 64), 0, st, s, NH, n_q, (int)total, scale);
     return launch_status("attention_f32");
 }
 }  // namespace
@@ -439,12 +443,14 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     }
     const float scale = (float)(1.0 / sqrtf((float)HS));
     const float scale2 = (float)(1.4426950408889634 / sqrt((double)HS));  // scores in powers of two: the exponentials are one instruction
-    if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 22) && a.ld_qkv[1] < (1 << 22)) {
+    if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 24) && a.ld_qkv[1] < (1 << 24)) {
         // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. (Not by the batch: a batch
         // element's result stays what it is alone.) Four key runs in both: eight, or the keys over several workgroups and a second
         // kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four
         // runs 32).
         const bool few = (long long)NH * ((TQ + 31) / 32) < 192;
+        if (a.ld_qkv[0] >= (1 << 22) || a.ld_qkv[1] >= (1 << 22))  // (tens of thousands of heads)
+            return HS == 64 ? launch_split<64, 2, 1, 4, true>(s, B, NH, scale2, st) : launch_split<128, 2, 1, 4, true>(s, B, NH, scale2, st);
         if (HS == 64) return few ? launch_split<64, 1, 2, 4>(s, B, NH, scale2, st) : launch_split<64, 2, 1, 4>(s, B, NH, scale2, st);
         return few ? launch_split<128, 1, 1, 4>(s, B, NH, scale2, st) : launch_split<128, 2, 1, 4>(s, B, NH, scale2, st);
     }

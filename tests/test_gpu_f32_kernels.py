@@ -122,6 +122,16 @@ def test_attention_f32(B, NH, hs, Tq, Tk):
     assert float((out.double() - want.transpose(1, 2).reshape(B, Tq, -1)).abs().max()) <= bound
 
 
+@pytest.mark.parametrize("NH,hs", [(65536, 64), (98304, 64), (32768, 128)])
+def test_attention_f32_of_long_rows(NH, hs):
+    """Rows of 2^22 floats and more: the heads have the bits that they have in calls of a quarter as many, partly empty tile and query block included."""
+    g = torch.Generator(device="cuda").manual_seed(NH)
+    q, k, v = (torch.randn((1, t, NH * hs), device="cuda", generator=g) for t in (3, 21, 21))
+    out = M.mha(q, k, v, NH)
+    for part, want in zip(zip(*(t.chunk(4, 2) for t in (q, k, v))), out.chunk(4, 2)):
+        assert torch.equal(M.mha(*(t.contiguous() for t in part), NH // 4), want)
+
+
 @pytest.mark.parametrize("m,k,n", [(1, 32, 4), (31, 96, 36), (130, 160, 132), (65, 192, 68)])
 def test_gemm_f32_depths_of_whole_k_tiles(m, k, n):
     """Depths of one to six whole K tiles of 32 (fewer than, as many as and more than the rings hold), whose operands are addressed by one scalar and a
