@@ -10,6 +10,7 @@
 
 #include "../../include/sd3_hip.h"
 #include "device.hpp"
+#include "offsets.hpp"
 #include "passengers.hpp"
 
 namespace sd3 {

@@ -97,8 +97,7 @@ typedef __attribute__((__vector_size__(4 * sizeof(int)))) int i32x4_t;
 
 // FP8: the operands are OCP e4m3 bytes (A (M,K) and Wp (N,K), both K-contiguous); a 128-byte LDS row then holds 128 k values and
 // the matrix instruction is v_mfma_f32_32x32x64_f8f6f4; the accumulators are multiplied by a_scale[m] * w_scale[n] in the epilogue.
-// WIDE: operand rows so long (more than LONG_K values) that offsets inside a tile do not fit 32 bits.
-constexpr int LONG_K = 1 << 22;
+// WIDE: operand rows so long that offsets inside a tile do not fit 32 bits (offsets_fit).
 template <int BM, int BN, int WM, int WN, int STAGES, int EPI, bool OUT_F32, bool FP8, bool WIDE>
 __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* smem) {
     constexpr int ESZ = FP8 ? 1 : 2;                  // bytes per operand element
@@ -589,17 +588,18 @@ int launch_cfg(ProbSet& args, int n, hipStream_t st) {
     return launch_status("gemm_bf16");
 }
 
-bool any_long(const ProbSet& set, int n) {
+// whether tiles of `rows` rows (of either operand) address their operands, `esz` bytes a value, by 32-bit offsets
+bool addresses(const ProbSet& set, int n, int rows, int esz) {
     for (int i = 0; i < n; i++)
-        if (set.p[i].K > LONG_K) return true;
-    return false;
+        if (!offsets_fit(rows, (long long)set.p[i].K * esz)) return false;
+    return true;
 }
 
 // fp8 operands: 256x256 tiles (variant 4) or 128x128 tiles with a ring of two stages (anything else)
 template <int EPI, bool OUT_F32>
 int launch_epi_fp8(int variant, ProbSet& args, int n, hipStream_t st) {
-    if (any_long(args, n)) return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32, true, true>(args, n, st);
-    if (variant == 4) return launch_cfg<256, 256, 2, 4, 2, EPI, OUT_F32, true>(args, n, st);
+    if (!addresses(args, n, 128, 1)) return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32, true, true>(args, n, st);
+    if (variant == 4 && addresses(args, n, 256, 1)) return launch_cfg<256, 256, 2, 4, 2, EPI, OUT_F32, true>(args, n, st);
     return launch_cfg<128, 128, 2, 2, 2, EPI, OUT_F32, true>(args, n, st);
 }
 
@@ -965,15 +965,20 @@ int cheapest_shape(const ProbSet& set, int n, int cus, double& cost) {
 // 2356 rows 90 against 81).
 template <int EPI, bool OUT_F32>
 int launch_shape(int shape, ProbSet& args, int n, int cus, hipStream_t st) {
+    const bool whole = all_whole(args, n);
+    if (!shape_takes(shape, whole)) shape = TILE_256;
+    // Rows of more than 2^23 values: the next smaller tiles that can address them. (64-bit addresses are built for one shape only, which takes 64 ms for 3 x 68 x
+    // (2^22 + 64) where 64x64 tiles take 12, and 90 ms for 1024 x 512 instead of 17.)
+    auto fits = [&](int s) { return addresses(args, n, tile_shapes[s].tm > tile_shapes[s].tn ? tile_shapes[s].tm : tile_shapes[s].tn, 2); };
+    while (shape > TILE_64 && !fits(shape)) shape--;
+    if (!fits(shape)) return launch_cfg<128, 256, 1, 4, 2, EPI, OUT_F32, false, true>(args, n, st);
     long long tiles = 0;
     for (int i = 0; i < n; i++) tiles += tiles_of(args.p[i], shape);
     const bool one_round = tiles <= cus;
-    if (any_long(args, n)) return launch_cfg<128, 256, 1, 4, 2, EPI, OUT_F32, false, true>(args, n, st);
-    if (!all_whole(args, n)) {
+    if (!whole) {
         if (shape == TILE_64) return launch_ring<64, 64, 4, 1, 5, 2, EPI, OUT_F32, false>(args, n, st);
         if (shape == TILE_128) return launch_ring<128, 128, 4, 2, 4, 2, EPI, OUT_F32, false>(args, n, st);
         if (shape == TILE_256_128) return launch_ring<256, 128, 4, 2, 3, 2, EPI, OUT_F32, false>(args, n, st);
-        if (!shape_takes(shape, false)) shape = TILE_256;
     }
     switch (shape) {
         case TILE_64: return launch_ring<64, 64, 4, 1, 5, 2, EPI, OUT_F32>(args, n, st);
