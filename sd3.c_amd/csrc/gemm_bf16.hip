@@ -92,6 +92,9 @@ struct ProbSet {
 };
 // the layers of a block, whose launches take modulation projections along and read ahead
 constexpr bool carries(int epi, bool out_f32) { return epi == EPI_GATE_RESID ? out_f32 : (epi == EPI_BIAS_GELU || epi == EPI_QKV_NORM) && !out_f32; }
+// ... among the ring kernels not those of two workgroups per compute unit (four wavefronts per SIMD, MW), which are launched only where the tiles are more
+// than the units, so that none is idle
+constexpr bool ring_carries(int epi, bool out_f32, bool whole_rows, int mw) { return carries(epi, out_f32) && whole_rows && mw == 2; }
 
 // One output tile: K loop + epilogue. `wg` is the tile's position in the XCD-aware order of its problem.
 typedef __attribute__((__vector_size__(8 * sizeof(int)))) int i32x8_t;
@@ -632,7 +635,7 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
     static_assert(NJ == 4 && TI >= 1 && TM * 8 % NT == 0 && TN * 8 % NT == 0, "tile shape");
     static_assert(STAGES >= 2 && (STAGES - 1) * (LA + LB) < 64, "the loads in flight must fit the 6-bit counter");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
-    if (carries(EPI, OUT_F32) && WHOLE_ROWS && (int)blockIdx.x >= args.tiles_wgs) {
+    if (ring_carries(EPI, OUT_F32, WHOLE_ROWS, MW) && (int)blockIdx.x >= args.tiles_wgs) {
         ada_carried<NT>(args.ada, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs, smem);
         read_ahead<NT>(args.ahead, blockIdx.x - args.tiles_wgs, gridDim.x - args.tiles_wgs);
         return;
@@ -889,7 +892,7 @@ int launch_ring(ProbSet& args, int n, hipStream_t st) {
     const int cus = compute_units();
     if (cus <= 0) return SD3_ERR_HIP;
     args.tiles_wgs = total;
-    hipLaunchKernelGGL(kern, dim3(total + carried_wgs<carries(EPI, OUT_F32) && WHOLE_ROWS>(args, total, cus, smem)), dim3(WM * WN * 64), smem, st, args);
+    hipLaunchKernelGGL(kern, dim3(total + carried_wgs<ring_carries(EPI, OUT_F32, WHOLE_ROWS, MW)>(args, total, cus, smem)), dim3(WM * WN * 64), smem, st, args);
     g_gemm_bf16_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_status("gemm_bf16");
 }
