@@ -10,8 +10,8 @@ from sd3_c_amd.params import block_param_shapes, dit_param_shapes
 pytestmark = pytest.mark.gpu
 
 
-# slices of 2, 14, 16, 18, 24, 30, 32, 34 and 76 rows
-@pytest.mark.parametrize("C", [64, 448, 512, 576, 768, 960, 1024, 1088, 2432])
+# slices of 2, 14, 16, 18, 24, 30, 32, 34, 76, 96 and 128 rows; the last two are as deep as eight rows of y and as the kernel allow
+@pytest.mark.parametrize("C", [64, 448, 512, 576, 768, 960, 1024, 1088, 2432, 3072, 4096])
 @pytest.mark.parametrize("B", [1, 2, 3, 9])
 def test_gates_of_any_depth(C, B):
     """With zero residual streams, zero output weights and one bias of ones the block's outputs are gates, i.e. columns of y @ W + b: against float64 on the
