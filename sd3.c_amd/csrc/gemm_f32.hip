@@ -7,6 +7,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "tiles_f32.hpp"
 
 namespace sd3 {
 
@@ -132,7 +133,7 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__
 // fp32 matrix instructions are slow (64 FLOP per cycle and SIMD: a 64x64 wavefront tile works 2048 cycles on 16 k values), so the
 // matrix unit is the bound as soon as every SIMD has a tile; LDS and global traffic are not. What costs is SIMDs without work: the
 // layers of a 512 x 512 image are 96 tiles of 128x128 on 256 compute units. Hence a range of tile shapes down to 32x32, chosen per
-// launch by the number of rounds (pick_tile), and one launch for the layers of the same kind of both token streams.
+// launch by the number of rounds (pick_f32_tile), and one launch for the layers of the same kind of both token streams.
 //
 // Both operands go global -> LDS by direct loads. A tile rows are 128 bytes (32 k values), 16-byte chunks XOR-swizzled by the row as
 // in the bf16 kernel's 16x16 layout: lane l reads chunk 4h + l/16 of row l%16, i.e. k values 16h + 4(l/16) .. +3 of one half h of the
@@ -388,20 +389,16 @@ int launch_tile_k(TileProbSet& set, int n, hipStream_t st) {
     return launch_status("gemm_f32");
 }
 
+// whether the launch takes the kernel of whole K tiles (whose offsets within a tile are 32 bits)
+bool whole_k_tiles(const TileProbSet& set, int n) {
+    for (int i = 0; i < n; i++)
+        if (set.p[i].K % TK || set.p[i].lda > (1 << 22) || set.p[i].ldw > (1 << 22)) return false;
+    return true;
+}
 template <int TM, int TN, int WM, int WN, int STAGES, int EPI>
 int launch_tile(TileProbSet& set, int n, hipStream_t st) {
-    bool whole = true;  // (and offsets within a tile of 32 bits)
-    for (int i = 0; i < n; i++) whole = whole && set.p[i].K % TK == 0 && set.p[i].lda <= (1 << 22) && set.p[i].ldw <= (1 << 22);
-    return whole ? launch_tile_k<TM, TN, WM, WN, STAGES, EPI, true>(set, n, st) : launch_tile_k<TM, TN, WM, WN, STAGES, EPI, false>(set, n, st);
+    return whole_k_tiles(set, n) ? launch_tile_k<TM, TN, WM, WN, STAGES, EPI, true>(set, n, st) : launch_tile_k<TM, TN, WM, WN, STAGES, EPI, false>(set, n, st);
 }
-
-// The tile shapes, largest first, and what one K tile (32 k values) of one output tile costs in cycles, measured over N = 1536 .. 6144
-// and K = 1536, 6144: alone on its compute unit, and with two or three workgroups sharing one (the matrix instructions alone: TM*TN/4).
-struct TileShape {
-    int tm, tn;
-    double alone, shared;
-};
-constexpr TileShape TILE_SHAPES[] = {{128, 128, 4270, 4250}, {128, 64, 2150, 2155}, {64, 64, 1150, 1100}, {32, 64, 670, 590}, {32, 32, 440, 325}};
 
 template <int EPI>
 int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
@@ -416,26 +413,10 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
     }
 }
 
-// The shape whose busiest compute unit is done first: with r output tiles on it, r * shared cycles per K tile (alone for r = 1).
 int pick_tile(const TileProbSet& set, int n, int cus) {
-    int best = 0;
-    double best_cost = 0;
-    for (int s = 0; s < (int)(sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0])); s++) {
-        const TileShape t = TILE_SHAPES[s];
-        long long tiles = 0, depth = 0;
-        for (int i = 0; i < n; i++) {
-            const long long c = (long long)((set.p[i].M + t.tm - 1) / t.tm) * ((set.p[i].N + t.tn - 1) / t.tn);
-            tiles += c;
-            depth += c * set.p[i].K;
-        }
-        const long long r = (tiles + cus - 1) / cus;
-        const double cost = (double)depth / tiles * (r == 1 ? t.alone : r * t.shared);
-        if (s == 0 || cost < best_cost) {
-            best = s;
-            best_cost = cost;
-        }
-    }
-    return best;
+    F32Layer layers[MAX_PROBS];
+    for (int i = 0; i < n; i++) layers[i] = F32Layer{set.p[i].M, set.p[i].N, set.p[i].K};
+    return pick_f32_tile(layers, n, cus, whole_k_tiles(set, n));
 }
 
 // What the tile kernel asks for: operands whose rows are made of aligned 16-byte chunks (its direct loads into LDS) and outputs in whole
@@ -495,6 +476,6 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, int n0, float* ou
     return gemm_f32_grouped(&q, 1, epi, st);
 }
 
-int g_gemm_f32_tile = -1;  // -1: chosen from the sizes; 0..4: that entry of TILE_SHAPES (sd3_tune)
+int g_gemm_f32_tile = -1;  // -1: chosen from the sizes; 0..4: that entry of f32_tiles (sd3_tune)
 
 }  // namespace sd3
