@@ -8,6 +8,8 @@
 //   S^T (keys x queries) = K . Q^T      -> C-layout: a lane owns ONE query column and 16 keys per 32-key block
 //   O^T (d x queries)   += V^T . P^T    -> the lane's own S^T registers are exactly the P^T operand it must supply
 // Online softmax statistics are per query = per lane (plus one exchange with lane^32).
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace sd3 {
@@ -176,8 +178,8 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(SegDev s, int HS, float s
 // and split the KEYS (tile t goes to wavefront t % KS); K and V rows come straight from memory (L2: all workgroups of a head run on one
 // XCD) into registers, half a tile of matrix work ahead of their use; the KS partial results are merged in a fixed tree at the end.
 // This gives every SIMD work also where there are few queries: 1178 tokens and 2 heads are 20 workgroups of 128 queries with the keys in
-// one run (290 us), 592 wavefronts this way (30 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 152 us, 70 -> 112 TFLOP/s of 155 (the matrix
-// instructions alone 130, the softmax 12, the loads 9).
+// one run (290 us), 592 wavefronts this way (30 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 148 us, 70 -> 115 TFLOP/s of 155 (the matrix
+// instructions alone about 127, the softmax 12, the loads 9).
 //
 // Contraction order: K and Q are read as float4 along d, so step s of 16-wide chunk c contracts d = 16c + 4g + s over the lane groups
 // g = l/16. S^T registers r of a 16x16 block are keys 4g + r of query l%16: as they are, the operand of step r of O^T += V^T P^T, whose
@@ -232,10 +234,10 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
         t0 = (seg ? t - nt0 : t) * TKEYS;
         return (seg ? T1 : T0) - t0;  // keys from here to the end of the segment
     };
-    // Where a lane's chunks of a tile's rows are: a scalar base and 32-bit row offsets in bytes, which the loads take as they are (as 64-bit addresses:
-    // 24 heads of 64, 1178 tokens, batch 2 160 us instead of 152, 4250 tokens 967 instead of 916; 2 heads of 128, batch 8 138 instead of 127). The
-    // chunks are requested one by one, each right behind the last use of the register it goes to, so that the requests are spread over the matrix
-    // work of a whole tile.
+    // Where a lane's chunks of a tile's rows are: a scalar base and 32-bit row offsets in bytes, which the loads take as they are (as 64-bit addresses,
+    // both before the last tile had a form of its own: 24 heads of 64, 1178 tokens, batch 2 160 us instead of 152, 4250 tokens 967 instead of 916; 2 heads
+    // of 128, batch 8 138 instead of 127; calls of few keys 1 to 2 % less). The chunks are requested one by one, each right behind the last use of the
+    // register it goes to, so that the requests are spread over the matrix work of a whole tile.
     auto row_at = [](int row, int ld) { return LONG_ROWS ? __umul24(row, ld) * 4u : (unsigned)__umul24(row, 4 * ld); };
     struct Rows {
         const char* base;
@@ -295,8 +297,12 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
         k_rows(t + KS < n_t ? t + KS : t, w);
         scores(sc, w);
     }
-    for (; t < n_t; t += KS) {
-        const int next = t + KS < n_t ? t + KS : t, next2 = t + 2 * KS < n_t ? t + 2 * KS : t;  // (past the end: any tile, never used)
+    // One key tile. MORE: this wavefront has another one behind it. Its last tile asks for no rows and computes no scores of a next one, which is most of what
+    // calls of few keys do: with them 4250 queries of 64 keys, 24 heads of 64, take 46.2 us instead of 38.5; 4 x 1024 of 154, 12 heads of 128 64.2 (1.1 %
+    // more than with 64-bit addresses) instead of 59.1; 2 x 1178 of 1178, 24 heads 150.8 instead of 148.0.
+    auto tile = [&](auto more) {
+        constexpr bool MORE = decltype(more)::value;
+        const int next = t + KS, next2 = t + 2 * KS < n_t ? t + 2 * KS : t;  // (past the end: any tile, never used)
         int seg, t0;
         const int left = keys_of(t, seg, t0);
         if (left < TKEYS) {
@@ -311,9 +317,11 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
         // the scores of the next tile on the matrix unit beside the softmax of this one on the vector unit (wavefronts of a SIMD fall
         // into step, so one of them does not fill the other's pauses)
         Rows wk, wv;
-        k_rows(next2, wk);
-        v_rows(next, wv);
-        scores(sn, wk);
+        if constexpr (MORE) {
+            k_rows(next2, wk);
+            v_rows(next, wv);
+            scores(sn, wk);
+        }
         float alpha[QB];
 #pragma unroll
         for (int i = 0; i < QB; i++) {
@@ -351,14 +359,17 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
                 for (int j = 0; j < 4; j++)
 #pragma unroll
                     for (int i = 0; i < QB; i++) o[i][u][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[x / 4][x % 4][u][j], sc[x / 4][i][x % 4], o[i][u][j], 0, 0, 0);
-            load_v(wv, x);
+            if constexpr (MORE) load_v(wv, x);
             __builtin_amdgcn_sched_barrier(VECTOR_ONLY);
         }
+        if constexpr (MORE)
 #pragma unroll
-        for (int kb = 0; kb < KB; kb++)
+            for (int kb = 0; kb < KB; kb++)
 #pragma unroll
-            for (int i = 0; i < QB; i++) sc[kb][i] = sn[kb][i];
-    }
+                for (int i = 0; i < QB; i++) sc[kb][i] = sn[kb][i];
+    };
+    for (; t + KS < n_t; t += KS) tile(std::true_type());
+    if (t < n_t) tile(std::false_type());
 
     // merge: in each step the upper half of the wavefronts hands its state to the lower half
 #pragma unroll

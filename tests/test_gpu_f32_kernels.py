@@ -122,6 +122,15 @@ def test_attention_f32(B, NH, hs, Tq, Tk):
     assert float((out.double() - want.transpose(1, 2).reshape(B, Tq, -1)).abs().max()) <= bound
 
 
+@pytest.mark.parametrize("NH", [2, 100])
+@pytest.mark.parametrize("hs", [64, 128])
+@pytest.mark.parametrize("Tk", [16, 63, 64, 65, 127, 128, 129, 193, 257])
+def test_attention_f32_by_the_key_tiles_of_a_wavefront(NH, hs, Tk):
+    """A wavefront's last key tile is its only one, its second or its third, for some wavefronts of a workgroup and not for others, and whole or not:
+    16 and 32 queries per workgroup (few and many heads)."""
+    test_attention_f32(1, NH, hs, 40, Tk)
+
+
 @pytest.mark.parametrize("NH,hs", [(65536, 64), (98304, 64), (32768, 128)])
 def test_attention_f32_of_long_rows(NH, hs):
     """Rows of 2^22 floats and more: the heads have the bits that they have in calls of a quarter as many, partly empty tile and query block included."""
