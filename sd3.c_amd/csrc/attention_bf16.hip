@@ -140,8 +140,8 @@ __global__ void __launch_bounds__(NW * 64, 2) flash_attn_bf16_kernel(const AttnS
     static_assert(NQ == 2 || (NQ == 1 && !NORM), "32-query blocks of a wavefront");
     __shared__ __attribute__((aligned(1024))) char smem[smem_bytes(NORM)];
     // The barrier in the middle of a tile, which publishes tile t+1 and retires the stage of tile t-1. In front of it a thread's own
-    // requests for tile t+1 must have landed -- every thread requests four 16-byte chunks per tile, so that is "all but the newest
-    // 4 (PF - 1)" -- and its LDS accesses must be done. A bare barrier between compiler fences: __syncthreads() would wait for
+    // requests for tile t+1 must have landed -- every thread requests CHUNKS 16-byte chunks of K and as many of V per tile, so that is "all but
+    // the newest 2 CHUNKS (PF - 1)" -- and its LDS accesses must be done. A bare barrier between compiler fences: __syncthreads() would wait for
     // every load in flight, the tiles requested further ahead included.
     auto tile_barrier = [&]() {
         __builtin_amdgcn_s_waitcnt(((2 * CHUNKS * (PF - 1)) & 15) | (7 << 4) | (0 << 8));  // lgkmcnt(0)

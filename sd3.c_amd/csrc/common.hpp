@@ -195,8 +195,8 @@ __device__ __forceinline__ void ada_stage_rows(const float* __restrict__ y, int 
 // One panel. A thread has 4 columns and one (NT = 512) or two of the 32 slices of K, 16 rows of weights in flight; the order of the sums does
 // not depend on NT or M (explicit multiply-adds), so that a row has the same bits in either kernel and in any batch.
 // ONCE: nobody reads these weights again in a forward, so they are not to push the blocks' activations and the weights that attention reads
-// ahead out of the last-level cache (non-temporal loads; forwards of 256px, 512px, its pair, 1024px 0.6, 0.7, 0.6, 0.9 % less). A block that
-// is called over and over finds them there (106.3 -> 104 us without).
+// ahead out of the last-level cache (non-temporal loads; forwards of 256px, 512px, its pair 0.6, 0.7, 0.6 % less). The launches that do nothing else
+// read them with plain loads: a block that is called over and over finds them in the cache (106.3 -> 104 us).
 template <int NT, int M, bool ONCE>
 __device__ __forceinline__ void ada_panel(const bf16_t* __restrict__ W, const float* __restrict__ bias, float* __restrict__ out, int ld, int B, int K,
                                           const float* xs, float* red) {

@@ -130,7 +130,8 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
     // ---- loader: chunk q = i*NT + tid lands at LDS byte q*16 of its tile, i.e. row q/8, physical chunk q%8 ----
     // Direct loads take one scalar address per operand, which moves on with the K tiles, and a 32-bit offset per thread, which does not: a 64-bit
     // address per load costs the vector unit an addition between the matrix instructions. 8192 + 308 rows, 256x256 tiles, warm: q|k|v 140 -> 132 us,
-    // mlp-1 175 -> 168; the smaller tiles of the ring kernel gain 0 to 1 %; forwards 0.9 (2048px) to 1.8 % (guided 512px pair), 256px 0.
+    // mlp-1 175 -> 168; the smaller tiles of the ring kernel gain 0 to 1 %; forwards 1.8 % (guided 512px pair), 256px 0, and nothing that lasts for the pair of
+    // 1024px and for 2048px, which the power limit holds.
     typedef typename std::conditional<WIDE, long long, unsigned>::type offset_t;
     offset_t a_off[LA], b_off[LB];
     const long long row_bytes = (long long)K * ESZ;
@@ -904,7 +905,7 @@ int launch_ring(ProbSet& args, int n, hipStream_t st) {
 // per tile but are there for what is left of a round: q|k|v of 2 x 1024 + 154 rows, 162 or 234 tiles, 50.2 -> 46.0 us; 128x256 beside 256x128
 // for rows that are not multiples of 256: mlp-1 of 1581 + 999 rows, 504 tiles instead of 528 in two rounds of 256, 73 -> 60 us.
 // Where 128x64 and 64x128 are the same number of rounds the former is taken: out-projection and mlp-2 of 1024 + 154 rows 16.7 -> 15.8 and 44.4 ->
-// 42.4 us; forwards of 24 x 40 patches -3.4 %, two of 256px -1.6 %, 512px +0.3 %.
+// 42.4 us; forwards of 24 x 40 patches -3.4 %, two of 256px -1.6 %, 512px +0.3 %. That is what its fixed cost says: 2.25 where the fit gives 2.3 for both.
 struct TileShape {
     int tm, tn;
     double fixed, per_k;

@@ -87,8 +87,10 @@ __global__ void __launch_bounds__(256) small_linear_kernel(const float* __restri
 }
 
 // The modulation projections of the bf16 path on their own (common.hpp: ada_panel): one workgroup per panel. Those of a block (216 or 360
-// panels of 1536 x 64): 16 us; of all 24 blocks, 1.53 GB, one / four / eight rows: 260 to 285 us (5.4 to 5.9 TB/s; from (K,N) weights, 128 columns
-// x 8 slices a workgroup, eight rows took 840).
+// panels of 1536 x 64): 16 us; of all 24 blocks, 1.53 GB, one / four / eight rows: 266, 291, 520 us (5.8, 5.3, 3.0 TB/s; from (K,N) weights, 128
+// columns x 8 slices a workgroup, eight rows took 840). Eight rows are neither the weights nor the vector units (40 % of the time) nor the LDS (41 %, of which 54 %
+// bank conflicts: the four slices of a wavefront read xs a multiple of 64 banks apart): with 114 KB of LDS a unit has one workgroup, whose staging of y,
+// streaming and summing up nothing else covers.
 struct AdaJobPack {
     AdaJob j[SMALL_LINEAR_JOBS_PER_LAUNCH];
 };
