@@ -317,7 +317,7 @@ struct GemmEpilogueArgs {
     const float* w_scale = nullptr;
 };
 
-// fp32 GEMM on the fp32 MFMA units: out(M,N) = A(M,K; lda) @ W(K, ldw)[:, n0:n0+N] (+ epilogue); out fp32 with row stride ldc.
+// fp32 GEMM: out(M,N) = A(M,K; lda) @ W(K, ldw)[:, n0:n0+N] (+ epilogue); out fp32 with row stride ldc.
 int gemm_f32(const float* A, int lda, const float* W, int ldw, int n0, float* out, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
              hipStream_t st);
 // Up to three independent fp32 GEMMs with the same epilogue kind: one launch where all rows are made of whole 16-byte chunks.
@@ -329,7 +329,7 @@ struct GemmF32Problem {
     GemmEpilogueArgs ea;
 };
 int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st);
-extern int g_gemm_f32_tile;
+extern int g_gemm_f32_tile, g_gemm_f32_no_pieces;
 // bf16 GEMM: A bf16 (M,K) row-major; Wp = packed weight, bf16, K-contiguous (see GemmBf16Problem::w_tiled); out bf16 (out_is_f32 = 0) or fp32.
 int gemm_bf16(const bf16_t* A, const bf16_t* Wp, bool w_tiled, void* out, int out_is_f32, int ldc, int M, int N, int K, int epi, const GemmEpilogueArgs& ea,
               hipStream_t st);

@@ -1475,8 +1475,12 @@ int sd3_tune(const char* name, int value) {
         return SD3_OK;
     }
     if (!std::strcmp(name, "gemm_f32_tile")) {
-        SD3_REQUIRE(value >= -1 && value <= 4, "sd3_tune(%s): -1 (automatic) or 0..4 (got %d)", name, value);
+        SD3_REQUIRE(value >= -1 && value <= 5, "sd3_tune(%s): -1 (automatic) or 0..5 (got %d)", name, value);
         g_gemm_f32_tile = value;
+        return SD3_OK;
+    }
+    if (!std::strcmp(name, "gemm_f32_no_pieces")) {
+        g_gemm_f32_no_pieces = value != 0;
         return SD3_OK;
     }
     if (!std::strcmp(name, "attention_context_splits")) {

@@ -1,9 +1,10 @@
-// fp32 GEMM on the gfx950 fp32 matrix cores, for the fp32 parity path and the fp32 operators:
+// fp32 GEMM on the gfx950 matrix cores, for the fp32 parity path and the fp32 operators:
 //   out(M,N) = A(M,K) @ W(K,N)[:, n0:n0+N] + epilogue
 // replacing linear / partial_linear of the reference (modules.cpp:475-511, naive triple loops).
 //
-// gemm_f32_tile_kernel (v_mfma_f32_16x16x4_f32) takes everything whose operand rows are made of whole 16-byte chunks, up to three problems
-// per launch; gemm_f32_kernel (v_mfma_f32_32x32x2_f32, 128x128x16 tiles, element-wise loads) takes operands of any other stride or alignment.
+// gemm_f32_pieces_kernel (operands as three bf16 pieces each, on the bf16 matrix instruction) takes depths from 512 on;
+// gemm_f32_tile_kernel (v_mfma_f32_16x16x4_f32) everything else whose operand rows are made of whole 16-byte chunks; both up to three problems
+// per launch. gemm_f32_kernel (v_mfma_f32_32x32x2_f32, 128x128x16 tiles, element-wise loads) takes operands of any other stride or alignment.
 #include <type_traits>
 
 #include "common.hpp"
@@ -182,6 +183,41 @@ __device__ __forceinline__ void store_cols(float* p, const float (&v)[NJ]) {
     *reinterpret_cast<typename Cols<NJ>::mem*>(p) = t;
 }
 
+// Epilogue and stores of TI x NJ blocks of 16x16. C layout of a block: lane = column l%16 (of block j: column NJ*(l%16) + j), register r = row 4*(l/16) + r;
+// m: the lane's first row, n: its first column
+template <int TI, int NJ, int EPI>
+__device__ __forceinline__ void store_tile(const TileProb& pr, const f32x4_t (&acc)[TI][NJ], int m0, int n) {
+    if (n >= pr.N) return;  // (N is a multiple of 4, so a lane's columns are all inside or all outside)
+    const EpiDev& e = pr.epi;
+    float bias[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; j++) bias[j] = e.bias ? e.bias[pr.n0 + n + j] : 0.f;
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int m = m0 + i * 16 + r;
+            if (m >= pr.M) continue;
+            const long long idx = (long long)m * pr.ldc + n;
+            float v[NJ], g[NJ], t[NJ];
+            if (EPI == EPI_GATE_RESID) {
+                load_cols<NJ>(e.gate + (long long)(m / e.rows_per_batch) * e.gate_ld + n, g);
+                load_cols<NJ>(e.resid + idx, t);
+            } else if (EPI == EPI_BIAS_ROWADD) {
+                load_cols<NJ>(e.table + (long long)(m % e.rows_per_batch) * e.gate_ld + n, t);
+            }
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                v[j] = acc[i][j][r] + bias[j];
+                if (EPI == EPI_BIAS_GELU) v[j] = gelu_tanh_precise(v[j]);
+                else if (EPI == EPI_BIAS_SILU) v[j] = silu_precise(v[j]);
+                else if (EPI == EPI_GATE_RESID) v[j] = v[j] * g[j] + t[j];
+                else if (EPI == EPI_BIAS_ROWADD) v[j] += t[j];
+            }
+            store_cols<NJ>(pr.out + idx, v);
+        }
+}
+
 // WHOLE_K: K is made of whole tiles in every problem
 template <int TM, int TN, int WM, int WN, int STAGES, int EPI, bool WHOLE_K>
 __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const TileProbSet set) {
@@ -341,37 +377,7 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const Til
         spread(std::true_type{});
     }
     wait_vmcnt<0>();  // no direct load may still be on its way into this workgroup's LDS when it ends
-    // C layout of a 16x16 block: lane = column l%16 (of block j: column NJ*(l%16) + j), register r = row 4*(l/16) + r
-    const int n = n_blk + wn * (TN / WN) + NJ * lr;
-    if (n >= N) return;  // (N is a multiple of 4, so a lane's columns are all inside or all outside)
-    const EpiDev& e = pr.epi;
-    float bias[NJ];
-#pragma unroll
-    for (int j = 0; j < NJ; j++) bias[j] = e.bias ? e.bias[pr.n0 + n + j] : 0.f;
-#pragma unroll
-    for (int i = 0; i < TI; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int m = m_blk + wm * (TM / WM) + i * 16 + 4 * lg + r;
-            if (m >= M) continue;
-            const long long idx = (long long)m * pr.ldc + n;
-            float v[NJ], g[NJ], t[NJ];
-            if (EPI == EPI_GATE_RESID) {
-                load_cols<NJ>(e.gate + (long long)(m / e.rows_per_batch) * e.gate_ld + n, g);
-                load_cols<NJ>(e.resid + idx, t);
-            } else if (EPI == EPI_BIAS_ROWADD) {
-                load_cols<NJ>(e.table + (long long)(m % e.rows_per_batch) * e.gate_ld + n, t);
-            }
-#pragma unroll
-            for (int j = 0; j < NJ; j++) {
-                v[j] = acc[i][j][r] + bias[j];
-                if (EPI == EPI_BIAS_GELU) v[j] = gelu_tanh_precise(v[j]);
-                else if (EPI == EPI_BIAS_SILU) v[j] = silu_precise(v[j]);
-                else if (EPI == EPI_GATE_RESID) v[j] = v[j] * g[j] + t[j];
-                else if (EPI == EPI_BIAS_ROWADD) v[j] += t[j];
-            }
-            store_cols<NJ>(pr.out + idx, v);
-        }
+    store_tile<TI, NJ, EPI>(pr, acc, m_blk + wm * (TM / WM) + 4 * lg, n_blk + wn * (TN / WN) + NJ * lr);
 }
 
 template <int TM, int TN, int WM, int WN, int STAGES, int EPI, bool WHOLE_K>
@@ -413,11 +419,359 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
     }
 }
 
-int pick_tile(const TileProbSet& set, int n, int cus) {
-    F32Layer layers[MAX_PROBS];
-    for (int i = 0; i < n; i++) layers[i] = F32Layer{set.p[i].M, set.p[i].N, set.p[i].K};
-    return pick_f32_tile(layers, n, cus, whole_k_tiles(set, n));
+// ---- the pieces kernel ----
+// The bf16 matrix instruction does sixteen times the operations of the fp32 one per cycle. An fp32 value is the sum of three bf16 values, x = h + m + l, without a
+// remainder (bf16_pieces), and a product of two values is the sum of nine products of pieces, which are exact. Six of them are formed: what l*m, m*l and l*l
+// would add is below 2^-25 of the product, the rounding of an fp32 product. The sums are fp32 as before, and fewer additions round: six per 32 k values and
+// block instead of 32. Relative error against 64 bits, normal operands, with this kernel (with the tile kernel): K = 256 2.3e-7 (2.9e-7), 768 4.2e-7 (5.0e-7),
+// 1536 6.0e-7 (7.0e-7), 6144 1.24e-6 (1.40e-6).
+//
+// Six products per K tile of 32 are 96 matrix instructions of 17 cycles for a wavefront of 64x64: 240 TFLOP/s if nothing else took time. Splitting the operands does:
+// 11 vector operations per pair of values. Done between the matrix instructions of the same wavefronts they added up (8192 x 3072 x 768: 200 us), so wavefronts
+// of their own do it: they fetch both operands from memory, K tiles ahead, and write the pieces to LDS, while the others read fragments and multiply (173 us;
+// what the vector unit does for one wavefront costs the matrix instructions of another nothing, and a lone wavefront issues a vector operation every 5 cycles,
+// three of them one every 2). One barrier per GROUP K tiles, two buffers.
+// With the LDS reads (256 bytes per cycle), writes (128) and the requests the 256x128 tile takes 3700 cycles per K tile, the matrix instructions 3280; smaller
+// tiles have more to split per product: 128x128 2120 (1640), 128x64 1140 (820), 64x64 800 (410), 32x64 590 (205), 32x32 465 (100; the tile kernel's 440).
+// us, tile kernel -> this one, rows x columns x depth: 8192 x 3072 x 768 280 -> 176 (219 TFLOP/s), 10656 x 768 x 1536 178 -> 110, 1178 x 6144 x 1536 184 -> 105,
+// 1178 x 4608 x 1536 141 -> 92, 1178 x 1536 x 6144 178 -> 130, 1178 x 1536 x 1536 48 -> 37, 333 x 1536 x 1536 25.3 -> 22.4, 64 x 1536 x 1536 12.1 -> 12.0; of 160 sizes
+// from 1 to 8192 rows the worst is 666 x 1536 x 768, 16.9 -> 18.4.
+//
+// An LDS row is the 32 k values of one plane of pieces (64 bytes); its four chunks of 8 lie where neither the reads (16 lanes at a time: rows 0-3 and 12-15 with
+// 4-11 of the next chunk) nor the writes (8 consecutive lanes) meet in a bank (piece_slot). Columns of W are assigned to lanes as in the tile kernel.
+// Splits H floats into three bf16 pieces each, x = h + m + l without a remainder: 8 significant bits rounded to nearest, the next 8 of what is left, and the
+// rest (at most 7 bits). The pairs' chains of operations go step by step side by side: one behind the other, as the compiler would have them, every
+// operation waits for the one before it.
+template <int H>
+__device__ __forceinline__ void bf16_pieces(float (&x)[H], uint32_t (&h)[H / 2], uint32_t (&m)[H / 2], uint32_t (&l)[H / 2]) {
+    constexpr int NOT_VECTOR = 0x94;  // what may cross: scalar operations, memory and LDS
+    auto cut = [&](uint32_t (&piece)[H / 2]) {
+        float t[H];
+#pragma unroll
+        for (int p = 0; p < H / 2; p++) piece[p] = pack_bf16x2(x[2 * p], x[2 * p + 1]);
+        __builtin_amdgcn_sched_barrier(NOT_VECTOR);
+#pragma unroll
+        for (int k = 0; k < H; k++) t[k] = __uint_as_float(k & 1 ? piece[k / 2] & 0xffff0000u : piece[k / 2] << 16);
+        __builtin_amdgcn_sched_barrier(NOT_VECTOR);
+#pragma unroll
+        for (int k = 0; k < H; k++) x[k] -= t[k];
+        __builtin_amdgcn_sched_barrier(NOT_VECTOR);
+    };
+    cut(h);
+    cut(m);
+#pragma unroll
+    for (int p = 0; p < H / 2; p++) l[p] = pack_bf16x2(x[2 * p], x[2 * p + 1]);
 }
+
+// Where the 8 k values `chunk` of a row of a plane lie
+template <int MULT>
+__device__ __forceinline__ unsigned piece_slot(unsigned row, unsigned chunk) {
+    return row * 64 + ((chunk ^ (0u - (row >> 2)) ^ ((row >> 1) & 1) ^ ((row >> 4) * MULT)) & 3) * 16;
+}
+template <int KEEP>  // all but the last KEEP LDS operations of this wavefront are done, and behind the barrier those of the others too
+__device__ __forceinline__ void barrier_behind_lds() {
+    __builtin_amdgcn_s_waitcnt(15 | (KEEP << 8) | (7 << 4) | (3 << 14));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// A wavefront that fetches operands and writes their pieces: per thread and K tile CA runs of H k values of rows of A and CW ones of columns of W, by PT threads
+template <int TM, int TN, int NJ, int CA, int CW, int H, int PT, int SETS, int GROUP>
+__device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, int n_blk, int nkt, unsigned tid, char* smem) {
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE), WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
+    static_assert((H == 8 || H == 4) && (CA == 0 || CA * PT == TM * RUNS) && (CW == 0 || CW * PT == TN * RUNS) && CW <= 2, "shares of a K tile");
+    unsigned a_off[CA + 1], w_off[H], a_dst[CA + 1], w_dst[CW + 1];
+#pragma unroll
+    for (int i = 0; i < CA; i++) {
+        const unsigned q = i * PT + tid, row = q / RUNS, k = q % RUNS * H;
+        a_off[i] = (min(row, (unsigned)(pr.M - 1 - m_blk)) * pr.lda + k) * 4;  // rows beyond M re-read the last one and are never stored
+        a_dst[i] = piece_slot<1>(row, k / 8) + k % 8 * 2;
+    }
+    if constexpr (CW > 0) {
+        const unsigned c = tid % (TN / CW) * CW, k0 = tid / (TN / CW) * H;
+#pragma unroll
+        for (int k = 0; k < H; k++) w_off[k] = ((k0 + k) * pr.ldw + min(n_blk + c, (unsigned)(pr.N - CW))) * 4;
+#pragma unroll
+        for (int x = 0; x < CW; x++) {
+            const unsigned cc = c + x, in = cc % (16 * NJ);
+            w_dst[x] = 3 * A_PLANE + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 8) + k0 % 8 * 2;
+        }
+    }
+    const char* a_tile = reinterpret_cast<const char*>(pr.A + (long long)m_blk * pr.lda);
+    const char* w_tile = reinterpret_cast<const char*>(pr.W + pr.n0);
+    const long long w_step = (long long)pr.ldw * 4 * TK;
+    f32x4_t ra[SETS][CA + 1][H / 4];  // K tiles on their way from memory
+    float rw[SETS][H][CW + 1];
+    auto load_a = [&](int set, int i) {
+        asm volatile("" : "+v"(a_off[i]));
+#pragma unroll
+        for (int x = 0; x < H / 4; x++) ra[set][i][x] = *reinterpret_cast<const f32x4_t*>(a_tile + a_off[i] + 16 * x);
+    };
+    auto load_w = [&](int set) {
+        if constexpr (CW > 0) {
+#pragma unroll
+            for (int k = 0; k < H; k++) {
+                asm volatile("" : "+v"(w_off[k]));
+                float t[CW];
+                load_as<typename Cols<CW>::lds>(reinterpret_cast<const float*>(w_tile + w_off[k]), t);
+#pragma unroll
+                for (int c = 0; c < CW; c++) rw[set][k][c] = t[c];
+            }
+        }
+    };
+    auto put = [&](char* at, int plane, float (&x)[H]) {
+        uint32_t piece[3][H / 2];
+        bf16_pieces<H>(x, piece[0], piece[1], piece[2]);
+#pragma unroll
+        for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * plane, H * 2), piece[p], H * 2);
+    };
+    auto advance = [&](int kt) {  // the addresses, to K tile kt (past the last one: that one again)
+        const bool more = kt < nkt;
+        if (CA) a_tile += more ? TK * 4 : 0;
+        if (CW) w_tile += more ? w_step : 0;
+    };
+    // the pieces of set `set` into `stage`, and the requests of the K tile SETS behind it, which is where the addresses are
+    auto stage_tile = [&](int set, char* stage) {
+        float x[H];
+#pragma unroll
+        for (int i = 0; i < CA; i++) {
+#pragma unroll
+            for (int k = 0; k < H; k++) x[k] = ra[set][i][k >> 2][k & 3];
+            put(stage + a_dst[i], A_PLANE, x);
+            load_a(set, i);
+            if (CA + CW > 4) __builtin_amdgcn_sched_barrier(0);  // (or the runs share too many registers)
+        }
+#pragma unroll
+        for (int c = 0; c < CW; c++) {
+#pragma unroll
+            for (int k = 0; k < H; k++) x[k] = rw[set][k][c];
+            put(stage + w_dst[c], B_PLANE, x);
+            if (CA + CW > 4) __builtin_amdgcn_sched_barrier(0);
+        }
+        load_w(set);
+    };
+#pragma unroll
+    for (int t = 0; t < SETS; t++) {
+#pragma unroll
+        for (int i = 0; i < CA; i++) load_a(t, i);
+        load_w(t);
+        advance(t + 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < GROUP; t++) {
+        stage_tile(t, smem + t * STAGE_BYTES);
+        advance(t + 1 + SETS);
+    }
+    barrier_behind_lds<0>();
+    for (int kt = 0; kt < nkt; kt += SETS) {  // (whole groups of SETS: an end in between would make every round wait for all loads in flight)
+#pragma unroll
+        for (int t = 0; t < SETS; t++) {
+            stage_tile((t + GROUP) % SETS, smem + (t + GROUP) % (2 * GROUP) * STAGE_BYTES);
+            advance(kt + t + GROUP + 1 + SETS);
+            if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
+        }
+    }
+    wait_vmcnt<0>();
+}
+
+// WM x WN wavefronts multiply; PA fetch and split A and PB W (PB = 0: PA both). GROUP: K tiles per barrier. SETS: K tiles on their way from memory. WAVES: wavefronts
+// per SIMD that the registers are to allow. The depth is made of whole groups of four K tiles.
+template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
+__global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_pieces_kernel(const TileProbSet set) {
+    constexpr int TI = TM / WM / 16, NJ = TN / WN / 16, CONSUMERS = WM * WN, REGS = 512 / WAVES - 40;  // REGS: for fragments and sums
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE);
+    static_assert(TI >= 1 && (NJ == 1 || NJ == 2 || NJ == 4), "tile shape");
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    const int w = blockIdx.x;
+    const int which = (w >= set.end[0]) + (w >= set.end[1]);
+    const TileProb& pr = set.p[which];
+    const int M = pr.M, N = pr.N;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int tile_m, tile_n;
+    tile_of_workgroup(w - (which ? set.end[which - 1] : 0), (M + TM - 1) / TM, (N + TN - 1) / TN, tile_m, tile_n);
+    const int m_blk = tile_m * TM, n_blk = tile_n * TN;
+    const int nkt = pr.K / TK;
+    if (wave >= CONSUMERS) {
+        const unsigned tid = threadIdx.x - CONSUMERS * 64;
+        constexpr int CA = TM * (TK / HA) / (PA * 64), CB = TN * (TK / HB) / ((PB ? PB : PA) * 64);
+        if constexpr (PB == 0) {
+            produce_pieces<TM, TN, NJ, CA, CB, HA, PA * 64, SETS, GROUP>(pr, m_blk, n_blk, nkt, tid, smem);
+        } else {
+            if (wave < CONSUMERS + PA) produce_pieces<TM, TN, NJ, CA, 0, HA, PA * 64, SETS, GROUP>(pr, m_blk, n_blk, nkt, tid, smem);
+            else produce_pieces<TM, TN, NJ, 0, CB, HB, PB * 64, SETS, GROUP>(pr, m_blk, n_blk, nkt, tid - PA * 64, smem);
+        }
+        return;
+    }
+
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4, wm = wave / WN, wn = wave % WN;
+    f32x4_t acc[TI][NJ];
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr int WMULT = NJ == 2 ? 2 : 1;
+    const unsigned a_src = piece_slot<1>(wm * (TM / WM) + lr, lg), b_src = 3 * A_PLANE + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
+    auto read_a = [&](bf16x8_t (&f)[TI], const char* stage, int plane) {
+#pragma unroll
+        for (int i = 0; i < TI; i++) {
+            const unsigned key = ((((wm * (TM / WM) >> 4) + i) ^ ((wm * (TM / WM)) >> 4)) & 3) * 16;  // (rows 16 apart have other chunks: slot())
+            f[i] = *reinterpret_cast<const bf16x8_t*>(stage + plane * A_PLANE + (a_src ^ key) + i * 1024);
+        }
+    };
+    auto read_b = [&](bf16x8_t (&f)[NJ], const char* stage, int plane) {
+#pragma unroll
+        for (int j = 0; j < NJ; j++) {
+            const unsigned key = ((((wn * (TN / WN) >> 4) + j) ^ ((wn * (TN / WN)) >> 4)) * WMULT & 3) * 16;
+            f[j] = *reinterpret_cast<const bf16x8_t*>(stage + plane * B_PLANE + (b_src ^ key) + j * 1024);
+        }
+    };
+    auto multiply = [&](const bf16x8_t (&a)[TI], const bf16x8_t (&b)[NJ]) {
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+    };
+    // an LDS read behind each of the first matrix instructions: issued in one go the matrix unit stands still meanwhile
+    auto spread = [](auto reads, auto products) {
+        constexpr int R = decltype(reads)::value, NM = TI * NJ * decltype(products)::value, EACH = R > NM ? (R + NM - 1) / NM : 1;
+#pragma unroll
+        for (int x = 0; x < R; x += EACH) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    typedef std::integral_constant<int, 1> One;
+    typedef std::integral_constant<int, TI> ReadA;
+    typedef std::integral_constant<int, NJ> ReadB;
+    // Products in the order l*h, m*h, m*m, h*m, h*l, h*h, whatever the tile: a row's result depends on neither the shape nor the grouping.
+    if constexpr (3 * (TI + NJ) * 4 * 2 + TI * NJ * 4 <= REGS) {  // all fragments of the next K tile are read beside the products of this one
+        bf16x8_t a[2][3][TI], b[2][3][NJ];
+        auto read = [&](int p, const char* stage) {
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                read_a(a[p][2 - x], stage, 2 - x);
+                read_b(b[p][x], stage, x);
+            }
+        };
+        barrier_behind_lds<0>();
+        read(0, smem);
+        for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
+#pragma unroll
+            for (int t = 0; t < 2 * GROUP; t++) {
+                const int p = t & 1;
+                if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
+                read(p ^ 1, smem + (t + 1) % (2 * GROUP) * STAGE_BYTES);
+                multiply(a[p][2], b[p][0]);
+                multiply(a[p][1], b[p][0]);
+                multiply(a[p][1], b[p][1]);
+                multiply(a[p][0], b[p][1]);
+                multiply(a[p][0], b[p][2]);
+                multiply(a[p][0], b[p][0]);
+                spread(std::integral_constant<int, 3 * (TI + NJ)>{}, std::integral_constant<int, 6>{});
+            }
+        }
+    } else {  // the fragments of one product beside the one before
+        bf16x8_t ah[TI], am[TI], al[TI], bh[2][NJ], bm[NJ], bl[NJ];
+        barrier_behind_lds<0>();
+        read_a(al, smem, 2);
+        read_b(bh[0], smem, 0);
+        for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
+#pragma unroll
+            for (int t = 0; t < 2 * GROUP; t++) {
+                const int p = t & 1;
+                const char *cur = smem + t * STAGE_BYTES, *next = smem + (t + 1) % (2 * GROUP) * STAGE_BYTES;
+                read_a(am, cur, 1);
+                read_b(bm, cur, 1);
+                multiply(al, bh[p]);
+                spread(std::integral_constant<int, TI + NJ>{}, One{});
+                read_a(ah, cur, 0);
+                multiply(am, bh[p]);
+                spread(ReadA{}, One{});
+                read_b(bl, cur, 2);
+                multiply(am, bm);
+                spread(ReadB{}, One{});
+                multiply(ah, bm);
+                spread(std::integral_constant<int, 0>{}, One{});
+                if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
+                read_a(al, next, 2);
+                multiply(ah, bl);
+                spread(ReadA{}, One{});
+                read_b(bh[p ^ 1], next, 0);
+                multiply(ah, bh[p]);
+                spread(ReadB{}, One{});
+            }
+        }
+    }
+    // A value beyond the bf16 range, an infinity or a NaN has no pieces: a sum that is not finite is formed anew from the operands themselves
+    const int m0 = m_blk + wm * (TM / WM), n0 = n_blk + wn * (TN / WN);
+    auto infinite = [](const f32x4_t& v) {
+        bool bad = false;
+#pragma unroll
+        for (int r = 0; r < 4; r++) bad |= (__float_as_uint(v[r]) & 0x7f800000u) == 0x7f800000u;
+        return bad;
+    };
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+        for (int j = 0; j < NJ; j++) bad |= infinite(acc[i][j]);
+    if (__builtin_amdgcn_ballot_w64(bad)) {
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) {
+                if (!__builtin_amdgcn_ballot_w64(infinite(acc[i][j]))) continue;
+                const float* pa = pr.A + (long long)min(m0 + i * 16 + lr, M - 1) * pr.lda + lg;
+                const float* pw = pr.W + (long long)lg * pr.ldw + pr.n0 + min(n0 + NJ * lr + j, N - 1);
+                f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+                for (int k = 0; k < pr.K; k += 4, pa += 4, pw += 4 * (long long)pr.ldw) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(*pa, *pw, sum, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if ((__float_as_uint(acc[i][j][r]) & 0x7f800000u) == 0x7f800000u) acc[i][j][r] = sum[r];
+            }
+    }
+    store_tile<TI, NJ, EPI>(pr, acc, m0 + 4 * lg, n0 + NJ * lr);
+}
+
+template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
+int launch_pieces(TileProbSet& set, int n, hipStream_t st) {
+    auto kern = gemm_f32_pieces_kernel<TM, TN, WM, WN, PA, PB, HA, HB, GROUP, SETS, WAVES, EPI>;
+    constexpr int smem = 2 * GROUP * 3 * (TM + TN) * 64;
+    static DynamicLds lds;
+    SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
+    int total = 0;
+    for (int i = 0; i < MAX_PROBS; i++) {
+        if (i < n) total += ((set.p[i].M + TM - 1) / TM) * ((set.p[i].N + TN - 1) / TN);
+        set.end[i] = total;
+    }
+    hipLaunchKernelGGL(kern, dim3(total), dim3((WM * WN + PA + PB) * 64), smem, st, set);
+    return launch_status("gemm_f32");
+}
+template <int EPI>
+int launch_pieces_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
+    switch (shape) {
+        case 0: return launch_pieces<128, 128, 2, 2, 4, 4, 8, 8, 1, 4, 3, EPI>(set, n, st);
+        // (columns of W by runs of four: a thread's eight loads, one per k value, were what it spent most time on. 128x64 at 512 rows, K = 1536 31 -> 29 us,
+        // 64x64 22.3 -> 20.7, 32x64 17.7 -> 15.4)
+        case 1: return launch_pieces<128, 64, 2, 2, 4, 8, 8, 4, 2, 4, 4, EPI>(set, n, st);
+        case 2: return launch_pieces<64, 64, 2, 2, 4, 8, 8, 4, 2, 4, 4, EPI>(set, n, st);
+        case 3: return launch_pieces<32, 64, 2, 2, 4, 8, 4, 4, 2, 4, 4, EPI>(set, n, st);
+        case 4: return launch_pieces<32, 32, 2, 2, 4, 4, 4, 4, 2, 4, 3, EPI>(set, n, st);
+        default: return launch_pieces<256, 128, 4, 2, 4, 0, 8, 8, 1, 2, 3, EPI>(set, n, st);
+    }
+}
+
+struct Layers {
+    F32Layer l[MAX_PROBS];
+    Layers(const TileProbSet& set, int n) {
+        for (int i = 0; i < n; i++) l[i] = F32Layer{set.p[i].M, set.p[i].N, set.p[i].K};
+    }
+};
 
 // What the tile kernel asks for: operands whose rows are made of aligned 16-byte chunks (its direct loads into LDS) and outputs in whole
 // groups of four columns. The output side may lie at any float with any stride (1024 x 4608 x 1536 into an output that is 4 bytes off: 314 us
@@ -459,7 +813,19 @@ int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st
     if (m == 0) return SD3_OK;
     const int cus = compute_units();
     if (cus <= 0) return SD3_ERR_HIP;
-    const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile : pick_tile(set, m, cus);
+    const Layers layers(set, m);
+    if (whole_k_tiles(set, m) && f32_by_pieces(layers.l, m) && !g_gemm_f32_no_pieces) {
+        const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile : pick_f32_piece_tile(layers.l, m, cus);
+        switch (epi) {
+            case EPI_BIAS: return launch_pieces_shape<EPI_BIAS>(shape, set, m, st);
+            case EPI_BIAS_GELU: return launch_pieces_shape<EPI_BIAS_GELU>(shape, set, m, st);
+            case EPI_BIAS_SILU: return launch_pieces_shape<EPI_BIAS_SILU>(shape, set, m, st);
+            case EPI_GATE_RESID: return launch_pieces_shape<EPI_GATE_RESID>(shape, set, m, st);
+            case EPI_BIAS_ROWADD: return launch_pieces_shape<EPI_BIAS_ROWADD>(shape, set, m, st);
+            default: return fail(SD3_ERR_INVALID_ARG, "gemm_f32: unknown epilogue %d", epi);
+        }
+    }
+    const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile % F32_TILES : pick_f32_tile(layers.l, m, cus, whole_k_tiles(set, m));
     switch (epi) {
         case EPI_BIAS: return launch_shape<EPI_BIAS>(shape, set, m, st);
         case EPI_BIAS_GELU: return launch_shape<EPI_BIAS_GELU>(shape, set, m, st);
@@ -476,6 +842,7 @@ int gemm_f32(const float* A, int lda, const float* W, int ldw, int n0, float* ou
     return gemm_f32_grouped(&q, 1, epi, st);
 }
 
-int g_gemm_f32_tile = -1;  // -1: chosen from the sizes; 0..4: that entry of f32_tiles (sd3_tune)
+int g_gemm_f32_tile = -1;  // -1: chosen from the sizes; 0..5: that entry of f32_tiles or f32_piece_tiles (sd3_tune)
+int g_gemm_f32_no_pieces = 0;  // 1: the kernels of the fp32 instruction at every depth (sd3_tune)
 
 }  // namespace sd3

@@ -1,4 +1,4 @@
-// Which tile shape a launch of fp32 products takes. Host code only.
+// Which kernel and tile shape a launch of fp32 products takes. Host code only.
 #pragma once
 
 namespace sd3 {
@@ -33,6 +33,48 @@ inline int pick_f32_tile(const F32Layer* layers, int n, int cus, bool whole_k) {
         }
         const long long r = (tiles + cus - 1) / cus;
         const double cost = (double)depth / tiles * (r == 1 ? t.alone : r * t.shared);
+        if (s == 0 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+// ---- products of bf16 pieces (gemm_f32_pieces_kernel) ----
+// Which launches: depths of 512 and more, in whole groups of the four K tiles that its loops take at a time. Shallower products are over before the split of the
+// operands is under way: us, fp32 instruction | pieces, 768 columns, K = 256: 64 rows 4.6 | 5.3, 512 6.0 | 6.4, 2356 12.5 | 11.4; K = 768: 64 rows 7.5 | 7.6, 512 10.9 | 10.3,
+// 2356 26.3 | 20.8. By the depth alone: the two kernels round differently, and a row's result is to be the same in every batch.
+inline bool f32_by_pieces(const F32Layer* layers, int n) {
+    for (int i = 0; i < n; i++)
+        if (layers[i].K % 128 || layers[i].K < 512) return false;
+    return true;
+}
+
+// The shapes (the first five as above) and their times in us, measured over N = 768 .. 6144 and K = 256 .. 6144: a launch's last round apart from its K tiles, each
+// round before it likewise, a K tile of a lone workgroup, and by how much longer that takes with every compute unit at work (the power limit; it grows with
+// the square of the share that is. Two and more of the smallest tiles share a unit, which gains more than that).
+struct F32PieceTile {
+    int tm, tn;
+    double last, before, step, crowd;
+};
+constexpr int F32_PIECE_TILES = 6;
+constexpr F32PieceTile f32_piece_tiles[F32_PIECE_TILES] = {{128, 128, 7.3, 7.3, 0.885, 0.24}, {128, 64, 6.4, 6.4, 0.474, 0.28}, {64, 64, 4.5, 3.0, 0.332, 0.14},
+                                                           {32, 64, 3.6, 2.5, 0.246, 0},      {32, 32, 2.8, 0, 0.194, -0.17},   {256, 128, 8.0, 8.0, 1.52, 0.36}};
+inline int pick_f32_piece_tile(const F32Layer* layers, int n, int cus) {
+    int best = 0;
+    double best_cost = 0;
+    for (int s = 0; s < F32_PIECE_TILES; s++) {
+        const F32PieceTile t = f32_piece_tiles[s];
+        long long tiles = 0, depth = 0;
+        for (int i = 0; i < n; i++) {
+            const long long c = (long long)((layers[i].M + t.tm - 1) / t.tm) * ((layers[i].N + t.tn - 1) / t.tn);
+            tiles += c;
+            depth += c * layers[i].K;
+        }
+        const long long full = (tiles - 1) / cus;
+        const double part = (double)(tiles - full * cus) / cus, steps = (double)depth / tiles / 32 * t.step;
+        const double cost = full * (t.before + steps * (1 + t.crowd)) + t.last + steps * (1 + t.crowd * part * part);
         if (s == 0 || cost < best_cost) {
             best = s;
             best_cost = cost;
