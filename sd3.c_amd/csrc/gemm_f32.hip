@@ -2,12 +2,13 @@
 //   out(M,N) = A(M,K) @ W(K,N)[:, n0:n0+N] + epilogue
 // replacing linear / partial_linear of the reference (modules.cpp:475-511, naive triple loops).
 //
-// gemm_f32_pieces_kernel (operands as three bf16 pieces each, on the bf16 matrix instruction) takes depths from 512 on;
+// gemm_f32_pieces_kernel (operands as two f16 pieces each, on the f16 matrix instruction) takes depths from 256 on;
 // gemm_f32_tile_kernel (v_mfma_f32_16x16x4_f32) everything else whose operand rows are made of whole 16-byte chunks; both up to three problems
 // per launch. gemm_f32_kernel (v_mfma_f32_32x32x2_f32, 128x128x16 tiles, element-wise loads) takes operands of any other stride or alignment.
 #include <type_traits>
 
 #include "common.hpp"
+#include "pieces.hpp"
 #include "tiles_f32.hpp"
 
 namespace sd3 {
@@ -420,82 +421,47 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 }
 
 // ---- the pieces kernel ----
-// The bf16 matrix instruction does sixteen times the operations of the fp32 one per cycle. An fp32 value is the sum of three bf16 values, x = h + m + l, without a
-// remainder (bf16_pieces), and a product of two values is the sum of nine products of pieces, which are exact. Six of them are formed: what l*m, m*l and l*l
-// would add is below 2^-25 of the product, the rounding of an fp32 product. The sums are fp32 as before, and fewer additions round: six per 32 k values and
-// block instead of 32. Relative error against 64 bits, normal operands, with this kernel (with the tile kernel): K = 256 2.3e-7 (2.9e-7), 768 4.2e-7 (5.0e-7),
-// 1536 6.0e-7 (7.0e-7), 6144 1.24e-6 (1.40e-6).
+// The f16 matrix instruction does sixteen times the operations of the fp32 one per cycle. A value times a power of two is the sum of two f16 values but for 2^-24
+// of itself (f16_pieces), which is what fp32 rounds away, and of the four products of pieces, which are exact, three are formed: what l*l would add is below 2^-24 of
+// the product. The sums are fp32 as before, and fewer additions round: three per 32 k values and block instead of 32. Relative error against 64 bits, normal
+// operands, with this kernel (with the tile kernel): K = 768 1.5e-7 (2.4e-7), 1536 2.7e-7 (4.3e-7), 6144 7.4e-7 (1.17e-6). (Three bf16 pieces and six products, which
+// need no powers of two: 2.1e-7, 3.7e-7, 1.04e-6, and 105 us where this takes 70.)
+// The powers of two belong to the rows of A and the columns of W and come from their first two K tiles, so that a result depends on neither its neighbours nor the
+// tile. They leave room for values 2^11 times as large as those; a sum that something larger has made infinite is formed anew by the fp32 instruction, as are
+// those of infinities and NaNs.
 //
-// Six products per K tile of 32 are 96 matrix instructions of 17 cycles for a wavefront of 64x64: 240 TFLOP/s if nothing else took time. Splitting the operands does:
-// 11 vector operations per pair of values. Done between the matrix instructions of the same wavefronts they added up (8192 x 3072 x 768: 200 us), so wavefronts
-// of their own do it: they fetch both operands from memory, K tiles ahead, and write the pieces to LDS, while the others read fragments and multiply (173 us;
-// what the vector unit does for one wavefront costs the matrix instructions of another nothing, and a lone wavefront issues a vector operation every 5 cycles,
-// three of them one every 2). One barrier per GROUP K tiles, two buffers.
-// With the LDS reads (256 bytes per cycle), writes (128) and the requests the 256x128 tile takes 3700 cycles per K tile, the matrix instructions 3280; smaller
-// tiles have more to split per product: 128x128 2120 (1640), 128x64 1140 (820), 64x64 800 (410), 32x64 590 (205), 32x32 465 (100; the tile kernel's 440).
-// us, tile kernel -> this one, rows x columns x depth: 8192 x 3072 x 768 280 -> 176 (219 TFLOP/s), 10656 x 768 x 1536 178 -> 110, 1178 x 6144 x 1536 184 -> 105,
-// 1178 x 4608 x 1536 141 -> 92, 1178 x 1536 x 6144 178 -> 130, 1178 x 1536 x 1536 48 -> 37, 333 x 1536 x 1536 25.3 -> 22.4, 64 x 1536 x 1536 12.1 -> 12.0; of 160 sizes
-// from 1 to 8192 rows the worst is 666 x 1536 x 768, 16.9 -> 18.4.
+// Three products per K tile of 32 are 48 matrix instructions of 17 cycles for a wavefront of 64x64. Splitting the operands takes 6 vector operations per pair of
+// values: wavefronts of their own do it. They fetch both operands from memory, K tiles ahead, and write the pieces to LDS, while the others read fragments and
+// multiply. One barrier per GROUP K tiles, two buffers. The splitting wavefronts set the pace (they wait for nobody, the others 40 to 60 % of the time), and not for their loads
+// but for the vector unit, on which matrix instructions of 16 cycles leave little room: 256x128 tiles take 2300 cycles per K tile, the matrix instructions 1540; 128x128 1380 (770),
+// 128x64 720 (390), 64x64 450 (190), 32x64 310 (100), 32x32 230 (50; the tile kernel's 440).
+// us, tile kernel -> this one, rows x columns x depth: 8192 x 3072 x 768 308 -> 115 (337 TFLOP/s), 10656 x 768 x 1536 175 -> 72, 1178 x 6144 x 1536 182 -> 69,
+// 1178 x 4608 x 1536 138 -> 61, 1178 x 1536 x 6144 184 -> 82, 1178 x 1536 x 1536 52 -> 27, 333 x 1536 x 1536 25 -> 16, 64 x 1536 x 6144 40 -> 27, 64 x 1536 x 1536 11.9 -> 10.9.
 //
 // An LDS row is the 32 k values of one plane of pieces (64 bytes); its four chunks of 8 lie where neither the reads (16 lanes at a time: rows 0-3 and 12-15 with
-// 4-11 of the next chunk) nor the writes (8 consecutive lanes) meet in a bank (piece_slot). Columns of W are assigned to lanes as in the tile kernel.
-// Splits H floats into three bf16 pieces each, x = h + m + l without a remainder: 8 significant bits rounded to nearest, the next 8 of what is left, and the
-// rest (at most 7 bits). The pairs' chains of operations go step by step side by side: one behind the other, as the compiler would have them, every
-// operation waits for the one before it.
-template <int H>
-__device__ __forceinline__ void bf16_pieces(float (&x)[H], uint32_t (&h)[H / 2], uint32_t (&m)[H / 2], uint32_t (&l)[H / 2]) {
-    constexpr int NOT_VECTOR = 0x94;  // what may cross: scalar operations, memory and LDS
-    auto cut = [&](uint32_t (&piece)[H / 2]) {
-        float t[H];
-#pragma unroll
-        for (int p = 0; p < H / 2; p++) piece[p] = pack_bf16x2(x[2 * p], x[2 * p + 1]);
-        __builtin_amdgcn_sched_barrier(NOT_VECTOR);
-#pragma unroll
-        for (int k = 0; k < H; k++) t[k] = __uint_as_float(k & 1 ? piece[k / 2] & 0xffff0000u : piece[k / 2] << 16);
-        __builtin_amdgcn_sched_barrier(NOT_VECTOR);
-#pragma unroll
-        for (int k = 0; k < H; k++) x[k] -= t[k];
-        __builtin_amdgcn_sched_barrier(NOT_VECTOR);
-    };
-    cut(h);
-    cut(m);
-#pragma unroll
-    for (int p = 0; p < H / 2; p++) l[p] = pack_bf16x2(x[2 * p], x[2 * p + 1]);
-}
-
-// Where the 8 k values `chunk` of a row of a plane lie
-template <int MULT>
-__device__ __forceinline__ unsigned piece_slot(unsigned row, unsigned chunk) {
-    return row * 64 + ((chunk ^ (0u - (row >> 2)) ^ ((row >> 1) & 1) ^ ((row >> 4) * MULT)) & 3) * 16;
-}
-template <int KEEP>  // all but the last KEEP LDS operations of this wavefront are done, and behind the barrier those of the others too
-__device__ __forceinline__ void barrier_behind_lds() {
-    __builtin_amdgcn_s_waitcnt(15 | (KEEP << 8) | (7 << 4) | (3 << 14));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
+// 4-11 of the next chunk) nor the writes (8 consecutive lanes) meet in a bank (piece_slot). Chunk c holds k = 4c .. 4c + 3 and 16 + 4c .. 16 + 4c + 3, so that the four lanes of a row
+// of A read 64 contiguous bytes at a time (3 % at 256x128). Columns of W are assigned to lanes as in the tile kernel.
 
 // A wavefront that fetches operands and writes their pieces: per thread and K tile CA runs of H k values of rows of A and CW ones of columns of W, by PT threads
 template <int TM, int TN, int NJ, int CA, int CW, int H, int PT, int SETS, int GROUP>
 __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, int n_blk, int nkt, unsigned tid, char* smem) {
-    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE), WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 2 * (A_PLANE + B_PLANE), WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
     static_assert((H == 8 || H == 4) && (CA == 0 || CA * PT == TM * RUNS) && (CW == 0 || CW * PT == TN * RUNS) && CW <= 2, "shares of a K tile");
     unsigned a_off[CA + 1], w_off[H], a_dst[CA + 1], w_dst[CW + 1];
 #pragma unroll
     for (int i = 0; i < CA; i++) {
-        const unsigned q = i * PT + tid, row = q / RUNS, k = q % RUNS * H;
+        const unsigned q = i * PT + tid, row = q / RUNS, k = q % RUNS * 4;
         a_off[i] = (min(row, (unsigned)(pr.M - 1 - m_blk)) * pr.lda + k) * 4;  // rows beyond M re-read the last one and are never stored
-        a_dst[i] = piece_slot<1>(row, k / 8) + k % 8 * 2;
+        a_dst[i] = piece_slot<1>(row, k / 4 % 4) + k / 16 * 8;
     }
     if constexpr (CW > 0) {
-        const unsigned c = tid % (TN / CW) * CW, k0 = tid / (TN / CW) * H;
+        const unsigned c = tid % (TN / CW) * CW, k0 = tid / (TN / CW) * 4;
 #pragma unroll
-        for (int k = 0; k < H; k++) w_off[k] = ((k0 + k) * pr.ldw + min(n_blk + c, (unsigned)(pr.N - CW))) * 4;
+        for (int k = 0; k < H; k++) w_off[k] = ((k0 + k % 4 + k / 4 * 16) * pr.ldw + min(n_blk + c, (unsigned)(pr.N - CW))) * 4;
 #pragma unroll
         for (int x = 0; x < CW; x++) {
             const unsigned cc = c + x, in = cc % (16 * NJ);
-            w_dst[x] = 3 * A_PLANE + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 8) + k0 % 8 * 2;
+            w_dst[x] = 2 * A_PLANE + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 4 % 4) + k0 / 16 * 8;
         }
     }
     const char* a_tile = reinterpret_cast<const char*>(pr.A + (long long)m_blk * pr.lda);
@@ -506,7 +472,7 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
     auto load_a = [&](int set, int i) {
         asm volatile("" : "+v"(a_off[i]));
 #pragma unroll
-        for (int x = 0; x < H / 4; x++) ra[set][i][x] = *reinterpret_cast<const f32x4_t*>(a_tile + a_off[i] + 16 * x);
+        for (int x = 0; x < H / 4; x++) ra[set][i][x] = *reinterpret_cast<const f32x4_t*>(a_tile + a_off[i] + 64 * x);
     };
     auto load_w = [&](int set) {
         if constexpr (CW > 0) {
@@ -520,17 +486,18 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
             }
         }
     };
-    auto put = [&](char* at, int plane, float (&x)[H]) {
-        uint32_t piece[3][H / 2];
-        bf16_pieces<H>(x, piece[0], piece[1], piece[2]);
+    auto put = [&](char* at, int plane, float (&x)[H], float scale) {
+        uint32_t piece[2][H / 2];
+        f16_pieces<H>(x, scale, piece[0], piece[1]);
 #pragma unroll
-        for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * plane, H * 2), piece[p], H * 2);
+        for (int p = 0; p < 2; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * plane, H * 2), piece[p], H * 2);
     };
     auto advance = [&](int kt) {  // the addresses, to K tile kt (past the last one: that one again)
         const bool more = kt < nkt;
         if (CA) a_tile += more ? TK * 4 : 0;
         if (CW) w_tile += more ? w_step : 0;
     };
+    float a_scale[CA + 1], w_scale[CW + 1];
     // the pieces of set `set` into `stage`, and the requests of the K tile SETS behind it, which is where the addresses are
     auto stage_tile = [&](int set, char* stage) {
         float x[H];
@@ -538,7 +505,7 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
         for (int i = 0; i < CA; i++) {
 #pragma unroll
             for (int k = 0; k < H; k++) x[k] = ra[set][i][k >> 2][k & 3];
-            put(stage + a_dst[i], A_PLANE, x);
+            put(stage + a_dst[i], A_PLANE, x, a_scale[i]);
             load_a(set, i);
             if (CA + CW > 4) __builtin_amdgcn_sched_barrier(0);  // (or the runs share too many registers)
         }
@@ -546,10 +513,11 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
         for (int c = 0; c < CW; c++) {
 #pragma unroll
             for (int k = 0; k < H; k++) x[k] = rw[set][k][c];
-            put(stage + w_dst[c], B_PLANE, x);
+            put(stage + w_dst[c], B_PLANE, x, w_scale[c]);
             if (CA + CW > 4) __builtin_amdgcn_sched_barrier(0);
         }
         load_w(set);
+        __builtin_amdgcn_sched_barrier(0);  // (or the products of all sets' values with their scales come first, and wait for all loads in flight)
     };
 #pragma unroll
     for (int t = 0; t < SETS; t++) {
@@ -559,6 +527,33 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
         advance(t + 1);
         __builtin_amdgcn_sched_barrier(0);
     }
+    // Powers of two for each row of A and column of W, from their largest value in the first two K tiles (two, whatever the tile: results depend on it)
+    unsigned* const most = reinterpret_cast<unsigned*>(smem + 2 * GROUP * STAGE_BYTES);  // rows, then columns
+    auto record = [&](unsigned* at, float x) { __hip_atomic_fetch_max(at, __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
+    barrier_behind_lds<0>();
+#pragma unroll
+    for (int i = 0; i < CA; i++) {
+        float x = 0.f;
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int k = 0; k < H; k++) x = larger(x, ra[t][i][k >> 2][k & 3]);
+        record(most + (i * PT + tid) / RUNS, x);
+    }
+#pragma unroll
+    for (int c = 0; c < CW; c++) {
+        float x = 0.f;
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int k = 0; k < H; k++) x = larger(x, rw[t][k][c]);
+        record(most + TM + tid % (TN / (CW + !CW)) * CW + c, x);
+    }
+    barrier_behind_lds<0>();
+#pragma unroll
+    for (int i = 0; i < CA; i++) a_scale[i] = power_of_exponent(scale_exponent(most[(i * PT + tid) / RUNS]));
+#pragma unroll
+    for (int c = 0; c < CW; c++) w_scale[c] = power_of_exponent(scale_exponent(most[TM + tid % (TN / (CW + !CW)) * CW + c]));
 #pragma unroll
     for (int t = 0; t < GROUP; t++) {
         stage_tile(t, smem + t * STAGE_BYTES);
@@ -581,7 +576,7 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
 template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
 __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_pieces_kernel(const TileProbSet set) {
     constexpr int TI = TM / WM / 16, NJ = TN / WN / 16, CONSUMERS = WM * WN, REGS = 512 / WAVES - 40;  // REGS: for fragments and sums
-    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE);
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 2 * (A_PLANE + B_PLANE);
     static_assert(TI >= 1 && (NJ == 1 || NJ == 2 || NJ == 4), "tile shape");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int w = blockIdx.x;
@@ -605,6 +600,9 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
         return;
     }
 
+    for (int i = threadIdx.x; i < TM + TN; i += CONSUMERS * 64) reinterpret_cast<unsigned*>(smem + 2 * GROUP * STAGE_BYTES)[i] = 0;
+    barrier_behind_lds<0>();
+    barrier_behind_lds<0>();
     const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4, wm = wave / WN, wn = wave % WN;
     f32x4_t acc[TI][NJ];
 #pragma unroll
@@ -612,26 +610,26 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     constexpr int WMULT = NJ == 2 ? 2 : 1;
-    const unsigned a_src = piece_slot<1>(wm * (TM / WM) + lr, lg), b_src = 3 * A_PLANE + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
-    auto read_a = [&](bf16x8_t (&f)[TI], const char* stage, int plane) {
+    const unsigned a_src = piece_slot<1>(wm * (TM / WM) + lr, lg), b_src = 2 * A_PLANE + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
+    auto read_a = [&](f16x8_t (&f)[TI], const char* stage, int plane) {
 #pragma unroll
         for (int i = 0; i < TI; i++) {
             const unsigned key = ((((wm * (TM / WM) >> 4) + i) ^ ((wm * (TM / WM)) >> 4)) & 3) * 16;  // (rows 16 apart have other chunks: slot())
-            f[i] = *reinterpret_cast<const bf16x8_t*>(stage + plane * A_PLANE + (a_src ^ key) + i * 1024);
+            f[i] = *reinterpret_cast<const f16x8_t*>(stage + plane * A_PLANE + (a_src ^ key) + i * 1024);
         }
     };
-    auto read_b = [&](bf16x8_t (&f)[NJ], const char* stage, int plane) {
+    auto read_b = [&](f16x8_t (&f)[NJ], const char* stage, int plane) {
 #pragma unroll
         for (int j = 0; j < NJ; j++) {
             const unsigned key = ((((wn * (TN / WN) >> 4) + j) ^ ((wn * (TN / WN)) >> 4)) * WMULT & 3) * 16;
-            f[j] = *reinterpret_cast<const bf16x8_t*>(stage + plane * B_PLANE + (b_src ^ key) + j * 1024);
+            f[j] = *reinterpret_cast<const f16x8_t*>(stage + plane * B_PLANE + (b_src ^ key) + j * 1024);
         }
     };
-    auto multiply = [&](const bf16x8_t (&a)[TI], const bf16x8_t (&b)[NJ]) {
+    auto multiply = [&](const f16x8_t (&a)[TI], const f16x8_t (&b)[NJ]) {
 #pragma unroll
         for (int i = 0; i < TI; i++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
     };
     // an LDS read behind each of the first matrix instructions: issued in one go the matrix unit stands still meanwhile
     auto spread = [](auto reads, auto products) {
@@ -647,13 +645,13 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
     typedef std::integral_constant<int, 1> One;
     typedef std::integral_constant<int, TI> ReadA;
     typedef std::integral_constant<int, NJ> ReadB;
-    // Products in the order l*h, m*h, m*m, h*m, h*l, h*h, whatever the tile: a row's result depends on neither the shape nor the grouping.
-    if constexpr (3 * (TI + NJ) * 4 * 2 + TI * NJ * 4 <= REGS) {  // all fragments of the next K tile are read beside the products of this one
-        bf16x8_t a[2][3][TI], b[2][3][NJ];
+    // Products in the order l*h, h*h, h*l, whatever the tile: a row's result depends on neither the shape nor the grouping.
+    if constexpr (2 * (TI + NJ) * 4 * 2 + TI * NJ * 4 <= REGS) {  // all fragments of the next K tile are read beside the products of this one
+        f16x8_t a[2][2][TI], b[2][2][NJ];
         auto read = [&](int p, const char* stage) {
 #pragma unroll
-            for (int x = 0; x < 3; x++) {
-                read_a(a[p][2 - x], stage, 2 - x);
+            for (int x = 0; x < 2; x++) {
+                read_a(a[p][1 - x], stage, 1 - x);
                 read_b(b[p][x], stage, x);
             }
         };
@@ -665,48 +663,47 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
                 const int p = t & 1;
                 if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
                 read(p ^ 1, smem + (t + 1) % (2 * GROUP) * STAGE_BYTES);
-                multiply(a[p][2], b[p][0]);
                 multiply(a[p][1], b[p][0]);
-                multiply(a[p][1], b[p][1]);
-                multiply(a[p][0], b[p][1]);
-                multiply(a[p][0], b[p][2]);
                 multiply(a[p][0], b[p][0]);
-                spread(std::integral_constant<int, 3 * (TI + NJ)>{}, std::integral_constant<int, 6>{});
+                multiply(a[p][0], b[p][1]);
+                spread(std::integral_constant<int, 2 * (TI + NJ)>{}, std::integral_constant<int, 3>{});
             }
         }
     } else {  // the fragments of one product beside the one before
-        bf16x8_t ah[TI], am[TI], al[TI], bh[2][NJ], bm[NJ], bl[NJ];
+        f16x8_t ah[TI], al[TI], bh[2][NJ], bl[NJ];
         barrier_behind_lds<0>();
-        read_a(al, smem, 2);
+        read_a(al, smem, 1);
         read_b(bh[0], smem, 0);
         for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
 #pragma unroll
             for (int t = 0; t < 2 * GROUP; t++) {
                 const int p = t & 1;
                 const char *cur = smem + t * STAGE_BYTES, *next = smem + (t + 1) % (2 * GROUP) * STAGE_BYTES;
-                read_a(am, cur, 1);
-                read_b(bm, cur, 1);
+                read_a(ah, cur, 0);
+                read_b(bl, cur, 1);
                 multiply(al, bh[p]);
                 spread(std::integral_constant<int, TI + NJ>{}, One{});
-                read_a(ah, cur, 0);
-                multiply(am, bh[p]);
-                spread(ReadA{}, One{});
-                read_b(bl, cur, 2);
-                multiply(am, bm);
-                spread(ReadB{}, One{});
-                multiply(ah, bm);
-                spread(std::integral_constant<int, 0>{}, One{});
                 if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
-                read_a(al, next, 2);
-                multiply(ah, bl);
+                read_a(al, next, 1);
+                multiply(ah, bh[p]);
                 spread(ReadA{}, One{});
                 read_b(bh[p ^ 1], next, 0);
-                multiply(ah, bh[p]);
+                multiply(ah, bl);
                 spread(ReadB{}, One{});
             }
         }
     }
-    // A value beyond the bf16 range, an infinity or a NaN has no pieces: a sum that is not finite is formed anew from the operands themselves
+    const unsigned* const most = reinterpret_cast<const unsigned*>(smem + 2 * GROUP * STAGE_BYTES);
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        const int column = scale_exponent(most[TM + wn * (TN / WN) + NJ * lr + j]);
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                acc[i][j][r] = __builtin_amdgcn_ldexpf(acc[i][j][r], 254 - column - (int)scale_exponent(most[wm * (TM / WM) + i * 16 + 4 * lg + r]));
+    }
+    // A sum that is not finite (values beyond the range of their pieces, infinities, NaNs) is formed anew from the operands themselves
     const int m0 = m_blk + wm * (TM / WM), n0 = n_blk + wn * (TN / WN);
     auto infinite = [](const f32x4_t& v) {
         bool bad = false;
@@ -728,8 +725,9 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
                 const float* pa = pr.A + (long long)min(m0 + i * 16 + lr, M - 1) * pr.lda + lg;
                 const float* pw = pr.W + (long long)lg * pr.ldw + pr.n0 + min(n0 + NJ * lr + j, N - 1);
                 f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-                for (int k = 0; k < pr.K; k += 4, pa += 4, pw += 4 * (long long)pr.ldw) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(*pa, *pw, sum, 0, 0, 0);
+                for (int k = 0; k < pr.K; k += TK, pa += TK, pw += TK * (long long)pr.ldw)
+#pragma unroll
+                    for (int step = 0; step < TK; step += 4) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[step], pw[step * (long long)pr.ldw], sum, 0, 0, 0);
 #pragma unroll
                 for (int r = 0; r < 4; r++)
                     if ((__float_as_uint(acc[i][j][r]) & 0x7f800000u) == 0x7f800000u) acc[i][j][r] = sum[r];
@@ -741,7 +739,7 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
 template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
 int launch_pieces(TileProbSet& set, int n, hipStream_t st) {
     auto kern = gemm_f32_pieces_kernel<TM, TN, WM, WN, PA, PB, HA, HB, GROUP, SETS, WAVES, EPI>;
-    constexpr int smem = 2 * GROUP * 3 * (TM + TN) * 64;
+    constexpr int smem = 2 * GROUP * 2 * (TM + TN) * 64 + (TM + TN) * 4;
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
     int total = 0;

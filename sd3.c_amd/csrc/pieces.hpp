@@ -1,0 +1,56 @@
+// fp32 values as pairs of f16 pieces (fp32 products on the f16 matrix instruction).
+#pragma once
+#include "common.hpp"
+
+namespace sd3 {
+namespace {
+
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {  // rounds to nearest even
+    typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+    const f32x2_t v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+}
+
+// x * scale = h + l: h the first 11 significant bits, rounded to nearest, l the next 11 of what is left; what remains is at most 2^-24 of x, as much as fp32
+// itself rounds away, where x * scale is at least 2^-2 (below that 2^-25 absolute) and less than 65520. Beyond, as for infinities and NaNs, h is infinite or a NaN.
+// A mixed-precision fma takes h as it is; the forms of it that round to f16 would save the conversions behind but take 8.7 cycles (this one and the conversion of
+// two values 4.5, a product 2.6, several wavefronts of a SIMD at it). Step by step for all values, as each step waits for the one before. N values, two to a register.
+template <int N>
+__device__ __forceinline__ void f16_pieces(float (&x)[N], float scale, uint32_t (&h)[N / 2], uint32_t (&l)[N / 2]) {
+#pragma unroll
+    for (int k = 0; k < N; k++) x[k] *= scale;
+#pragma unroll
+    for (int p = 0; p < N / 2; p++) h[p] = pack_f16x2(x[2 * p], x[2 * p + 1]);
+#pragma unroll
+    for (int p = 0; p < N / 2; p++) {
+        asm("v_fma_mix_f32 %0, %0, 1.0, -%1 op_sel_hi:[0,0,1]" : "+v"(x[2 * p]) : "v"(h[p]));
+        asm("v_fma_mix_f32 %0, %0, 1.0, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(x[2 * p + 1]) : "v"(h[p]));
+    }
+#pragma unroll
+    for (int p = 0; p < N / 2; p++) l[p] = pack_f16x2(x[2 * p], x[2 * p + 1]);
+}
+// The exponent field of the power of two that takes values of up to `most` (the bits of an absolute value) to 2^4 .. 2^5: what comes later may be 2^11 times as
+// large. All zero: 2^126, so that anything that comes later is infinite. Infinite or NaN: any.
+__device__ __forceinline__ unsigned scale_exponent(unsigned most) { return (unsigned)min(max(258 - (int)(most >> 23), 1), 253); }
+__device__ __forceinline__ float power_of_exponent(unsigned exponent) { return __uint_as_float(exponent << 23); }
+
+__device__ __forceinline__ float larger(float most, float x) { return fmaxf(most, fabsf(x)); }
+
+// Where `chunk`, 8 k values, of a row of a plane lies
+template <int MULT>
+__device__ __forceinline__ unsigned piece_slot(unsigned row, unsigned chunk) {
+    return row * 64 + ((chunk ^ (0u - (row >> 2)) ^ ((row >> 1) & 1) ^ ((row >> 4) * MULT)) & 3) * 16;
+}
+template <int KEEP>  // all but the last KEEP LDS operations of this wavefront are done, and behind the barrier those of the others too
+__device__ __forceinline__ void barrier_behind_lds() {
+    __builtin_amdgcn_s_waitcnt(15 | (KEEP << 8) | (7 << 4) | (3 << 14));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ bool finite(float x) { return (__float_as_uint(x) & 0x7f800000u) != 0x7f800000u; }
+
+}  // namespace
+}  // namespace sd3

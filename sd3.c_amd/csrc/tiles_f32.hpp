@@ -41,26 +41,27 @@ inline int pick_f32_tile(const F32Layer* layers, int n, int cus, bool whole_k) {
     return best;
 }
 
-// ---- products of bf16 pieces (gemm_f32_pieces_kernel) ----
-// Which launches: depths of 512 and more, in whole groups of the four K tiles that its loops take at a time. Shallower products are over before the split of the
-// operands is under way: us, fp32 instruction | pieces, 768 columns, K = 256: 64 rows 4.6 | 5.3, 512 6.0 | 6.4, 2356 12.5 | 11.4; K = 768: 64 rows 7.5 | 7.6, 512 10.9 | 10.3,
-// 2356 26.3 | 20.8. By the depth alone: the two kernels round differently, and a row's result is to be the same in every batch.
+// ---- products of f16 pieces (gemm_f32_pieces_kernel) ----
+// Which launches: depths of 256 and more, in whole groups of the four K tiles that its loops take at a time. Shallower products are over before the split of the
+// operands is under way. us, fp32 instruction | pieces, a call each: K = 256: 1178 x 3072 21.8 | 15.9, 2356 x 768 12.6 | 11.2, 8192 x 768 29.6 | 20.1; smaller ones are
+// lost in the 11 us that a call costs (forward of 1178 tokens, width 256: 324 us with K = 256 on the fp32 instruction, 319 without). By the depth alone: the two kernels
+// round differently, and a row's result is to be the same in every batch.
 inline bool f32_by_pieces(const F32Layer* layers, int n) {
     for (int i = 0; i < n; i++)
-        if (layers[i].K % 128 || layers[i].K < 512) return false;
+        if (layers[i].K % 128 || layers[i].K < 256) return false;
     return true;
 }
 
-// The shapes (the first five as above) and their times in us, measured over N = 768 .. 6144 and K = 256 .. 6144: a launch's last round apart from its K tiles, each
+// The shapes (the first five as above) and their times in us, measured over M = 1 .. 8192, N = 768 .. 6144 and K = 512 .. 6144 (to 3 to 9 %): a launch's last round apart from its K tiles, each
 // round before it likewise, a K tile of a lone workgroup, and by how much longer that takes with every compute unit at work (the power limit; it grows with
-// the square of the share that is. Two and more of the smallest tiles share a unit, which gains more than that).
+// the square of the share that is).
 struct F32PieceTile {
     int tm, tn;
     double last, before, step, crowd;
 };
 constexpr int F32_PIECE_TILES = 6;
-constexpr F32PieceTile f32_piece_tiles[F32_PIECE_TILES] = {{128, 128, 7.3, 7.3, 0.885, 0.24}, {128, 64, 6.4, 6.4, 0.474, 0.28}, {64, 64, 4.5, 3.0, 0.332, 0.14},
-                                                           {32, 64, 3.6, 2.5, 0.246, 0},      {32, 32, 2.8, 0, 0.194, -0.17},   {256, 128, 8.0, 8.0, 1.52, 0.36}};
+constexpr F32PieceTile f32_piece_tiles[F32_PIECE_TILES] = {{128, 128, 8.6, 6.9, 0.574, 0.38}, {128, 64, 6.6, 6.0, 0.298, 0.45}, {64, 64, 6.2, 2.0, 0.189, 0.42},
+                                                           {32, 64, 6.4, 0.8, 0.128, 0.37},    {32, 32, 6.1, 0.5, 0.095, 0.17},  {256, 128, 9.0, 5.2, 0.974, 0.52}};
 inline int pick_f32_piece_tile(const F32Layer* layers, int n, int cus) {
     int best = 0;
     double best_cost = 0;

@@ -1,4 +1,4 @@
-"""fp32 products of bf16 pieces at the edges of their tiles, beyond the bf16 range and in blocks, against float64 arithmetic and the fp32 instruction."""
+"""fp32 products of f16 pieces at the edges of their tiles, beyond the range of the pieces and in blocks, against float64 arithmetic and the fp32 instruction."""
 import pytest
 import torch
 
@@ -17,10 +17,11 @@ def _automatic_choice_afterwards():
     L.call("sd3_tune", b"gemm_f32_no_pieces", 0)
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 512, 4), (31, 512, 36), (33, 640, 68), (65, 768, 64), (129, 512, 132), (257, 640, 260), (300, 1536, 1540)])
+@pytest.mark.parametrize("m,k,n", [(1, 512, 4), (31, 256, 36), (33, 384, 68), (65, 768, 64), (129, 512, 132), (257, 640, 260), (300, 1536, 1540)])
 def test_every_tile_shape(m, k, n):
-    """Rows and columns on and beside the multiples of the tiles (32 to 256), depths from the smallest on. Bound: a product of pieces lacks less than u of itself, and
-    of the sums no more are rounded than one per value: that of a sum of k products in any order, (k + 2) u (|x| |W| + |b|). The shapes agree bit for bit."""
+    """Rows and columns on and beside the multiples of the tiles (32 to 256), depths from the smallest on. Bound: a product of pieces lacks less than 3 u of itself
+    (u of either value, u for l*l), and of its additions three per 32 values round: less than a sum of k products in any order, (k + 2) u (|x| |W| + |b|). The
+    shapes agree bit for bit."""
     g = torch.Generator(device="cuda").manual_seed(m * 31 + k)
     x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, n), (n,)))
     want = x.double() @ W.double() + b.double()
@@ -36,7 +37,7 @@ def test_every_tile_shape(m, k, n):
 
 @pytest.mark.parametrize("scale_x,scale_w", [(1e-18, 1e-12), (1e15, 1e18), (1e-30, 1e28)])
 def test_small_and_large_values(scale_x, scale_w):
-    """The pieces have the exponents of fp32: the error is that of the tile kernel at any scale (twice it, as two sums of one product may differ)."""
+    """Powers of two bring the values into the range of the pieces: the error is that of the tile kernel at any scale (twice it, as two sums of one product may differ)."""
     g = torch.Generator(device="cuda").manual_seed(7)
     x, W, b = scale_x * torch.randn((200, 512), device="cuda", generator=g), scale_w * torch.randn((512, 192), device="cuda", generator=g), torch.zeros(192, device="cuda")
     want = x.double() @ W.double()
@@ -49,7 +50,7 @@ def test_small_and_large_values(scale_x, scale_w):
 
 @pytest.mark.parametrize("shape", [0, 1, 2, 3, 4, 5])
 def test_infinities_nans_and_values_beyond_bf16(shape):
-    """What has no pieces (infinities, NaNs, finite values that bf16 rounds to infinity, in x and in W) gives what the fp32 instruction gives, and changes nothing else."""
+    """What has no pieces (infinities, NaNs, values much larger than the first of their row, in x and in W) gives what the fp32 instruction gives, and changes nothing else."""
     g = torch.Generator(device="cuda").manual_seed(shape)
     m, k, n = 150, 512, 140
     x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, n), (n,)))
@@ -72,6 +73,27 @@ def test_infinities_nans_and_values_beyond_bf16(shape):
     cols[7] = False
     assert torch.equal(got[rows][:, cols], plain[rows][:, cols])
     assert float(((got[90] - want[90])[finite[90]]).abs().max()) <= (k + 2) * U * 3.4e38 * 4
+
+
+@pytest.mark.parametrize("shape", [0, 1, 2, 3, 4, 5])
+def test_rows_and_columns_of_any_scale(shape):
+    """Rows of x and columns of W from 2^-40 to 2^40, a row whose first 64 and one whose first 200 values are zero, one of zeros, one that grows by 2^20 and a column that does (formed anew
+    by the fp32 instruction), one that starts 2^9 above the rest and one that grows by 2^10. Bound as above: relative to |x| |W| of the element itself."""
+    g = torch.Generator(device="cuda").manual_seed(shape + 50)
+    m, k, n = 150, 512, 140
+    x, W, b = torch.randn((m, k), device="cuda", generator=g), torch.randn((k, n), device="cuda", generator=g), torch.zeros(n, device="cuda")
+    x *= torch.ldexp(torch.ones(m), torch.randint(-40, 41, (m,), generator=torch.Generator().manual_seed(1))).cuda()[:, None]
+    W *= torch.ldexp(torch.ones(n), torch.randint(-40, 41, (n,), generator=torch.Generator().manual_seed(2))).cuda()
+    x[3, :64], x[4, :200], x[5] = 0, 0, 0
+    x[9, 64:] *= 2.0 ** 20
+    x[70, :64] *= 2.0 ** 9
+    x[71, 64:] *= 2.0 ** 10
+    W[100:, 17] *= 2.0 ** 20
+    W[:64, 130] = 0
+    L.call("sd3_tune", b"gemm_f32_tile", shape)
+    y = M.linear(x, W, b)
+    bound = (k + 2) * U * (x.double().abs() @ W.double().abs())
+    assert ((y.double() - x.double() @ W.double()).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("Tc,Tx,dual", [(77, 1000, True), (5, 2049, False)])
