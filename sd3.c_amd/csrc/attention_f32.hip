@@ -3,14 +3,16 @@
 // concatenation / split around it (modules.cpp:1427-1432): keys/values/queries of the joint sequence are read
 // straight from the context buffers (first T[0] tokens) and the latent buffers (next T[1] tokens).
 //
-// Two kernels: attn_f32_split_kernel for head_dim 64 and 128 with 16-byte aligned rows (below), attn_f32_kernel for any other head_dim up
-// to 128. Formulation of both: everything is kept transposed so that the probabilities never leave registers.
+// Three kernels: attn_f32_pieces_kernel (operands as two f16 pieces each, on the f16 matrix instruction) and attn_f32_split_kernel (fp32 matrix instruction, for
+// few queries and heads) for head_dim 64 and 128 with 16-byte aligned rows, attn_f32_kernel for any other head_dim up to 128. Formulation of all: everything is
+// kept transposed so that the probabilities never leave registers.
 //   S^T (keys x queries) = K . Q^T      -> C-layout: a lane owns ONE query column and 16 keys per 32-key block
 //   O^T (d x queries)   += V^T . P^T    -> the lane's own S^T registers are exactly the P^T operand it must supply
 // Online softmax statistics are per query = per lane (plus one exchange with lane^32).
 #include <type_traits>
 
 #include "common.hpp"
+#include "pieces.hpp"
 
 namespace sd3 {
 namespace {
@@ -172,7 +174,7 @@ __global__ void __launch_bounds__(256) attn_f32_kernel(SegDev s, int HS, float s
     }
 }
 
-// ---- head_dim 64 and 128 ----
+// ---- head_dim 64 and 128, few queries ----
 // The matrix unit (v_mfma_f32_16x16x4_f32: 64 FLOP per cycle and SIMD) is the bound, and everything it needs fits the registers of one
 // wavefront: 16*QB queries and 16*KB keys at a time. So no LDS tiles and no barriers: the KS wavefronts of a workgroup share its queries
 // and split the KEYS (tile t goes to wavefront t % KS); K and V rows come straight from memory (L2: all workgroups of a head run on one
@@ -432,7 +434,558 @@ int launch_split(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
     hipLaunchKernelGGL((attn_f32_split_kernel<HS, QB, KB, KS, LONG_ROWS>), dim3((unsigned)total), dim3(KS * 64), 0, st, s, NH, n_q, (int)total, scale);
     return launch_status("attention_f32");
 }
+
+// ---- head_dim 64 and 128 by f16 pieces ----
+// Products as in gemm_f32_pieces_kernel: values times powers of two as two f16 pieces each, three products of pieces on the f16 matrix instruction, fp32 sums. Powers of
+// two: a query's own; one for the K and one for the V of a (batch, head), from three of its tiles of 32 keys, with room for values 2^9 times as large; 2^6 for
+// the probabilities. Results that are not finite (values beyond that, infinities, NaNs) are formed anew on the fp32 instruction (attend_in_f32). Scores, probabilities, their
+// sums and the outputs are fp32 throughout. Relative error against 64 bits, normal inputs (fp32 instruction): 24 heads of 64, 1178 keys 2.9e-7 (4.2e-7), 4250
+// keys 3.9e-7 (6.6e-7), 64 keys 2.0e-7 (2.5e-7); 12 heads of 128, 1178 keys 4.0e-7 (5.2e-7).
+//
+// A wavefront has 32 queries; QG of them share the K and V tiles, which each splits a share of, into LDS. Per tile of 32 keys a wavefront of head_dim 64 issues 24 matrix instructions
+// (768 cycles) and 220 vector operations (about 700), and the two hardly overlap however they are interleaved: the vector unit gets few slots beside matrix
+// instructions, which is also why these are the ones of 32 cycles and not of 16. So it is vector operations that count: two pieces instead of three bf16 ones
+// (350 -> 250 operations, mha of 2 x 1178 tokens, 24 heads 105 -> 81 us), a reference that moves only past a margin, offsets that stay from tile to tile (81 -> 67).
+// The keys are two runs, even and odd tiles, with a reference and sums of their own, merged at the end: half the additions to one sum (error 3.4e-7 -> 2.9e-7),
+// and few queries get twice the wavefronts. KR = 2: side by side; SEQ = 2: one after the other, with the same bits.
+// us, fp32 instruction -> pieces: 2 x 1178 tokens, 24 heads of 64 148 -> 71 (240 TFLOP/s), 4250 tokens 902 -> 400 (277), 16 x 666 tokens, 12 heads of 64 195 -> 102, 4 x 1024
+// queries of 154 keys, 24 heads 57 -> 32, 8 x 1178 tokens, 12 heads of 128 551 -> 251.
+// What f16 pieces cannot give (values beyond their range, infinities, NaNs): the lane's query `qt`, all lanes 32 of them, over all keys on the fp32
+// matrix instruction; out (null: not stored): the query's result from d = 4(l/32) on. For the rare case, so as plain as can be.
+template <int HS>
+__device__ void attend_in_f32(const SegDev& s, int b, int h, int qt, float scale, float* out) {
+    const int l32 = threadIdx.x & 31, lk = threadIdx.x >> 5 & 1;
+    const int qseg = qt < s.Tq[0] ? 0 : 1;
+    const float* q = s.q[qseg] + ((long long)b * s.Tq[qseg] + (qseg ? qt - s.Tq[0] : qt)) * s.ld_qkv[qseg] + h * HS + lk;
+    float m = -1e30f, l = 0.f;
+    f32x16_t o[HS / 32];
+#pragma unroll
+    for (int j = 0; j < HS / 32; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[j][r] = 0.f;
+    for (int seg = 0; seg < 2; seg++)
+        for (int t0 = 0; t0 < s.T[seg]; t0 += 32) {
+            const int last = s.T[seg] - 1;
+            const long long ld = s.ld_qkv[seg], first = (long long)b * s.T[seg];
+            const float* k = s.k[seg] + (first + min(t0 + l32, last)) * ld + h * HS + lk;
+            f32x16_t x;
+#pragma unroll
+            for (int r = 0; r < 16; r++) x[r] = 0.f;
+            for (int d = 0; d < HS; d += 2) x = __builtin_amdgcn_mfma_f32_32x32x2f32(k[d], q[d] * scale, x, 0, 0, 0);
+            float mx = m;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                if (t0 + 8 * (r >> 2) + 4 * lk + (r & 3) > last) x[r] = -1e30f;
+                mx = fmaxf(mx, x[r]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            const float alpha = __builtin_amdgcn_exp2f(m - mx);
+            m = mx;
+            l *= alpha;
+#pragma unroll
+            for (int j = 0; j < HS / 32; j++) o[j] *= alpha;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const float p = __builtin_amdgcn_exp2f(x[r] - mx);
+                l += p;
+                const float* v = s.v[seg] + (first + min(t0 + 8 * (r >> 2) + 4 * lk + (r & 3), last)) * ld + h * HS + l32;
+#pragma unroll
+                for (int j = 0; j < HS / 32; j++) o[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[32 * j], p, o[j], 0, 0, 0);
+            }
+        }
+    const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));
+    if (out)
+#pragma unroll
+        for (int j = 0; j < HS / 32; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) out[32 * j + 8 * (r >> 2) + (r & 3)] = o[j][r] * inv;
+}
+
+// The split of eight values into pieces (f16_pieces) in steps, to be spread over matrix instructions
+struct Split {
+    float x[8];
+    uint32_t piece[2][4];
+    __device__ __forceinline__ void step(int n) {
+        if (n == 0) f16_high<8>(x, piece[0]);
+        else if (n == 1) f16_rest<8>(x, piece[0]);
+        else f16_high<8>(x, piece[1]);
+    }
+};
+
+template <int HS, int QG, int KR, int SEQ>
+struct PiecesShape {
+    static constexpr int QWG = 32 * QG, THREADS = QG * KR * 64;
+    static constexpr int K_PLANE = 32 * 64, V_PLANE = HS * 64;  // bytes: 32 k values of 32 keys; 32 keys of HS values
+    static constexpr int K_BYTES = HS / 32 * 2 * K_PLANE, V_BYTES = 2 * V_PLANE, RUN_BYTES = K_BYTES + 2 * V_BYTES;
+    static constexpr int PITCH = HS / 2 + 4;                    // floats per lane of a run's result
+    static constexpr int MERGE_BYTES = KR / 2 * QG * 64 * PITCH * 4, KEPT_BYTES = SEQ > 1 ? QG * 64 * PITCH * 4 : 0;
+    static constexpr int LDS = (KR * RUN_BYTES > MERGE_BYTES ? KR * RUN_BYTES : MERGE_BYTES) + KEPT_BYTES + 8;
+};
+
+// Where 16 bytes (8 k values) of a 64-byte row lie: neither the reads (32 rows, 16 of them at a time: 0-3, 12-15, 20-27 and the others) nor the writes
+// (8 consecutive lanes) meet in a bank
+__device__ __forceinline__ unsigned row_slot(unsigned row, unsigned chunk) { return row * 64 + ((chunk ^ (row >> 2)) & 3) * 16; }
+
+template <int HS, int QG, int KR, int SEQ>
+__global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces_kernel(SegDev s, int NH, int n_q, int total, float scale) {
+    typedef PiecesShape<HS, QG, KR, SEQ> S;
+    constexpr int NC = HS / 16, ND = HS / 32, PT = QG * 64, CK = 4 * HS / PT, TKEYS = 32, RUNS = KR * SEQ;
+    static_assert(SEQ == 1 || (KR == 1 && SEQ == 2), "runs side by side or two one after the other");
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
+    const int lane = threadIdx.x & 63, l32 = lane & 31, lk = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), run = wave / QG, group = wave % QG;
+    const unsigned tid = threadIdx.x - run * PT;  // among the threads of the run
+    // consecutive workgroup ids go to the 8 XCDs in turn: every XCD gets a contiguous run of (batch, head, query tile)
+    const int xcd = blockIdx.x % 8, local = blockIdx.x / 8, per = (total + 7) / 8, tall = (total % 8) ? (total % 8) : 8;
+    const int item = xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
+    const int bh = item / n_q, h = bh % NH, b = bh / NH, qt = (item % n_q) * S::QWG + group * 32 + l32;
+    const int T0 = s.T[0], T1 = s.T[1], Tq0 = s.Tq[0], TQ = s.Tq[0] + s.Tq[1];
+
+    // pieces of the lane's query: of step c the 8 values d = 32(c/2) + 8(c%2) + 4(l/32) .. +3 and 16 behind them, times a power of two of its own
+    f16x8_t q[2][NC];
+    int q_exponent;
+    {
+        const int t = min(qt, TQ - 1), seg = t < Tq0 ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
+        const float* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? t - Tq0 : t)) * s.ld_qkv[seg] + h * HS + 4 * lk;
+        float x[NC][8], most = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8), hi = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8 + 16);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                x[c][k] = (k < 4 ? lo[k & 3] : hi[k & 3]) * scale;
+                most = larger(most, x[c][k]);
+            }
+        }
+        most = fmaxf(most, __shfl_xor(most, 32, 64));
+        q_exponent = scale_exponent<14>(__float_as_uint(most));
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            uint32_t piece[2][4];
+            f16_pieces<8>(x[c], power_of_exponent(q_exponent), piece[0], piece[1]);
+#pragma unroll
+            for (int w = 0; w < 2; w++) __builtin_memcpy(&q[w][c], piece[w], 16);
+        }
+    }
+    constexpr bool REST = HS == 64;
+    f32x16_t o[ND], o_rest[REST ? ND : 1];  // the products of first pieces, and the others where there are registers for them: so o is rounded once per k step and not three times
+    float m_run = -1e30f, l_run = 0.f;  // l_run: over the keys of this lane
+#pragma unroll
+    for (int j = 0; j < ND; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[j][r] = o_rest[REST ? j : 0][r] = 0.f;
+
+    const int nt0 = (T0 + TKEYS - 1) / TKEYS, n_t = nt0 + (T1 + TKEYS - 1) / TKEYS, first = (n_t + RUNS - 1) / RUNS;
+    const int ld0 = s.ld_qkv[0], ld1 = s.ld_qkv[1];
+    const float* k0 = s.k[0] + (long long)b * T0 * ld0 + h * HS;
+    const float* k1 = s.k[1] + (long long)b * T1 * ld1 + h * HS;
+    const float* v0 = s.v[0] + (long long)b * T0 * ld0 + h * HS;
+    const float* v1 = s.v[1] + (long long)b * T1 * ld1 + h * HS;
+    auto keys_of = [&](int t, int& seg, int& t0) {  // tile t: its segment, its first key in it
+        seg = t < nt0 ? 0 : 1;
+        t0 = (seg ? t - nt0 : t) * TKEYS;
+        return (seg ? T1 : T0) - t0;  // keys from here to the end of the segment
+    };
+    char* const k_lds = smem + run * S::RUN_BYTES;
+    char* const v_lds = k_lds + S::K_BYTES;
+
+    // This thread's share of a tile: CK runs of 8 values of a K row, and CK squares of 4 keys x 2 values of V: d = 16 * (u / 64) + 2 * (u % 8); keys 4 * quad ..: bits
+    // 3, 4, 5 of u are bits 1, 0, 2 of the quad.
+    auto quad_of = [](unsigned u) { return (u >> 3 & 1) << 1 | (u >> 4 & 1) | (u >> 5 & 1) << 2; };
+    f32x4_t kr[CK][2];
+    f32x2_t vr[CK][4];
+    // Where they are: a scalar base per tile, and offsets in bytes that stay as they are from one whole tile of a segment to the next
+    const char *k_base, *v_base;
+    unsigned k_off[CK], v_off[CK][4];
+    int k_rows = -1, v_rows = -1;  // segment and rows of the tile that the offsets are for
+    auto rows_of = [&](int& t, int& ld, int& rows) {  // (tiles past the end: the last one)
+        t = min(t, n_t - 1);
+        const int seg = t < nt0 ? 0 : 1;
+        t = (seg ? t - nt0 : t) * TKEYS;
+        ld = seg ? ld1 : ld0;
+        rows = min((seg ? T1 : T0) - t, TKEYS);
+        return seg;
+    };
+    auto find_k = [&](int t) {
+        int ld, rows;
+        const int seg = rows_of(t, ld, rows), state = seg * 64 + rows;
+        k_base = reinterpret_cast<const char*>((seg ? k1 : k0) + (long long)t * ld);
+        if (state == k_rows) return;
+        k_rows = state;
+#pragma unroll
+        for (int i = 0; i < CK; i++) {
+            const unsigned u = i * PT + tid;
+            k_off[i] = __umul24(min((int)(u / 4 % 32), rows - 1), ld) * 4u + (u / 128 * 32 + u % 4 * 4) * 4;
+        }
+    };
+    auto find_v = [&](int t) {
+        int ld, rows;
+        const int seg = rows_of(t, ld, rows), state = seg * 64 + rows;
+        v_base = reinterpret_cast<const char*>((seg ? v1 : v0) + (long long)t * ld);
+        if (state == v_rows) return;
+        v_rows = state;
+#pragma unroll
+        for (int i = 0; i < CK; i++) {
+            const unsigned u = i * PT + tid;
+#pragma unroll
+            for (int x = 0; x < 4; x++) v_off[i][x] = __umul24(min((int)quad_of(u) * 4 + x, rows - 1), ld) * 4u + (u / 64 * 16 + u % 8 * 2) * 4;
+        }
+    };
+    auto load_k = [&]() {
+#pragma unroll
+        for (int i = 0; i < CK; i++) {
+            kr[i][0] = *reinterpret_cast<const f32x4_t*>(k_base + k_off[i]);
+            kr[i][1] = *reinterpret_cast<const f32x4_t*>(k_base + k_off[i] + 64);
+        }
+    };
+    auto load_v = [&]() {
+#pragma unroll
+        for (int i = 0; i < CK; i++)
+#pragma unroll
+            for (int x = 0; x < 4; x++) vr[i][x] = *reinterpret_cast<const f32x2_t*>(v_base + v_off[i][x]);
+    };
+    Split part;
+    auto put_k = [&](int i) {
+        const unsigned u = i * PT + tid, key = u / 4 % 32, c = u / 128;
+        char* at = k_lds + c * 2 * S::K_PLANE + row_slot(key, u % 4);
+#pragma unroll
+        for (int p = 0; p < 2; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * S::K_PLANE, 16), part.piece[p], 16);
+    };
+    auto put_v = [&](int i, int buffer) {
+        // of 16 keys, 4(l/32) .. +3 of either half are the k values 8(l/32) .. +7 of the matrix instruction, as the scores have them
+        const unsigned u = i * PT + tid, d = u / 64 * 16 + u % 8 * 2, quad = quad_of(u), chunk = quad / 4 * 2 + quad % 2, half = quad / 2 % 2;
+#pragma unroll
+        for (int y = 0; y < 2; y++) {
+            char* at = v_lds + buffer * S::V_BYTES + row_slot(d + y, chunk) + half * 8;
+#pragma unroll
+            for (int p = 0; p < 2; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * S::V_PLANE, 8), &part.piece[p][2 * y], 8);
+        }
+    };
+    // fragments: row l%32, chunk l/32 of one of the two k steps of a 64-byte row
+    const unsigned src = row_slot(l32, lk);
+    auto k_frag = [&](int c, int p) { return *reinterpret_cast<const f16x8_t*>(k_lds + (c / 2 * 2 + p) * S::K_PLANE + (src ^ c % 2 * 32)); };
+    auto v_frag = [&](int buffer, int n, int p) {  // n: d block n / 2, k step n % 2
+        return *reinterpret_cast<const f16x8_t*>(v_lds + buffer * S::V_BYTES + p * S::V_PLANE + n / 2 * 2048 + (src ^ n % 2 * 32));
+    };
+    // The products of pieces of a k step in the order l*h, h*l, h*h; `beside(n)`, n = 0 .. COUNT - 1, is what the vector unit does meanwhile, spread over
+    // the k steps.
+    auto spread = [](bool reads) {
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (reads && x < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x402, 8, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    f32x16_t sc, sn;
+    f16x8_t frag[2][2], p[2][2];
+    float unit;                        // of the scores as they leave the matrix unit
+    constexpr int P_EXPONENT = 6, MARGIN = 8;  // probabilities are kept times 2^6, those of scores up to 2^8 above the reference included
+    auto scores = [&](f32x16_t& x, auto count, auto beside) {
+        constexpr int COUNT = decltype(count)::value;
+        frag[0][1] = k_frag(0, 1);
+        frag[0][0] = k_frag(0, 0);
+#pragma unroll
+        for (int r = 0; r < 16; r++) x[r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int now = c & 1;
+            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][1], q[0][c], x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], q[1][c], x, 0, 0, 0);
+            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], q[0][c], x, 0, 0, 0);
+            if (c + 1 < NC)
+#pragma unroll
+                for (int w = 1; w >= 0; w--) frag[now ^ 1][w] = k_frag(c + 1, w);
+#pragma unroll
+            for (int z = c * COUNT / NC; z < (c + 1) * COUNT / NC; z++) beside(z);
+            spread(c + 1 < NC);
+        }
+    };
+    auto outputs = [&](int buffer, auto count, auto beside) {
+        constexpr int COUNT = decltype(count)::value;
+        frag[0][1] = v_frag(buffer, 0, 1);
+        frag[0][0] = v_frag(buffer, 0, 0);
+#pragma unroll
+        for (int n = 0; n < 2 * ND; n++) {
+            const int now = n & 1, j = n / 2, step = n % 2;
+            f32x16_t& rest = REST ? o_rest[j] : o[j];
+            rest = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][1], p[0][step], rest, 0, 0, 0);
+            rest = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], p[1][step], rest, 0, 0, 0);
+            o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], p[0][step], o[j], 0, 0, 0);
+            if (n + 1 < 2 * ND)
+#pragma unroll
+                for (int w = 1; w >= 0; w--) frag[now ^ 1][w] = v_frag(buffer, n + 1, w);
+#pragma unroll
+            for (int z = n * COUNT / (2 * ND); z < (n + 1) * COUNT / (2 * ND); z++) beside(z);
+            spread(n + 1 < 2 * ND);
+        }
+    };
+    // The softmax of the current tile in steps, for each half of the lane's keys: their probabilities, the sum and the pieces
+    constexpr int SOFTMAX = 6 * 2;
+    auto softmax = [&](f32x16_t& x, int n) {
+        const int half = n / 6, step = n % 6;
+        if (step == 0) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) part.x[k] = __builtin_fmaf(x[8 * half + k], unit, P_EXPONENT - m_run);
+        } else if (step == 1) {
+#pragma unroll
+            for (int k = 0; k < 8; k++) part.x[k] = __builtin_amdgcn_exp2f(part.x[k]);
+        } else if (step == 2) {
+            l_run += ((part.x[0] + part.x[1]) + (part.x[2] + part.x[3])) + ((part.x[4] + part.x[5]) + (part.x[6] + part.x[7]));
+        } else {
+            part.step(step - 3);
+            if (step == 5)
+#pragma unroll
+                for (int w = 0; w < 2; w++) __builtin_memcpy(&p[w][half], part.piece[w], 16);
+        }
+    };
+    // The largest score of a tile, in two steps
+    float most_a, most_b, top;
+    auto largest = [&](const f32x16_t& x, int n) {
+        if (n == 0) {
+            most_a = x[0];
+            most_b = x[8];
+#pragma unroll
+            for (int r = 1; r < 8; r++) {
+                most_a = fmaxf(most_a, x[r]);
+                most_b = fmaxf(most_b, x[8 + r]);
+            }
+        } else {
+            most_a = fmaxf(most_a, most_b);
+            const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(most_a), __float_as_uint(most_a), false, false);
+            top = fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+        }
+    };
+
+    // A run's tiles are run, run + RUNS, ...; one without a tile in the last iteration keeps the barriers' company only. With SEQ = 2 a wavefront has the tiles of the
+    // second run behind those of the first.
+    const int n_it = SEQ > 1 ? n_t : first;
+    auto tile_of = [&](int it) { return SEQ > 1 && it >= first ? it < n_t ? (it - first) * 2 + 1 : n_t : it * RUNS + run; };
+    // K and V tiles to LDS and the requests of the next ones, in steps
+    constexpr int STAGING = 8 * CK;
+    float k_scale, v_scale;
+    auto stage_k = [&](int i, int n) {
+        if (n == 0)
+#pragma unroll
+            for (int k = 0; k < 8; k++) part.x[k] = kr[i][k >> 2][k & 3] * k_scale;
+        if (n < 3) part.step(n);
+        if (n == 2) put_k(i);
+        if (n == 3 && i == CK - 1) load_k();
+    };
+    auto stage_v = [&](int i, int n, int buffer) {
+        if (n == 0)
+#pragma unroll
+            for (int k = 0; k < 8; k++) part.x[k] = vr[i][k & 3][k >> 2] * v_scale;
+        if (n < 3) part.step(n);
+        if (n == 2) put_v(i, buffer);
+        if (n == 3 && i == CK - 1) load_v();
+    };
+    typedef std::integral_constant<int, 0> None;
+    // Powers of two for K and V, from the largest values in the first tile of each run and in the one in the middle, which is the latents' if the first is the context's
+    unsigned* const most = reinterpret_cast<unsigned*>(smem + S::LDS - 8);
+    if (threadIdx.x < 2) most[threadIdx.x] = 0;
+    auto sample = [&](int t) {
+        find_k(t);
+        find_v(t);
+        load_k();
+        load_v();
+    };
+    sample(n_t / 2);
+    float k_most = 0.f, v_most = 0.f;
+    auto look = [&]() {
+#pragma unroll
+        for (int i = 0; i < CK; i++)
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                k_most = larger(k_most, kr[i][k >> 2][k & 3]);
+                v_most = larger(v_most, vr[i][k & 3][k >> 2]);
+            }
+    };
+    look();
+    if (SEQ > 1) {
+        sample(1);
+        look();
+    }
+    sample(tile_of(0));
+    look();
+    barrier_behind_lds<0>();
+    k_most = wave_max(k_most);
+    v_most = wave_max(v_most);
+    if (lane < 2) __hip_atomic_fetch_max(most + lane, __float_as_uint(lane ? v_most : k_most), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    barrier_behind_lds<0>();
+    const int k_exponent = __builtin_amdgcn_readfirstlane(scale_exponent<6>(most[0])), v_exponent = __builtin_amdgcn_readfirstlane(scale_exponent<6>(most[1]));
+    k_scale = power_of_exponent(k_exponent);
+    v_scale = power_of_exponent(v_exponent);
+    unit = power_of_exponent((unsigned)min(max(127 + 254 - q_exponent - k_exponent, 1), 254));
+    find_k(tile_of(1));
+    find_v(tile_of(1));
+#pragma unroll
+    for (int n = 0; n < 4 * CK; n++) stage_k(n / 4, n % 4);
+#pragma unroll
+    for (int n = 0; n < 4 * CK; n++) stage_v(n / 4, n % 4, 0);
+    barrier_behind_lds<0>();
+    scores(sc, None(), [](int) {});
+    barrier_behind_lds<0>();
+    find_k(tile_of(2));
+#pragma unroll
+    for (int n = 0; n < 4 * CK; n++) stage_k(n / 4, n % 4);
+    auto mask = [&](f32x16_t& x, int it) {  // keys past the end of the tile's segment
+        int seg, t0;
+        const int left = keys_of(tile_of(it), seg, t0);
+        if (left < TKEYS) {
+#pragma unroll
+            for (int r = 0; r < 16; r++)
+                if (8 * (r >> 2) + 4 * lk + (r & 3) >= left) x[r] = -__builtin_inff();
+        }
+    };
+    mask(sc, 0);
+    largest(sc, 0);
+    largest(sc, 1);
+    barrier_behind_lds<0>();
+    // Tile `it` of the run, whose scores are x and their largest `top`; y: the scores of the next one. Two barriers: the scores of the next tile beside the softmax of this one;
+    // the outputs beside the split of the K tile after the next and of the next V tile.
+    float* const kept = reinterpret_cast<float*>(smem + S::LDS - 8 - S::KEPT_BYTES) + threadIdx.x * S::PITCH;
+    auto keep = [&](float* at) {
+        at[0] = m_run;
+        at[1] = l_run;
+#pragma unroll
+        for (int j = 0; j < ND; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                f32x4_t four;
+#pragma unroll
+                for (int k = 0; k < 4; k++) four[k] = REST ? o[j][r + k] + o_rest[REST ? j : 0][r + k] : o[j][r + k];
+                *reinterpret_cast<f32x4_t*>(at + 4 + j * 16 + r) = four;
+            }
+    };
+    auto add_rest = [&]() {
+        if (REST)
+#pragma unroll
+            for (int j = 0; j < ND; j++) o[j] += o_rest[REST ? j : 0];
+    };
+    // This wavefront's run and another one; EARLIER: the other one is the earlier of the two (the sums round the same either way round)
+    auto merge_with = [&](const float* at, auto earlier) {
+        constexpr bool EARLIER = decltype(earlier)::value;
+        const float om = at[0], mx = fmaxf(m_run, om);
+        const float wa = __builtin_amdgcn_exp2f(m_run - mx), wb = __builtin_amdgcn_exp2f(om - mx);  // (a run that had no tile: its factor is 0)
+        auto sum = [&](float mine, float other) { return EARLIER ? __builtin_fmaf(other, wb, mine * wa) : __builtin_fmaf(mine, wa, other * wb); };
+        m_run = mx;
+        l_run = sum(l_run, at[1]);
+#pragma unroll
+        for (int j = 0; j < ND; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) o[j][r] = sum(o[j][r], at[4 + j * 16 + r]);
+    };
+    auto tile = [&](int it, f32x16_t& x, f32x16_t& y, auto buffer_tag) {
+        constexpr int buffer = decltype(buffer_tag)::value;
+        const bool mine = tile_of(it) < n_t;
+        if (SEQ > 1 && it == first) {  // the second run starts
+            keep(kept);
+            m_run = -1e30f;
+            l_run = 0.f;
+#pragma unroll
+            for (int j = 0; j < ND; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) o[j][r] = o_rest[REST ? j : 0][r] = 0.f;
+        }
+        if (mine) {
+            // The reference moves only where a score exceeds it by 2^MARGIN: in the first tile and hardly ever again (with the largest score as the reference some of
+            // 32 queries have a larger one in most tiles)
+            const bool moves = top * unit > m_run + MARGIN;
+            if (__builtin_amdgcn_ballot_w64(moves)) {
+                const float m = moves ? top * unit : m_run, alpha = __builtin_amdgcn_exp2f(m_run - m);
+                m_run = m;
+                l_run *= alpha;
+#pragma unroll
+                for (int j = 0; j < ND; j++) {
+                    o[j] *= alpha;
+                    if (REST) o_rest[j] *= alpha;
+                }
+            }
+            find_k(tile_of(it + 3));
+            find_v(tile_of(it + 2));
+            scores(y, std::integral_constant<int, SOFTMAX>(), [&](int n) { softmax(x, n); });
+            // (named here, or the compiler moves what makes them behind the branches that follow, away from the products that it is to run beside)
+            asm volatile("" : "+v"(y), "+v"(l_run));
+#pragma unroll
+            for (int w = 0; w < 2; w++) asm volatile("" : "+v"(p[w][0]), "+v"(p[w][1]));
+        }
+        barrier_behind_lds<0>();
+        if (mine) {
+            mask(y, it + 1);
+            outputs(buffer, std::integral_constant<int, STAGING + 2>(), [&](int n) {
+                if (n < 4 * CK) stage_k(n / 4, n % 4);
+                else if (n < STAGING) stage_v(n / 4 - CK, n % 4, buffer ^ 1);
+                else largest(y, n - STAGING);
+            });
+        }
+        barrier_behind_lds<0>();
+    };
+    for (int it = 0; it < n_it; it += 2) {
+        tile(it, sc, sn, std::integral_constant<int, 0>());
+        if (it + 1 < n_it) tile(it + 1, sn, sc, std::integral_constant<int, 1>());
+    }
+
+    // merge: in each step the upper half of the runs hands its state to the lower half
+    float* merge = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int half = KR / 2; half >= 1; half /= 2) {
+        float* at = merge + (((run < half ? run : run - half) * QG + group) * 64 + lane) * S::PITCH;
+        __syncthreads();
+        if (run >= half && run < 2 * half) keep(at);
+        __syncthreads();
+        if (run < half) {
+            add_rest();
+            merge_with(at, std::false_type());
+        }
+    }
+    if (SEQ > 1 || KR == 1) add_rest();
+    if (SEQ > 1 && n_t > 1) merge_with(kept, std::true_type());
+    l_run *= 1.f / (1 << P_EXPONENT);
+#pragma unroll
+    for (int j = 0; j < ND; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o[j][r] = __builtin_amdgcn_ldexpf(o[j][r], 127 - v_exponent - P_EXPONENT);
+    if (run) return;
+    const float l = l_run + __shfl_xor(l_run, 32, 64), inv = 1.0f / l;
+    bool bad = !finite(l);
+#pragma unroll
+    for (int j = 0; j < ND; j++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            bad |= !finite(o[j][r]);
+            o[j][r] *= inv;
+        }
+    const int seg = qt < Tq0 ? 0 : 1;
+    const bool store = qt < TQ && s.out[seg];
+    float* out = store ? s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_out[seg] + h * HS + 4 * lk : nullptr;
+    if (__builtin_amdgcn_ballot_w64(bad)) {
+        attend_in_f32<HS>(s, b, h, min(qt, TQ - 1), scale, out);
+        return;
+    }
+    if (store)
+#pragma unroll
+        for (int j = 0; j < ND; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) *reinterpret_cast<f32x4_t*>(out + 32 * j + 2 * r) = f32x4_t{o[j][r], o[j][r + 1], o[j][r + 2], o[j][r + 3]};
+}
+
+template <int HS, int QG, int KR, int SEQ>
+int launch_attn_pieces(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
+    typedef PiecesShape<HS, QG, KR, SEQ> S;
+    auto kern = attn_f32_pieces_kernel<HS, QG, KR, SEQ>;
+    static DynamicLds lds;
+    SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), S::LDS));
+    const int TQ = s.Tq[0] + s.Tq[1], n_q = (TQ + S::QWG - 1) / S::QWG;
+    const long long total = (long long)B * NH * n_q;
+    if (total > 0x7fffffff) return fail(SD3_ERR_UNSUPPORTED, "attention (fp32): too many work items");
+    hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(S::THREADS), S::LDS, st, s, NH, n_q, (int)total, scale);
+    return launch_status("attention_f32");
+}
 }  // namespace
+
+int g_attention_f32_no_pieces = 0;  // 1: fp32 matrix instruction in every call (sd3_tune)
 
 int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) {
     const int T = a.T[0] + a.T[1], TQ = a.Tq[0] + a.Tq[1];
@@ -455,9 +1008,24 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     const float scale = (float)(1.0 / sqrtf((float)HS));
     const float scale2 = (float)(1.4426950408889634 / sqrt((double)HS));  // scores in powers of two: the exponentials are one instruction
     if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 24) && a.ld_qkv[1] < (1 << 24)) {
-        // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. (Not by the batch: a batch
-        // element's result stays what it is alone.) Four key runs in both: eight, or the keys over several workgroups and a second
-        // kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four
+        // By pieces where an element has enough for workgroups of 128 queries: heads x blocks of 128 queries from 64 on. us, fp32 instruction | pieces: one element
+        // of 24 heads of 64: 1178 tokens 93 | 38, 384 20.6 | 17.0, 333 17.7 | 15.2, 256 (48 workgroups) 10.7 | 14.4, 128 queries of 2000 keys (24) 24.5 | 49; 12 heads of
+        // 64, 640 tokens (60) 18.5 | 21.7, 666 (72) 20.0 | 20.5; 12 heads of 128, 1178 tokens (120) 90 | 56, 300 queries of 2000 keys (36) 45 | 81. Up to 64 queries
+        // more than half of a block would be empty. (Not by the batch: a batch element's result stays what it is alone.)
+        if (TQ > 64 && (long long)NH * ((TQ + 127) / 128) >= 64 && !g_attention_f32_no_pieces) {
+            // How the two runs of keys are computed, which their results do not depend on: side by side in workgroups of 64 or of 128 queries as long as all of these
+            // find a compute unit, then one after the other in workgroups of half the wavefronts, two to a unit and independent of each other's
+            // barriers. us: 24 heads, 333 tokens 15.2 | 16.4 | 19.3; 1178 tokens 44 | 38 | 48, a batch of two 84 | 77 | 72; 16 x 12 heads, 666 tokens 121 | 118 | 103.
+            if (HS == 128) return launch_attn_pieces<128, 4, 2, 1>(s, B, NH, scale2, st);
+            const int cus = compute_units();
+            if (cus <= 0) return SD3_ERR_HIP;
+            const long long blocks = (long long)B * NH * ((TQ + 127) / 128);
+            if (2 * blocks <= cus) return launch_attn_pieces<64, 2, 2, 1>(s, B, NH, scale2, st);
+            if (blocks <= cus) return launch_attn_pieces<64, 4, 2, 1>(s, B, NH, scale2, st);
+            return launch_attn_pieces<64, 4, 1, 2>(s, B, NH, scale2, st);
+        }
+        // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. Four key runs in both: eight, or the keys over several
+        // workgroups and a second kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four
         // runs 32).
         const bool few = (long long)NH * ((TQ + 31) / 32) < 192;
         if (a.ld_qkv[0] >= (1 << 22) || a.ld_qkv[1] >= (1 << 22))  // (tens of thousands of heads)

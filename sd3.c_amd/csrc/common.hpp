@@ -442,6 +442,7 @@ struct AttnSegments {
     const float* rms_k[2];
 };
 int attention_f32(const AttnSegments& s, int B, int NH, int HS, hipStream_t st);
+extern int g_attention_f32_no_pieces;
 int attention_bf16(const AttnSegments& s, int B, int NH, int HS, hipStream_t st);
 // Up to three attention problems in one launch. kv_splits[i] > 1 (or null: all 1) splits the keys of set i into that many runs, one
 // work item each, whose partial results go through split_ws[i] (attention_bf16_split_workspace_floats floats) and are merged by a

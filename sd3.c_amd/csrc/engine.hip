@@ -1479,6 +1479,10 @@ int sd3_tune(const char* name, int value) {
         g_gemm_f32_tile = value;
         return SD3_OK;
     }
+    if (!std::strcmp(name, "attention_f32_no_pieces")) {
+        g_attention_f32_no_pieces = value != 0;
+        return SD3_OK;
+    }
     if (!std::strcmp(name, "gemm_f32_no_pieces")) {
         g_gemm_f32_no_pieces = value != 0;
         return SD3_OK;

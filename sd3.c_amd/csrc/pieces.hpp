@@ -17,22 +17,32 @@ __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {  // rounds 
 // A mixed-precision fma takes h as it is; the forms of it that round to f16 would save the conversions behind but take 8.7 cycles (this one and the conversion of
 // two values 4.5, a product 2.6, several wavefronts of a SIMD at it). Step by step for all values, as each step waits for the one before. N values, two to a register.
 template <int N>
-__device__ __forceinline__ void f16_pieces(float (&x)[N], float scale, uint32_t (&h)[N / 2], uint32_t (&l)[N / 2]) {
-#pragma unroll
-    for (int k = 0; k < N; k++) x[k] *= scale;
+__device__ __forceinline__ void f16_high(const float (&x)[N], uint32_t (&h)[N / 2]) {
 #pragma unroll
     for (int p = 0; p < N / 2; p++) h[p] = pack_f16x2(x[2 * p], x[2 * p + 1]);
+}
+template <int N>
+__device__ __forceinline__ void f16_rest(float (&x)[N], const uint32_t (&h)[N / 2]) {
 #pragma unroll
     for (int p = 0; p < N / 2; p++) {
         asm("v_fma_mix_f32 %0, %0, 1.0, -%1 op_sel_hi:[0,0,1]" : "+v"(x[2 * p]) : "v"(h[p]));
         asm("v_fma_mix_f32 %0, %0, 1.0, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(x[2 * p + 1]) : "v"(h[p]));
     }
-#pragma unroll
-    for (int p = 0; p < N / 2; p++) l[p] = pack_f16x2(x[2 * p], x[2 * p + 1]);
 }
-// The exponent field of the power of two that takes values of up to `most` (the bits of an absolute value) to 2^4 .. 2^5: what comes later may be 2^11 times as
-// large. All zero: 2^126, so that anything that comes later is infinite. Infinite or NaN: any.
-__device__ __forceinline__ unsigned scale_exponent(unsigned most) { return (unsigned)min(max(258 - (int)(most >> 23), 1), 253); }
+template <int N>
+__device__ __forceinline__ void f16_pieces(float (&x)[N], float scale, uint32_t (&h)[N / 2], uint32_t (&l)[N / 2]) {
+#pragma unroll
+    for (int k = 0; k < N; k++) x[k] *= scale;
+    f16_high<N>(x, h);
+    f16_rest<N>(x, h);
+    f16_high<N>(x, l);
+}
+// The exponent field of the power of two that takes values of up to `most` (the bits of an absolute value) to 2^TARGET .. 2^(TARGET + 1): what comes later may be
+// 2^(15 - TARGET) times as large. All zero: 2^126, so that anything that comes later is infinite. Infinite or NaN: any.
+template <int TARGET = 4>
+__device__ __forceinline__ unsigned scale_exponent(unsigned most) {
+    return (unsigned)min(max(254 + TARGET - (int)(most >> 23), 1), 253);
+}
 __device__ __forceinline__ float power_of_exponent(unsigned exponent) { return __uint_as_float(exponent << 23); }
 
 __device__ __forceinline__ float larger(float most, float x) { return fmaxf(most, fabsf(x)); }
