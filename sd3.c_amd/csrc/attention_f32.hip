@@ -522,6 +522,18 @@ struct PiecesShape {
     static constexpr int LDS = (KR * RUN_BYTES > MERGE_BYTES ? KR * RUN_BYTES : MERGE_BYTES) + KEPT_BYTES + 8;
 };
 
+// The largest of the wavefront's values, in all lanes
+__device__ __forceinline__ float max_of_lanes(float x) {
+    x = fmaxf(x, dpp_move<0x128>(x));  // rotations of 16 lanes by 8, 4, 2 and 1
+    x = fmaxf(x, dpp_move<0x124>(x));
+    x = fmaxf(x, dpp_move<0x122>(x));
+    x = fmaxf(x, dpp_move<0x121>(x));
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+
 // Where 16 bytes (8 k values) of a 64-byte row lie: neither the reads (32 rows, 16 of them at a time: 0-3, 12-15, 20-27 and the others) nor the writes
 // (8 consecutive lanes) meet in a bank
 __device__ __forceinline__ unsigned row_slot(unsigned row, unsigned chunk) { return row * 64 + ((chunk ^ (row >> 2)) & 3) * 16; }
@@ -541,32 +553,6 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     const int bh = item / n_q, h = bh % NH, b = bh / NH, qt = (item % n_q) * S::QWG + group * 32 + l32;
     const int T0 = s.T[0], T1 = s.T[1], Tq0 = s.Tq[0], TQ = s.Tq[0] + s.Tq[1];
 
-    // pieces of the lane's query: of step c the 8 values d = 32(c/2) + 8(c%2) + 4(l/32) .. +3 and 16 behind them, times a power of two of its own
-    f16x8_t q[2][NC];
-    int q_exponent;
-    {
-        const int t = min(qt, TQ - 1), seg = t < Tq0 ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
-        const float* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? t - Tq0 : t)) * s.ld_qkv[seg] + h * HS + 4 * lk;
-        float x[NC][8], most = 0.f;
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8), hi = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8 + 16);
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                x[c][k] = (k < 4 ? lo[k & 3] : hi[k & 3]) * scale;
-                most = larger(most, x[c][k]);
-            }
-        }
-        most = fmaxf(most, __shfl_xor(most, 32, 64));
-        q_exponent = scale_exponent<14>(__float_as_uint(most));
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            uint32_t piece[2][4];
-            f16_pieces<8>(x[c], power_of_exponent(q_exponent), piece[0], piece[1]);
-#pragma unroll
-            for (int w = 0; w < 2; w++) __builtin_memcpy(&q[w][c], piece[w], 16);
-        }
-    }
     constexpr bool REST = HS == 64;
     f32x16_t o[ND], o_rest[REST ? ND : 1];  // the products of first pieces, and the others where there are registers for them: so o is rounded once per k step and not three times
     float m_run = -1e30f, l_run = 0.f;  // l_run: over the keys of this lane
@@ -644,6 +630,49 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
 #pragma unroll
             for (int x = 0; x < 4; x++) vr[i][x] = *reinterpret_cast<const f32x2_t*>(v_base + v_off[i][x]);
     };
+    // (all requests before the first wait)
+    struct Share {
+        f32x4_t k[CK][2];
+        f32x2_t v[CK][4];
+    } middle, second;
+    auto sample = [&](int t, Share& to) {
+        find_k(t);
+        find_v(t);
+        load_k();
+        load_v();
+        __builtin_memcpy(to.k, kr, sizeof(kr));
+        __builtin_memcpy(to.v, vr, sizeof(vr));
+    };
+    Share now;
+    sample(n_t / 2, middle);
+    if (SEQ > 1) sample(1, second);
+    sample(SEQ > 1 ? 0 : run, now);
+    // pieces of the lane's query: of step c the 8 values d = 32(c/2) + 8(c%2) + 4(l/32) .. +3 and 16 behind them, times a power of two of its own
+    f16x8_t q[2][NC];
+    int q_exponent;
+    {
+        const int t = min(qt, TQ - 1), seg = t < Tq0 ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
+        const float* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? t - Tq0 : t)) * s.ld_qkv[seg] + h * HS + 4 * lk;
+        float x[NC][8], most = 0.f;
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8), hi = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8 + 16);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                x[c][k] = (k < 4 ? lo[k & 3] : hi[k & 3]) * scale;
+                most = larger(most, x[c][k]);
+            }
+        }
+        most = fmaxf(most, __shfl_xor(most, 32, 64));
+        q_exponent = scale_exponent<14>(__float_as_uint(most));
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            uint32_t piece[2][4];
+            f16_pieces<8>(x[c], power_of_exponent(q_exponent), piece[0], piece[1]);
+#pragma unroll
+            for (int w = 0; w < 2; w++) __builtin_memcpy(&q[w][c], piece[w], 16);
+        }
+    }
     Split part;
     auto put_k = [&](int i) {
         const unsigned u = i * PT + tid, key = u / 4 % 32, c = u / 128;
@@ -785,33 +814,22 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     // Powers of two for K and V, from the largest values in the first tile of each run and in the one in the middle, which is the latents' if the first is the context's
     unsigned* const most = reinterpret_cast<unsigned*>(smem + S::LDS - 8);
     if (threadIdx.x < 2) most[threadIdx.x] = 0;
-    auto sample = [&](int t) {
-        find_k(t);
-        find_v(t);
-        load_k();
-        load_v();
-    };
-    sample(n_t / 2);
     float k_most = 0.f, v_most = 0.f;
-    auto look = [&]() {
+    auto look = [&](const Share& at) {
 #pragma unroll
         for (int i = 0; i < CK; i++)
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                k_most = larger(k_most, kr[i][k >> 2][k & 3]);
-                v_most = larger(v_most, vr[i][k & 3][k >> 2]);
+                k_most = larger(k_most, at.k[i][k >> 2][k & 3]);
+                v_most = larger(v_most, at.v[i][k & 3][k >> 2]);
             }
     };
-    look();
-    if (SEQ > 1) {
-        sample(1);
-        look();
-    }
-    sample(tile_of(0));
-    look();
+    look(middle);
+    if (SEQ > 1) look(second);
+    look(now);
     barrier_behind_lds<0>();
-    k_most = wave_max(k_most);
-    v_most = wave_max(v_most);
+    k_most = max_of_lanes(k_most);
+    v_most = max_of_lanes(v_most);
     if (lane < 2) __hip_atomic_fetch_max(most + lane, __float_as_uint(lane ? v_most : k_most), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     barrier_behind_lds<0>();
     const int k_exponent = __builtin_amdgcn_readfirstlane(scale_exponent<6>(most[0])), v_exponent = __builtin_amdgcn_readfirstlane(scale_exponent<6>(most[1]));
@@ -846,23 +864,18 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     // Tile `it` of the run, whose scores are x and their largest `top`; y: the scores of the next one. Two barriers: the scores of the next tile beside the softmax of this one;
     // the outputs beside the split of the K tile after the next and of the next V tile.
     float* const kept = reinterpret_cast<float*>(smem + S::LDS - 8 - S::KEPT_BYTES) + threadIdx.x * S::PITCH;
+    auto add_rest = [&]() {
+        if (REST)
+#pragma unroll
+            for (int j = 0; j < ND; j++) o[j] += o_rest[REST ? j : 0];
+    };
     auto keep = [&](float* at) {
         at[0] = m_run;
         at[1] = l_run;
 #pragma unroll
         for (int j = 0; j < ND; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r += 4) {
-                f32x4_t four;
-#pragma unroll
-                for (int k = 0; k < 4; k++) four[k] = REST ? o[j][r + k] + o_rest[REST ? j : 0][r + k] : o[j][r + k];
-                *reinterpret_cast<f32x4_t*>(at + 4 + j * 16 + r) = four;
-            }
-    };
-    auto add_rest = [&]() {
-        if (REST)
-#pragma unroll
-            for (int j = 0; j < ND; j++) o[j] += o_rest[REST ? j : 0];
+            for (int r = 0; r < 16; r += 4) *reinterpret_cast<f32x4_t*>(at + 4 + j * 16 + r) = f32x4_t{o[j][r], o[j][r + 1], o[j][r + 2], o[j][r + 3]};
     };
     // This wavefront's run and another one; EARLIER: the other one is the earlier of the two (the sums round the same either way round)
     auto merge_with = [&](const float* at, auto earlier) {
@@ -881,6 +894,7 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
         constexpr int buffer = decltype(buffer_tag)::value;
         const bool mine = tile_of(it) < n_t;
         if (SEQ > 1 && it == first) {  // the second run starts
+            add_rest();
             keep(kept);
             m_run = -1e30f;
             l_run = 0.f;
@@ -928,6 +942,7 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     }
 
     // merge: in each step the upper half of the runs hands its state to the lower half
+    add_rest();
     float* merge = reinterpret_cast<float*>(smem);
 #pragma unroll
     for (int half = KR / 2; half >= 1; half /= 2) {
@@ -935,12 +950,8 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
         __syncthreads();
         if (run >= half && run < 2 * half) keep(at);
         __syncthreads();
-        if (run < half) {
-            add_rest();
-            merge_with(at, std::false_type());
-        }
+        if (run < half) merge_with(at, std::false_type());
     }
-    if (SEQ > 1 || KR == 1) add_rest();
     if (SEQ > 1 && n_t > 1) merge_with(kept, std::true_type());
     l_run *= 1.f / (1 << P_EXPONENT);
 #pragma unroll
@@ -1008,18 +1019,19 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     const float scale = (float)(1.0 / sqrtf((float)HS));
     const float scale2 = (float)(1.4426950408889634 / sqrt((double)HS));  // scores in powers of two: the exponentials are one instruction
     if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 24) && a.ld_qkv[1] < (1 << 24)) {
-        // By pieces where an element has enough for workgroups of 128 queries: heads x blocks of 128 queries from 64 on. us, fp32 instruction | pieces: one element
-        // of 24 heads of 64: 1178 tokens 93 | 38, 384 20.6 | 17.0, 333 17.7 | 15.2, 256 (48 workgroups) 10.7 | 14.4, 128 queries of 2000 keys (24) 24.5 | 49; 12 heads of
-        // 64, 640 tokens (60) 18.5 | 21.7, 666 (72) 20.0 | 20.5; 12 heads of 128, 1178 tokens (120) 90 | 56, 300 queries of 2000 keys (36) 45 | 81. Up to 64 queries
-        // more than half of a block would be empty. (Not by the batch: a batch element's result stays what it is alone.)
-        if (TQ > 64 && (long long)NH * ((TQ + 127) / 128) >= 64 && !g_attention_f32_no_pieces) {
+        // By pieces where an element has enough for workgroups of 128 queries: heads x blocks of 128 queries from 64 on, with more than 256 queries from 48. us, fp32
+        // instruction | pieces: one element of 24 heads of 64: 1178 tokens 89 | 37, 333 17.8 | 14.7, 256 (48 workgroups) 11.0 | 12.5, 128 queries of 2000 keys (24)
+        // 25 | 45; 12 heads of 64, 512 tokens (48) 16.1 | 17.0, two of these 24.5 | 17.3, 16 118 | 57; 12 heads of 128, 1178 tokens (120) 90 | 56, 300 queries of 2000 keys
+        // (36) 45 | 81. Up to 64 queries more than half of a block would be empty. (Not by the batch: a batch element's result stays what it is alone.)
+        const long long element_blocks = (long long)NH * ((TQ + 127) / 128);
+        if (TQ > 64 && element_blocks >= (TQ > 256 ? 48 : 64) && !g_attention_f32_no_pieces) {
             // How the two runs of keys are computed, which their results do not depend on: side by side in workgroups of 64 or of 128 queries as long as all of these
             // find a compute unit, then one after the other in workgroups of half the wavefronts, two to a unit and independent of each other's
-            // barriers. us: 24 heads, 333 tokens 15.2 | 16.4 | 19.3; 1178 tokens 44 | 38 | 48, a batch of two 84 | 77 | 72; 16 x 12 heads, 666 tokens 121 | 118 | 103.
+            // barriers. us: 24 heads, 333 tokens 14.7 | 16.6 | 19.1; 1178 tokens 45 | 37 | 47, a batch of two 89 | 77 | 72; 16 x 12 heads, 666 tokens 117 | 119 | 104.
             if (HS == 128) return launch_attn_pieces<128, 4, 2, 1>(s, B, NH, scale2, st);
             const int cus = compute_units();
             if (cus <= 0) return SD3_ERR_HIP;
-            const long long blocks = (long long)B * NH * ((TQ + 127) / 128);
+            const long long blocks = B * element_blocks;
             if (2 * blocks <= cus) return launch_attn_pieces<64, 2, 2, 1>(s, B, NH, scale2, st);
             if (blocks <= cus) return launch_attn_pieces<64, 4, 2, 1>(s, B, NH, scale2, st);
             return launch_attn_pieces<64, 4, 1, 2>(s, B, NH, scale2, st);

@@ -36,7 +36,7 @@ def on_fp32_instruction(*args):
 
 
 @pytest.mark.parametrize("B,NH,hs,Tq,Tk", [(1, 64, 64, 65, 1), (1, 64, 64, 127, 31), (1, 64, 64, 128, 32), (1, 32, 64, 129, 33), (2, 64, 64, 129, 63), (1, 22, 64, 257, 97),
-                                           (5, 64, 64, 65, 64), (5, 64, 64, 100, 1), (5, 64, 64, 128, 65), (3, 64, 64, 257, 191), (1, 64, 128, 65, 33), (2, 32, 128, 129, 65),
+                                           (5, 64, 64, 65, 64), (5, 64, 64, 100, 1), (5, 64, 64, 128, 65), (3, 64, 64, 257, 191), (1, 12, 64, 512, 97), (1, 64, 128, 65, 33), (2, 32, 128, 129, 65),
                                            (5, 64, 128, 100, 127)])
 def test_edges(B, NH, hs, Tq, Tk):
     """One key tile (a run without keys) to six, whole and not, query blocks of 64 and 128, the runs side by side (up to 256 blocks of 128 queries) and one after the other."""
