@@ -424,7 +424,7 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 // The f16 matrix instruction does sixteen times the operations of the fp32 one per cycle. A value times a power of two is the sum of two f16 values but for 2^-24
 // of itself (f16_pieces), which is what fp32 rounds away, and of the four products of pieces, which are exact, three are formed: what l*l would add is below 2^-24 of
 // the product. The sums are fp32 as before, and fewer additions round: three per 32 k values and block instead of 32. Relative error against 64 bits, normal
-// operands, with this kernel (with the tile kernel): K = 768 1.5e-7 (2.4e-7), 1536 2.7e-7 (4.3e-7), 6144 7.4e-7 (1.17e-6). (Three bf16 pieces and six products, which
+// operands, with this kernel (with the tile kernel): K = 256 1.9e-7 (2.9e-7), 768 3.1e-7 (4.9e-7), 1536 4.4e-7 (7.0e-7), 6144 8.8e-7 (1.41e-6). (Three bf16 pieces and six products, which
 // need no powers of two: 0.85 of the tile kernel's error, and 105 us where this takes 70.)
 // The powers of two belong to the rows of A and the columns of W and come from their first two K tiles, so that a result depends on neither its neighbours nor the
 // tile. They leave room for values 2^11 times as large as those; a sum that something larger has made infinite is formed anew by the fp32 instruction, as are
