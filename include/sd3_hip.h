@@ -262,7 +262,7 @@ int sd3_gemm_bf16_force_tile(int tile);
  * with the number of splits); "gemm_bf16_row_split": 0 / 1 (default), whether a many-row problem that leaves a partial round of
  * 256x256 tiles may send its last rows to a second launch of smaller tiles; "gemm_f32_tile": -1 chosen from the sizes (default), 0..5 a
  * fixed tile shape of the fp32 GEMM (128x128, 128x64, 64x64, 32x64, 32x32; 256x128 where there is one, else 128x128); "gemm_f32_no_pieces": 1 forms
- * fp32 products of every depth on the fp32 matrix instruction (results change in the last bits), 0 deep ones of two f16 pieces per value
+ * fp32 products of every depth on the fp32 matrix instruction (results change in the last bits), 0 deep ones of three bf16 pieces per value
  * (default); "attention_f32_no_pieces": the same for fp32 attention. Unknown names return SD3_ERR_INVALID_ARG. */
 int sd3_tune(const char* name, int value);
 /* Measurement aid with no counterpart in the reference: the rate (in TFLOP/s) at which the device's matrix cores run the

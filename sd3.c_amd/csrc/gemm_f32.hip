@@ -2,7 +2,7 @@
 //   out(M,N) = A(M,K) @ W(K,N)[:, n0:n0+N] + epilogue
 // replacing linear / partial_linear of the reference (modules.cpp:475-511, naive triple loops).
 //
-// gemm_f32_pieces_kernel (operands as two f16 pieces each, on the f16 matrix instruction) takes depths from 256 on;
+// gemm_f32_pieces_kernel (operands as three bf16 pieces each, on the bf16 matrix instruction) takes depths from 256 on;
 // gemm_f32_tile_kernel (v_mfma_f32_16x16x4_f32) everything else whose operand rows are made of whole 16-byte chunks; both up to three problems
 // per launch. gemm_f32_kernel (v_mfma_f32_32x32x2_f32, 128x128x16 tiles, element-wise loads) takes operands of any other stride or alignment.
 #include <type_traits>
@@ -421,22 +421,26 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 }
 
 // ---- the pieces kernel ----
-// The f16 matrix instruction does sixteen times the operations of the fp32 one per cycle. A value times a power of two is the sum of two f16 values but for 2^-24
-// of itself (f16_pieces), which is what fp32 rounds away, and of the four products of pieces, which are exact, three are formed: what l*l would add is below 2^-24 of
-// the product. The sums are fp32 as before, and fewer additions round: three per 32 k values and block instead of 32. Relative error against 64 bits, normal
-// operands, with this kernel (with the tile kernel): K = 256 1.9e-7 (2.9e-7), 768 3.1e-7 (4.9e-7), 1536 4.4e-7 (7.0e-7), 6144 8.8e-7 (1.41e-6). (Three bf16 pieces and six products, which
-// need no powers of two: 0.85 of the tile kernel's error, and 105 us where this takes 70.)
-// The powers of two belong to the rows of A and the columns of W and come from their first two K tiles, so that a result depends on neither its neighbours nor the
-// tile. They leave room for values 2^11 times as large as those; a sum that something larger has made infinite is formed anew by the fp32 instruction, as are
-// those of infinities and NaNs: 16 rows at a time from memory, for 1178 x 1536 x 1536 32 us more for a row of them and 340 us where all rows have some.
+// The bf16 matrix instruction does sixteen times the operations of the fp32 one per cycle. An fp32 value is the sum of three bf16 values, h + m + l, without a
+// remainder (bf16_pieces), and a product of two values that of nine products of pieces, which are exact. Six of them are formed: what m*l, l*m and l*l would add is at
+// most 2^-24 + 2^-34 of the product, half a unit in its last place. No value is lost beside a larger one of its row, column or product. (Two f16 pieces per value and
+// three products took 0.65 of this time, 1178 x 6144 x 1536 69 us, but hold 22 of the 24 bits, and only of values within 2^-7 of the largest that the scale is
+// made for: rows of one channel 2^20 times the others, which W leaves out, came out with an error of 9e-4.)
+// The products of a K tile (32 k values) are summed by themselves, and that sum is then added to the fp32 sum of the tiles before: one rounding per K tile that counts,
+// where the fp32 instruction has eight. Relative error against 64 bits, normal operands, with this kernel (with the tile kernel): K = 256 7.0e-8 (2.9e-7), 1536
+// 1.4e-7 (7.0e-7), 6144 2.7e-7 (1.41e-6); one in 16 values of A not zero 1536 1.4e-7 (1.8e-7); all values 1 + 2^-11 1.6e-7 (1.6e-7). All six products added to one sum:
+// 0.85 of the tile kernel's error for normal operands but 1.9 times it for one in 16, 8192 x 3072 x 768 177 us instead of 189; the five small products in a second
+// sum: 0.34 of it, but 256x128 tiles have no registers for that, 219 us.
+// Sums that are not finite (infinities, NaNs, values from 2^112 and sums from 2^96 on) are formed anew by the fp32 instruction, 16 rows at a time from memory: 1178 x 1536 x
+// 1536 43 us, 104 with one such row, 250 with one in 16 or all (tile kernel 50 to 55).
 //
-// Three products per K tile of 32 are 48 matrix instructions of 17 cycles for a wavefront of 64x64. Splitting the operands takes 6 vector operations per pair of
-// values: wavefronts of their own do it. They fetch both operands from memory, K tiles ahead, and write the pieces to LDS, while the others read fragments and
-// multiply. One barrier per GROUP K tiles, two buffers. The splitting wavefronts set the pace (they wait for nobody, the others 40 to 60 % of the time), and not for their loads
-// but for the vector unit, on which matrix instructions of 16 cycles leave little room: 256x128 tiles take 2300 cycles per K tile, the matrix instructions 1540; 128x128 1380 (770),
-// 128x64 720 (390), 64x64 450 (190), 32x64 310 (100), 32x32 230 (50; the tile kernel's 440).
-// us, tile kernel -> this one, rows x columns x depth: 8192 x 3072 x 768 308 -> 115 (337 TFLOP/s), 10656 x 768 x 1536 175 -> 72, 1178 x 6144 x 1536 182 -> 69,
-// 1178 x 4608 x 1536 138 -> 61, 1178 x 1536 x 6144 184 -> 82, 1178 x 1536 x 1536 52 -> 27, 333 x 1536 x 1536 25 -> 16, 64 x 1536 x 6144 40 -> 27, 64 x 1536 x 1536 11.9 -> 10.9.
+// Six products per K tile of 32 are 96 matrix instructions of 17 cycles for a wavefront of 64x64. Splitting the operands takes 12 vector operations per pair of values:
+// wavefronts of their own do it. They fetch both operands from memory, K tiles ahead, and write the pieces to LDS, while the others read fragments and
+// multiply. One barrier per GROUP K tiles, two buffers. (x - h as one v_dot2c_f32_bf16 instead of two operations: it takes turns with the matrix instructions,
+// 168 -> 188 us for 8192 x 3072 x 768 with one sum and no scale.) Matrix instructions of 16 cycles leave the vector unit little room: 256x128 tiles take 4460 cycles per K tile, the matrix
+// instructions 3260; 128x128 2290 (1630), 128x64 1290 (820), 64x64 740 (410), 32x64 545 (205), 32x32 370 (100; the tile kernel's 440).
+// us, tile kernel -> this one, rows x columns x depth: 8192 x 3072 x 768 312 -> 189 (205 TFLOP/s), 10656 x 768 x 1536 181 -> 121, 1178 x 6144 x 1536 182 -> 116,
+// 1178 x 4608 x 1536 139 -> 107, 1178 x 1536 x 6144 187 -> 142, 1178 x 1536 x 1536 52 -> 40, 333 x 1536 x 1536 24.6 -> 22.2, 64 x 1536 x 6144 39 -> 41, 64 x 1536 x 1536 11.9 -> 12.6.
 //
 // An LDS row is the 32 k values of one plane of pieces (64 bytes); its four chunks of 8 lie where neither the reads (16 lanes at a time: rows 0-3 and 12-15 with
 // 4-11 of the next chunk) nor the writes (8 consecutive lanes) meet in a bank (piece_slot). Chunk c holds k = 4c .. 4c + 3 and 16 + 4c .. 16 + 4c + 3, so that the four lanes of a row
@@ -445,14 +449,14 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 // A wavefront that fetches operands and writes their pieces: per thread and K tile CA runs of H k values of rows of A and CW ones of columns of W, by PT threads
 template <int TM, int TN, int NJ, int CA, int CW, int H, int PT, int SETS, int GROUP>
 __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, int n_blk, int nkt, unsigned tid, char* smem) {
-    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 2 * (A_PLANE + B_PLANE), WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE), WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
     static_assert((H == 8 || H == 4) && (CA == 0 || CA * PT == TM * RUNS) && (CW == 0 || CW * PT == TN * RUNS) && CW <= 2, "shares of a K tile");
     unsigned a_off[CA + 1], w_off[H], a_dst[CA + 1], w_dst[CW + 1];
 #pragma unroll
     for (int i = 0; i < CA; i++) {
         const unsigned q = i * PT + tid, row = q / RUNS, k = q % RUNS * 4;
         a_off[i] = (min(row, (unsigned)(pr.M - 1 - m_blk)) * pr.lda + k) * 4;  // rows beyond M re-read the last one and are never stored
-        a_dst[i] = piece_slot<1>(row, k / 4 % 4) + k / 16 * 8;
+        a_dst[i] = piece_slot<0>(row, k / 4 % 4) + k / 16 * 8;
     }
     if constexpr (CW > 0) {
         const unsigned c = tid % (TN / CW) * CW, k0 = tid / (TN / CW) * 4;
@@ -461,7 +465,7 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
 #pragma unroll
         for (int x = 0; x < CW; x++) {
             const unsigned cc = c + x, in = cc % (16 * NJ);
-            w_dst[x] = 2 * A_PLANE + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 4 % 4) + k0 / 16 * 8;
+            w_dst[x] = 3 * A_PLANE + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 4 % 4) + k0 / 16 * 8;
         }
     }
     const char* a_tile = reinterpret_cast<const char*>(pr.A + (long long)m_blk * pr.lda);
@@ -486,26 +490,25 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
             }
         }
     };
-    auto put = [&](char* at, int plane, float (&x)[H], float scale) {
-        uint32_t piece[2][H / 2];
-        f16_pieces<H>(x, scale, piece[0], piece[1]);
-#pragma unroll
-        for (int p = 0; p < 2; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * plane, H * 2), piece[p], H * 2);
-    };
     auto advance = [&](int kt) {  // the addresses, to K tile kt (past the last one: that one again)
         const bool more = kt < nkt;
         if (CA) a_tile += more ? TK * 4 : 0;
         if (CW) w_tile += more ? w_step : 0;
     };
-    float a_scale[CA + 1], w_scale[CW + 1];
     // the pieces of set `set` into `stage`, and the requests of the K tile SETS behind it, which is where the addresses are
     auto stage_tile = [&](int set, char* stage) {
         float x[H];
+        auto put = [&](char* at, int plane) {
+            uint32_t piece[3][H / 2];
+            bf16_pieces<H>(x, piece[0], piece[1], piece[2]);
+#pragma unroll
+            for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * plane, H * 2), piece[p], H * 2);
+        };
 #pragma unroll
         for (int i = 0; i < CA; i++) {
 #pragma unroll
             for (int k = 0; k < H; k++) x[k] = ra[set][i][k >> 2][k & 3];
-            put(stage + a_dst[i], A_PLANE, x, a_scale[i]);
+            put(stage + a_dst[i], A_PLANE);
             load_a(set, i);
             if (CA + CW > 4) __builtin_amdgcn_sched_barrier(0);  // (or the runs share too many registers)
         }
@@ -513,11 +516,11 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
         for (int c = 0; c < CW; c++) {
 #pragma unroll
             for (int k = 0; k < H; k++) x[k] = rw[set][k][c];
-            put(stage + w_dst[c], B_PLANE, x, w_scale[c]);
+            put(stage + w_dst[c], B_PLANE);
             if (CA + CW > 4) __builtin_amdgcn_sched_barrier(0);
         }
         load_w(set);
-        __builtin_amdgcn_sched_barrier(0);  // (or the products of all sets' values with their scales come first, and wait for all loads in flight)
+        __builtin_amdgcn_sched_barrier(0);  // (or the products of all sets' values with their scale come first, and wait for all loads in flight)
     };
 #pragma unroll
     for (int t = 0; t < SETS; t++) {
@@ -527,33 +530,6 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
         advance(t + 1);
         __builtin_amdgcn_sched_barrier(0);
     }
-    // Powers of two for each row of A and column of W, from their largest value in the first two K tiles (two, whatever the tile: results depend on it)
-    unsigned* const most = reinterpret_cast<unsigned*>(smem + 2 * GROUP * STAGE_BYTES);  // rows, then columns
-    auto record = [&](unsigned* at, float x) { __hip_atomic_fetch_max(at, __float_as_uint(x), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); };
-    barrier_behind_lds<0>();
-#pragma unroll
-    for (int i = 0; i < CA; i++) {
-        float x = 0.f;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int k = 0; k < H; k++) x = larger(x, ra[t][i][k >> 2][k & 3]);
-        record(most + (i * PT + tid) / RUNS, x);
-    }
-#pragma unroll
-    for (int c = 0; c < CW; c++) {
-        float x = 0.f;
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-#pragma unroll
-            for (int k = 0; k < H; k++) x = larger(x, rw[t][k][c]);
-        record(most + TM + tid % (TN / (CW + !CW)) * CW + c, x);
-    }
-    barrier_behind_lds<0>();
-#pragma unroll
-    for (int i = 0; i < CA; i++) a_scale[i] = power_of_exponent(scale_exponent(most[(i * PT + tid) / RUNS]));
-#pragma unroll
-    for (int c = 0; c < CW; c++) w_scale[c] = power_of_exponent(scale_exponent(most[TM + tid % (TN / (CW + !CW)) * CW + c]));
 #pragma unroll
     for (int t = 0; t < GROUP; t++) {
         stage_tile(t, smem + t * STAGE_BYTES);
@@ -575,8 +551,8 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
 // per SIMD that the registers are to allow. The depth is made of whole groups of four K tiles.
 template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
 __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_pieces_kernel(const TileProbSet set) {
-    constexpr int TI = TM / WM / 16, NJ = TN / WN / 16, CONSUMERS = WM * WN, REGS = 512 / WAVES - 40;  // REGS: for fragments and sums
-    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 2 * (A_PLANE + B_PLANE);
+    constexpr int TI = TM / WM / 16, NJ = TN / WN / 16, CONSUMERS = WM * WN;
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE);
     static_assert(TI >= 1 && (NJ == 1 || NJ == 2 || NJ == 4), "tile shape");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int w = blockIdx.x;
@@ -600,9 +576,6 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
         return;
     }
 
-    for (int i = threadIdx.x; i < TM + TN; i += CONSUMERS * 64) reinterpret_cast<unsigned*>(smem + 2 * GROUP * STAGE_BYTES)[i] = 0;
-    barrier_behind_lds<0>();
-    barrier_behind_lds<0>();
     const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4, wm = wave / WN, wn = wave % WN;
     f32x4_t acc[TI][NJ];
 #pragma unroll
@@ -610,100 +583,92 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     constexpr int WMULT = NJ == 2 ? 2 : 1;
-    const unsigned a_src = piece_slot<1>(wm * (TM / WM) + lr, lg), b_src = 2 * A_PLANE + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
-    auto read_a = [&](f16x8_t (&f)[TI], const char* stage, int plane) {
+    const unsigned a_src = piece_slot<0>(wm * (TM / WM) + lr, lg), b_src = 3 * A_PLANE + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
+    auto read_a = [&](bf16x8_t (&f)[TI], const char* stage, int plane) {
 #pragma unroll
-        for (int i = 0; i < TI; i++) {
-            const unsigned key = ((((wm * (TM / WM) >> 4) + i) ^ ((wm * (TM / WM)) >> 4)) & 3) * 16;  // (rows 16 apart have other chunks: slot())
-            f[i] = *reinterpret_cast<const f16x8_t*>(stage + plane * A_PLANE + (a_src ^ key) + i * 1024);
-        }
+        for (int i = 0; i < TI; i++) f[i] = *reinterpret_cast<const bf16x8_t*>(stage + plane * A_PLANE + a_src + i * 1024);
     };
-    auto read_b = [&](f16x8_t (&f)[NJ], const char* stage, int plane) {
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const unsigned key = ((((wn * (TN / WN) >> 4) + j) ^ ((wn * (TN / WN)) >> 4)) * WMULT & 3) * 16;
-            f[j] = *reinterpret_cast<const f16x8_t*>(stage + plane * B_PLANE + (b_src ^ key) + j * 1024);
-        }
+    auto read_b = [&](const char* stage, int plane, int j) {
+        const unsigned key = ((((wn * (TN / WN) >> 4) + j) ^ ((wn * (TN / WN)) >> 4)) * WMULT & 3) * 16;  // (columns 16 apart have other chunks: piece_slot())
+        return *reinterpret_cast<const bf16x8_t*>(stage + plane * B_PLANE + (b_src ^ key) + j * 1024);
     };
-    auto multiply = [&](const f16x8_t (&a)[TI], const f16x8_t (&b)[NJ]) {
+    auto multiply = [&](const bf16x8_t (&x)[TI], const bf16x8_t& y, f32x4_t (&to)[TI]) {
 #pragma unroll
-        for (int i = 0; i < TI; i++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < TI; i++) to[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i], y, to[i], 0, 0, 0);
     };
-    // an LDS read behind each of the first matrix instructions: issued in one go the matrix unit stands still meanwhile
-    auto spread = [](auto reads, auto products) {
-        constexpr int R = decltype(reads)::value, NM = TI * NJ * decltype(products)::value, EACH = R > NM ? (R + NM - 1) / NM : 1;
+    // an LDS read behind each of the first matrix instructions: issued in one go the matrix unit stands still meanwhile; ADDS vector operations behind each
+    auto spread = [](auto reads, auto products, auto adds) {
+        constexpr int R = decltype(reads)::value, NM = decltype(products)::value, ADDS = decltype(adds)::value;
 #pragma unroll
-        for (int x = 0; x < R; x += EACH) {
+        for (int x = 0; x < NM; x++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, EACH, 0);
+            if (x < R) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (ADDS) __builtin_amdgcn_sched_group_barrier(0x002, ADDS, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, NM, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
+    typedef std::integral_constant<int, 0> None;
     typedef std::integral_constant<int, 1> One;
-    typedef std::integral_constant<int, TI> ReadA;
-    typedef std::integral_constant<int, NJ> ReadB;
-    // Products in the order l*h, h*h, h*l, whatever the tile: a row's result depends on neither the shape nor the grouping.
-    if constexpr (2 * (TI + NJ) * 4 * 2 + TI * NJ * 4 <= REGS) {  // all fragments of the next K tile are read beside the products of this one
-        f16x8_t a[2][2][TI], b[2][2][NJ];
-        auto read = [&](int p, const char* stage) {
+    typedef std::integral_constant<int, 4> Four;
+    typedef std::integral_constant<int, TI> Rows;
+    // Column block by column block: its products over the 32 k values of the tile in the order l*h, m*h, m*m, h*m, h*l, h*h, whatever the tile shape (a row's result depends on
+    // neither the shape nor the grouping), in sums of their own (u), which are added to acc beside the first products of the block after. A register is
+    // loaded for the next block or K tile behind its last use; behind the barrier nothing of the current stage is read any more.
+    bf16x8_t ah[TI], am[TI], al[TI], bh[2], bm, bl;
+    f32x4_t u[2][TI];
+    barrier_behind_lds<0>();
+    bh[0] = read_b(smem, 0, 0);
+    read_a(al, smem, 2);
+    read_a(am, smem, 1);
+    bm = read_b(smem, 1, 0);
+    read_a(ah, smem, 0);
+    bl = read_b(smem, 2, 0);
 #pragma unroll
-            for (int x = 0; x < 2; x++) {
-                read_a(a[p][1 - x], stage, 1 - x);
-                read_b(b[p][x], stage, x);
-            }
-        };
-        barrier_behind_lds<0>();
-        read(0, smem);
-        for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
+    for (int i = 0; i < TI; i++) u[1][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
 #pragma unroll
-            for (int t = 0; t < 2 * GROUP; t++) {
-                const int p = t & 1;
-                if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
-                read(p ^ 1, smem + (t + 1) % (2 * GROUP) * STAGE_BYTES);
-                multiply(a[p][1], b[p][0]);
-                multiply(a[p][0], b[p][0]);
-                multiply(a[p][0], b[p][1]);
-                spread(std::integral_constant<int, 2 * (TI + NJ)>{}, std::integral_constant<int, 3>{});
-            }
-        }
-    } else {  // the fragments of one product beside the one before
-        f16x8_t ah[TI], al[TI], bh[2][NJ], bl[NJ];
-        barrier_behind_lds<0>();
-        read_a(al, smem, 1);
-        read_b(bh[0], smem, 0);
-        for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
+        for (int t = 0; t < 2 * GROUP; t++) {
+            const char *cur = smem + t * STAGE_BYTES, *next = smem + (t + 1) % (2 * GROUP) * STAGE_BYTES;
 #pragma unroll
-            for (int t = 0; t < 2 * GROUP; t++) {
-                const int p = t & 1;
-                const char *cur = smem + t * STAGE_BYTES, *next = smem + (t + 1) % (2 * GROUP) * STAGE_BYTES;
-                read_a(ah, cur, 0);
-                read_b(bl, cur, 1);
-                multiply(al, bh[p]);
-                spread(std::integral_constant<int, TI + NJ>{}, One{});
-                if (t % GROUP == GROUP - 1) barrier_behind_lds<0>();
-                read_a(al, next, 1);
-                multiply(ah, bh[p]);
-                spread(ReadA{}, One{});
-                read_b(bh[p ^ 1], next, 0);
-                multiply(ah, bl);
-                spread(ReadB{}, One{});
+            for (int j = 0; j < NJ; j++) {
+                const int p = (t * NJ + j) & 1;
+                const bool last = j == NJ - 1;
+                const char* const stage = last ? next : cur;
+                const int column = last ? 0 : j + 1;
+                if (last && t % GROUP == GROUP - 1) barrier_behind_lds<0>();
+                bh[p ^ 1] = read_b(stage, 0, column);
+#pragma unroll
+                for (int i = 0; i < TI; i++) u[p][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                multiply(al, bh[p], u[p]);
+#pragma unroll
+                for (int i = 0; i < TI; i++) acc[i][(j + NJ - 1) % NJ] += u[p ^ 1][i];
+                spread(One{}, Rows{}, Four{});
+                if (last) read_a(al, next, 2);
+                multiply(am, bh[p], u[p]);
+                multiply(am, bm, u[p]);
+                if (last) spread(Rows{}, std::integral_constant<int, 2 * TI>{}, None{});
+                else spread(None{}, std::integral_constant<int, 2 * TI>{}, None{});
+                if (last) read_a(am, next, 1);
+                multiply(ah, bm, u[p]);
+                if (last) spread(Rows{}, Rows{}, None{});
+                else spread(None{}, Rows{}, None{});
+                bm = read_b(stage, 1, column);
+                multiply(ah, bl, u[p]);
+                spread(One{}, Rows{}, None{});
+                bl = read_b(stage, 2, column);
+                multiply(ah, bh[p], u[p]);
+                spread(One{}, Rows{}, None{});
+                if (last) read_a(ah, next, 0);
             }
         }
     }
-    const unsigned* const most = reinterpret_cast<const unsigned*>(smem + 2 * GROUP * STAGE_BYTES);
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const int column = scale_exponent(most[TM + wn * (TN / WN) + NJ * lr + j]);
+    for (int i = 0; i < TI; i++) acc[i][NJ - 1] += u[1][i];
 #pragma unroll
-        for (int i = 0; i < TI; i++)
+    for (int i = 0; i < TI; i++)
 #pragma unroll
-            for (int r = 0; r < 4; r++)
-                acc[i][j][r] = __builtin_amdgcn_ldexpf(acc[i][j][r], 254 - column - (int)scale_exponent(most[wm * (TM / WM) + i * 16 + 4 * lg + r]));
-    }
-    // A sum that is not finite (values beyond the range of their pieces, infinities, NaNs) is formed anew from the operands themselves
+        for (int j = 0; j < NJ; j++) acc[i][j] *= 1.0f / (PIECES_SCALE * PIECES_SCALE);
+    // A sum that is not finite (values or sums too large for the pieces, infinities, NaNs) is formed anew from the operands themselves
     const int m0 = m_blk + wm * (TM / WM), n0 = n_blk + wn * (TN / WN);
     auto infinite = [](const f32x4_t& v) {
         bool bad = false;
@@ -749,7 +714,7 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
 template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
 int launch_pieces(TileProbSet& set, int n, hipStream_t st) {
     auto kern = gemm_f32_pieces_kernel<TM, TN, WM, WN, PA, PB, HA, HB, GROUP, SETS, WAVES, EPI>;
-    constexpr int smem = 2 * GROUP * 2 * (TM + TN) * 64 + (TM + TN) * 4;
+    constexpr int smem = 2 * GROUP * 3 * (TM + TN) * 64;
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
     int total = 0;
@@ -763,10 +728,10 @@ int launch_pieces(TileProbSet& set, int n, hipStream_t st) {
 template <int EPI>
 int launch_pieces_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
     switch (shape) {
-        case 0: return launch_pieces<128, 128, 2, 2, 4, 4, 8, 8, 1, 4, 3, EPI>(set, n, st);
+        case 0: return launch_pieces<128, 128, 2, 4, 4, 4, 8, 8, 1, 2, 4, EPI>(set, n, st);
+        case 1: return launch_pieces<128, 64, 4, 2, 4, 4, 8, 4, 2, 4, 4, EPI>(set, n, st);
         // (columns of W by runs of four: a thread's eight loads, one per k value, were what it spent most time on. 128x64 at 512 rows, K = 1536 31 -> 29 us,
         // 64x64 22.3 -> 20.7, 32x64 17.7 -> 15.4)
-        case 1: return launch_pieces<128, 64, 2, 2, 4, 8, 8, 4, 2, 4, 4, EPI>(set, n, st);
         case 2: return launch_pieces<64, 64, 2, 2, 4, 8, 8, 4, 2, 4, 4, EPI>(set, n, st);
         case 3: return launch_pieces<32, 64, 2, 2, 4, 8, 4, 4, 2, 4, 4, EPI>(set, n, st);
         case 4: return launch_pieces<32, 32, 2, 2, 4, 4, 4, 4, 2, 4, 3, EPI>(set, n, st);

@@ -41,10 +41,11 @@ inline int pick_f32_tile(const F32Layer* layers, int n, int cus, bool whole_k) {
     return best;
 }
 
-// ---- products of f16 pieces (gemm_f32_pieces_kernel) ----
+// ---- products of bf16 pieces (gemm_f32_pieces_kernel) ----
 // Which launches: depths of 256 and more, in whole groups of the four K tiles that its loops take at a time. Shallower products are over before the split of the
-// operands is under way. us, fp32 instruction | pieces, a call each: K = 256: 1178 x 3072 21.8 | 15.9, 2356 x 768 12.6 | 11.2, 8192 x 768 29.6 | 20.1; smaller ones are
-// lost in the 11 us that a call costs (forward of 1178 tokens, width 256: 324 us with K = 256 on the fp32 instruction, 319 without). By the depth alone: the two kernels
+// operands is under way. us, fp32 instruction | pieces: K = 256: 8192 x 1536 57 | 49, 1178 x 4608 30.4 | 27.7, 2356 x 768 13.1 | 12.2, what is smaller is lost in the 11 us that a
+// call costs; over 1 to 8192 rows, 256 to 6144 columns the mean is 0.96 of the fp32 instruction's time at K = 256, 0.93 at 512, 0.90 from 768 on. One round of small
+// tiles is up to a tenth slower (154 x 1536 x 1536 12.1 | 13.0, 666 x 1536 x 1536 28.7 | 31.2), from 1178 rows and 768 columns on it is 0.6 to 0.9. By the depth alone: the two kernels
 // round differently, and a row's result is to be the same in every batch.
 inline bool f32_by_pieces(const F32Layer* layers, int n) {
     for (int i = 0; i < n; i++)
@@ -52,7 +53,7 @@ inline bool f32_by_pieces(const F32Layer* layers, int n) {
     return true;
 }
 
-// The shapes (the first five as above) and their times in us, measured over M = 1 .. 8192, N = 768 .. 6144 and K = 512 .. 6144 (to 3 to 9 %): a launch's last round apart from its K tiles, each
+// The shapes (the first five as above) and their times in us, measured over M = 1 .. 8192, N = 768 .. 6144 and K = 256 .. 6144 (to 2 to 9 %): a launch's last round apart from its K tiles, each
 // round before it likewise, a K tile of a lone workgroup, and by how much longer that takes with every compute unit at work (the power limit; it grows with
 // the square of the share that is).
 struct F32PieceTile {
@@ -60,8 +61,8 @@ struct F32PieceTile {
     double last, before, step, crowd;
 };
 constexpr int F32_PIECE_TILES = 6;
-constexpr F32PieceTile f32_piece_tiles[F32_PIECE_TILES] = {{128, 128, 8.6, 6.9, 0.574, 0.38}, {128, 64, 6.6, 6.0, 0.298, 0.45}, {64, 64, 6.2, 2.0, 0.189, 0.42},
-                                                           {32, 64, 6.4, 0.8, 0.128, 0.37},    {32, 32, 6.1, 0.5, 0.095, 0.17},  {256, 128, 9.0, 5.2, 0.974, 0.52}};
+constexpr F32PieceTile f32_piece_tiles[F32_PIECE_TILES] = {{128, 128, 6.7, 5.2, 0.954, 0.32}, {128, 64, 6.1, 3.8, 0.538, 0.32}, {64, 64, 6.3, 2.9, 0.309, 0.32},
+                                                           {32, 64, 6.5, 0.7, 0.227, 0.11},    {32, 32, 6.5, 0.5, 0.154, 0.04},  {256, 128, 8.6, 5.7, 1.860, 0.35}};
 inline int pick_f32_piece_tile(const F32Layer* layers, int n, int cus) {
     int best = 0;
     double best_cost = 0;

@@ -1,4 +1,4 @@
-"""fp32 products of f16 pieces at the edges of their tiles, beyond the range of the pieces and in blocks, against float64 arithmetic and the fp32 instruction."""
+"""fp32 products of bf16 pieces at the edges of their tiles, beyond the range of the pieces and in blocks, against float64 arithmetic and the fp32 instruction."""
 import pytest
 import torch
 
@@ -19,9 +19,9 @@ def _automatic_choice_afterwards():
 
 @pytest.mark.parametrize("m,k,n", [(1, 512, 4), (31, 256, 36), (33, 384, 68), (65, 768, 64), (129, 512, 132), (257, 640, 260), (300, 1536, 1540)])
 def test_every_tile_shape(m, k, n):
-    """Rows and columns on and beside the multiples of the tiles (32 to 256), depths from the smallest on. Bound: a product of pieces lacks less than 3 u of itself
-    (u of either value, u for l*l), and of its additions three per 32 values round: less than a sum of k products in any order, (k + 2) u (|x| |W| + |b|). The
-    shapes agree bit for bit."""
+    """Rows and columns on and beside the multiples of the tiles (32 to 256), depths from the smallest on. Bound: a product of pieces lacks at most
+    u of itself (m*l, l*m: 2^-25 each), and the additions of 32 products and of their sum to the sum of those before round less often than a sum of k products in any
+    order does, (k + 2) u (|x| |W| + |b|). The shapes agree bit for bit."""
     g = torch.Generator(device="cuda").manual_seed(m * 31 + k)
     x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, n), (n,)))
     want = x.double() @ W.double() + b.double()
@@ -35,9 +35,10 @@ def test_every_tile_shape(m, k, n):
         assert torch.equal(y, first), shape
 
 
-@pytest.mark.parametrize("scale_x,scale_w", [(1e-18, 1e-12), (1e15, 1e18), (1e-30, 1e28)])
+@pytest.mark.parametrize("scale_x,scale_w", [(1e-18, 1e-12), (1e15, 1e18), (1e-30, 1e28), (1e-36, 1e34), (1e-41, 1e37), (1e37, 1e-41), (1e-20, 1e-20)])
 def test_small_and_large_values(scale_x, scale_w):
-    """Powers of two bring the values into the range of the pieces: the error is that of the tile kernel at any scale (twice it, as two sums of one product may differ)."""
+    """The error is that of the tile kernel at any scale, values below 2^-110 (whose pieces would be below the bf16 range) and subnormal ones, sums of 2^96 and more (formed anew) and
+    subnormal results included (twice it, as two sums of one product may differ)."""
     g = torch.Generator(device="cuda").manual_seed(7)
     x, W, b = scale_x * torch.randn((200, 512), device="cuda", generator=g), scale_w * torch.randn((512, 192), device="cuda", generator=g), torch.zeros(192, device="cuda")
     want = x.double() @ W.double()
@@ -49,8 +50,8 @@ def test_small_and_large_values(scale_x, scale_w):
 
 
 @pytest.mark.parametrize("shape", [0, 1, 2, 3, 4, 5])
-def test_infinities_nans_and_values_beyond_bf16(shape):
-    """What has no pieces (infinities, NaNs, values much larger than the first of their row, in x and in W) gives what the fp32 instruction gives, and changes nothing else."""
+def test_infinities_nans_and_values_beyond_the_pieces(shape):
+    """What has no pieces (infinities, NaNs, values of 2^112 and more, in x and in W) gives what the fp32 instruction gives, and changes nothing else."""
     g = torch.Generator(device="cuda").manual_seed(shape)
     m, k, n = 150, 512, 140
     x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, n), (n,)))
@@ -77,8 +78,8 @@ def test_infinities_nans_and_values_beyond_bf16(shape):
 
 @pytest.mark.parametrize("shape", [0, 1, 2, 3, 4, 5])
 def test_rows_and_columns_of_any_scale(shape):
-    """Rows of x and columns of W from 2^-40 to 2^40, a row whose first 64 and one whose first 200 values are zero, one of zeros, one that grows by 2^20 and a column that does (formed anew
-    by the fp32 instruction), one that starts 2^9 above the rest and one that grows by 2^10. Bound as above: relative to |x| |W| of the element itself."""
+    """Rows of x and columns of W from 2^-40 to 2^40, a row whose first 64 and one whose first 200 values are zero, one of zeros, one that grows by 2^20 and a column that does,
+    one that starts 2^9 above the rest and one that grows by 2^10. Bound as above: relative to |x| |W| of the element itself."""
     g = torch.Generator(device="cuda").manual_seed(shape + 50)
     m, k, n = 150, 512, 140
     x, W, b = torch.randn((m, k), device="cuda", generator=g), torch.randn((k, n), device="cuda", generator=g), torch.zeros(n, device="cuda")
@@ -94,6 +95,88 @@ def test_rows_and_columns_of_any_scale(shape):
     y = M.linear(x, W, b)
     bound = (k + 2) * U * (x.double().abs() @ W.double().abs())
     assert ((y.double() - x.double() @ W.double()).abs() <= bound).all()
+
+
+def spread(kind, e, m, k, n):
+    """Operands whose values differ by powers of two of up to e within a row of x, a column of W or both, so that a result can consist of the small ones."""
+    g = torch.Generator(device="cuda").manual_seed(k + e)
+    x, W = torch.randn((m, k), device="cuda", generator=g), torch.randn((k, n), device="cuda", generator=g)
+    channel = 0 if kind.endswith("first") else k // 2 + 3
+    if kind.startswith("a large channel of x that W leaves out"):
+        x[:, channel] *= 2.0 ** e
+        W[channel] = 0
+    elif kind.startswith("a large channel of W that x leaves out"):
+        W[channel] *= 2.0 ** e
+        x[:, channel] = 0
+    elif kind.startswith("a channel in another unit"):
+        x[:, channel] *= 2.0 ** e
+        W[channel] *= 2.0 ** -e
+    else:  # every channel in a unit of its own
+        d = torch.exp2((torch.rand(k, device="cuda", generator=g) * 2 - 1) * e).clamp_(2.0 ** -60, 2.0 ** 60)
+        x *= d
+        W /= d[:, None]
+    return x, W
+
+
+@pytest.mark.parametrize("e", [-40, 7, 12, 16, 20, 27, 60])
+@pytest.mark.parametrize("kind", ["a large channel of x that W leaves out, the first", "a large channel of x that W leaves out", "a large channel of W that x leaves out, the first",
+                                  "a large channel of W that x leaves out", "a channel in another unit, the first", "a channel in another unit", "every channel in a unit of its own"])
+@pytest.mark.parametrize("k", [512, 1536])
+def test_channels_of_any_magnitude(kind, e, k):
+    """Values far below the largest of their row or column count in full: element by element the bound of a sum of k products (as above), and in all no more error than
+    the fp32 instruction's (1.25 times it, as the errors of two sums of the same products may differ by chance)."""
+    x, W = spread(kind, e, 150, k, 140)
+    b = torch.zeros(140, device="cuda")
+    want, bound = x.double() @ W.double(), (k + 2) * U * (x.double().abs() @ W.double().abs())
+    err = []
+    for choice in (1, 0):
+        L.call("sd3_tune", b"gemm_f32_no_pieces", choice)
+        diff = (M.linear(x, W, b).double() - want).abs()
+        err.append(float(diff.norm()))
+    assert (diff <= bound).all()
+    assert err[1] <= 1.25 * err[0]
+
+
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 4, 5])
+def test_single_products(shape):
+    """Rows of x with one value that is not zero: every result is one product, which lacks at most 2^-24 of itself for the products of pieces that are not formed and is added
+    to what is small beside it within a unit in the last place (2 u) whichever way that rounds: 3 u and 2^-8 of it for the sums of the smaller ones. Powers of two of
+    2^-60 to 2^60, and values of 1 + 2^-11 and 1 + 2^-12 + 2^-23, whose low bits all count."""
+    m, k, n = 256, 256, 140
+    g = torch.Generator(device="cuda").manual_seed(shape + 3)
+    value = torch.randn(m, device="cuda", generator=g) * torch.exp2(torch.randint(-60, 61, (m,), device="cuda", generator=g).float())
+    value[:3] = 1 + 2.0 ** -11
+    value[3:6] = 1 + 2.0 ** -12 + 2.0 ** -23
+    W = torch.randn((k, n), device="cuda", generator=g) * torch.exp2(torch.randint(-20, 21, (k, 1), device="cuda", generator=g).float())
+    W[:, :3] = 1 + 2.0 ** -11
+    W[:, 3:6] = 1 + 2.0 ** -12 + 2.0 ** -23
+    x = torch.zeros((m, k), device="cuda")
+    x[torch.arange(m), torch.randperm(k, generator=torch.Generator().manual_seed(1)).cuda()] = value
+    L.call("sd3_tune", b"gemm_f32_tile", shape)
+    want = x.double() @ W.double()
+    assert ((M.linear(x, W, torch.zeros(n, device="cuda")).double() - want).abs() <= 3.02 * U * want.abs()).all()
+
+
+@pytest.mark.parametrize("x_of,w_of", [("normal", "normal"), ("positive", "positive"), ("1 + 2^-11", "1 + 2^-11"), ("positive", "1 + 2^-12 + 2^-23"), ("gelu", "normal"), ("one in 16", "normal")])
+@pytest.mark.parametrize("k", [256, 1536, 6144])
+def test_error_is_no_larger_than_the_fp32_instructions(x_of, w_of, k):
+    """Sums whose terms cancel, whose terms all have one sign (where rounding to one side would add up), constants, and few terms. 1.25: two sums of the same
+    products may differ by chance; u: results that one of the two happens to hold exactly."""
+    g = torch.Generator(device="cuda").manual_seed(k)
+
+    def make(kind, *shape):
+        t = torch.randn(shape, device="cuda", generator=g)
+        return {"normal": t, "positive": t.abs(), "1 + 2^-11": torch.full_like(t, 1 + 2.0 ** -11), "1 + 2^-12 + 2^-23": torch.full_like(t, 1 + 2.0 ** -12 + 2.0 ** -23),
+                "gelu": torch.nn.functional.gelu(t, approximate="tanh"), "one in 16": t * (torch.rand(shape, device="cuda", generator=g) < 1 / 16)}[kind]
+
+    x, W, b = make(x_of, 300, k), make(w_of, k, 260), torch.zeros(260, device="cuda")
+    want = x.double() @ W.double()
+    err = []
+    for choice in (1, 0):
+        L.call("sd3_tune", b"gemm_f32_no_pieces", choice)
+        err.append(float((M.linear(x, W, b).double() - want).norm() / want.norm()))
+    print(f"fp32 instruction {err[0]:.2e}, pieces {err[1]:.2e}")
+    assert err[1] <= 1.25 * err[0] + U
 
 
 @pytest.mark.parametrize("Tc,Tx,dual", [(77, 1000, True), (5, 2049, False)])
