@@ -3,9 +3,9 @@
 // concatenation / split around it (modules.cpp:1427-1432): keys/values/queries of the joint sequence are read
 // straight from the context buffers (first T[0] tokens) and the latent buffers (next T[1] tokens).
 //
-// Three kernels: attn_f32_pieces_kernel (operands as two f16 pieces each, on the f16 matrix instruction) and attn_f32_split_kernel (fp32 matrix instruction, for
-// few queries and heads) for head_dim 64 and 128 with 16-byte aligned rows, attn_f32_kernel for any other head_dim up to 128. Formulation of all: everything is
-// kept transposed so that the probabilities never leave registers.
+// Three kernels: attn_f32_split_kernel (fp32 matrix instruction) for head_dim 64 and 128 with 16-byte aligned rows, attn_f32_pieces_kernel (values as three bf16
+// pieces each, on the bf16 matrix instruction) for head_dim 64 where there are many queries and heads, attn_f32_kernel for any other head_dim up to 128. Formulation of
+// all: everything is kept transposed so that the probabilities never leave registers.
 //   S^T (keys x queries) = K . Q^T      -> C-layout: a lane owns ONE query column and 16 keys per 32-key block
 //   O^T (d x queries)   += V^T . P^T    -> the lane's own S^T registers are exactly the P^T operand it must supply
 // Online softmax statistics are per query = per lane (plus one exchange with lane^32).
@@ -181,22 +181,14 @@ __device__ __forceinline__ float max_of_groups(float x) {
     const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
     return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
 }
-// The largest of the wavefront's values, in all lanes
-__device__ __forceinline__ float max_of_lanes(float x) {
-    x = fmaxf(x, dpp_move<0x128>(x));  // rotations of 16 lanes by 8, 4, 2 and 1
-    x = fmaxf(x, dpp_move<0x124>(x));
-    x = fmaxf(x, dpp_move<0x122>(x));
-    x = fmaxf(x, dpp_move<0x121>(x));
-    return max_of_groups(x);
-}
 
-// ---- head_dim 64 and 128, few queries ----
+// ---- head_dim 64 and 128 ----
 // The matrix unit (v_mfma_f32_16x16x4_f32: 64 FLOP per cycle and SIMD) is the bound, and everything it needs fits the registers of one
 // wavefront: 16*QB queries and 16*KB keys at a time. So no LDS tiles and no barriers: the KS wavefronts of a workgroup share its queries
 // and split the KEYS (tile t goes to wavefront t % KS); K and V rows come straight from memory (L2: all workgroups of a head run on one
 // XCD) into registers, half a tile of matrix work ahead of their use; the KS partial results are merged in a fixed tree at the end.
 // This gives every SIMD work also where there are few queries: 1178 tokens and 2 heads are 20 workgroups of 128 queries with the keys in
-// one run (290 us), 592 wavefronts this way (28 us). 2 x 24 heads of 64, 1178 tokens: 244 -> 148 us, 70 -> 115 TFLOP/s of 155 (the matrix
+// one run (290 us), 592 wavefronts this way (28 us). 2 x 24 heads of 64, 1178 tokens (which go by pieces now): 244 -> 148 us, 70 -> 115 TFLOP/s of 155 (the matrix
 // instructions alone about 127, the softmax 12, the loads 9).
 //
 // Contraction order: K and Q are read as float4 along d, so step s of 16-wide chunk c contracts d = 16c + 4g + s over the lane groups
@@ -451,25 +443,33 @@ int launch_split(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
     return launch_status("attention_f32");
 }
 
-// ---- head_dim 64 and 128 by f16 pieces ----
-// Products as in gemm_f32_pieces_kernel: values times powers of two as two f16 pieces each, three products of pieces on the f16 matrix instruction, fp32 sums. Powers of
-// two: a query's own; one for the K and one for the V of a (batch, head), from three of its tiles of 32 keys, with room for values 2^9 times as large; 2^6 for
-// the probabilities. Results that are not finite (values beyond that, infinities, NaNs) are formed anew on the fp32 instruction (attend_in_f32). Scores, probabilities, their
-// sums and the outputs are fp32 throughout. Relative error against 64 bits, normal inputs (fp32 instruction): 24 heads of 64, 1178 keys 2.9e-7 (4.2e-7), 4250
-// keys 3.9e-7 (6.6e-7), 64 keys 2.0e-7 (2.5e-7); 12 heads of 128, 1178 keys 4.0e-7 (5.2e-7).
+// ---- head_dim 64 by bf16 pieces ----
+// Products as in gemm_f32_pieces_kernel: an fp32 value is the sum of three bf16 values without a remainder (bf16_pieces), six of the nine products of pieces are formed. No
+// value is lost beside a larger one of its head, channel or token. Probabilities are split as they are, so those below 2^-110 keep the bits down to 2^-133. Scores, probabilities,
+// their sums and the outputs are fp32 throughout. Two sums per score, of the products of first pieces and of the others, because the matrix instruction does not round to nearest;
+// the products of a key tile are summed by themselves before they join the outputs, one rounding per tile. Relative error against 64 bits, 24 heads of 64 (fp32
+// instruction): 32 keys 1.1e-7 (2.3e-7), 77 1.3e-7 (2.7e-7), 1178 1.8e-7 (4.3e-7), 4250 2.4e-7 (6.6e-7); equal weights, 77 keys 7.7e-8 (1.1e-7), constant values 7.0e-8
+// (7.9e-8). (Two f16 pieces per value and three products took 68 us for 2 x 1178 tokens, 24 heads, but hold 22 of the 24 bits, and only of values within 2^-7 of the
+// largest of the head: with one channel of V 2^16 times the others these came out with an error of 4e-5, beside a key that takes 1 - 2^-20 of the weight 7e-5. One sum per
+// score 104 us instead of 108, and up to 1.25 times the fp32 instruction's error where a score is one large product.)
+// Results that are not finite (infinities, NaNs, values from 2^112 and sums from 2^96 on) are formed anew on the fp32 instruction (attend_in_f32), 32 queries at a time: 2 x 1178
+// tokens, 24 heads, 108 us, with one such query 200, with one such head 260, with 24 of the 48 380. (A score of -2^96 and below counts as minus infinity: its rounding error in
+// fp32 is 2^72.)
 //
-// A wavefront has 32 queries; QG of them share the K and V tiles, which each splits a share of, into LDS. Per tile of 32 keys a wavefront of head_dim 64 issues 24 matrix instructions
-// (768 cycles) and 220 vector operations (about 700), and the two hardly overlap however they are interleaved: the vector unit gets few slots beside matrix
-// instructions, which is also why these are the ones of 32 cycles and not of 16. So it is vector operations that count: two pieces instead of three bf16 ones
-// (350 -> 250 operations, mha of 2 x 1178 tokens, 24 heads 105 -> 81 us), a reference that moves only past a margin, offsets that stay from tile to tile (81 -> 67).
-// The keys are two runs, even and odd tiles, with a reference and sums of their own, merged at the end: half the additions to one sum (error 3.4e-7 -> 2.9e-7),
-// and few queries get twice the wavefronts. KR = 2: side by side; SEQ = 2: one after the other, with the same bits.
-// us, fp32 instruction -> pieces: 2 x 1178 tokens, 24 heads of 64 148 -> 71 (240 TFLOP/s), 4250 tokens 902 -> 400 (277), 16 x 666 tokens, 12 heads of 64 195 -> 102, 4 x 1024
-// queries of 154 keys, 24 heads 57 -> 32, 8 x 1178 tokens, 12 heads of 128 551 -> 251.
-// What f16 pieces cannot give (values beyond their range, infinities, NaNs): the lane's query `qt`, all lanes 32 of them, over all keys on the fp32
+// A wavefront has 32 queries; QG of them share the K and V tiles, which each splits a share of, into LDS. Per tile of 32 keys a wavefront issues 48 matrix instructions
+// (1536 cycles) and 370 vector operations (about 1400), and the two hardly overlap however they are interleaved: the vector unit gets few slots beside matrix
+// instructions, which is also why these are the ones of 32 cycles and not of 16. So vector operations count: a reference that moves only past a margin, offsets that stay from
+// tile to tile.
+// The keys are two runs, even and odd tiles, with a reference and sums of their own, merged at the end: half the additions to one sum, and few queries get twice the
+// wavefronts. KR = 2: side by side; SEQ = 2: one after the other, with the same bits.
+// us, fp32 instruction -> pieces, 24 heads: 2 x 1178 tokens 145 -> 108 (158 TFLOP/s, 950 of products of pieces), 4250 tokens 901 -> 695, 8 x 512 tokens 114 -> 81, 3 x 860
+// 121 -> 85, one element of 1178 85 -> 57.
+// head_dim 128 has no registers for the pieces of its queries beside a second wavefront: with one per SIMD 12 heads, 1178 tokens 84 -> 83, two of these 159 -> 121, but 3 x 1000
+// tokens 173 -> 206, 666 tokens 30 -> 52. It stays on the fp32 instruction.
+// What the pieces cannot give (values beyond their range, infinities, NaNs): the lane's query `qt`, all lanes 32 of them, over all keys on the fp32
 // matrix instruction; out (null: not stored): the query's result from d = 4(l/32) on. For the rare case, so as plain as can be.
-template <int HS>
 __device__ void attend_in_f32(const SegDev& s, int b, int h, int qt, float scale, float* out) {
+    constexpr int HS = 64;
     const int l32 = threadIdx.x & 31, lk = threadIdx.x >> 5 & 1;
     const int qseg = qt < s.Tq[0] ? 0 : 1;
     const float* q = s.q[qseg] + ((long long)b * s.Tq[qseg] + (qseg ? qt - s.Tq[0] : qt)) * s.ld_qkv[qseg] + h * HS + lk;
@@ -517,35 +517,35 @@ __device__ void attend_in_f32(const SegDev& s, int b, int h, int qt, float scale
             for (int r = 0; r < 16; r++) out[32 * j + 8 * (r >> 2) + (r & 3)] = o[j][r] * inv;
 }
 
-// The split of eight values into pieces (f16_pieces) in steps, to be spread over matrix instructions
+// The split of eight values into pieces (bf16_pieces) in steps, to be spread over matrix instructions
 struct Split {
+    static constexpr int STEPS = 5;
     float x[8];
-    uint32_t piece[2][4];
+    uint32_t piece[3][4];
     __device__ __forceinline__ void step(int n) {
-        if (n == 0) f16_high<8>(x, piece[0]);
-        else if (n == 1) f16_rest<8>(x, piece[0]);
-        else f16_high<8>(x, piece[1]);
+        if (n % 2 == 0) bf16_high<8>(x, piece[n / 2]);
+        else bf16_rest<8, false>(x, piece[n / 2]);
     }
 };
 
-template <int HS, int QG, int KR, int SEQ>
+template <int QG, int KR, int SEQ>
 struct PiecesShape {
-    static constexpr int QWG = 32 * QG, THREADS = QG * KR * 64;
+    static constexpr int HS = 64, QWG = 32 * QG, THREADS = QG * KR * 64;
     static constexpr int K_PLANE = 32 * 64, V_PLANE = HS * 64;  // bytes: 32 k values of 32 keys; 32 keys of HS values
-    static constexpr int K_BYTES = HS / 32 * 2 * K_PLANE, V_BYTES = 2 * V_PLANE, RUN_BYTES = K_BYTES + 2 * V_BYTES;
+    static constexpr int K_BYTES = HS / 32 * 3 * K_PLANE, V_BYTES = 3 * V_PLANE, RUN_BYTES = K_BYTES + 2 * V_BYTES;
     static constexpr int PITCH = HS / 2 + 4;                    // floats per lane of a run's result
     static constexpr int MERGE_BYTES = KR / 2 * QG * 64 * PITCH * 4, KEPT_BYTES = SEQ > 1 ? QG * 64 * PITCH * 4 : 0;
-    static constexpr int LDS = (KR * RUN_BYTES > MERGE_BYTES ? KR * RUN_BYTES : MERGE_BYTES) + KEPT_BYTES + 8;
+    static constexpr int LDS = (KR * RUN_BYTES > MERGE_BYTES ? KR * RUN_BYTES : MERGE_BYTES) + KEPT_BYTES;
 };
 
 // Where 16 bytes (8 k values) of a 64-byte row lie: neither the reads (32 rows, 16 of them at a time: 0-3, 12-15, 20-27 and the others) nor the writes
 // (8 consecutive lanes) meet in a bank
 __device__ __forceinline__ unsigned row_slot(unsigned row, unsigned chunk) { return row * 64 + ((chunk ^ (row >> 2)) & 3) * 16; }
 
-template <int HS, int QG, int KR, int SEQ>
-__global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces_kernel(SegDev s, int NH, int n_q, int total, float scale) {
-    typedef PiecesShape<HS, QG, KR, SEQ> S;
-    constexpr int NC = HS / 16, ND = HS / 32, PT = QG * 64, CK = 4 * HS / PT, TKEYS = 32, RUNS = KR * SEQ;
+template <int QG, int KR, int SEQ>
+__global__ void __launch_bounds__(QG* KR * 64, SEQ * QG * KR / 4) attn_f32_pieces_kernel(SegDev s, int NH, int n_q, int total, float scale) {
+    typedef PiecesShape<QG, KR, SEQ> S;
+    constexpr int HS = S::HS, NC = HS / 16, ND = HS / 32, PT = QG * 64, CK = 4 * HS / PT, TKEYS = 32, RUNS = KR * SEQ;
     static_assert(SEQ == 1 || (KR == 1 && SEQ == 2), "runs side by side or two one after the other");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int lane = threadIdx.x & 63, l32 = lane & 31, lk = lane >> 5;
@@ -557,13 +557,12 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     const int bh = item / n_q, h = bh % NH, b = bh / NH, qt = (item % n_q) * S::QWG + group * 32 + l32;
     const int T0 = s.T[0], T1 = s.T[1], Tq0 = s.Tq[0], TQ = s.Tq[0] + s.Tq[1];
 
-    constexpr bool REST = HS == 64;
-    f32x16_t o[ND], o_rest[REST ? ND : 1];  // the products of first pieces, and the others where there are registers for them: so o is rounded once per k step and not three times
+    f32x16_t o[ND];
     float m_run = -1e30f, l_run = 0.f;  // l_run: over the keys of this lane
 #pragma unroll
     for (int j = 0; j < ND; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[j][r] = o_rest[REST ? j : 0][r] = 0.f;
+        for (int r = 0; r < 16; r++) o[j][r] = 0.f;
 
     const int nt0 = (T0 + TKEYS - 1) / TKEYS, n_t = nt0 + (T1 + TKEYS - 1) / TKEYS, first = (n_t + RUNS - 1) / RUNS;
     const int ld0 = s.ld_qkv[0], ld1 = s.ld_qkv[1];
@@ -635,54 +634,34 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
             for (int x = 0; x < 4; x++) vr[i][x] = *reinterpret_cast<const f32x2_t*>(v_base + v_off[i][x]);
     };
     // (all requests before the first wait)
-    struct Share {
-        f32x4_t k[CK][2];
-        f32x2_t v[CK][4];
-    } middle, second;
-    auto sample = [&](int t, Share& to) {
-        find_k(t);
-        find_v(t);
-        load_k();
-        load_v();
-        __builtin_memcpy(to.k, kr, sizeof(kr));
-        __builtin_memcpy(to.v, vr, sizeof(vr));
-    };
-    Share now;
-    sample(n_t / 2, middle);
-    if (SEQ > 1) sample(1, second);
-    sample(SEQ > 1 ? 0 : run, now);
-    // pieces of the lane's query: of step c the 8 values d = 32(c/2) + 8(c%2) + 4(l/32) .. +3 and 16 behind them, times a power of two of its own
-    f16x8_t q[2][NC];
-    int q_exponent;
+    const int first_tile = SEQ > 1 ? 0 : run;
+    find_k(first_tile);
+    find_v(first_tile);
+    load_k();
+    load_v();
+    // pieces of the lane's query: of step c the 8 values d = 32(c/2) + 8(c%2) + 4(l/32) .. +3 and 16 behind them
+    bf16x8_t q[3][NC];
     {
         const int t = min(qt, TQ - 1), seg = t < Tq0 ? 0 : 1;  // (queries past the end repeat the last one and are not stored)
         const float* p = s.q[seg] + ((long long)b * s.Tq[seg] + (seg ? t - Tq0 : t)) * s.ld_qkv[seg] + h * HS + 4 * lk;
-        float x[NC][8], most = 0.f;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8), hi = *reinterpret_cast<const f32x4_t*>(p + c / 2 * 32 + c % 2 * 8 + 16);
+            float x[8];
 #pragma unroll
-            for (int k = 0; k < 8; k++) {
-                x[c][k] = (k < 4 ? lo[k & 3] : hi[k & 3]) * scale;
-                most = larger(most, x[c][k]);
-            }
-        }
-        most = fmaxf(most, __shfl_xor(most, 32, 64));
-        q_exponent = scale_exponent<14>(__float_as_uint(most));
+            for (int k = 0; k < 8; k++) x[k] = (k < 4 ? lo[k & 3] : hi[k & 3]) * scale;
+            uint32_t piece[3][4];
+            bf16_pieces<8>(x, piece[0], piece[1], piece[2]);
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-            uint32_t piece[2][4];
-            f16_pieces<8>(x[c], power_of_exponent(q_exponent), piece[0], piece[1]);
-#pragma unroll
-            for (int w = 0; w < 2; w++) __builtin_memcpy(&q[w][c], piece[w], 16);
+            for (int w = 0; w < 3; w++) __builtin_memcpy(&q[w][c], piece[w], 16);
         }
     }
     Split part;
     auto put_k = [&](int i) {
         const unsigned u = i * PT + tid, key = u / 4 % 32, c = u / 128;
-        char* at = k_lds + c * 2 * S::K_PLANE + row_slot(key, u % 4);
+        char* at = k_lds + c * 3 * S::K_PLANE + row_slot(key, u % 4);
 #pragma unroll
-        for (int p = 0; p < 2; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * S::K_PLANE, 16), part.piece[p], 16);
+        for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * S::K_PLANE, 16), part.piece[p], 16);
     };
     auto put_v = [&](int i, int buffer) {
         // of 16 keys, 4(l/32) .. +3 of either half are the k values 8(l/32) .. +7 of the matrix instruction, as the scores have them
@@ -691,76 +670,95 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
         for (int y = 0; y < 2; y++) {
             char* at = v_lds + buffer * S::V_BYTES + row_slot(d + y, chunk) + half * 8;
 #pragma unroll
-            for (int p = 0; p < 2; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * S::V_PLANE, 8), &part.piece[p][2 * y], 8);
+            for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * S::V_PLANE, 8), &part.piece[p][2 * y], 8);
         }
     };
     // fragments: row l%32, chunk l/32 of one of the two k steps of a 64-byte row
     const unsigned src = row_slot(l32, lk);
-    auto k_frag = [&](int c, int p) { return *reinterpret_cast<const f16x8_t*>(k_lds + (c / 2 * 2 + p) * S::K_PLANE + (src ^ c % 2 * 32)); };
+    auto k_frag = [&](int c, int p) { return *reinterpret_cast<const bf16x8_t*>(k_lds + (c / 2 * 3 + p) * S::K_PLANE + (src ^ c % 2 * 32)); };
     auto v_frag = [&](int buffer, int n, int p) {  // n: d block n / 2, k step n % 2
-        return *reinterpret_cast<const f16x8_t*>(v_lds + buffer * S::V_BYTES + p * S::V_PLANE + n / 2 * 2048 + (src ^ n % 2 * 32));
+        return *reinterpret_cast<const bf16x8_t*>(v_lds + buffer * S::V_BYTES + p * S::V_PLANE + n / 2 * 2048 + (src ^ n % 2 * 32));
     };
-    // The products of pieces of a k step in the order l*h, h*l, h*h; `beside(n)`, n = 0 .. COUNT - 1, is what the vector unit does meanwhile, spread over
-    // the k steps.
-    auto spread = [](bool reads) {
+    // The products of pieces of a k step in the order l*h, m*m, h*l, m*h, h*m, h*h. `beside(n)`, n = 0 .. COUNT - 1, is what the vector unit does meanwhile, spread
+    // over the k steps.
+    auto spread = [](int products, int reads) {
 #pragma unroll
-        for (int x = 0; x < 3; x++) {
+        for (int x = 0; x < products; x++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (reads && x < 2) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            if (x < reads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x402, 8, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    auto mfma = [](const bf16x8_t& a, const bf16x8_t& b, const f32x16_t& c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); };
+    auto five = [&](const bf16x8_t (&a)[3], const bf16x8_t& h, const bf16x8_t& m, const bf16x8_t& l, f32x16_t& x) {
+        x = mfma(a[2], h, x);
+        x = mfma(a[1], m, x);
+        x = mfma(a[0], l, x);
+        x = mfma(a[1], h, x);
+        x = mfma(a[0], m, x);
+    };
     f32x16_t sc, sn;
-    f16x8_t frag[2][2], p[2][2];
-    float unit;                        // of the scores as they leave the matrix unit
-    constexpr int P_EXPONENT = 6, MARGIN = 8;  // probabilities are kept times 2^6, those of scores up to 2^8 above the reference included
+    bf16x8_t p[3][2];
+    constexpr float UNIT = 1.f / (PIECES_SCALE * PIECES_SCALE);  // of the scores as they leave the matrix unit
+    constexpr int MARGIN = 8;
     auto scores = [&](f32x16_t& x, auto count, auto beside) {
         constexpr int COUNT = decltype(count)::value;
-        frag[0][1] = k_frag(0, 1);
-        frag[0][0] = k_frag(0, 0);
+        bf16x8_t frag[2][3];
 #pragma unroll
-        for (int r = 0; r < 16; r++) x[r] = 0.f;
+        for (int w = 2; w >= 0; w--) frag[0][w] = k_frag(0, w);
+        f32x16_t large;
+#pragma unroll
+        for (int r = 0; r < 16; r++) x[r] = large[r] = 0.f;
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int now = c & 1;
-            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][1], q[0][c], x, 0, 0, 0);
-            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], q[1][c], x, 0, 0, 0);
-            x = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], q[0][c], x, 0, 0, 0);
+            five(frag[now], q[0][c], q[1][c], q[2][c], x);
+            large = mfma(frag[now][0], q[0][c], large);
             if (c + 1 < NC)
 #pragma unroll
-                for (int w = 1; w >= 0; w--) frag[now ^ 1][w] = k_frag(c + 1, w);
+                for (int w = 2; w >= 0; w--) frag[now ^ 1][w] = k_frag(c + 1, w);
 #pragma unroll
             for (int z = c * COUNT / NC; z < (c + 1) * COUNT / NC; z++) beside(z);
-            spread(c + 1 < NC);
+            spread(6, c + 1 < NC ? 3 : 0);
         }
+        x += large;
     };
     auto outputs = [&](int buffer, auto count, auto beside) {
         constexpr int COUNT = decltype(count)::value;
-        frag[0][1] = v_frag(buffer, 0, 1);
-        frag[0][0] = v_frag(buffer, 0, 0);
+        bf16x8_t frag[2][3];
 #pragma unroll
-        for (int n = 0; n < 2 * ND; n++) {
-            const int now = n & 1, j = n / 2, step = n % 2;
-            f32x16_t& rest = REST ? o_rest[j] : o[j];
-            rest = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][1], p[0][step], rest, 0, 0, 0);
-            rest = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], p[1][step], rest, 0, 0, 0);
-            o[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(frag[now][0], p[0][step], o[j], 0, 0, 0);
-            if (n + 1 < 2 * ND)
+        for (int w = 2; w >= 0; w--) frag[0][w] = v_frag(buffer, 0, w);
 #pragma unroll
-                for (int w = 1; w >= 0; w--) frag[now ^ 1][w] = v_frag(buffer, n + 1, w);
+        for (int j = 0; j < ND; j++) {
+            f32x16_t x;  // of this tile, so that o is rounded once per tile
 #pragma unroll
-            for (int z = n * COUNT / (2 * ND); z < (n + 1) * COUNT / (2 * ND); z++) beside(z);
-            spread(n + 1 < 2 * ND);
+            for (int r = 0; r < 16; r++) x[r] = 0.f;
+#pragma unroll
+            for (int step = 0; step < 2; step++) {
+                const int n = 2 * j + step;
+                five(frag[step], p[0][step], p[1][step], p[2][step], x);
+                if (step == 1) {
+                    x = mfma(frag[0][0], p[0][0], x);
+                    x = mfma(frag[1][0], p[0][1], x);
+                }
+                if (step == 0 || j + 1 < ND)
+#pragma unroll
+                    for (int w = 2; w >= 0; w--) frag[step ^ 1][w] = v_frag(buffer, n + 1, w);
+#pragma unroll
+                for (int z = n * COUNT / (2 * ND); z < (n + 1) * COUNT / (2 * ND); z++) beside(z);
+                spread(step ? 7 : 5, step == 0 || j + 1 < ND ? 3 : 0);
+            }
+            o[j] += x;
         }
     };
     // The softmax of the current tile in steps, for each half of the lane's keys: their probabilities, the sum and the pieces
-    constexpr int SOFTMAX = 6 * 2;
+    constexpr int SOFTMAX = (3 + Split::STEPS) * 2;
     auto softmax = [&](f32x16_t& x, int n) {
-        const int half = n / 6, step = n % 6;
+        const int half = n / (3 + Split::STEPS), step = n % (3 + Split::STEPS);
         if (step == 0) {
 #pragma unroll
-            for (int k = 0; k < 8; k++) part.x[k] = __builtin_fmaf(x[8 * half + k], unit, P_EXPONENT - m_run);
+            for (int k = 0; k < 8; k++) part.x[k] = __builtin_fmaf(x[8 * half + k], UNIT, -m_run);
         } else if (step == 1) {
 #pragma unroll
             for (int k = 0; k < 8; k++) part.x[k] = __builtin_amdgcn_exp2f(part.x[k]);
@@ -768,9 +766,9 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
             l_run += ((part.x[0] + part.x[1]) + (part.x[2] + part.x[3])) + ((part.x[4] + part.x[5]) + (part.x[6] + part.x[7]));
         } else {
             part.step(step - 3);
-            if (step == 5)
+            if (step == 2 + Split::STEPS)
 #pragma unroll
-                for (int w = 0; w < 2; w++) __builtin_memcpy(&p[w][half], part.piece[w], 16);
+                for (int w = 0; w < 3; w++) __builtin_memcpy(&p[w][half], part.piece[w], 16);
         }
     };
     // The largest score of a tile, in two steps
@@ -796,62 +794,36 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     const int n_it = SEQ > 1 ? n_t : first;
     auto tile_of = [&](int it) { return SEQ > 1 && it >= first ? it < n_t ? (it - first) * 2 + 1 : n_t : it * RUNS + run; };
     // K and V tiles to LDS and the requests of the next ones, in steps
-    constexpr int STAGING = 8 * CK;
-    float k_scale, v_scale;
+    constexpr int STEPS = Split::STEPS + 1, STAGING = 2 * STEPS * CK;
     auto stage_k = [&](int i, int n) {
         if (n == 0)
 #pragma unroll
-            for (int k = 0; k < 8; k++) part.x[k] = kr[i][k >> 2][k & 3] * k_scale;
-        if (n < 3) part.step(n);
-        if (n == 2) put_k(i);
-        if (n == 3 && i == CK - 1) load_k();
+            for (int k = 0; k < 8; k++) part.x[k] = kr[i][k >> 2][k & 3] * PIECES_SCALE;
+        if (n < Split::STEPS) part.step(n);
+        if (n == Split::STEPS - 1) put_k(i);
+        if (n == Split::STEPS && i == CK - 1) load_k();
     };
     auto stage_v = [&](int i, int n, int buffer) {
         if (n == 0)
 #pragma unroll
-            for (int k = 0; k < 8; k++) part.x[k] = vr[i][k & 3][k >> 2] * v_scale;
-        if (n < 3) part.step(n);
-        if (n == 2) put_v(i, buffer);
-        if (n == 3 && i == CK - 1) load_v();
+            for (int k = 0; k < 8; k++) part.x[k] = vr[i][k & 3][k >> 2] * PIECES_SCALE;
+        if (n < Split::STEPS) part.step(n);
+        if (n == Split::STEPS - 1) put_v(i, buffer);
+        if (n == Split::STEPS && i == CK - 1) load_v();
     };
     typedef std::integral_constant<int, 0> None;
-    // Powers of two for K and V, from the largest values in the first tile of each run and in the one in the middle, which is the latents' if the first is the context's
-    unsigned* const most = reinterpret_cast<unsigned*>(smem + S::LDS - 8);
-    if (threadIdx.x < 2) most[threadIdx.x] = 0;
-    float k_most = 0.f, v_most = 0.f;
-    auto look = [&](const Share& at) {
-#pragma unroll
-        for (int i = 0; i < CK; i++)
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                k_most = larger(k_most, at.k[i][k >> 2][k & 3]);
-                v_most = larger(v_most, at.v[i][k & 3][k >> 2]);
-            }
-    };
-    look(middle);
-    if (SEQ > 1) look(second);
-    look(now);
-    barrier_behind_lds<0>();
-    k_most = max_of_lanes(k_most);
-    v_most = max_of_lanes(v_most);
-    if (lane < 2) __hip_atomic_fetch_max(most + lane, __float_as_uint(lane ? v_most : k_most), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    barrier_behind_lds<0>();
-    const int k_exponent = __builtin_amdgcn_readfirstlane(scale_exponent<6>(most[0])), v_exponent = __builtin_amdgcn_readfirstlane(scale_exponent<6>(most[1]));
-    k_scale = power_of_exponent(k_exponent);
-    v_scale = power_of_exponent(v_exponent);
-    unit = power_of_exponent((unsigned)min(max(127 + 254 - q_exponent - k_exponent, 1), 254));
     find_k(tile_of(1));
     find_v(tile_of(1));
 #pragma unroll
-    for (int n = 0; n < 4 * CK; n++) stage_k(n / 4, n % 4);
+    for (int n = 0; n < STEPS * CK; n++) stage_k(n / STEPS, n % STEPS);
 #pragma unroll
-    for (int n = 0; n < 4 * CK; n++) stage_v(n / 4, n % 4, 0);
+    for (int n = 0; n < STEPS * CK; n++) stage_v(n / STEPS, n % STEPS, 0);
     barrier_behind_lds<0>();
     scores(sc, None(), [](int) {});
     barrier_behind_lds<0>();
     find_k(tile_of(2));
 #pragma unroll
-    for (int n = 0; n < 4 * CK; n++) stage_k(n / 4, n % 4);
+    for (int n = 0; n < STEPS * CK; n++) stage_k(n / STEPS, n % STEPS);
     auto mask = [&](f32x16_t& x, int it) {  // keys past the end of the tile's segment
         int seg, t0;
         const int left = keys_of(tile_of(it), seg, t0);
@@ -867,12 +839,7 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     barrier_behind_lds<0>();
     // Tile `it` of the run, whose scores are x and their largest `top`; y: the scores of the next one. Two barriers: the scores of the next tile beside the softmax of this one;
     // the outputs beside the split of the K tile after the next and of the next V tile.
-    float* const kept = reinterpret_cast<float*>(smem + S::LDS - 8 - S::KEPT_BYTES) + threadIdx.x * S::PITCH;
-    auto add_rest = [&]() {
-        if (REST)
-#pragma unroll
-            for (int j = 0; j < ND; j++) o[j] += o_rest[REST ? j : 0];
-    };
+    float* const kept = reinterpret_cast<float*>(smem + S::LDS - S::KEPT_BYTES) + threadIdx.x * S::PITCH;
     auto keep = [&](float* at) {
         at[0] = m_run;
         at[1] = l_run;
@@ -898,28 +865,24 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
         constexpr int buffer = decltype(buffer_tag)::value;
         const bool mine = tile_of(it) < n_t;
         if (SEQ > 1 && it == first) {  // the second run starts
-            add_rest();
             keep(kept);
             m_run = -1e30f;
             l_run = 0.f;
 #pragma unroll
             for (int j = 0; j < ND; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) o[j][r] = o_rest[REST ? j : 0][r] = 0.f;
+                for (int r = 0; r < 16; r++) o[j][r] = 0.f;
         }
         if (mine) {
             // The reference moves only where a score exceeds it by 2^MARGIN: in the first tile and hardly ever again (with the largest score as the reference some of
             // 32 queries have a larger one in most tiles)
-            const bool moves = top * unit > m_run + MARGIN;
+            const bool moves = top * UNIT > m_run + MARGIN;
             if (__builtin_amdgcn_ballot_w64(moves)) {
-                const float m = moves ? top * unit : m_run, alpha = __builtin_amdgcn_exp2f(m_run - m);
+                const float m = moves ? top * UNIT : m_run, alpha = __builtin_amdgcn_exp2f(m_run - m);
                 m_run = m;
                 l_run *= alpha;
 #pragma unroll
-                for (int j = 0; j < ND; j++) {
-                    o[j] *= alpha;
-                    if (REST) o_rest[j] *= alpha;
-                }
+                for (int j = 0; j < ND; j++) o[j] *= alpha;
             }
             find_k(tile_of(it + 3));
             find_v(tile_of(it + 2));
@@ -927,14 +890,14 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
             // (named here, or the compiler moves what makes them behind the branches that follow, away from the products that it is to run beside)
             asm volatile("" : "+v"(y), "+v"(l_run));
 #pragma unroll
-            for (int w = 0; w < 2; w++) asm volatile("" : "+v"(p[w][0]), "+v"(p[w][1]));
+            for (int w = 0; w < 3; w++) asm volatile("" : "+v"(p[w][0]), "+v"(p[w][1]));
         }
         barrier_behind_lds<0>();
         if (mine) {
             mask(y, it + 1);
             outputs(buffer, std::integral_constant<int, STAGING + 2>(), [&](int n) {
-                if (n < 4 * CK) stage_k(n / 4, n % 4);
-                else if (n < STAGING) stage_v(n / 4 - CK, n % 4, buffer ^ 1);
+                if (n < STEPS * CK) stage_k(n / STEPS, n % STEPS);
+                else if (n < STAGING) stage_v(n / STEPS - CK, n % STEPS, buffer ^ 1);
                 else largest(y, n - STAGING);
             });
         }
@@ -946,7 +909,6 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     }
 
     // merge: in each step the upper half of the runs hands its state to the lower half
-    add_rest();
     float* merge = reinterpret_cast<float*>(smem);
 #pragma unroll
     for (int half = KR / 2; half >= 1; half /= 2) {
@@ -957,14 +919,13 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
         if (run < half) merge_with(at, std::false_type());
     }
     if (SEQ > 1 && n_t > 1) merge_with(kept, std::true_type());
-    l_run *= 1.f / (1 << P_EXPONENT);
 #pragma unroll
     for (int j = 0; j < ND; j++)
 #pragma unroll
-        for (int r = 0; r < 16; r++) o[j][r] = __builtin_amdgcn_ldexpf(o[j][r], 127 - v_exponent - P_EXPONENT);
+        for (int r = 0; r < 16; r++) o[j][r] = o[j][r] * (1.f / PIECES_SCALE);
     if (run) return;
     const float l = l_run + __shfl_xor(l_run, 32, 64), inv = 1.0f / l;
-    bool bad = !finite(l);
+    bool bad = !finite(l) || l == 0.f;
 #pragma unroll
     for (int j = 0; j < ND; j++)
 #pragma unroll
@@ -976,7 +937,7 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
     const bool store = qt < TQ && s.out[seg];
     float* out = store ? s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_out[seg] + h * HS + 4 * lk : nullptr;
     if (__builtin_amdgcn_ballot_w64(bad)) {
-        attend_in_f32<HS>(s, b, h, min(qt, TQ - 1), scale, out);
+        attend_in_f32(s, b, h, min(qt, TQ - 1), scale, out);
         return;
     }
     if (store)
@@ -986,10 +947,10 @@ __global__ void __launch_bounds__(QG* KR * 64, HS == 64 ? 2 : 1) attn_f32_pieces
             for (int r = 0; r < 16; r += 4) *reinterpret_cast<f32x4_t*>(out + 32 * j + 2 * r) = f32x4_t{o[j][r], o[j][r + 1], o[j][r + 2], o[j][r + 3]};
 }
 
-template <int HS, int QG, int KR, int SEQ>
+template <int QG, int KR, int SEQ>
 int launch_attn_pieces(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
-    typedef PiecesShape<HS, QG, KR, SEQ> S;
-    auto kern = attn_f32_pieces_kernel<HS, QG, KR, SEQ>;
+    typedef PiecesShape<QG, KR, SEQ> S;
+    auto kern = attn_f32_pieces_kernel<QG, KR, SEQ>;
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), S::LDS));
     const int TQ = s.Tq[0] + s.Tq[1], n_q = (TQ + S::QWG - 1) / S::QWG;
@@ -1023,22 +984,22 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     const float scale = (float)(1.0 / sqrtf((float)HS));
     const float scale2 = (float)(1.4426950408889634 / sqrt((double)HS));  // scores in powers of two: the exponentials are one instruction
     if (vec && vec_io && (HS == 64 || HS == 128) && a.ld_qkv[0] < (1 << 24) && a.ld_qkv[1] < (1 << 24)) {
-        // By pieces where an element has enough for workgroups of 128 queries: heads x blocks of 128 queries from 64 on, with more than 256 queries from 48. us, fp32
-        // instruction | pieces: one element of 24 heads of 64: 1178 tokens 89 | 37, 333 17.8 | 14.7, 256 (48 workgroups) 11.0 | 12.5, 128 queries of 2000 keys (24)
-        // 25 | 45; 12 heads of 64, 512 tokens (48) 16.1 | 17.0, two of these 24.5 | 17.3, 16 118 | 57; 12 heads of 128, 1178 tokens (120) 90 | 56, 300 queries of 2000 keys
-        // (36) 45 | 81. Up to 64 queries more than half of a block would be empty. (Not by the batch: a batch element's result stays what it is alone.)
+        // By pieces where an element alone is not slower: heads x blocks of 128 queries from 96 on, and these x tiles of 32 keys from 1536. us, fp32 instruction | pieces: one
+        // element of 24 heads: 333 tokens (72 blocks) 17.2 | 18.6, 400 (96 blocks, 1248 with tiles) 20.4 | 21.6, 512 23.9 | 23.7, 640 28.3 | 28.2, 700 42 | 34, 1024 58 | 46, 512
+        // queries of 77 keys 10.2 | 11.5, 1024 of 333 25.0 | 22.8; 12 heads, 666 tokens (72) 19 | 29, 1000 (96) 40.5 | 39.6. 24 heads, 666 tokens (144) 29.8 | 33.2: one more query and the
+        // fp32 kernel takes 42. Batches gain more, 8 x 24 heads, 333 tokens 63 | 56, 16 x 12 heads, 666 tokens 187 | 155, but an element's result stays what it is alone.
+        // (Up to 64 queries more than half of a block would be empty.)
         const long long element_blocks = (long long)NH * ((TQ + 127) / 128);
-        if (TQ > 64 && element_blocks >= (TQ > 256 ? 48 : 64) && !g_attention_f32_no_pieces) {
-            // How the two runs of keys are computed, which their results do not depend on: side by side in workgroups of 64 or of 128 queries as long as all of these
-            // find a compute unit, then one after the other in workgroups of half the wavefronts, two to a unit and independent of each other's
-            // barriers. us: 24 heads, 333 tokens 14.7 | 16.6 | 19.1; 1178 tokens 45 | 37 | 47, a batch of two 89 | 77 | 72; 16 x 12 heads, 666 tokens 117 | 119 | 104.
-            if (HS == 128) return launch_attn_pieces<128, 4, 2, 1>(s, B, NH, scale2, st);
+        if (HS == 64 && TQ > 64 && element_blocks >= 96 && element_blocks * ((T + 31) / 32) >= 1536 && !g_attention_f32_no_pieces) {
             const int cus = compute_units();
             if (cus <= 0) return SD3_ERR_HIP;
             const long long blocks = B * element_blocks;
-            if (2 * blocks <= cus) return launch_attn_pieces<64, 2, 2, 1>(s, B, NH, scale2, st);
-            if (blocks <= cus) return launch_attn_pieces<64, 4, 2, 1>(s, B, NH, scale2, st);
-            return launch_attn_pieces<64, 4, 1, 2>(s, B, NH, scale2, st);
+            // How the two runs of keys are computed, which their results do not depend on: side by side in workgroups of 64 or of 128 queries as long as all of these
+            // find a compute unit, then one after the other in workgroups of half the wavefronts, two to a unit and independent of each other's
+            // barriers. us, 24 heads: 512 tokens 25 | 27 | 32; 700 58 | 34 | 42, a batch of two 86 | 69 | 60; 1178 90 | 57 | 67, a batch of two 178 | 113 | 106.
+            if (2 * blocks <= cus) return launch_attn_pieces<2, 2, 1>(s, B, NH, scale2, st);
+            if (blocks <= cus) return launch_attn_pieces<4, 2, 1>(s, B, NH, scale2, st);
+            return launch_attn_pieces<4, 1, 2>(s, B, NH, scale2, st);
         }
         // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. Four key runs in both: eight, or the keys over several
         // workgroups and a second kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four

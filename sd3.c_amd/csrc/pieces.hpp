@@ -5,48 +5,6 @@
 namespace sd3 {
 namespace {
 
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi) {  // rounds to nearest even
-    typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
-    const f32x2_t v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-}
-
-// x * scale = h + l: h the first 11 significant bits, rounded to nearest, l the next 11 of what is left; what remains is at most 2^-24 of x, as much as fp32
-// itself rounds away, where x * scale is at least 2^-2 (below that 2^-25 absolute) and less than 65520. Beyond, as for infinities and NaNs, h is infinite or a NaN.
-// A mixed-precision fma takes h as it is; the forms of it that round to f16 would save the conversions behind but take 8.7 cycles (this one and the conversion of
-// two values 4.5, a product 2.6, several wavefronts of a SIMD at it). Step by step for all values, as each step waits for the one before. N values, two to a register.
-template <int N>
-__device__ __forceinline__ void f16_high(const float (&x)[N], uint32_t (&h)[N / 2]) {
-#pragma unroll
-    for (int p = 0; p < N / 2; p++) h[p] = pack_f16x2(x[2 * p], x[2 * p + 1]);
-}
-template <int N>
-__device__ __forceinline__ void f16_rest(float (&x)[N], const uint32_t (&h)[N / 2]) {
-#pragma unroll
-    for (int p = 0; p < N / 2; p++) {
-        asm("v_fma_mix_f32 %0, %0, 1.0, -%1 op_sel_hi:[0,0,1]" : "+v"(x[2 * p]) : "v"(h[p]));
-        asm("v_fma_mix_f32 %0, %0, 1.0, -%1 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "+v"(x[2 * p + 1]) : "v"(h[p]));
-    }
-}
-template <int N>
-__device__ __forceinline__ void f16_pieces(float (&x)[N], float scale, uint32_t (&h)[N / 2], uint32_t (&l)[N / 2]) {
-#pragma unroll
-    for (int k = 0; k < N; k++) x[k] *= scale;
-    f16_high<N>(x, h);
-    f16_rest<N>(x, h);
-    f16_high<N>(x, l);
-}
-// The exponent field of the power of two that takes values of up to `most` (the bits of an absolute value) to 2^TARGET .. 2^(TARGET + 1): what comes later may be
-// 2^(15 - TARGET) times as large. All zero: 2^126, so that anything that comes later is infinite. Infinite or NaN: any.
-template <int TARGET = 4>
-__device__ __forceinline__ unsigned scale_exponent(unsigned most) {
-    return (unsigned)min(max(254 + TARGET - (int)(most >> 23), 1), 253);
-}
-__device__ __forceinline__ float power_of_exponent(unsigned exponent) { return __uint_as_float(exponent << 23); }
-
-__device__ __forceinline__ float larger(float most, float x) { return fmaxf(most, fabsf(x)); }
-
 // x * 2^16 = h + m + l, each a bf16 value: h the first 8 significant bits, rounded to nearest, m the next 8 of what is left, l the rest, at most 8 bits. Without a
 // remainder for every |x| < 2^112, subnormal numbers included: the last bit of the smallest, 2^-149, becomes the last bit of the smallest bf16 value, which the matrix instructions take as
 // it is (with no scale, values below 2^-110 would lose bits; the scale costs 4 %). Beyond, as for infinities and NaNs, h is infinite or a NaN. |m| <= 2^-8 |x| and
@@ -58,15 +16,15 @@ __device__ __forceinline__ void bf16_high(const float (&x)[N], uint32_t (&piece)
 #pragma unroll
     for (int p = 0; p < N / 2; p++) piece[p] = pack_bf16x2(x[2 * p], x[2 * p + 1]);
 }
-template <int N>
+template <int N, bool FENCES = true>
 __device__ __forceinline__ void bf16_rest(float (&x)[N], const uint32_t (&piece)[N / 2]) {
     float t[N];
 #pragma unroll
     for (int k = 0; k < N; k++) t[k] = __uint_as_float(k & 1 ? piece[k / 2] & 0xffff0000u : piece[k / 2] << 16);
-    __builtin_amdgcn_sched_barrier(NOT_VECTOR);
+    if constexpr (FENCES) __builtin_amdgcn_sched_barrier(NOT_VECTOR);
 #pragma unroll
     for (int k = 0; k < N; k++) x[k] -= t[k];
-    __builtin_amdgcn_sched_barrier(NOT_VECTOR);
+    if constexpr (FENCES) __builtin_amdgcn_sched_barrier(NOT_VECTOR);
 }
 template <int N>
 __device__ __forceinline__ void bf16_pieces(float (&x)[N], uint32_t (&h)[N / 2], uint32_t (&m)[N / 2], uint32_t (&l)[N / 2]) {
