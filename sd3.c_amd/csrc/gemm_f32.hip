@@ -2,7 +2,7 @@
 //   out(M,N) = A(M,K) @ W(K,N)[:, n0:n0+N] + epilogue
 // replacing linear / partial_linear of the reference (modules.cpp:475-511, naive triple loops).
 //
-// gemm_f32_pieces_kernel (operands as three bf16 pieces each, on the bf16 matrix instruction) takes depths from 256 on;
+// gemm_f32_pieces_kernel (operands as three bf16 pieces each, on the bf16 matrix instruction) takes depths from 512 on;
 // gemm_f32_tile_kernel (v_mfma_f32_16x16x4_f32) everything else whose operand rows are made of whole 16-byte chunks; both up to three problems
 // per launch. gemm_f32_kernel (v_mfma_f32_32x32x2_f32, 128x128x16 tiles, element-wise loads) takes operands of any other stride or alignment.
 #include <type_traits>

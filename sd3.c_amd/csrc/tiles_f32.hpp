@@ -42,14 +42,14 @@ inline int pick_f32_tile(const F32Layer* layers, int n, int cus, bool whole_k) {
 }
 
 // ---- products of bf16 pieces (gemm_f32_pieces_kernel) ----
-// Which launches: depths of 256 and more, in whole groups of the four K tiles that its loops take at a time. Shallower products are over before the split of the
-// operands is under way. us, fp32 instruction | pieces: K = 256: 8192 x 1536 57 | 49, 1178 x 4608 30.4 | 27.7, 2356 x 768 13.1 | 12.2, what is smaller is lost in the 11 us that a
-// call costs; over 1 to 8192 rows, 256 to 6144 columns the mean is 0.96 of the fp32 instruction's time at K = 256, 0.93 at 512, 0.90 from 768 on. One round of small
-// tiles is up to a tenth slower (154 x 1536 x 1536 12.1 | 13.0, 666 x 1536 x 1536 28.7 | 31.2), from 1178 rows and 768 columns on it is 0.6 to 0.9. By the depth alone: the two kernels
+// Which launches: depths of 512 and more, in whole groups of the four K tiles that its loops take at a time. us, fp32 instruction | pieces: over 1 to 8192 rows, 256 to 6144
+// columns the mean is 0.93 of the fp32 instruction's time at K = 512, 0.90 from 768 on, 0.96 at 256, where large products gain (8192 x 1536 57 | 49) and small ones lose, which
+// are what such models consist of (width 256, 2 heads, three blocks, 1178 tokens: a forward 327 us, with pieces from K = 256 on 334). One round of small
+// tiles is up to a tenth slower (154 x 1536 x 1536 12.9 | 13.8, 666 x 1536 x 1536 29.4 | 30.5), from 1178 rows and 768 columns on it is 0.6 to 0.9. By the depth alone: the two kernels
 // round differently, and a row's result is to be the same in every batch.
 inline bool f32_by_pieces(const F32Layer* layers, int n) {
     for (int i = 0; i < n; i++)
-        if (layers[i].K % 128 || layers[i].K < 256) return false;
+        if (layers[i].K % 128 || layers[i].K < 512) return false;
     return true;
 }
 

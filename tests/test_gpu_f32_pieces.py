@@ -17,7 +17,7 @@ def _automatic_choice_afterwards():
     L.call("sd3_tune", b"gemm_f32_no_pieces", 0)
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 512, 4), (31, 256, 36), (33, 384, 68), (65, 768, 64), (129, 512, 132), (257, 640, 260), (300, 1536, 1540)])
+@pytest.mark.parametrize("m,k,n", [(1, 512, 4), (31, 640, 36), (33, 1152, 68), (65, 768, 64), (129, 512, 132), (257, 640, 260), (300, 1536, 1540)])
 def test_every_tile_shape(m, k, n):
     """Rows and columns on and beside the multiples of the tiles (32 to 256), depths from the smallest on. Bound: a product of pieces lacks at most
     u of itself (m*l, l*m: 2^-25 each), and the additions of 32 products and of their sum to the sum of those before round less often than a sum of k products in any
@@ -142,7 +142,7 @@ def test_single_products(shape):
     """Rows of x with one value that is not zero: every result is one product, which lacks at most 2^-24 of itself for the products of pieces that are not formed and is added
     to what is small beside it within a unit in the last place (2 u) whichever way that rounds: 3 u and 2^-8 of it for the sums of the smaller ones. Powers of two of
     2^-60 to 2^60, and values of 1 + 2^-11 and 1 + 2^-12 + 2^-23, whose low bits all count."""
-    m, k, n = 256, 256, 140
+    m, k, n = 512, 512, 140
     g = torch.Generator(device="cuda").manual_seed(shape + 3)
     value = torch.randn(m, device="cuda", generator=g) * torch.exp2(torch.randint(-60, 61, (m,), device="cuda", generator=g).float())
     value[:3] = 1 + 2.0 ** -11
@@ -158,7 +158,7 @@ def test_single_products(shape):
 
 
 @pytest.mark.parametrize("x_of,w_of", [("normal", "normal"), ("positive", "positive"), ("1 + 2^-11", "1 + 2^-11"), ("positive", "1 + 2^-12 + 2^-23"), ("gelu", "normal"), ("one in 16", "normal")])
-@pytest.mark.parametrize("k", [256, 1536, 6144])
+@pytest.mark.parametrize("k", [512, 1536, 6144])
 def test_error_is_no_larger_than_the_fp32_instructions(x_of, w_of, k):
     """Sums whose terms cancel, whose terms all have one sign (where rounding to one side would add up), constants, and few terms. 1.25: two sums of the same
     products may differ by chance; u: results that one of the two happens to hold exactly."""
