@@ -5,6 +5,7 @@ import torch
 from gpu_util import M
 from sd3_c_amd import lib as L
 from sd3_c_amd.params import block_param_shapes
+from test_gpu_f32_kernels import test_gemm_f32_every_tile_shape as check_tile_kernel
 
 pytestmark = pytest.mark.gpu
 U = 2.0 ** -24  # unit roundoff of fp32
@@ -206,3 +207,35 @@ def test_blocks_in_batches(Tc, Tx, dual):
     L.call("sd3_tune", b"gemm_f32_no_pieces", 1)
     for a, b in zip(run(2), both):
         assert not torch.equal(a, b) and float((a - b).norm()) <= 1e-5 * float(a.norm())
+
+
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 4, 5])
+@pytest.mark.parametrize("k", [512, 640])
+def test_column_windows_and_outputs_at_any_float(k, shape):
+    """Columns n0.. of a wider weight have the bits of that part of the weight by itself, outputs may begin at any float and nothing beside them is written, also in rows and
+    columns that are formed anew (values of 2^113 and more, an infinity). Bound as above."""
+    m, nmax, n0, n = 70, 240, 100, 132
+    g = torch.Generator(device="cuda").manual_seed(k)
+    x, W, b = (torch.randn(s, device="cuda", generator=g) for s in ((m, k), (k, nmax), (nmax,)))
+    x[33] *= 2.0 ** 113
+    W[7, n0 + 66] = float("inf")
+    L.call("sd3_tune", b"gemm_f32_tile", shape)
+    part, bias = W[:, n0:n0 + n].contiguous(), b[n0:n0 + n].contiguous()
+    want = M.linear(x, part, bias)
+    assert torch.equal(M.partial_linear(x, W, b, n0, n), want)
+    fine = torch.arange(n, device="cuda") != 66
+    exact = x.double() @ part[:, fine].double() + bias[fine].double()
+    assert ((want[:, fine].double() - exact).abs() <= (k + 2) * U * (x.double().abs() @ part[:, fine].double().abs() + bias[fine].double().abs())).all()
+    assert torch.isinf(want[:, 66]).all()
+    for off in (1, 2, 3):
+        buf = torch.full((m * n + 8,), 7.0, device="cuda")
+        L.call("sd3_linear", x.data_ptr(), part.data_ptr(), bias.data_ptr(), buf.data_ptr() + 4 * off, m, k, n, None)
+        torch.cuda.synchronize()
+        assert torch.equal(buf[off:off + m * n].view(m, n), want) and bool((buf[:off] == 7).all()) and bool((buf[off + m * n:] == 7).all()), off
+
+
+@pytest.mark.parametrize("m,k,n", [(154, 1536, 1540), (154, 1568, 1540), (257, 480, 64)])
+def test_deep_products_of_the_tile_kernel(m, k, n):
+    """The fp32 instruction at depths of many whole K tiles: asked for, and where they are not whole groups of four."""
+    L.call("sd3_tune", b"gemm_f32_no_pieces", 1)
+    check_tile_kernel(m, k, n)
