@@ -427,7 +427,7 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 // three products took 0.65 of this time, 1178 x 6144 x 1536 69 us, but hold 22 of the 24 bits, and only of values within 2^-7 of the largest that the scale is
 // made for: rows of one channel 2^20 times the others, which W leaves out, came out with an error of 9e-4.)
 // The products of a K tile (32 k values) are summed by themselves, and that sum is then added to the fp32 sum of the tiles before: one rounding per K tile that counts,
-// where the fp32 instruction has eight. Relative error against 64 bits, normal operands, with this kernel (with the tile kernel): K = 256 7.0e-8 (2.9e-7), 1536
+// where the fp32 instruction has eight. Relative error against 64 bits, normal operands, with this kernel (with the tile kernel): K = 512 9.0e-8 (4.1e-7), 1536
 // 1.4e-7 (7.0e-7), 6144 2.7e-7 (1.41e-6); one in 16 values of A not zero 1536 1.4e-7 (1.8e-7); all values 1 + 2^-11 1.6e-7 (1.6e-7). All six products added to one sum:
 // 0.85 of the tile kernel's error for normal operands but 1.9 times it for one in 16, 8192 x 3072 x 768 177 us instead of 189; the five small products in a second
 // sum: 0.34 of it, but 256x128 tiles have no registers for that, 219 us.

@@ -102,8 +102,11 @@ def test_infinities_nans_and_values_beyond_the_pieces(hs, B):
     for h in range(11):
         g, w = got[0, :, at(h)], want[0, :, at(h)]
         fine = torch.isfinite(w)
-        # scores of up to 2^10 * 30 carry errors of 2^-24 of that, and an output as many; elsewhere rounding
-        assert float((g - w)[fine].abs().max() / w[fine].abs().max()) <= (2e-2 if h == 7 else 1e-5) if fine.any() else True
+        if h == 7:  # scores of up to 2^10 * 30, whose own rounding shows: no further from float64 than the fp32 instruction (1.25 as below)
+            truth = exact(q[:1, :, at(7)], k[:1, :, at(7)], v[:1, :, at(7)], 1)[0]
+            assert float((g.double() - truth).norm()) <= 1.25 * float((w.double() - truth).norm())
+        elif fine.any():
+            assert float((g - w)[fine].abs().max() / w[fine].abs().max()) <= 1e-5
     assert torch.equal(got[0, :, 11 * hs:], plain[0, :, 11 * hs:])
     assert torch.equal(got[1:], plain[1:])
 
