@@ -445,9 +445,10 @@ int launch_split(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
 
 // ---- head_dim 64 by bf16 pieces ----
 // Products as in gemm_f32_pieces_kernel: an fp32 value is the sum of three bf16 values without a remainder (bf16_pieces), six of the nine products of pieces are formed. No
-// value is lost beside a larger one of its head, channel or token. Probabilities are split as they are: those below 2^-110 keep the bits down to 2^-133,
-// and an exponential below 2^-126 is 0 in any case (times 2^16 first: 2 x 1178 tokens 109 -> 112 us, the same error where a result is made of weights of 2^-118). Scores, probabilities, their sums and the outputs are fp32 throughout. Two sums per score, of the products of first pieces and of the others, because the matrix instruction does not round to nearest;
-// the products of a key tile are summed by themselves before they join the outputs, one rounding per tile. Relative error against 64 bits, 24 heads of 64 (fp32
+// value is lost beside a larger one of its head, channel or token. Probabilities are split as they are: those below 2^-110 keep the bits down to 2^-133, and an exponential
+// below 2^-126 is 0 in any case (times 2^16 first: 2 x 1178 tokens 109 -> 112 us, the same error where a result is made of weights of 2^-118). Scores, probabilities, their
+// sums and the outputs are fp32 throughout. Two sums per score, of the products of first pieces and of the others, because the matrix instruction does not round to
+// nearest; the products of a key tile are summed by themselves before they join the outputs, one rounding per tile. Relative error against 64 bits, 24 heads of 64 (fp32
 // instruction): 32 keys 1.1e-7 (2.3e-7), 77 1.3e-7 (2.7e-7), 1178 1.8e-7 (4.3e-7), 4250 2.4e-7 (6.6e-7); equal weights, 77 keys 7.7e-8 (1.1e-7), constant values 7.0e-8
 // (7.9e-8). (Two f16 pieces per value and three products took 68 us for 2 x 1178 tokens, 24 heads, but hold 22 of the 24 bits, and only of values within 2^-7 of the
 // largest of the head: with one channel of V 2^16 times the others these came out with an error of 4e-5, beside a key that takes 1 - 2^-20 of the weight 7e-5. One sum per
