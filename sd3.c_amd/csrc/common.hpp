@@ -68,9 +68,13 @@ __device__ __forceinline__ float gelu_tanh_f(float x) {
     const float e = __builtin_amdgcn_exp2f(x * (k3 * x2 + k1));
     return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
+// The same to fp32 precision: the quotient x / d and the sum d = 1 + 2^t with their remainders. 11 full-rate operations and two others instead of tanhf's, whose time stood behind every tile of
+// the fp32 MLP (10656 x 3072 x 768 286 -> 277 us).
 __device__ __forceinline__ float gelu_tanh_precise(float x) {
-    const float p = 0.7978845608028654f;
-    return 0.5f * x * (1.0f + tanhf(p * (x + 0.044715f * x * x * x)));
+    const float k1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f;
+    const float e = __builtin_amdgcn_exp2f(x * fmaf(k1 * 0.044715f, x * x, k1)), d = 1.0f + e, r = __builtin_amdgcn_rcpf(d), q = x * r;
+    const float rest = fmaf(-q, e - (d - 1.0f), fmaf(-q, d, x));
+    return __builtin_amdgcn_div_fixupf(fmaf(rest, r, q), d, x);  // (infinities)
 }
 __device__ __forceinline__ float silu_precise(float x) { return x / (1.0f + expf(-x)); }
 
