@@ -28,7 +28,14 @@ struct SegDev {
     int ld_out[2];
     int T[2];   // keys/values per batch element in each segment
     int Tq[2];  // queries per batch element in each segment
+    int B;
 };
+// Four values of an output row, from column `col` on. PIECES: AttnSegments::out_pieces
+template <bool PIECES>
+__device__ __forceinline__ void put_output(const SegDev& s, int seg, long long row, int col, const f32x4_t& v) {
+    if constexpr (PIECES) put_pieces<4>(PieceMatrix(s.out[seg], (long long)s.B * s.Tq[seg], s.ld_out[seg]), row, col, {v[0], v[1], v[2], v[3]});
+    else *reinterpret_cast<f32x4_t*>(s.out[seg] + row * s.ld_out[seg] + col) = v;
+}
 
 template <int HSP, bool VEC>
 __global__ void __launch_bounds__(256) attn_f32_kernel(SegDev s, int HS, float scale) {
@@ -197,7 +204,7 @@ __device__ __forceinline__ float max_of_groups(float x) {
 // LONG_ROWS: rows are 2^22 floats or more apart (and less than 2^24): four times the stride does not fit the 24-bit product of the row offsets. An
 // instantiation of its own, since the shift behind the product, done in every case, costs the others up to 2 %. 65536 heads of 64, 2 queries, 40 keys:
 // 691 us, with attn_f32_kernel 2204.
-template <int HS, int QB, int KB, int KS, bool LONG_ROWS>
+template <int HS, int QB, int KB, int KS, bool LONG_ROWS, bool PIECES>
 __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, int NH, int n_q, int total, float scale) {
     constexpr int NC = HS / 16, NU = HS / 64, TKEYS = 16 * KB, QW = 16 * QB;
     constexpr int PITCH = NU * 16 * QB + 2 * QB;  // floats per lane in the merge buffer
@@ -424,23 +431,28 @@ __global__ void __launch_bounds__(KS * 64, 2) attn_f32_split_kernel(SegDev s, in
         l += __shfl_xor(l, 32, 64);
         if (qt >= TQ || !s.out[seg]) continue;
         const float inv = 1.0f / l;
-        float* p = s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_out[seg] + h * HS + 16 * lg;
+        const long long row = (long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt);
 #pragma unroll
         for (int u = 0; u < NU; u++)
 #pragma unroll
             for (int r = 0; r < 4; r++)
-                *reinterpret_cast<f32x4_t*>(p + 64 * u + 4 * r) =
-                    f32x4_t{o[i][u][0][r] * inv, o[i][u][1][r] * inv, o[i][u][2][r] * inv, o[i][u][3][r] * inv};
+                put_output<PIECES>(s, seg, row, h * HS + 16 * lg + 64 * u + 4 * r,
+                           f32x4_t{o[i][u][0][r] * inv, o[i][u][1][r] * inv, o[i][u][2][r] * inv, o[i][u][3][r] * inv});
     }
 }
 
-template <int HS, int QB, int KB, int KS, bool LONG_ROWS = false>
-int launch_split(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
+template <int HS, int QB, int KB, int KS, bool LONG_ROWS, bool PIECES>
+int launch_split_as(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
     const int TQ = s.Tq[0] + s.Tq[1], n_q = (TQ + 16 * QB - 1) / (16 * QB);
     const long long total = (long long)B * NH * n_q;
     if (total > 0x7fffffff) return fail(SD3_ERR_UNSUPPORTED, "attention (fp32): too many work items");
-    hipLaunchKernelGGL((attn_f32_split_kernel<HS, QB, KB, KS, LONG_ROWS>), dim3((unsigned)total), dim3(KS * 64), 0, st, s, NH, n_q, (int)total, scale);
+    hipLaunchKernelGGL((attn_f32_split_kernel<HS, QB, KB, KS, LONG_ROWS, PIECES>), dim3((unsigned)total), dim3(KS * 64), 0, st, s, NH, n_q, (int)total, scale);
     return launch_status("attention_f32");
+}
+
+template <int HS, int QB, int KB, int KS>
+int launch_split(const SegDev& s, int B, int NH, float scale, bool pieces, hipStream_t st) {
+    return pieces ? launch_split_as<HS, QB, KB, KS, false, true>(s, B, NH, scale, st) : launch_split_as<HS, QB, KB, KS, false, false>(s, B, NH, scale, st);
 }
 
 // ---- head_dim 64 by bf16 pieces ----
@@ -468,8 +480,9 @@ int launch_split(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
 // head_dim 128 has no registers for the pieces of its queries beside a second wavefront: with one per SIMD 12 heads, 1178 tokens 84 -> 83, two of these 159 -> 121, but 3 x 1000
 // tokens 173 -> 206, 666 tokens 30 -> 52. It stays on the fp32 instruction.
 // What the pieces cannot give (values beyond their range, infinities, NaNs): the lane's query `qt`, all lanes 32 of them, over all keys on the fp32
-// matrix instruction; out (null: not stored): the query's result from d = 4(l/32) on. For the rare case, so as plain as can be.
-__device__ void attend_in_f32(const SegDev& s, int b, int h, int qt, float scale, float* out) {
+// matrix instruction; row: where the query's result goes in its segment (-1: not stored). For the rare case, so as plain as can be.
+template <bool PIECES>
+__device__ void attend_in_f32(const SegDev& s, int b, int h, int qt, float scale, long long row) {
     constexpr int HS = 64;
     const int l32 = threadIdx.x & 31, lk = threadIdx.x >> 5 & 1;
     const int qseg = qt < s.Tq[0] ? 0 : 1;
@@ -511,11 +524,12 @@ __device__ void attend_in_f32(const SegDev& s, int b, int h, int qt, float scale
             }
         }
     const float inv = 1.0f / (l + __shfl_xor(l, 32, 64));
-    if (out)
+    if (row >= 0)
 #pragma unroll
         for (int j = 0; j < HS / 32; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) out[32 * j + 8 * (r >> 2) + (r & 3)] = o[j][r] * inv;
+            for (int r = 0; r < 16; r += 4)
+                put_output<PIECES>(s, qseg, row, h * HS + 4 * lk + 32 * j + 2 * r, f32x4_t{o[j][r] * inv, o[j][r + 1] * inv, o[j][r + 2] * inv, o[j][r + 3] * inv});
 }
 
 // The split of eight values into pieces (bf16_pieces) in steps, to be spread over matrix instructions
@@ -543,7 +557,7 @@ struct PiecesShape {
 // (8 consecutive lanes) meet in a bank
 __device__ __forceinline__ unsigned row_slot(unsigned row, unsigned chunk) { return row * 64 + ((chunk ^ (row >> 2)) & 3) * 16; }
 
-template <int QG, int KR, int SEQ>
+template <int QG, int KR, int SEQ, bool PIECES>
 __global__ void __launch_bounds__(QG* KR * 64, SEQ * QG * KR / 4) attn_f32_pieces_kernel(SegDev s, int NH, int n_q, int total, float scale) {
     typedef PiecesShape<QG, KR, SEQ> S;
     constexpr int HS = S::HS, NC = HS / 16, ND = HS / 32, PT = QG * 64, CK = 4 * HS / PT, TKEYS = 32, RUNS = KR * SEQ;
@@ -936,22 +950,22 @@ __global__ void __launch_bounds__(QG* KR * 64, SEQ * QG * KR / 4) attn_f32_piece
         }
     const int seg = qt < Tq0 ? 0 : 1;
     const bool store = qt < TQ && s.out[seg];
-    float* out = store ? s.out[seg] + ((long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt)) * s.ld_out[seg] + h * HS + 4 * lk : nullptr;
+    const long long row = store ? (long long)b * s.Tq[seg] + (seg ? qt - Tq0 : qt) : -1;
     if (__builtin_amdgcn_ballot_w64(bad)) {
-        attend_in_f32(s, b, h, min(qt, TQ - 1), scale, out);
+        attend_in_f32<PIECES>(s, b, h, min(qt, TQ - 1), scale, row);
         return;
     }
     if (store)
 #pragma unroll
         for (int j = 0; j < ND; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r += 4) *reinterpret_cast<f32x4_t*>(out + 32 * j + 2 * r) = f32x4_t{o[j][r], o[j][r + 1], o[j][r + 2], o[j][r + 3]};
+            for (int r = 0; r < 16; r += 4) put_output<PIECES>(s, seg, row, h * HS + 4 * lk + 32 * j + 2 * r, f32x4_t{o[j][r], o[j][r + 1], o[j][r + 2], o[j][r + 3]});
 }
 
-template <int QG, int KR, int SEQ>
-int launch_attn_pieces(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
+template <int QG, int KR, int SEQ, bool PIECES>
+int launch_attn_pieces_as(const SegDev& s, int B, int NH, float scale, hipStream_t st) {
     typedef PiecesShape<QG, KR, SEQ> S;
-    auto kern = attn_f32_pieces_kernel<QG, KR, SEQ>;
+    auto kern = attn_f32_pieces_kernel<QG, KR, SEQ, PIECES>;
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), S::LDS));
     const int TQ = s.Tq[0] + s.Tq[1], n_q = (TQ + S::QWG - 1) / S::QWG;
@@ -959,6 +973,10 @@ int launch_attn_pieces(const SegDev& s, int B, int NH, float scale, hipStream_t 
     if (total > 0x7fffffff) return fail(SD3_ERR_UNSUPPORTED, "attention (fp32): too many work items");
     hipLaunchKernelGGL(kern, dim3((unsigned)total), dim3(S::THREADS), S::LDS, st, s, NH, n_q, (int)total, scale);
     return launch_status("attention_f32");
+}
+template <int QG, int KR, int SEQ>
+int launch_attn_pieces(const SegDev& s, int B, int NH, float scale, bool pieces, hipStream_t st) {
+    return pieces ? launch_attn_pieces_as<QG, KR, SEQ, true>(s, B, NH, scale, st) : launch_attn_pieces_as<QG, KR, SEQ, false>(s, B, NH, scale, st);
 }
 }  // namespace
 
@@ -970,6 +988,7 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
     if (T <= 0) return fail(SD3_ERR_INVALID_ARG, "attention: no keys");
     if (HS <= 0 || HS > 128) return fail(SD3_ERR_UNSUPPORTED, "attention (fp32): head_dim %d not in 1..128", HS);
     SegDev s;
+    s.B = B;
     bool vec = (HS % 4 == 0), vec_io = true;  // vec_io: queries and outputs too are made of aligned 16-byte chunks
     for (int i = 0; i < 2; i++) {
         s.q[i] = (const float*)a.q[i]; s.k[i] = (const float*)a.k[i]; s.v[i] = (const float*)a.v[i]; s.out[i] = (float*)a.out[i];
@@ -998,19 +1017,22 @@ int attention_f32(const AttnSegments& a, int B, int NH, int HS, hipStream_t st) 
             // How the two runs of keys are computed, which their results do not depend on: side by side in workgroups of 64 or of 128 queries as long as all of these
             // find a compute unit, then one after the other in workgroups of half the wavefronts, two to a unit and independent of each other's
             // barriers. us, 24 heads: 512 tokens 25 | 27 | 32; 700 58 | 34 | 42, a batch of two 86 | 69 | 60; 1178 90 | 57 | 67, a batch of two 178 | 113 | 106.
-            if (2 * blocks <= cus) return launch_attn_pieces<2, 2, 1>(s, B, NH, scale2, st);
-            if (blocks <= cus) return launch_attn_pieces<4, 2, 1>(s, B, NH, scale2, st);
-            return launch_attn_pieces<4, 1, 2>(s, B, NH, scale2, st);
+            if (2 * blocks <= cus) return launch_attn_pieces<2, 2, 1>(s, B, NH, scale2, a.out_pieces, st);
+            if (blocks <= cus) return launch_attn_pieces<4, 2, 1>(s, B, NH, scale2, a.out_pieces, st);
+            return launch_attn_pieces<4, 1, 2>(s, B, NH, scale2, a.out_pieces, st);
         }
         // 32 queries per workgroup; with so few (queries, heads) that this leaves compute units idle, 16. Four key runs in both: eight, or the keys over several
         // workgroups and a second kernel to merge, cost as much in starts and merging as they save in the runs (2 heads of 128, 1178 tokens: 36 and 36 us, four
         // runs 32).
         const bool few = (long long)NH * ((TQ + 31) / 32) < 192;
-        if (a.ld_qkv[0] >= (1 << 22) || a.ld_qkv[1] >= (1 << 22))  // (tens of thousands of heads)
-            return HS == 64 ? launch_split<64, 2, 1, 4, true>(s, B, NH, scale2, st) : launch_split<128, 2, 1, 4, true>(s, B, NH, scale2, st);
-        if (HS == 64) return few ? launch_split<64, 1, 2, 4>(s, B, NH, scale2, st) : launch_split<64, 2, 1, 4>(s, B, NH, scale2, st);
-        return few ? launch_split<128, 1, 1, 4>(s, B, NH, scale2, st) : launch_split<128, 2, 1, 4>(s, B, NH, scale2, st);
+        if (a.ld_qkv[0] >= (1 << 22) || a.ld_qkv[1] >= (1 << 22)) {  // (tens of thousands of heads)
+            if (a.out_pieces) return fail(SD3_ERR_INVALID_ARG, "attention (fp32): no outputs in pieces for rows as long as these");
+            return HS == 64 ? launch_split_as<64, 2, 1, 4, true, false>(s, B, NH, scale2, st) : launch_split_as<128, 2, 1, 4, true, false>(s, B, NH, scale2, st);
+        }
+        if (HS == 64) return few ? launch_split<64, 1, 2, 4>(s, B, NH, scale2, a.out_pieces, st) : launch_split<64, 2, 1, 4>(s, B, NH, scale2, a.out_pieces, st);
+        return few ? launch_split<128, 1, 1, 4>(s, B, NH, scale2, a.out_pieces, st) : launch_split<128, 2, 1, 4>(s, B, NH, scale2, a.out_pieces, st);
     }
+    if (a.out_pieces) return fail(SD3_ERR_INVALID_ARG, "attention (fp32): no outputs in pieces for these heads, strides or alignments");
     dim3 grid((TQ + BQ - 1) / BQ, NH, B), block(256);
     const int hsp = HS <= 32 ? 32 : (HS <= 64 ? 64 : 128);
 #define SD3_ATTN_LAUNCH(P)                                                                              \

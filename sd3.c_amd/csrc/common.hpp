@@ -331,7 +331,10 @@ struct GemmF32Problem {
     float* out;
     int lda, ldw, n0, ldc, M, N, K;
     GemmEpilogueArgs ea;
+    bool a_pieces = false;    // A: a matrix of pieces (pieces.hpp), in all problems of the launch and where gemm_f32_takes_a_pieces
+    bool out_pieces = false;  // EPI_BIAS_GELU: the output as a matrix of pieces of ldc columns
 };
+bool gemm_f32_takes_a_pieces(const float* W, int ldw, int n0, int N, int K);
 int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st);
 extern int g_gemm_f32_tile, g_gemm_f32_no_pieces;
 // bf16 GEMM: A bf16 (M,K) row-major; Wp = packed weight, bf16, K-contiguous (see GemmBf16Problem::w_tiled); out bf16 (out_is_f32 = 0) or fp32.
@@ -382,7 +385,8 @@ struct LayerNormJob {
     const float* scale2;
     int mod_ld, B, T;
 };
-int layernorm_modulate_pair(const LayerNormJob* jobs, int n, float eps, int C, int out_bf16, hipStream_t st);
+enum LayerNormOut : int { LN_F32 = 0, LN_BF16 = 1, LN_PIECES = 2 };  // fp32, bf16, a matrix of bf16 pieces (pieces.hpp)
+int layernorm_modulate_pair(const LayerNormJob* jobs, int n, float eps, int C, int out, hipStream_t st);
 int layernorm_modulate(const float* x, void* out, void* out2, const float* shift, const float* scale, const float* shift2, const float* scale2,
                        int mod_ld, float eps, int B, int T, int C, int out_bf16, hipStream_t st);
 int layernorm_full(const float* x, float* y, float* mean, float* rstd, const float* w, const float* bias, float eps, long long rows, int C,
@@ -444,6 +448,7 @@ struct AttnSegments {
     int Tq[2];      // queries per batch element in each segment (equal to T for self-attention)
     const float* rms_q[2];  // bf16 kernel only: fused per-head RMSNorm weights (null = no norm)
     const float* rms_k[2];
+    bool out_pieces = false;  // fp32 kernel, heads of 64 or 128: the outputs as matrices of bf16 pieces (pieces.hpp) of ld_out columns
 };
 int attention_f32(const AttnSegments& s, int B, int NH, int HS, hipStream_t st);
 extern int g_attention_f32_no_pieces;

@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "pieces.hpp"
 
 namespace sd3 {
 
@@ -267,28 +268,75 @@ struct Dims {
     bool dual, qk, discard;
 };
 
-size_t block_workspace_bytes(const Dims& d, int prec) {
+// fp32: which operands of a block's products are written as bf16 pieces by what produces them (pieces.hpp), six bytes a value, so that the products'
+// workgroups need not split them, each for itself. Results are the same bits either way.
+struct Pieces {
+    bool rows = false;    // LayerNorm's outputs, for q|k|v and the first MLP layers
+    bool att = false;     // attention's outputs, for the out-projections
+    bool hidden = false;  // the first MLP layers' outputs, for the second ones
+    static size_t bytes(bool pieces, size_t M, size_t K) { return pieces ? pieces_bytes(M, K) : M * K * 4; }
+};
+// Where the kernels take them (by depths, widths and the weights' addresses) and where it pays. By rows x width, us of a block without | with LayerNorm's outputs in pieces | all
+// three, width 1536: 333 rows 259 | 257 | 266, 560 317 | 316 | 320, 700 442 | 397 | 397, 900 510 | 475 | 475, 1178 561 | 535 | 535, 4250 2226 | 2146 | 1935; 768: 450 119 | 122 | 124, 1178 202 |
+// 202 | 207, 16 x 666 1237 | 1200 | 1156; the forward at 512px (1178 rows of 1536) 15400 | 14140 | 14020.
+Pieces pieces_of(const Dims& d, int prec, const sd3_block_weights& w) {
+    Pieces p;
+    const double values = (double)d.B * (d.Tc + d.Tx) * d.C;  // of a layer of the block's width
+    if (is_bf(prec) || values < 1.0e6) return p;
+    const int C = d.C, H = d.E * d.C;
+    auto takes = [](const float* W, int K, int N) { return !W || gemm_f32_takes_a_pieces(W, N, 0, N, K); };
+    // (wider rows take LayerNorm's element-wise kernel)
+    p.rows = C <= 3072 && takes(w.c_qkv_w, C, 3 * C) && takes(w.x_qkv_w, C, 3 * C) && takes(w.x2_qkv_w, C, 3 * C) && takes(w.c_mlp_w1, C, H) && takes(w.x_mlp_w1, C, H);
+    if (!p.rows || values < 1.7e6) return p;
+    p.att = (d.HS == 64 || d.HS == 128) && takes(w.c_out_w, C, C) && takes(w.x_out_w, C, C) && takes(w.x2_out_w, C, C);
+    p.hidden = takes(w.c_mlp_w2, H, C) && takes(w.x_mlp_w2, H, C);
+    return p;
+}
+
+size_t block_workspace_bytes(const Dims& d, int prec, Pieces pieces = {}) {
     Bump b(nullptr, 0);
     const size_t es = is_bf(prec) ? 2 : 4;
     const size_t mc = (size_t)d.B * d.Tc, mx = (size_t)d.B * d.Tx;
     auto act = [&](size_t n) { b.take<char>(n * es); };
+    auto rows = [&](size_t m) { b.take<char>(is_bf(prec) ? m * d.C * 2 : Pieces::bytes(pieces.rows, m, d.C)); };
+    auto att = [&](size_t m) { b.take<char>(is_bf(prec) ? m * d.C * 2 : Pieces::bytes(pieces.att, m, d.C)); };
+    auto hidden = [&](size_t m) { b.take<char>(is_bf(prec) ? m * d.E * d.C * 2 : Pieces::bytes(pieces.hidden, m, (size_t)d.E * d.C)); };
     if (fp8_kind(prec)) {  // fp8 copies of the MLP inputs and one factor per row
         b.take<char>(mc * d.E * d.C); b.take<char>(mx * d.E * d.C);
         b.take<float>(mc); b.take<float>(mx);
     }
-    act(mc * d.C); act(mx * d.C); act(mx * d.C);           // c_hid, x_hid, x_hid2
+    rows(mc); rows(mx); rows(mx);                          // c_hid, x_hid, x_hid2
     act(mc * 3 * d.C); act(mx * 3 * d.C);                  // c_qkv, x_qkv
     if (d.dual) act(mx * 3 * d.C);                         // x_qkv2
-    act(mc * d.C); act(mx * d.C);                          // c_att, x_att
+    att(mc); att(mx);                                      // c_att, x_att
     if (is_bf(prec)) {
         if (d.dual) act(mx * d.C);                         // x_att2: both attentions of a dual block run in one launch
         // (a forward's blocks share one layout: room for the split of either kind of block)
         const int S = std::max(attention_bf16_context_splits(d.Tc, d.Tx, d.NH, false), attention_bf16_context_splits(d.Tc, d.Tx, d.NH, true));
         if (S) b.take<float>(attention_bf16_split_workspace_floats(d.B, d.NH, d.Tc, S));
     }
-    act(mc * d.E * d.C); act(mx * d.E * d.C);              // c_mlp, x_mlp
+    hidden(mc); hidden(mx);                                // c_mlp, x_mlp
     b.take<float>((size_t)d.B * 6 * d.C); b.take<float>((size_t)d.B * 9 * d.C);  // ada_c, ada_x
     return b.off;
+}
+
+// Room for `front` bytes and a block's intermediates behind them. Operands in pieces are larger: where they don't fit, in a capture that what there is would do for or for lack of
+// memory, *pieces becomes none.
+int ensure_block_workspace(sd3_ctx* ctx, size_t front, const Dims& d, int prec, Pieces* pieces) {
+    const size_t plain = front + block_workspace_bytes(d, prec), bytes = front + block_workspace_bytes(d, prec, *pieces);
+    if (bytes == plain || bytes <= ctx->ws_bytes) return ensure_workspace(ctx, bytes);
+    if (plain <= ctx->ws_bytes) {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            *pieces = Pieces{};
+            return SD3_OK;
+        }
+    }
+    const int rc = ensure_workspace(ctx, bytes);
+    if (rc != SD3_ERR_OOM) return rc;
+    *pieces = Pieces{};
+    return ensure_workspace(ctx, plain);
 }
 
 // One linear layer: out = epilogue(A @ W + b). fp32: W used in place; bf16: the packed copy.
@@ -316,6 +364,7 @@ struct LayerCall {
     void* out;
     int ldc, M, N, K;
     GemmEpilogueArgs ea;
+    bool a_pieces = false, out_pieces = false;  // fp32 (GemmF32Problem)
 };
 int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f32, int epi, const LayerCall* then = nullptr, AdaCarry* carry = nullptr) {
     if (n > 3) return fail(SD3_ERR_INVALID_ARG, "linear_pair: at most three layers per group");
@@ -329,6 +378,8 @@ int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f
             if (!c.W) return fail(SD3_ERR_MISSING_PARAM, "a weight needed by this configuration is not bound (N=%d K=%d)", c.N, c.K);
             probs[m] = GemmF32Problem{(const float*)c.A, c.W, (float*)c.out, c.K, c.N, 0, c.ldc, c.M, c.N, c.K, c.ea};
             probs[m].ea.bias = c.bias;
+            probs[m].a_pieces = c.a_pieces;
+            probs[m].out_pieces = c.out_pieces;
             flop += 2.0 * c.M * c.N * c.K;
             m++;
         }
@@ -402,15 +453,15 @@ int ln_mod(sd3_ctx* ctx, const float* x, void* out, void* out2, const float* shi
 }
 
 // The LayerNorms of the latent and of the context stream at the same point of the block: one launch
-int ln_mod_pair(sd3_ctx* ctx, const LayerNormJob* jobs, int n, float eps, int C, int bf) {
+int ln_mod_pair(sd3_ctx* ctx, const LayerNormJob* jobs, int n, float eps, int C, LayerNormOut out) {
     double bytes = 0;
     for (int i = 0; i < n; i++) {
         const double e = (double)jobs[i].B * jobs[i].T * C;
-        bytes += e * 4 + e * (bf ? 2 : 4) * (jobs[i].out2 ? 2 : 1);
+        bytes += e * 4 + e * (out == LN_BF16 ? 2 : out == LN_PIECES ? 6 : 4) * (jobs[i].out2 ? 2 : 1);
     }
     if (bytes == 0) return SD3_OK;
     ProfScope ps(ctx, SD3_PROF_LAYERNORM, bytes);
-    return layernorm_modulate_pair(jobs, n, eps, C, bf, ctx->stream);
+    return layernorm_modulate_pair(jobs, n, eps, C, out, ctx->stream);
 }
 
 int attention(sd3_ctx* ctx, const AttnSegments& a, int B, int NH, int HS, bool bf) {
@@ -425,7 +476,7 @@ struct AheadWeight {
 };
 // The block. ada_c / ada_x: modulation vectors (B, chunks*C) already computed, or null to compute them here. carry, next (the block behind
 // this one): what its GEMM launches take along, see carried_wgs.
-int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const sd3_block_weights& w, const Dims& d, const float* ada_c,
+int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const sd3_block_weights& w, const Dims& d, Pieces pieces, const float* ada_c,
               const float* ada_x, Bump& ws, AdaCarry* carry = nullptr, const sd3_block_weights* next = nullptr, bool next_dual = false) {
     hipStream_t st = ctx->stream;
     const int B = d.B, Tc = d.Tc, Tx = d.Tx, C = d.C;
@@ -434,22 +485,26 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     const bool bf = is_bf(prec);
     const int f8 = fp8_kind(prec);
     const size_t es = bf ? 2 : 4;
+    const LayerNormOut ln_out = bf ? LN_BF16 : pieces.rows ? LN_PIECES : LN_F32;
     const bool in_forward = ada_c && ada_x;  // one of many blocks: its weights have long left the caches
     auto act = [&](size_t n) -> void* { return ws.take<char>(n * es); };
+    auto rows = [&](size_t m) -> void* { return ws.take<char>(bf ? m * C * 2 : Pieces::bytes(pieces.rows, m, C)); };
+    auto att = [&](size_t m) -> void* { return ws.take<char>(bf ? m * C * 2 : Pieces::bytes(pieces.att, m, C)); };
+    auto hidden = [&](size_t m) -> void* { return ws.take<char>(bf ? m * d.E * C * 2 : Pieces::bytes(pieces.hidden, m, (size_t)d.E * C)); };
     uint8_t *cq = nullptr, *xq = nullptr;
     float *cs = nullptr, *xs = nullptr;
     if (f8) {
         cq = ws.take<uint8_t>((size_t)mc * d.E * C); xq = ws.take<uint8_t>((size_t)mx * d.E * C);
         cs = ws.take<float>((size_t)mc); xs = ws.take<float>((size_t)mx);
     }
-    void* c_hid = act((size_t)mc * C);
-    void* x_hid = act((size_t)mx * C);
-    void* x_hid2 = act((size_t)mx * C);
+    void* c_hid = rows(mc);
+    void* x_hid = rows(mx);
+    void* x_hid2 = rows(mx);
     void* c_qkv = act((size_t)mc * 3 * C);
     void* x_qkv = act((size_t)mx * 3 * C);
     void* x_qkv2 = d.dual ? act((size_t)mx * 3 * C) : nullptr;  // q,k,v of the extra self-attention branch
-    void* c_att = act((size_t)mc * C);
-    void* x_att = act((size_t)mx * C);
+    void* c_att = att(mc);
+    void* x_att = att(mx);
     void* x_att2 = x_att;  // output of the extra self-attention (bf16 path: a buffer of its own, the two attentions share a launch)
     float* split_ws = nullptr;
     const int ctx_splits = is_bf(prec) ? attention_bf16_context_splits(Tc, Tx, d.NH, d.dual) : 0;
@@ -457,8 +512,8 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         if (d.dual) x_att2 = act((size_t)mx * C);
         if (ctx_splits) split_ws = ws.take<float>(attention_bf16_split_workspace_floats(B, d.NH, Tc, ctx_splits));
     }
-    void* c_mlp = act((size_t)mc * d.E * C);
-    void* x_mlp = act((size_t)mx * d.E * C);
+    void* c_mlp = hidden(mc);
+    void* x_mlp = hidden(mx);
     float* ada_c_buf = ws.take<float>((size_t)B * 6 * C);
     float* ada_x_buf = ws.take<float>((size_t)B * 9 * C);
 
@@ -505,7 +560,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         const LayerNormJob ln1[2] = {{x, x_hid, d.dual ? x_hid2 : nullptr, xchunk(0), xchunk(1), d.dual ? xchunk(6) : nullptr, d.dual ? xchunk(7) : nullptr,
                                       ldx_ada, B, Tx},
                                      {c, c_hid, nullptr, c_shift, c_scale, nullptr, nullptr, ldc_ada, B, Tc}};
-        SD3_TRY(ln_mod_pair(ctx, ln1, 2, 1e-6f, C, bf));
+        SD3_TRY(ln_mod_pair(ctx, ln1, 2, 1e-6f, C, ln_out));
     }
     {
         // bf16 path: the per-head RMSNorm of q and k (modules.cpp:1396-1399, 1420-1423) runs in the projection's epilogue, on the
@@ -517,9 +572,9 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         GemmEpilogueArgs n2;
         n2.gate = w.x2_rms_q; n2.resid = w.x2_rms_k;
         // the dual branch's projection reads the other output of the same LayerNorm pass: same kind, same launch
-        LayerCall qkv[3] = {{x_hid, w.x_qkv_w, w.x_qkv_b, x_qkv, 3 * C, mx, 3 * C, C, fused_norm ? nx : none},
-                            {x_hid2, w.x2_qkv_w, w.x2_qkv_b, x_qkv2, 3 * C, d.dual ? mx : 0, 3 * C, C, fused_norm ? n2 : none},
-                            {c_hid, w.c_qkv_w, w.c_qkv_b, c_qkv, 3 * C, mc, 3 * C, C, fused_norm ? nc : none}};
+        LayerCall qkv[3] = {{x_hid, w.x_qkv_w, w.x_qkv_b, x_qkv, 3 * C, mx, 3 * C, C, fused_norm ? nx : none, pieces.rows},
+                            {x_hid2, w.x2_qkv_w, w.x2_qkv_b, x_qkv2, 3 * C, d.dual ? mx : 0, 3 * C, C, fused_norm ? n2 : none, pieces.rows},
+                            {c_hid, w.c_qkv_w, w.c_qkv_b, c_qkv, 3 * C, mc, 3 * C, C, fused_norm ? nc : none, pieces.rows}};
         SD3_TRY(linear_pair(ctx, prec, qkv, 3, !bf, fused_norm ? EPI_QKV_NORM : EPI_BIAS, nullptr, carry));
     }
 
@@ -530,6 +585,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         SD3_TRY(qk_norm_rows(norms, d.dual ? 3 : 2, 1e-6f, d.NH, d.HS, 3 * C, st));
     }
     AttnSegments joint{}, dual_set{};
+    joint.out_pieces = dual_set.out_pieces = pieces.att;
     joint.q[0] = c_qkv; joint.k[0] = seg_ptr(c_qkv, 1); joint.v[0] = seg_ptr(c_qkv, 2); joint.out[0] = d.discard ? nullptr : c_att;
     joint.q[1] = x_qkv; joint.k[1] = seg_ptr(x_qkv, 1); joint.v[1] = seg_ptr(x_qkv, 2); joint.out[1] = x_att;
     joint.ld_qkv[0] = joint.ld_qkv[1] = 3 * C; joint.ld_out[0] = joint.ld_out[1] = C;
@@ -597,7 +653,8 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     gc.rows_per_batch = Tc; gc.gate = cchunk(2); gc.gate_ld = ldc_ada; gc.resid = c;
     gx.rows_per_batch = Tx; gx.gate = xchunk(2); gx.gate_ld = ldx_ada; gx.resid = x;
     {
-        LayerCall proj[2] = {{x_att, w.x_out_w, w.x_out_b, x, C, mx, C, C, gx}, {c_att, w.c_out_w, w.c_out_b, c, C, d.discard ? 0 : mc, C, C, gc}};
+        LayerCall proj[2] = {{x_att, w.x_out_w, w.x_out_b, x, C, mx, C, C, gx, pieces.att},
+                             {c_att, w.c_out_w, w.c_out_b, c, C, d.discard ? 0 : mc, C, C, gc, pieces.att}};
         // with dual attention, bf16: the second projection of the latent rows (modules.cpp:1450-1453, 1486) rides behind the first, in its launch
         GemmEpilogueArgs g2;
         g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;
@@ -611,7 +668,8 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         SD3_TRY(attention(ctx, dual_set, B, d.NH, d.HS, bf));
         GemmEpilogueArgs g2;
         g2.rows_per_batch = Tx; g2.gate = xchunk(8); g2.gate_ld = ldx_ada; g2.resid = x;
-        SD3_TRY(linear_layer(ctx, prec, x_att2, w.x2_out_w, w.x2_out_b, x, 1, C, mx, C, C, EPI_GATE_RESID, g2));
+        const LayerCall proj2{x_att2, w.x2_out_w, w.x2_out_b, x, C, mx, C, C, g2, pieces.att};
+        SD3_TRY(linear_pair(ctx, prec, &proj2, 1, 1, EPI_GATE_RESID));
     }
 
     // ---- MLPs of both streams (modules.cpp:1463-1476, 1488-1504)
@@ -619,7 +677,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
     {
         const LayerNormJob ln2[2] = {{x, x_hid, nullptr, xchunk(3), xchunk(4), nullptr, nullptr, ldx_ada, B, Tx},
                                      {c, c_hid, nullptr, cchunk(3), cchunk(4), nullptr, nullptr, ldc_ada, B, d.discard ? 0 : Tc}};
-        SD3_TRY(ln_mod_pair(ctx, ln2, 2, 1e-6f, C, bf));
+        SD3_TRY(ln_mod_pair(ctx, ln2, 2, 1e-6f, C, ln_out));
     }
     if (f8) {
         // fp8 MLPs: the inputs of both layers are quantised row by row (one factor per token), the weights column by column (one
@@ -660,13 +718,13 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         return SD3_OK;
     }
     {
-        LayerCall up[2] = {{x_hid, w.x_mlp_w1, w.x_mlp_b1, x_mlp, d.E * C, mx, d.E * C, C, none},
-                           {c_hid, w.c_mlp_w1, w.c_mlp_b1, c_mlp, d.E * C, mcm, d.E * C, C, none}};
+        LayerCall up[2] = {{x_hid, w.x_mlp_w1, w.x_mlp_b1, x_mlp, d.E * C, mx, d.E * C, C, none, pieces.rows, pieces.hidden},
+                           {c_hid, w.c_mlp_w1, w.c_mlp_b1, c_mlp, d.E * C, mcm, d.E * C, C, none, pieces.rows, pieces.hidden}};
         SD3_TRY(read_ahead_of({{w.x_mlp_w2, d.E * C, C}, {mcm ? w.c_mlp_w2 : nullptr, d.E * C, C}}));
         SD3_TRY(linear_pair(ctx, prec, up, 2, !bf, EPI_BIAS_GELU, nullptr, carry));
         gc.gate = cchunk(5);
         gx.gate = xchunk(5);
-        LayerCall down[2] = {{x_mlp, w.x_mlp_w2, w.x_mlp_b2, x, C, mx, C, d.E * C, gx}, {c_mlp, w.c_mlp_w2, w.c_mlp_b2, c, C, mcm, C, d.E * C, gc}};
+        LayerCall down[2] = {{x_mlp, w.x_mlp_w2, w.x_mlp_b2, x, C, mx, C, d.E * C, gx, pieces.hidden}, {c_mlp, w.c_mlp_w2, w.c_mlp_b2, c, C, mcm, C, d.E * C, gc, pieces.hidden}};
         if (carry) carry->last = true;
         if (next) SD3_TRY(read_ahead_of({{next->x_qkv_w, C, 3 * C}, {mc ? next->c_qkv_w : nullptr, C, 3 * C}, {next_dual ? next->x2_qkv_w : nullptr, C, 3 * C}}));
         SD3_TRY(linear_pair(ctx, prec, down, 2, 1, EPI_GATE_RESID, nullptr, carry));
@@ -1082,9 +1140,10 @@ int sd3_dit_block_w(sd3_ctx* ctx, const float* y, float* c, float* x, const sd3_
     DeviceGuard g(ctx->device);
     if (!g.ok) return fail(SD3_ERR_HIP, "cannot select device %d", ctx->device);
     OrderScope order(ctx);
-    SD3_TRY(ensure_workspace(ctx, block_workspace_bytes(d, precision)));
+    Pieces pieces = pieces_of(d, precision, *w);
+    SD3_TRY(ensure_block_workspace(ctx, 0, d, precision, &pieces));
     Bump ws(ctx->ws, ctx->ws_bytes);
-    return run_block(ctx, precision, y, c, x, *w, d, nullptr, nullptr, ws);
+    return run_block(ctx, precision, y, c, x, *w, d, pieces, nullptr, nullptr, ws);
 }
 
 int sd3_dit_block(sd3_ctx* ctx, const float* y, float* c, float* x, const char* prefix, int B, int Tc, int Tx, int emb_dim, int attn_heads, int mlp_expand,
@@ -1120,7 +1179,9 @@ int sd3_dit_block_static(sd3_ctx* ctx, const float* y, float* c, float* x, const
     OrderScope order(ctx);  // (records an event that exists since the context was created: no allocation)
     Bump ws(ctx->static_scratch, SD3_STATIC_SCRATCH_BYTES);
     ctx->no_alloc = true;
-    const int rc = run_block(ctx, precision, y, c, x, w, d, nullptr, nullptr, ws);
+    Pieces pieces = pieces_of(d, precision, w);
+    if (block_workspace_bytes(d, precision, pieces) > (size_t)SD3_STATIC_SCRATCH_BYTES) pieces = Pieces{};  // (the same results, a little later)
+    const int rc = run_block(ctx, precision, y, c, x, w, d, pieces, nullptr, nullptr, ws);
     ctx->no_alloc = false;
     return rc;
 }
@@ -1203,7 +1264,16 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     void *cap_in, *patches;
     Bump probe(nullptr, 0);
     layout(probe, &temb, &h1, &h2, &yt, &yp, &y, &c, &x, &cap_in, &patches, &ada_all, &ada_out, &tokens);
-    SD3_TRY(ensure_workspace(ctx, probe.off + block_workspace_bytes(dmax, precision)));
+    std::vector<Pieces> pieces(num_layers);
+    Pieces any;
+    for (int l = 0; l < num_layers; l++) {
+        pieces[l] = pieces_of(bd[l], precision, bw[l]);
+        any.rows |= pieces[l].rows;
+        any.att |= pieces[l].att;
+        any.hidden |= pieces[l].hidden;
+    }
+    SD3_TRY(ensure_block_workspace(ctx, probe.off, dmax, precision, &any));
+    if (!any.rows) pieces.assign(num_layers, Pieces{});
     Bump ws(ctx->ws, ctx->ws_bytes);
     layout(ws, &temb, &h1, &h2, &yt, &yp, &y, &c, &x, &cap_in, &patches, &ada_all, &ada_out, &tokens);
     const size_t block_ws_off = ws.off;
@@ -1301,7 +1371,7 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
                 carry.total += q.N / 64;
             }
         }
-        SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], base, base + (size_t)B * 6 * C, bws, few_rows ? &carry : nullptr, l + 1 < num_layers ? &bw[l + 1] : nullptr, l + 1 < num_layers && bd[l + 1].dual));
+        SD3_TRY(run_block(ctx, precision, y, c, x, bw[l], bd[l], pieces[l], base, base + (size_t)B * 6 * C, bws, few_rows ? &carry : nullptr, l + 1 < num_layers ? &bw[l + 1] : nullptr, l + 1 < num_layers && bd[l + 1].dual));
         if (carry.left() > 0) {  // what no launch had room for
             std::vector<AdaJob> rest;
             int skip = carry.work.first;

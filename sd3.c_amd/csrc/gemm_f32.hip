@@ -144,10 +144,11 @@ __global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__
 // consecutive columns NJ*(l%16) .. of its k row, one for each of its NJ column blocks, so column block j holds columns NJ*c + j and
 // a lane ends with NJ consecutive columns of a row: the epilogue stores straight from the accumulators, 16 lanes covering 16*NJ columns.
 struct TileProb {
-    const float* A;
+    const float* A;  // (A in pieces: a matrix of them, pieces.hpp)
     const float* W;
     float* out;
     int lda, ldw, ldc, M, N, K, n0;
+    bool out_pieces;  // EPI_BIAS_GELU: a matrix of pieces of ldc columns
     EpiDev epi;
 };
 constexpr int MAX_PROBS = 3;
@@ -188,8 +189,8 @@ __device__ __forceinline__ void store_cols(float* p, const float (&v)[NJ]) {
 // m0: the lane's first row, n: its first column. Everything that is to be read is requested before the first store and waited for together: row by row, each behind the other's store,
 // 16 rows were 16 trips to memory. With the gate, 10656 x 768 x 768: tiles of 128x128 93 -> 84 us, of
 // 64x64 132 -> 116; 333 x 1536 x 1536 25.7 -> 23.5.
-// LEAN: row by row all the same, for the 256x128 tiles of the kernel that splits A itself, whose K loop spills registers beside anything else (K = 6144 370 -> 486 us).
-template <int TI, int NJ, int EPI, bool LEAN = false>
+// LEAN: row by row all the same, for the 256x128 tiles of the kernel that splits A itself, whose K loop spills registers beside anything else (K = 6144 370 -> 486 us). PIECES: the output may be one of pieces.
+template <int TI, int NJ, int EPI, bool PIECES, bool LEAN = false>
 __device__ __forceinline__ void store_tile(const TileProb& pr, const f32x4_t (&acc)[TI][NJ], int m0, int n) {
     asm volatile("" : "+v"(m0), "+v"(n));  // (or addresses are formed in front of the K loop and held through it)
     const int m_wave = __builtin_amdgcn_readfirstlane(m0) & ~15;  // the wavefront's first row
@@ -202,6 +203,31 @@ __device__ __forceinline__ void store_tile(const TileProb& pr, const f32x4_t (&a
 #pragma unroll
         for (int j = 0; j < NJ; j++) asm volatile("" : "+v"(v[j]));
     };
+    if constexpr (EPI == EPI_BIAS_GELU && PIECES) {
+        if (pr.out_pieces) {
+            // Rows m0 + 16 i + r, m0 = 4(l/16) mod 16: the places of a block's rows in 32-bit offsets, the blocks in a scalar address (a 64-bit address for every
+            // store and plane costs more than the split)
+            const PieceMatrix to(pr.out, pr.M, pr.ldc);
+            const unsigned at[2] = {(unsigned)piece_index(m0 & 15, n, to.K) * 2, (unsigned)(piece_index((m0 & 15) + 2, n, to.K) - 64) * 2};
+            arrived(bias);
+#pragma unroll
+            for (int i = 0; i < TI; i++) {
+                char* const block = reinterpret_cast<char*>(to.p) + (long long)(m_wave / 16 + i) * to.K * 32;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    float v[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) v[j] = gelu_tanh_precise(acc[i][j][r] + bias[j]);
+                    uint32_t piece[3][(NJ + 1) / 2];
+                    pieces_for_memory<NJ>(v, piece);
+                    if (m0 + i * 16 + r < pr.M)
+#pragma unroll
+                        for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(block + p * to.plane * 2 + at[r / 2] + r * 64, NJ * 2), piece[p], NJ * 2);
+                }
+            }
+            return;
+        }
+    }
     const int rpb = e.rows_per_batch;
     // Rows of at most two batch elements, as all but those of very few rows: a gate for each
     const int b_first = EPI == EPI_GATE_RESID ? m_wave / rpb : 0, b_last = EPI == EPI_GATE_RESID ? min(m_wave + TI * 16 - 1, pr.M - 1) / rpb : 0;
@@ -461,7 +487,7 @@ __global__ void __launch_bounds__(WM* WN * 64, 2) gemm_f32_tile_kernel(const Til
         spread(std::true_type{});
     }
     wait_vmcnt<0>();  // no direct load may still be on its way into this workgroup's LDS when it ends
-    store_tile<TI, NJ, EPI>(pr, acc, m_blk + wm * (TM / WM) + 4 * lg, n_blk + wn * (TN / WN) + NJ * lr);
+    store_tile<TI, NJ, EPI, false>(pr, acc, m_blk + wm * (TM / WM) + 4 * lg, n_blk + wn * (TN / WN) + NJ * lr);
 }
 
 template <int TM, int TN, int WM, int WN, int STAGES, int EPI, bool WHOLE_K>
@@ -530,9 +556,9 @@ int launch_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
 // of A read 64 contiguous bytes at a time (3 % at 256x128). Columns of W are assigned to lanes as in the tile kernel.
 
 // A wavefront that fetches operands and writes their pieces: per thread and K tile CA runs of H k values of rows of A and CW ones of columns of W, by PT threads
-template <int TM, int TN, int NJ, int CA, int CW, int H, int PT, int SETS, int GROUP>
+template <int TM, int TN, int NJ, int CA, int CW, int H, int PT, int SETS, int GROUP, int W_AT = TM * 192, int STAGE_BYTES = (TM + TN) * 192>
 __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, int n_blk, int nkt, unsigned tid, char* smem) {
-    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE), WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H;
     static_assert((H == 8 || H == 4) && (CA == 0 || CA * PT == TM * RUNS) && (CW == 0 || CW * PT == TN * RUNS) && CW <= 2, "shares of a K tile");
     unsigned a_off[CA + 1], w_off[H], a_dst[CA + 1], w_dst[CW + 1];
 #pragma unroll
@@ -548,7 +574,7 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
 #pragma unroll
         for (int x = 0; x < CW; x++) {
             const unsigned cc = c + x, in = cc % (16 * NJ);
-            w_dst[x] = 3 * A_PLANE + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 4 % 4) + k0 / 16 * 8;
+            w_dst[x] = W_AT + piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 4 % 4) + k0 / 16 * 8;
         }
     }
     const char* a_tile = reinterpret_cast<const char*>(pr.A + (long long)m_blk * pr.lda);
@@ -630,12 +656,184 @@ __device__ __forceinline__ void produce_pieces(const TileProb& pr, int m_blk, in
     wait_vmcnt<0>();
 }
 
+// Where what produces A has written its pieces (TileProb::A) they go from memory to LDS by direct loads, requested by PA wavefronts: a ring of RING K tiles (whole pairs of groups),
+// RING - GROUP of them ahead.
+template <int TM, int PA, int GROUP, int RING>
+__device__ __forceinline__ void request_a_pieces(const TileProb& pr, int m_blk, int nkt, unsigned tid, char* smem) {
+    constexpr int A_STAGE = TM * 192, REQUESTS = A_STAGE / 1024, LA = (REQUESTS + PA - 1) / PA;  // direct loads of a K tile: all wavefronts' and one's
+    static_assert(RING % (2 * GROUP) == 0 && (RING / GROUP - 1) * GROUP * LA < 64, "whole rounds, and the requests in flight must fit the 6-bit counter");
+    const unsigned lane = tid & 63, block_row = (unsigned)pr.K * 32;
+    const long long plane_bytes = (pr.M + 15) / 16 * (long long)block_row;
+    const unsigned wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    unsigned off[LA], dst[LA];
+    long long plane_at[LA];
+#pragma unroll
+    for (int i = 0; i < LA; i++) {
+        // request q: a plane of a block. (Where the requests do not divide evenly, several wavefronts make the last one.)
+        const unsigned q = min(i * PA + wave, (unsigned)REQUESTS - 1), block = q / 3, plane = q % 3;
+        off[i] = min(block, (unsigned)(pr.M - 1 - m_blk) / 16) * block_row + lane * 16;  // blocks beyond M re-read the last one and are never stored
+        plane_at[i] = plane * plane_bytes;
+        dst[i] = plane * (TM * 64) + block * 1024;
+    }
+    const char* tile = reinterpret_cast<const char*>(pr.A) + (m_blk / 16) * (long long)block_row;
+    int next = 0;
+    unsigned slot = 0;
+    auto request = [&]() {  // the next K tile; past the end the last one once more, into a stage that nobody reads again
+#pragma unroll
+        for (int i = 0; i < LA; i++) {
+            asm volatile("" : "+v"(off[i]));
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(tile + plane_at[i] + off[i]), (lds_ptr_t)(smem + dst[i] + slot), 16, 0, 0);
+        }
+        next++;
+        tile += next < nkt ? 1024 : 0;
+        slot = slot == (RING - 1) * A_STAGE ? 0 : slot + A_STAGE;
+    };
+    auto publish = []() {  // all but the groups that are requested ahead of the one to publish
+        wait_vmcnt<(RING / GROUP - 2) * GROUP * LA>();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int t = 0; t < RING - GROUP; t++) request();
+    publish();
+    for (int kt = 0; kt < nkt; kt += GROUP) {
+#pragma unroll
+        for (int t = 0; t < GROUP; t++) request();  // into the stages that the last barrier has freed
+        publish();
+    }
+    wait_vmcnt<0>();  // no direct load may still be on its way into this workgroup's LDS when it ends
+}
+
+// LDS writes as assembly: behind direct loads into LDS the compiler has every write that it knows of wait for all of them (publish() waits for these)
+__device__ __forceinline__ void write_lds(char* at, const uint32_t (&v)[4]) {
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    asm volatile("ds_write_b128 %0, %1" ::"v"((uint32_t)(uintptr_t)(lds_ptr_t)at), "v"(u32x4_t{v[0], v[1], v[2], v[3]}) : "memory");
+}
+__device__ __forceinline__ void write_lds(char* at, const uint32_t (&v)[2]) {
+    asm volatile("ds_write_b64 %0, %1" ::"v"((uint32_t)(uintptr_t)(lds_ptr_t)at), "v"((unsigned long long)v[1] << 32 | v[0]) : "memory");
+}
+// Both by the same PT threads: the requests of A's pieces, and W's split.
+template <int TM, int TN, int NJ, int CW, int H, int PT, int SETS, int GROUP, int RING>
+__device__ __forceinline__ void produce_with_a_pieces(const TileProb& pr, int m_blk, int n_blk, int nkt, unsigned tid, char* smem) {
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, W_STAGE = 3 * B_PLANE, A_STAGE = 3 * A_PLANE, WMULT = NJ == 2 ? 2 : 1, RUNS = TK / H, PW = PT / 64;
+    constexpr int REQUESTS = A_STAGE / 1024, LA = (REQUESTS + PW - 1) / PW;  // direct loads of a K tile: all wavefronts' and one's
+    static_assert((H == 8 || H == 4) && CW * PT == TN * RUNS && CW <= 2 && SETS % GROUP == 0 && RING % (2 * GROUP) == 0, "shares of a K tile");
+    const unsigned lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const unsigned block_row = (unsigned)pr.K * 32;
+    const long long plane_bytes = (pr.M + 15) / 16 * (long long)block_row;
+    unsigned a_off[LA], a_dst[LA], w_off[H], w_dst[CW];
+    long long plane_at[LA];
+#pragma unroll
+    for (int i = 0; i < LA; i++) {
+        const unsigned q = min(i * PW + wave, REQUESTS - 1), block = q / 3, plane = q % 3;
+        a_off[i] = min(block, (unsigned)(pr.M - 1 - m_blk) / 16) * block_row + lane * 16;
+        plane_at[i] = plane * plane_bytes;
+        a_dst[i] = 2 * GROUP * W_STAGE + plane * A_PLANE + block * 1024;
+    }
+    const unsigned c = tid % (TN / CW) * CW, k0 = tid / (TN / CW) * 4;
+#pragma unroll
+    for (int k = 0; k < H; k++) w_off[k] = ((k0 + k % 4 + k / 4 * 16) * pr.ldw + min(n_blk + c, (unsigned)(pr.N - CW))) * 4;
+#pragma unroll
+    for (int x = 0; x < CW; x++) {
+        const unsigned cc = c + x, in = cc % (16 * NJ);
+        w_dst[x] = piece_slot<WMULT>(cc / (16 * NJ) * (16 * NJ) + in % NJ * 16 + in / NJ, k0 / 4 % 4) + k0 / 16 * 8;
+    }
+    const char* a_tile = reinterpret_cast<const char*>(pr.A) + (m_blk / 16) * (long long)block_row;
+    const char* w_tile = reinterpret_cast<const char*>(pr.W + pr.n0);
+    const long long w_step = (long long)pr.ldw * 4 * TK;
+    float rw[SETS][H][CW];
+    int w_next = 0, a_next = 0;  // the K tiles that the addresses are at
+    unsigned a_slot = 0;         // and where in the ring
+    // requests of the next K tile; past the end the last one once more, into a stage that nobody reads again
+    auto request_a = [&]() {
+#pragma unroll
+        for (int i = 0; i < LA; i++) {
+            asm volatile("" : "+v"(a_off[i]));
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(a_tile + plane_at[i] + a_off[i]), (lds_ptr_t)(smem + a_dst[i] + a_slot), 16, 0, 0);
+        }
+        a_next++;
+        a_tile += a_next < nkt ? 1024 : 0;
+        a_slot = a_slot == (RING - 1) * A_STAGE ? 0 : a_slot + A_STAGE;
+    };
+    auto request_w = [&](int set) {
+#pragma unroll
+        for (int k = 0; k < H; k++) {
+            asm volatile("" : "+v"(w_off[k]));
+            float t[CW];
+            load_as<typename Cols<CW>::lds>(reinterpret_cast<const float*>(w_tile + w_off[k]), t);
+#pragma unroll
+            for (int x = 0; x < CW; x++) rw[set][k][x] = t[x];
+        }
+        w_next++;
+        w_tile += w_next < nkt ? w_step : 0;
+    };
+    auto stage_w = [&](int set, char* stage) {
+#pragma unroll
+        for (int x = 0; x < CW; x++) {
+            float v[H];
+#pragma unroll
+            for (int k = 0; k < H; k++) v[k] = rw[set][k][x];
+            uint32_t piece[3][H / 2];
+            bf16_pieces<H>(v, piece[0], piece[1], piece[2]);
+#pragma unroll
+            for (int p = 0; p < 3; p++) write_lds(stage + w_dst[x] + p * B_PLANE, piece[p]);
+        }
+        request_w(set);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Everything but the newest NEWER requests of this wavefront has landed, its LDS writes are done; behind the barrier that holds for the others too
+    auto publish = [](auto newer) {
+        constexpr int NEWER = decltype(newer)::value < 63 ? decltype(newer)::value : 63;
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt((NEWER & 15) | (7 << 4) | ((NEWER >> 4) << 14));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    auto fence = []() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr int AHEAD = RING / GROUP - 2;  // groups of K tiles between the one that a round requests and the one it publishes
+#pragma unroll
+    for (int t = 0; t < RING - GROUP; t++) request_a();
+    fence();
+#pragma unroll
+    for (int t = 0; t < SETS; t++) {
+        request_w(t);
+        fence();
+    }
+#pragma unroll
+    for (int t = 0; t < GROUP; t++) stage_w(t, smem + t * W_STAGE);
+    publish(std::integral_constant<int, AHEAD * GROUP * LA + (SETS + GROUP) * H>());
+    for (int kt = 0; kt < nkt; kt += SETS) {
+#pragma unroll
+        for (int t = 0; t < SETS; t++) {
+            if (t % GROUP == 0) {
+#pragma unroll
+                for (int i = 0; i < GROUP; i++) request_a();  // into the stages that the last barrier has freed
+                fence();
+            }
+            stage_w((t + GROUP) % SETS, smem + (t + GROUP) % (2 * GROUP) * W_STAGE);
+            // (newer than the A tiles to publish: the W tiles of the round that requested them and all that the rounds behind it requested; in the first rounds more)
+            if (t % GROUP == GROUP - 1) publish(std::integral_constant<int, GROUP * H + AHEAD * GROUP * (LA + H)>());
+        }
+    }
+    wait_vmcnt<0>();  // no direct load may still be on its way into this workgroup's LDS when it ends
+}
+
 // WM x WN wavefronts multiply; PA fetch and split A and PB W (PB = 0: PA both). GROUP: K tiles per barrier. SETS: K tiles on their way from memory. WAVES: wavefronts
-// per SIMD that the registers are to allow. The depth is made of whole groups of four K tiles.
-template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
+// per SIMD that the registers are to allow. RING: A comes in pieces, in a ring of so many K tiles, which PA request; 0: it does not. The depth
+// is made of whole groups of four K tiles.
+template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int RING, int EPI>
 __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_pieces_kernel(const TileProbSet set) {
     constexpr int TI = TM / WM / 16, NJ = TN / WN / 16, CONSUMERS = WM * WN;
-    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, STAGE_BYTES = 3 * (A_PLANE + B_PLANE);
+    // A stage holds A and W; with RING the W stages come first and A's ring behind them
+    constexpr int A_PLANE = TM * 64, B_PLANE = TN * 64, W_STAGE = 3 * (RING ? B_PLANE : A_PLANE + B_PLANE), A_STAGE = RING ? 3 * A_PLANE : W_STAGE;
+    constexpr int A_AT = RING ? 2 * GROUP * W_STAGE : 0, W_AT = RING ? 0 : 3 * A_PLANE;
     static_assert(TI >= 1 && (NJ == 1 || NJ == 2 || NJ == 4), "tile shape");
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int w = blockIdx.x;
@@ -649,8 +847,12 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
     const int nkt = pr.K / TK;
     if (wave >= CONSUMERS) {
         const unsigned tid = threadIdx.x - CONSUMERS * 64;
-        constexpr int CA = TM * (TK / HA) / (PA * 64), CB = TN * (TK / HB) / ((PB ? PB : PA) * 64);
-        if constexpr (PB == 0) {
+        constexpr int CA = RING ? 0 : TM * (TK / HA) / (PA * 64), CB = TN * (TK / HB) / ((PB ? PB : PA) * 64);
+        if constexpr (RING > 0) {
+            if constexpr (PA == 0) produce_with_a_pieces<TM, TN, NJ, CB, HB, PB * 64, SETS, GROUP, RING>(pr, m_blk, n_blk, nkt, tid, smem);
+            else if (wave < CONSUMERS + PA) request_a_pieces<TM, PA, GROUP, RING>(pr, m_blk, nkt, tid, smem + A_AT);
+            else produce_pieces<TM, TN, NJ, 0, CB, HB, PB * 64, SETS, GROUP, W_AT, W_STAGE>(pr, m_blk, n_blk, nkt, tid - PA * 64, smem);
+        } else if constexpr (PB == 0) {
             produce_pieces<TM, TN, NJ, CA, CB, HA, PA * 64, SETS, GROUP>(pr, m_blk, n_blk, nkt, tid, smem);
         } else {
             if (wave < CONSUMERS + PA) produce_pieces<TM, TN, NJ, CA, 0, HA, PA * 64, SETS, GROUP>(pr, m_blk, n_blk, nkt, tid, smem);
@@ -666,7 +868,7 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     constexpr int WMULT = NJ == 2 ? 2 : 1;
-    const unsigned a_src = piece_slot<0>(wm * (TM / WM) + lr, lg), b_src = 3 * A_PLANE + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
+    const unsigned a_src = A_AT + piece_slot<0>(wm * (TM / WM) + lr, lg), b_src = W_AT + piece_slot<WMULT>(wn * (TN / WN) + lr, lg);
     auto read_a = [&](bf16x8_t (&f)[TI], const char* stage, int plane) {
 #pragma unroll
         for (int i = 0; i < TI; i++) f[i] = *reinterpret_cast<const bf16x8_t*>(stage + plane * A_PLANE + a_src + i * 1024);
@@ -708,10 +910,13 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
     bl = read_b(smem, 2, 0);
 #pragma unroll
     for (int i = 0; i < TI; i++) u[1][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    unsigned ring = 0;  // where in A's ring this round's K tiles begin
     for (int kt = 0; kt < nkt; kt += 2 * GROUP) {
+        const unsigned ring_next = RING > 2 * GROUP ? (ring + 2 * GROUP * A_STAGE) % (RING * A_STAGE) : 0;
 #pragma unroll
         for (int t = 0; t < 2 * GROUP; t++) {
-            const char *cur = smem + t * STAGE_BYTES, *next = smem + (t + 1) % (2 * GROUP) * STAGE_BYTES;
+            const char *cur = smem + t * W_STAGE, *next = smem + (t + 1) % (2 * GROUP) * W_STAGE;
+            const char* const next_a = smem + (t + 1 < 2 * GROUP ? ring + (t + 1) * A_STAGE : ring_next);
 #pragma unroll
             for (int j = 0; j < NJ; j++) {
                 const int p = (t * NJ + j) & 1;
@@ -726,12 +931,12 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
 #pragma unroll
                 for (int i = 0; i < TI; i++) acc[i][(j + NJ - 1) % NJ] += u[p ^ 1][i];
                 spread(One{}, Rows{}, Four{});
-                if (last) read_a(al, next, 2);
+                if (last) read_a(al, next_a, 2);
                 multiply(am, bh[p], u[p]);
                 multiply(am, bm, u[p]);
                 if (last) spread(Rows{}, std::integral_constant<int, 2 * TI>{}, None{});
                 else spread(None{}, std::integral_constant<int, 2 * TI>{}, None{});
-                if (last) read_a(am, next, 1);
+                if (last) read_a(am, next_a, 1);
                 multiply(ah, bm, u[p]);
                 if (last) spread(Rows{}, Rows{}, None{});
                 else spread(None{}, Rows{}, None{});
@@ -741,9 +946,10 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
                 bl = read_b(stage, 2, column);
                 multiply(ah, bh[p], u[p]);
                 spread(One{}, Rows{}, None{});
-                if (last) read_a(ah, next, 0);
+                if (last) read_a(ah, next_a, 0);
             }
         }
+        ring = ring_next;
     }
 #pragma unroll
     for (int i = 0; i < TI; i++) acc[i][NJ - 1] += u[1][i];
@@ -753,25 +959,26 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
         for (int j = 0; j < NJ; j++) acc[i][j] *= 1.0f / (PIECES_SCALE * PIECES_SCALE);
     // A sum that is not finite (values or sums too large for the pieces, infinities, NaNs) is formed anew from the operands themselves
     const int m0 = m_blk + wm * (TM / WM), n0 = n_blk + wn * (TN / WN);
-    auto infinite = [](const f32x4_t& v) {
+    auto infinite = [&](const f32x4_t& v, int i) {  // (rows beyond M may be anything)
         bool bad = false;
 #pragma unroll
-        for (int r = 0; r < 4; r++) bad |= (__float_as_uint(v[r]) & 0x7f800000u) == 0x7f800000u;
+        for (int r = 0; r < 4; r++) bad |= (!RING || m0 + i * 16 + 4 * lg + r < M) && (__float_as_uint(v[r]) & 0x7f800000u) == 0x7f800000u;
         return bad;
     };
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < TI; i++)
 #pragma unroll
-        for (int j = 0; j < NJ; j++) bad |= infinite(acc[i][j]);
+        for (int j = 0; j < NJ; j++) bad |= infinite(acc[i][j], i);
     if (__builtin_amdgcn_ballot_w64(bad)) {
 #pragma unroll
         for (int i = 0; i < TI; i++) {
             bad = false;
 #pragma unroll
-            for (int j = 0; j < NJ; j++) bad |= infinite(acc[i][j]);
+            for (int j = 0; j < NJ; j++) bad |= infinite(acc[i][j], i);
             if (!__builtin_amdgcn_ballot_w64(bad)) continue;
-            const float* pa = pr.A + (long long)min(m0 + i * 16 + lr, M - 1) * pr.lda + lg;
+            const int row = min(m0 + i * 16 + lr, M - 1);
+            const float* pa = pr.A + (long long)row * pr.lda + lg;
             const float* pw = pr.W + (long long)lg * pr.ldw + pr.n0 + min(n0 + NJ * lr, N - NJ);
             f32x4_t sum[NJ];
 #pragma unroll
@@ -782,7 +989,7 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
                     float w[NJ];
                     load_cols<NJ>(pw + step * (long long)pr.ldw, w);
 #pragma unroll
-                    for (int j = 0; j < NJ; j++) sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[step], w[j], sum[j], 0, 0, 0);
+                    for (int j = 0; j < NJ; j++) sum[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(RING ? of_pieces(PieceMatrix(const_cast<float*>(pr.A), M, pr.K), row, k + step + lg) : pa[step], w[j], sum[j], 0, 0, 0);
                 }
 #pragma unroll
             for (int j = 0; j < NJ; j++)
@@ -791,13 +998,13 @@ __global__ void __launch_bounds__((WM * WN + PA + PB) * 64, WAVES) gemm_f32_piec
                     if (!finite(acc[i][j][r])) acc[i][j][r] = sum[j][r];
         }
     }
-    store_tile<TI, NJ, EPI, TI * NJ >= 16>(pr, acc, m0 + 4 * lg, n0 + NJ * lr);
+    store_tile<TI, NJ, EPI, (RING > 0), RING == 0 && TI * NJ >= 16>(pr, acc, m0 + 4 * lg, n0 + NJ * lr);
 }
 
-template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int EPI>
+template <int TM, int TN, int WM, int WN, int PA, int PB, int HA, int HB, int GROUP, int SETS, int WAVES, int RING, int EPI>
 int launch_pieces(TileProbSet& set, int n, hipStream_t st) {
-    auto kern = gemm_f32_pieces_kernel<TM, TN, WM, WN, PA, PB, HA, HB, GROUP, SETS, WAVES, EPI>;
-    constexpr int smem = 2 * GROUP * 3 * (TM + TN) * 64;
+    auto kern = gemm_f32_pieces_kernel<TM, TN, WM, WN, PA, PB, HA, HB, GROUP, SETS, WAVES, RING, EPI>;
+    constexpr int smem = (RING ? RING * TM + 2 * GROUP * TN : 2 * GROUP * (TM + TN)) * 3 * 64;
     static DynamicLds lds;
     SD3_TRY(lds.allow(reinterpret_cast<const void*>(kern), smem));
     int total = 0;
@@ -811,14 +1018,33 @@ int launch_pieces(TileProbSet& set, int n, hipStream_t st) {
 template <int EPI>
 int launch_pieces_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
     switch (shape) {
-        case 0: return launch_pieces<128, 128, 2, 4, 4, 4, 8, 8, 1, 2, 4, EPI>(set, n, st);
-        case 1: return launch_pieces<128, 64, 4, 2, 4, 4, 8, 4, 2, 4, 4, EPI>(set, n, st);
+        case 0: return launch_pieces<128, 128, 2, 4, 4, 4, 8, 8, 1, 2, 4, 0, EPI>(set, n, st);
+        case 1: return launch_pieces<128, 64, 4, 2, 4, 4, 8, 4, 2, 4, 4, 0, EPI>(set, n, st);
         // (columns of W by runs of four: a thread's eight loads, one per k value, were what it spent most time on. 128x64 at 512 rows, K = 1536 31 -> 29 us,
         // 64x64 22.3 -> 20.7, 32x64 17.7 -> 15.4)
-        case 2: return launch_pieces<64, 64, 2, 2, 4, 8, 8, 4, 2, 4, 4, EPI>(set, n, st);
-        case 3: return launch_pieces<32, 64, 2, 2, 4, 8, 4, 4, 2, 4, 4, EPI>(set, n, st);
-        case 4: return launch_pieces<32, 32, 2, 2, 4, 4, 4, 4, 2, 4, 3, EPI>(set, n, st);
-        default: return launch_pieces<256, 128, 4, 2, 4, 0, 8, 8, 1, 2, 3, EPI>(set, n, st);
+        case 2: return launch_pieces<64, 64, 2, 2, 4, 8, 8, 4, 2, 4, 4, 0, EPI>(set, n, st);
+        case 3: return launch_pieces<32, 64, 2, 2, 4, 8, 4, 4, 2, 4, 4, 0, EPI>(set, n, st);
+        case 4: return launch_pieces<32, 32, 2, 2, 4, 4, 4, 4, 2, 4, 3, 0, EPI>(set, n, st);
+        default: return launch_pieces<256, 128, 4, 2, 4, 0, 8, 8, 1, 2, 3, 0, EPI>(set, n, st);
+    }
+}
+
+// A in pieces. What the launch of a layer costs then: two thirds (128x64, 256x128) or half of the splitting is gone, A moves half as many bytes more. us, A split here | A in pieces, cold
+// weights: 1178 x 4608 x 1536 117 | 90, 1178 x 6144 x 1536 with the GELU and its output in pieces 126 | 110, 1178 x 1536 x 1536 44.5 | 39, 1178 x 1536 x 6144 153 | 144, 3226 x 4608 x
+// 1536 240 | 205, 10656 x 768 x 3072 248 | 219, 10656 x 3072 x 768 286 | 246, 18848 x 2304 x 768 369 | 326; below some 600 rows nothing (333 x 1536 x 1536 24.4 | 25.4, 333 x 1536 x 6144
+// 77 | 84). With operands of zeros, so without the power limit, 256x128 tiles gain up to a quarter (1178 x 6144 x 1536 103 | 81).
+// Wavefronts of their own request A: behind the requests of the same wavefront the split of W started a third of a K tile late (128x128 1178 x 1536 x 1536 65 -> 59 us). 256x128 tiles
+// have no registers for a fourth wavefront per SIMD and keep both in one (produce_with_a_pieces). 128x64 as waves of 32x64 instead of 32x32: a quarter of the LDS reads less, 1178 x 1536 x
+// 6144 149 -> 139; 64x64 as waves of 16x64, two workgroups to a unit, 57 -> 45.
+template <int EPI>
+int launch_a_pieces_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
+    switch (shape) {
+        case 0: return launch_pieces<128, 128, 4, 2, 4, 4, 8, 8, 1, 2, 4, 4, EPI>(set, n, st);
+        case 1: return launch_pieces<128, 64, 4, 1, 4, 4, 8, 4, 2, 4, 3, 4, EPI>(set, n, st);
+        case 2: return launch_pieces<64, 64, 4, 1, 2, 4, 8, 4, 1, 4, 5, 4, EPI>(set, n, st);
+        case 3: return launch_pieces<32, 64, 2, 2, 4, 8, 4, 4, 2, 4, 4, 4, EPI>(set, n, st);
+        case 4: return launch_pieces<32, 32, 2, 2, 2, 4, 4, 4, 2, 4, 4, 8, EPI>(set, n, st);
+        default: return launch_pieces<256, 128, 4, 2, 0, 4, 8, 8, 1, 2, 3, 2, EPI>(set, n, st);
     }
 }
 
@@ -838,14 +1064,24 @@ bool whole_chunks(const GemmF32Problem& q) {
 }
 }  // namespace
 
+// (the widths as in whole_chunks and whole_k_tiles, the depth as in f32_by_pieces)
+bool gemm_f32_takes_a_pieces(const float* W, int ldw, int n0, int N, int K) {
+    const F32Layer layer{1, N, K};
+    return (reinterpret_cast<uintptr_t>(W) & 15) == 0 && ldw % 4 == 0 && ldw <= (1 << 22) && n0 % 4 == 0 && N % 4 == 0 && K <= (1 << 22) && f32_by_pieces(&layer, 1) &&
+           !g_gemm_f32_no_pieces;
+}
+
 int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st) {
     if (n < 1 || n > MAX_PROBS) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: 1 to %d problems (got %d)", MAX_PROBS, n);
     TileProbSet set{};
     int m = 0;
+    const bool a_pieces = probs[0].a_pieces;
     for (int i = 0; i < n; i++) {
         const GemmF32Problem& q = probs[i];
         if (q.M <= 0 || q.N <= 0) continue;
         if (q.K <= 0) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: K must be positive");
+        if (q.a_pieces != a_pieces || (a_pieces && !gemm_f32_takes_a_pieces(q.W, q.ldw, q.n0, q.N, q.K)) || (q.out_pieces && (epi != EPI_BIAS_GELU || !whole_chunks(q))))
+            return fail(SD3_ERR_INVALID_ARG, "gemm_f32: operands or outputs in pieces that this launch does not take");
         EpiDev e{q.ea.bias, q.ea.gate, q.ea.resid, q.ea.table, q.ea.gate_ld, q.ea.rows_per_batch > 0 ? q.ea.rows_per_batch : 1};
         if (epi == EPI_BIAS_ROWADD) e.gate_ld = q.N;
         if (!whole_chunks(q)) {
@@ -864,13 +1100,24 @@ int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st
             SD3_TRY(launch_status("gemm_f32"));
             continue;
         }
-        set.p[m++] = TileProb{q.A, q.W, q.out, q.lda, q.ldw, q.ldc, q.M, q.N, q.K, q.n0, e};
+        set.p[m++] = TileProb{q.A, q.W, q.out, q.lda, q.ldw, q.ldc, q.M, q.N, q.K, q.n0, q.out_pieces, e};
     }
     if (m == 0) return SD3_OK;
     const int cus = compute_units();
     if (cus <= 0) return SD3_ERR_HIP;
     const Layers layers(set, m);
+    if (a_pieces) {
+        const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile : pick_f32_piece_tile(layers.l, m, cus, f32_a_piece_tiles);
+        switch (epi) {
+            case EPI_BIAS: return launch_a_pieces_shape<EPI_BIAS>(shape, set, m, st);
+            case EPI_BIAS_GELU: return launch_a_pieces_shape<EPI_BIAS_GELU>(shape, set, m, st);
+            case EPI_GATE_RESID: return launch_a_pieces_shape<EPI_GATE_RESID>(shape, set, m, st);
+            default: return fail(SD3_ERR_INVALID_ARG, "gemm_f32: no epilogue %d with A in pieces", epi);
+        }
+    }
     if (whole_k_tiles(set, m) && f32_by_pieces(layers.l, m) && !g_gemm_f32_no_pieces) {
+        for (int i = 0; i < m; i++)
+            if (set.p[i].out_pieces) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: no output in pieces from the kernel that splits A itself");
         const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile : pick_f32_piece_tile(layers.l, m, cus);
         switch (epi) {
             case EPI_BIAS: return launch_pieces_shape<EPI_BIAS>(shape, set, m, st);

@@ -44,6 +44,66 @@ template <int MULT>
 __device__ __forceinline__ unsigned piece_slot(unsigned row, unsigned chunk) {
     return row * 64 + ((chunk ^ (0u - (row >> 2)) ^ ((row >> 1) & 1) ^ ((row >> 4) * MULT)) & 3) * 16;
 }
+
+// A matrix in pieces in memory, as what produces an operand writes it for the kernel that multiplies it: three planes (h, m, l), each in blocks of 16 rows x 32 k values
+// of 1024 bytes that are the GEMM's LDS rows as they are (piece_slot; chunk c of 8 values: k = 4c .. 4c + 3 and 16 + 4c ..): a direct load of a wavefront is a block,
+// whole cache lines; the blocks of 16 rows follow each other along k. (As rows of 192
+// bytes per K tile, whose lines neighbouring K tiles share, 10656 x 768 x 3072 took 227 us, with the planes of a block side by side, 3 KB that few memory channels
+// hold, 233, so 215; few workgroups of 256x128 tiles 1.42, 1.63 and 1.41 us a K tile.) K is a multiple of 32; a
+// last block of fewer rows has room for 16. What the pieces cannot hold (|x| from 2^112 on, infinities, NaNs) has a NaN for h and its own bits for m and l: products
+// with it are NaNs, and it can be had back.
+constexpr unsigned PIECES_NAN = 0x7fc0;
+__host__ __device__ inline size_t pieces_bytes(size_t rows, size_t K) { return (rows + 15) / 16 * 16 * K * 6; }
+struct PieceMatrix {
+    bf16_t* p;
+    long long plane;  // values
+    int K;
+    __device__ __forceinline__ PieceMatrix(void* q, long long M, int K_) : p(reinterpret_cast<bf16_t*>(q)), plane((M + 15) / 16 * 16 * K_), K(K_) {}
+};
+__device__ __forceinline__ long long piece_index(long long row, unsigned k, int K) {
+    return ((row >> 4) * (K / 32) + k / 32) * 512 + piece_slot<0>((unsigned)row & 15, k % 16 / 4) / 2 + k / 16 % 2 * 4 + k % 4;
+}
+// The pieces of N values as they are written
+template <int N>
+__device__ __forceinline__ void pieces_for_memory(const float (&v)[N], uint32_t (&piece)[3][(N + 1) / 2]) {
+    constexpr int P = N == 1 ? 2 : N;
+    float x[P];
+#pragma unroll
+    for (int i = 0; i < P; i++) x[i] = i < N ? v[i] : 0.f;
+    bf16_pieces<P>(x, piece[0], piece[1], piece[2]);
+    // what is left of a value that has no pieces is a NaN (infinity less infinity)
+    float rest = x[0];
+#pragma unroll
+    for (int i = 1; i < P; i++) rest += x[i];
+    if (__builtin_expect(rest != rest, 0)) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const unsigned sh = i & 1 ? 16 : 0;
+            if ((piece[0][i / 2] >> sh & 0x7f80u) == 0x7f80u) {
+                const uint32_t bits = __float_as_uint(v[i]), others = ~(0xffffu << sh);
+                piece[0][i / 2] = (piece[0][i / 2] & others) | PIECES_NAN << sh;
+                piece[1][i / 2] = (piece[1][i / 2] & others) | (bits >> 16) << sh;
+                piece[2][i / 2] = (piece[2][i / 2] & others) | (bits & 0xffffu) << sh;
+            }
+        }
+    }
+}
+// N = 1, 2 or 4 consecutive values of a row from k on, k a multiple of N
+template <int N>
+__device__ __forceinline__ void put_pieces(const PieceMatrix& to, long long row, unsigned k, const float (&v)[N]) {
+    uint32_t piece[3][(N + 1) / 2];
+    pieces_for_memory<N>(v, piece);
+    bf16_t* at = to.p + piece_index(row, k, to.K);
+#pragma unroll
+    for (int p = 0; p < 3; p++) __builtin_memcpy(__builtin_assume_aligned(at + p * to.plane, N * 2), piece[p], N * 2);
+}
+__device__ __forceinline__ float of_pieces(const PieceMatrix& of, long long row, unsigned k) {
+    const bf16_t* at = of.p + piece_index(row, k, of.K);
+    const uint32_t h = at[0], m = at[of.plane], l = at[2 * of.plane];
+    if ((h & 0x7f80u) == 0x7f80u) return __uint_as_float(m << 16 | l);
+    return ((__uint_as_float(h << 16) + __uint_as_float(m << 16)) + __uint_as_float(l << 16)) * (1.0f / PIECES_SCALE);
+}
+
 template <int KEEP>  // all but the last KEEP LDS operations of this wavefront are done, and behind the barrier those of the others too
 __device__ __forceinline__ void barrier_behind_lds() {
     __builtin_amdgcn_s_waitcnt(15 | (KEEP << 8) | (7 << 4) | (3 << 14));

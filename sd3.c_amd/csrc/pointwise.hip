@@ -1,6 +1,7 @@
 // Memory-bound kernels: LayerNorm(+adaLN modulation), per-head RMSNorm, activations, gating, embeddings,
 // patch gather / scatter, casts. All are sized so that one launch streams its tensors once through HBM.
 #include "common.hpp"
+#include "pieces.hpp"
 
 namespace sd3 {
 
@@ -24,6 +25,19 @@ template <>
 __device__ __forceinline__ void store1<float>(float* p, float a) { *p = a; }
 template <>
 __device__ __forceinline__ void store1<bf16_t>(bf16_t* p, float a) { *p = f32_to_bf16(a); }
+
+// Four values of a row of C from k on (k a multiple of 4), or one. Pieces: a matrix of bf16 pieces (pieces.hpp)
+struct Pieces {};
+template <typename T>
+__device__ __forceinline__ void put4(T* out, long long row, long long rows, int C, int k, float a, float b, float c, float d) {
+    if constexpr (std::is_same<T, Pieces>::value) put_pieces<4>(PieceMatrix(out, rows, C), row, k, {a, b, c, d});
+    else store4<T>(out + row * C + k, a, b, c, d);
+}
+template <typename T>
+__device__ __forceinline__ void put1(T* out, long long row, long long rows, int C, int k, float a) {
+    if constexpr (std::is_same<T, Pieces>::value) put_pieces<1>(PieceMatrix(out, rows, C), row, k, {a});
+    else store1<T>(out + row * C + k, a);
+}
 
 // One wavefront per row, the row held in registers (NV float4 per lane), two-pass mean / variance like the
 // reference (modules.cpp:22-37), then up to two modulated outputs (modules.cpp:1207-1221 fused in).
@@ -114,13 +128,13 @@ __global__ void __launch_bounds__(256) ln_mod_vec_kernel(const LnSegPair<OutT> s
             float n0 = rstd * (v[i].x - mu), n1 = rstd * (v[i].y - mu), n2 = rstd * (v[i].z - mu), n3 = rstd * (v[i].w - mu);
             if (sc) {
                 const float4 a = EARLY ? msc[i] : sc[j], c = EARLY ? msh[i] : sh[j];
-                store4<OutT>(out + row * C + 4 * j, n0 * (1.0f + a.x) + c.x, n1 * (1.0f + a.y) + c.y, n2 * (1.0f + a.z) + c.z, n3 * (1.0f + a.w) + c.w);
+                put4<OutT>(out, row, g.rows, C, 4 * j, n0 * (1.0f + a.x) + c.x, n1 * (1.0f + a.y) + c.y, n2 * (1.0f + a.z) + c.z, n3 * (1.0f + a.w) + c.w);
             } else {
-                store4<OutT>(out + row * C + 4 * j, n0, n1, n2, n3);
+                put4<OutT>(out, row, g.rows, C, 4 * j, n0, n1, n2, n3);
             }
             if (out2) {
                 const float4 a = EARLY ? msc2[i] : sc2[j], c = EARLY ? msh2[i] : sh2[j];
-                store4<OutT>(out2 + row * C + 4 * j, n0 * (1.0f + a.x) + c.x, n1 * (1.0f + a.y) + c.y, n2 * (1.0f + a.z) + c.z, n3 * (1.0f + a.w) + c.w);
+                put4<OutT>(out2, row, g.rows, C, 4 * j, n0 * (1.0f + a.x) + c.x, n1 * (1.0f + a.y) + c.y, n2 * (1.0f + a.z) + c.z, n3 * (1.0f + a.w) + c.w);
             }
         }
     }
@@ -158,8 +172,8 @@ __global__ void __launch_bounds__(256) ln_mod_generic_kernel(const float* __rest
         if (w) o *= w[j];
         if (bias) o += bias[j];
         if (scale) o = o * (1.0f + scale[b * mod_ld + j]) + shift[b * mod_ld + j];
-        store1<OutT>(out + row * C + j, o);
-        if (out2) store1<OutT>(out2 + row * C + j, n * (1.0f + scale2[b * mod_ld + j]) + shift2[b * mod_ld + j]);
+        put1<OutT>(out, row, rows, C, j, o);
+        if (out2) put1<OutT>(out2, row, rows, C, j, n * (1.0f + scale2[b * mod_ld + j]) + shift2[b * mod_ld + j]);
     }
 }
 
@@ -227,9 +241,13 @@ int layernorm_modulate(const float* x, void* out, void* out2, const float* shift
     return layernorm_modulate_pair(&j, 1, eps, C, out_bf16, st);
 }
 
-int layernorm_modulate_pair(const LayerNormJob* jobs, int n, float eps, int C, int out_bf16, hipStream_t st) {
+int layernorm_modulate_pair(const LayerNormJob* jobs, int n, float eps, int C, int out, hipStream_t st) {
     if (n < 1 || n > 2) return fail(SD3_ERR_INVALID_ARG, "layernorm_modulate_pair: 1 or 2 tensors (got %d)", n);
-    return out_bf16 ? ln_mod_pair_t<bf16_t>(jobs, n, eps, C, st) : ln_mod_pair_t<float>(jobs, n, eps, C, st);
+    switch (out) {
+        case LN_BF16: return ln_mod_pair_t<bf16_t>(jobs, n, eps, C, st);
+        case LN_PIECES: return ln_mod_pair_t<Pieces>(jobs, n, eps, C, st);
+        default: return ln_mod_pair_t<float>(jobs, n, eps, C, st);
+    }
 }
 
 int layernorm_full(const float* x, float* y, float* mean, float* rstd, const float* w, const float* bias, float eps, long long rows, int C,

@@ -1,0 +1,86 @@
+"""fp32 blocks whose operands are written as bf16 pieces by what produces them: the same bits as from products that split fp32 operands themselves.
+
+`sd3_dit_block_static` has a fixed 64 MiB for its intermediates and goes without the pieces where these, six bytes a value instead of four, do not fit; the
+context's workspace grows. Blocks between the two sizes are computed both ways."""
+import numpy as np
+import pytest
+
+from gpu_util import M, dev, dev_params, host
+from sd3_c_amd import lib as L
+from sd3_c_amd.params import block_param_shapes, synthetic_params_numpy
+
+pytestmark = pytest.mark.gpu
+
+
+def _plain_and_pieces_bytes(B, Tc, Tx, C, E, dual):
+    """The block's activations (fp32; pieces of LayerNorm's outputs, and from 1.7e6 values on of attention's and the first MLP layer's too)."""
+    rows = B * (Tc + Tx)
+    qkv = 12 * C * (rows + (B * Tx if dual else 0))
+    wide = rows * C >= 1.7e6
+    plain = qkv + 4 * C * (rows + B * Tx) + 4 * C * rows + 4 * E * C * rows
+    return plain, qkv + 6 * C * (rows + B * Tx) + (6 if wide else 4) * (C * rows + E * C * rows)
+
+
+def _both_ways(B, Tc, Tx, C, NH, E, dual, discard, spoil=None):
+    plain, pieces = _plain_and_pieces_bytes(B, Tc, Tx, C, E, dual)
+    limit = 64 << 20
+    assert plain + (1 << 19) < limit < pieces  # (room for the modulation vectors, and the case tells the two apart)
+    rng = np.random.Generator(np.random.Philox(Tx))
+    P = synthetic_params_numpy(block_param_shapes(C, E, dual, True, discard, C // NH), 11, 0.05, 0.05)
+    y, c, x = (rng.standard_normal(s, dtype=np.float32) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
+    if spoil:
+        spoil(P, c, x)
+    ctx = M.Context()
+    try:
+        ctx.bind(dev_params(P))
+        out = []
+        for run in (ctx.block, ctx.block_static):
+            cg, xg = dev(c.copy()), dev(x.copy())
+            run(dev(y), cg, xg, B, Tc, Tx, C, NH, E, dual, True, discard, precision="fp32")
+            out.append((host(cg), host(xg)))
+        return out
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("B,Tc,Tx,C,NH,E,dual,discard", [
+    (1, 77, 1100, 1536, 24, 2, False, False),   # all three, heads of 64, rows that are no whole blocks of 16
+    (3, 50, 351, 1536, 12, 2, False, False),    # heads of 128, several elements
+    (1, 20, 930, 1536, 24, 2, True, False),     # LayerNorm's outputs only; two of them
+    (1, 33, 1090, 1536, 24, 2, False, True),    # no context behind attention
+    (5, 1, 500, 768, 12, 2, False, False),      # 768 deep
+    (2, 15, 1701, 512, 8, 2, False, False),     # the least depth of the kernel
+])
+def test_the_same_bits_with_operands_in_pieces(B, Tc, Tx, C, NH, E, dual, discard):
+    (ca, xa), (cb, xb) = _both_ways(B, Tc, Tx, C, NH, E, dual, discard)
+    assert np.isfinite(xa).all()
+    assert np.array_equal(xa, xb) and np.array_equal(ca, cb)
+
+
+@pytest.mark.parametrize("tile", range(6))
+def test_the_same_bits_for_every_tile_shape(tile):
+    L.check(L.load().sd3_tune(b"gemm_f32_tile", tile))
+    try:
+        (ca, xa), (cb, xb) = _both_ways(1, 37, 3361, 512, 8, 2, False, False)
+    finally:
+        L.check(L.load().sd3_tune(b"gemm_f32_tile", -1))
+    assert np.array_equal(xa, xb) and np.array_equal(ca, cb)
+
+
+@pytest.mark.parametrize("what", ["scales", "tokens"])
+def test_values_without_pieces(what):
+    """Infinities, NaNs and values from 2^112 on in LayerNorm's, attention's and the MLP's outputs are formed anew by the fp32 instruction, from the bits that stand in the pieces' place."""
+    C = 1536
+
+    def spoil(P, c, x):
+        if what == "tokens":
+            x[0, 5, 3] = np.inf
+            x[0, 700, 8] = np.nan
+            return
+        for n, q in P.items():
+            if "ada" in n and n.endswith(".bias"):
+                q[1 * C + 7] = 2.0 ** 115   # the scale of LayerNorm's channel 7 in front of q|k|v: values, too, and what attention makes of them
+                q[4 * C + 9] = -2.0 ** 115  # ... in front of the MLP: some of the hidden values
+    (ca, xa), (cb, xb) = _both_ways(1, 77, 1100, C, 24, 2, False, False, spoil)
+    assert np.isfinite(xa).all() == (what == "scales")
+    assert np.array_equal(xa, xb, equal_nan=True) and np.array_equal(ca, cb, equal_nan=True)
