@@ -83,6 +83,17 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
+// RMSNorm's factor of a head of 64 * NV values (modules.cpp:192-198), of which each of 16 consecutive lanes has the squares of NV groups of four. For the fp32 path's two forms of it, in the
+// projection's epilogue and in a kernel of its own: explicit multiply-adds and one order of the sums, so that they have the same bits.
+__device__ __forceinline__ float head_squares(const float (&v)[4]) { return fmaf(v[0], v[0], v[1] * v[1]) + fmaf(v[2], v[2], v[3] * v[3]); }
+template <int NV>
+__device__ __forceinline__ float head_factor(float ss, float eps) {
+    ss += dpp_move<0xB1>(ss);   // quad_perm [1,0,3,2]
+    ss += dpp_move<0x4E>(ss);   // quad_perm [2,3,0,1]
+    ss += dpp_move<0x141>(ss);  // row_half_mirror
+    ss += dpp_move<0x140>(ss);  // row_mirror
+    return 1.0f / sqrtf(fmaf(ss, 1.0f / (64 * NV), eps));
+}
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -307,7 +318,7 @@ enum Epilogue : int {
     EPI_GATE_RESID = 3,   // out = resid + gate[m / rows_per_batch][n] * (acc + bias)   (out may alias resid)
     EPI_BIAS_ROWADD = 4,  // out = acc + bias + table[m % rows_per_batch][n]
     EPI_QKV_NORM = 5,     // packed q|k|v projection (N = 3C): acc + bias, then per-head RMSNorm (64 columns, eps 1e-6) of the q and k thirds
-                          // with weights `gate` (q) and `resid` (k), each 64 floats; C is given in gate_ld
+                          // with weights `gate` (q) and `resid` (k), each 64 floats; C is given in gate_ld. fp32: A in pieces
 };
 
 struct GemmEpilogueArgs {

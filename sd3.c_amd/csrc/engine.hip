@@ -562,13 +562,14 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
                                      {c, c_hid, nullptr, c_shift, c_scale, nullptr, nullptr, ldc_ada, B, Tc}};
         SD3_TRY(ln_mod_pair(ctx, ln1, 2, 1e-6f, C, ln_out));
     }
+    bool fused_norm;
     {
-        // bf16 path: the per-head RMSNorm of q and k (modules.cpp:1396-1399, 1420-1423) runs in the projection's epilogue, on the
-        // fp32 accumulators, so the attention kernel streams K tiles straight into LDS
+        // the per-head RMSNorm of q and k (modules.cpp:1396-1399, 1420-1423) runs in the projection's epilogue, on the fp32 accumulators, in the bf16 path, so that the
+        // attention kernel streams K tiles straight into LDS, and with heads of 64 in fp32 where the inputs come in pieces
         GemmEpilogueArgs nx, nc;
         nx.gate = w.x_rms_q; nx.resid = w.x_rms_k;
         nc.gate = w.c_rms_q; nc.resid = w.c_rms_k;
-        const bool fused_norm = bf && d.qk;
+        fused_norm = d.qk && (bf || (pieces.rows && d.HS == 64));
         GemmEpilogueArgs n2;
         n2.gate = w.x2_rms_q; n2.resid = w.x2_rms_k;
         // the dual branch's projection reads the other output of the same LayerNorm pass: same kind, same launch
@@ -578,9 +579,9 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
         SD3_TRY(linear_pair(ctx, prec, qkv, 3, !bf, fused_norm ? EPI_QKV_NORM : EPI_BIAS, nullptr, carry));
     }
 
-    // ---- joint attention over [context ; latent] (modules.cpp:1427-1432); fp32 path: qk-norm in place first
+    // ---- joint attention over [context ; latent] (modules.cpp:1427-1432); qk-norm in place first where the projection has left it
     auto seg_ptr = [&](void* base, int third) -> void* { return (char*)base + (size_t)third * C * es; };
-    if (!bf && d.qk) {
+    if (d.qk && !fused_norm) {
         const QkNormJob norms[3] = {{(float*)x_qkv, w.x_rms_q, w.x_rms_k, mx}, {(float*)c_qkv, w.c_rms_q, w.c_rms_k, mc}, {(float*)x_qkv2, w.x2_rms_q, w.x2_rms_k, mx}};
         SD3_TRY(qk_norm_rows(norms, d.dual ? 3 : 2, 1e-6f, d.NH, d.HS, 3 * C, st));
     }

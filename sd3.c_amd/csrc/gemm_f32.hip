@@ -229,6 +229,31 @@ __device__ __forceinline__ void store_tile(const TileProb& pr, const f32x4_t (&a
         }
     }
     const int rpb = e.rows_per_batch;
+    if constexpr (EPI == EPI_QKV_NORM) {
+        // q and k: a wavefront's 64 columns are one head, four a lane. (16 x 666 tokens, width 768: 368 us and 49 in a kernel of its own -> 370)
+        static_assert(NJ == 4, "a head per wavefront");
+        const int third = __builtin_amdgcn_readfirstlane(n / e.gate_ld);
+        float w[NJ] = {};
+        if (third < 2) load_cols<NJ>((third ? e.resid : e.gate) + n % 64, w);
+        arrived(bias);
+        arrived(w);
+#pragma unroll
+        for (int i = 0; i < TI; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int m = m0 + i * 16 + r;
+                float v[NJ];
+#pragma unroll
+                for (int j = 0; j < NJ; j++) v[j] = acc[i][j][r] + bias[j];
+                if (third < 2) {
+                    const float inv = head_factor<1>(head_squares(v), 1e-6f);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) v[j] = (v[j] * inv) * w[j];
+                }
+                if (m < pr.M) store_cols<NJ>(pr.out + (long long)m * pr.ldc + n, v);
+            }
+        return;
+    }
     // Rows of at most two batch elements, as all but those of very few rows: a gate for each
     const int b_first = EPI == EPI_GATE_RESID ? m_wave / rpb : 0, b_last = EPI == EPI_GATE_RESID ? min(m_wave + TI * 16 - 1, pr.M - 1) / rpb : 0;
     if (!LEAN && b_last - b_first <= 1) {
@@ -1048,6 +1073,16 @@ int launch_a_pieces_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
     }
 }
 
+// ... with the norms of q and k: the shapes whose wavefronts have 64 columns (by the number of rows from which on A comes in pieces the others are never the better ones)
+int launch_qkv_norm_shape(int shape, TileProbSet& set, int n, hipStream_t st) {
+    switch (shape) {
+        case 0: return launch_pieces<128, 128, 4, 2, 4, 4, 8, 8, 1, 2, 4, 4, EPI_QKV_NORM>(set, n, st);
+        case 1: return launch_pieces<128, 64, 4, 1, 4, 4, 8, 4, 2, 4, 3, 4, EPI_QKV_NORM>(set, n, st);
+        case 5: return launch_pieces<256, 128, 4, 2, 0, 4, 8, 8, 1, 2, 3, 2, EPI_QKV_NORM>(set, n, st);
+        default: return launch_pieces<64, 64, 4, 1, 2, 4, 8, 4, 1, 4, 5, 4, EPI_QKV_NORM>(set, n, st);
+    }
+}
+
 struct Layers {
     F32Layer l[MAX_PROBS];
     Layers(const TileProbSet& set, int n) {
@@ -1082,8 +1117,11 @@ int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st
         if (q.K <= 0) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: K must be positive");
         if (q.a_pieces != a_pieces || (a_pieces && !gemm_f32_takes_a_pieces(q.W, q.ldw, q.n0, q.N, q.K)) || (q.out_pieces && (epi != EPI_BIAS_GELU || !whole_chunks(q))))
             return fail(SD3_ERR_INVALID_ARG, "gemm_f32: operands or outputs in pieces that this launch does not take");
+        if (epi == EPI_QKV_NORM && (!a_pieces || q.n0 || q.N % 192))
+            return fail(SD3_ERR_INVALID_ARG, "gemm_f32: the norms of q and k are for A in pieces and heads of 64");
         EpiDev e{q.ea.bias, q.ea.gate, q.ea.resid, q.ea.table, q.ea.gate_ld, q.ea.rows_per_batch > 0 ? q.ea.rows_per_batch : 1};
         if (epi == EPI_BIAS_ROWADD) e.gate_ld = q.N;
+        if (epi == EPI_QKV_NORM) e.gate_ld = q.N / 3;
         if (!whole_chunks(q)) {
             dim3 grid((q.N + BN - 1) / BN, (q.M + BM - 1) / BM), block(256);
 #define SD3_GEMM_F32_LAUNCH(E) \
@@ -1112,6 +1150,7 @@ int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st
             case EPI_BIAS: return launch_a_pieces_shape<EPI_BIAS>(shape, set, m, st);
             case EPI_BIAS_GELU: return launch_a_pieces_shape<EPI_BIAS_GELU>(shape, set, m, st);
             case EPI_GATE_RESID: return launch_a_pieces_shape<EPI_GATE_RESID>(shape, set, m, st);
+            case EPI_QKV_NORM: return launch_qkv_norm_shape(shape, set, m, st);
             default: return fail(SD3_ERR_INVALID_ARG, "gemm_f32: no epilogue %d with A in pieces", epi);
         }
     }

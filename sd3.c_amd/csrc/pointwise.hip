@@ -319,11 +319,9 @@ __global__ void __launch_bounds__(256) qk_norm_kernel(const QkNormDev jobs, floa
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         v[i] = p[sub + 16 * i];
-        s += (v[i].x * v[i].x + v[i].y * v[i].y) + (v[i].z * v[i].z + v[i].w * v[i].w);
+        s += head_squares({v[i].x, v[i].y, v[i].z, v[i].w});
     }
-#pragma unroll
-    for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
-    const float inv = 1.0f / sqrtf(eps + s / (NV * 64));
+    const float inv = head_factor<NV>(s, eps);
 #pragma unroll
     for (int i = 0; i < NV; i++) {
         const float4 a = w[sub + 16 * i];
