@@ -18,6 +18,7 @@ namespace {
 
 constexpr int BK = 64;  // bf16 elements per K tile = 128 bytes per LDS row
 
+typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));  // four floats at any float
 struct EpiDev {
     const float* a_scale;  // fp8 operands: one factor per row of A (null: 1)
     const float* w_scale;  // fp8 operands: one factor per output column (null: 1)
@@ -407,6 +408,51 @@ __device__ __forceinline__ void gemm_tile(const Prob& pr, const int wg, char* sm
     // 4-byte scattered stores; each wavefront instead transposes one 32-row slab at a time through its private LDS
     // region (the tile ring is free now) and leaves with 16 lanes covering 64 contiguous columns of one row.
     __syncthreads();
+    if constexpr (EPI == EPI_GATE_RESID && OUT_F32 && M16 && WNC % 64 == 0) {
+        // Gated tiles that lie inside the matrix, with rows of at most two batch elements per wavefront: nothing is read or stored under a condition, so that the waits are counted
+        // exactly: a slab's residual rows, requested a slab ahead, are waited for without the stores behind them, and the gates are read once. (Else every row's gate waits for
+        // everything in flight, 32 times a tile: the pair of 1024px 22915 -> 22845 us without this form and 23426 -> 22919 with
+        // it, 2048px 82564 -> 81467.)
+        const int m_wave = m_blk + wm * (BM / WM), first = m_wave / rpb, last = (m_wave + BM / WM - 1) / rpb;
+        if (vec_ok && m_blk + BM <= M && n_blk + BN <= N && last - first <= 1) {
+            const long long lane_at = (long long)(m_wave + e_row) * ldc + n0;
+            auto at4 = [](const float* p) { return *reinterpret_cast<const f32x4_t*>(p); };
+            f32x4_t bias = epi.bias ? *reinterpret_cast<const f32x4_any_t*>(epi.bias + n0) : f32x4_any_t{0.f, 0.f, 0.f, 0.f};
+            f32x4_t gate_first = at4(epi.gate + (long long)first * epi.gate_ld + n0), gate_last = at4(epi.gate + (long long)last * epi.gate_ld + n0), next[NP];
+            auto request = [&](int i) {
+#pragma unroll
+                for (int p = 0; p < NP; p++) next[p] = at4(epi.resid + lane_at + (long long)(i * SR + p * RPI) * ldc);
+            };
+            request(0);
+            asm volatile("" : "+v"(bias), "+v"(gate_first), "+v"(gate_last));  // (named, so that they are waited for here)
+#pragma unroll
+            for (int i = 0; i < NSLAB; i++) {
+                f32x4_t cur[NP], vals[NP];
+#pragma unroll
+                for (int p = 0; p < NP; p++) cur[p] = next[p];
+                if (i + 1 < NSLAB) request(i + 1);
+#pragma unroll
+                for (int ii = 0; ii < SR / 16; ii++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) slab[(16 * ii + 4 * lg + r) * EP + j * 16 + lr] = acc16[(SR / 16) * i + ii][j][r];
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int p = 0; p < NP; p++) vals[p] = at4(&slab[(p * RPI + e_row) * EP + e_col]);
+#pragma unroll
+                for (int p = 0; p < NP; p++) {
+                    const bool second = m_wave + i * SR + p * RPI + e_row >= last * rpb;
+                    f32x4_t v;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) v[c] = fmaf(second ? gate_last[c] : gate_first[c], vals[p][c] + bias[c], cur[p][c]);
+                    *reinterpret_cast<f32x4_t*>(outf + lane_at + (long long)(i * SR + p * RPI) * ldc) = v;
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+            return;
+        }
+    }
     float bias4[4] = {0.f, 0.f, 0.f, 0.f};
     if (epi.bias)
 #pragma unroll
@@ -798,29 +844,113 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
             }
         }
     };
+    const int n0 = n_blk + wn * WC + NJ * lr, m_wave = m_blk + wm * (TM / WM);  // the lane's first column, the wavefront's first row
+    // What the epilogue of whole rows reads, requested together and waited for once (row by row, each behind the store of the one before, a tile's
+    // 4 to 16 rows were as many trips to memory; outputs the same bits: forwards of 256px 2519 -> 2456 us, 512px 4015 -> 3951, its pair 6153 -> 6089, 496x272 6657 -> 6499, 1024px 12650
+    // -> 12399, the block of 256 + 77 tokens 103.7 -> 100.1. In front of the K loop they would hide altogether, but spill in it: +1 to +2.4 %). Gates: of the batch elements of the wavefront's first and last row; rows of more than
+    // two (`few` is false) read theirs one by one.
+    constexpr bool READS = EPI == EPI_GATE_RESID || EPI == EPI_BIAS_ROWADD;
+    f32x4_t bias4, norm_w, gate_first, gate_last, rows[READS ? TI : 1][4];
+    int third = 0, second_from = 0;
+    bool few = true;
+    auto request = [&](const Prob& pr) {
+        if (!WHOLE_ROWS) return;
+        const EpiDev& epi = pr.epi;
+        const int n = min(n0, N - 4), rpb = epi.rows_per_batch;
+        bias4 = epi.bias ? *reinterpret_cast<const f32x4_any_t*>(epi.bias + n) : f32x4_any_t{0.f, 0.f, 0.f, 0.f};
+        if (EPI == EPI_QKV_NORM) {
+            third = n / epi.gate_ld;
+            norm_w = third < 2 ? *reinterpret_cast<const f32x4_t*>((third == 0 ? epi.gate : epi.resid) + (n & 63)) : f32x4_t{1.f, 1.f, 1.f, 1.f};
+        }
+        if (EPI == EPI_GATE_RESID) {
+            const int first = min(m_wave, M - 1) / rpb, last = min(m_wave + TI * 16, M) - 1 > 0 ? (min(m_wave + TI * 16, M) - 1) / rpb : 0;
+            few = last - first <= 1;
+            second_from = last * rpb;
+            gate_first = *reinterpret_cast<const f32x4_t*>(epi.gate + (long long)first * epi.gate_ld + n);
+            gate_last = *reinterpret_cast<const f32x4_t*>(epi.gate + (long long)last * epi.gate_ld + n);
+        }
+        if constexpr (READS) {
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = min(m_wave + i * 16 + 4 * lg + r, M - 1);
+                    rows[i][r] = *reinterpret_cast<const f32x4_t*>(EPI == EPI_GATE_RESID ? epi.resid + (long long)m * ldc + n : epi.table + (long long)(m % rpb) * epi.gate_ld + n);
+                }
+        }
+    };
+    auto arrived = [](f32x4_t& v) { asm volatile("" : "+v"(v)); };  // (named, so that it is waited for here)
     auto epilogue = [&](const Prob& pr) {
-        const int n0 = n_blk + wn * WC + NJ * lr;
         if (n0 >= N) return;
+        int n = n0, row0 = m_wave + 4 * lg;
+        asm volatile("" : "+v"(n), "+v"(row0));  // (or addresses are formed in front of the K loop and held through it)
         const EpiDev& epi = pr.epi;
         const int rpb = epi.rows_per_batch;
+        if constexpr (WHOLE_ROWS) {
+            arrived(bias4);
+            if (EPI == EPI_QKV_NORM) arrived(norm_w);
+            if (EPI == EPI_GATE_RESID) {
+                arrived(gate_first);
+                arrived(gate_last);
+            }
+            if constexpr (READS) {
+#pragma unroll
+                for (int i = 0; i < TI; i++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) arrived(rows[i][r]);
+            }
+#pragma unroll
+            for (int i = 0; i < TI; i++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int m = row0 + i * 16 + r;  // (uniform over the 16 lanes that share a head)
+                    float v[4] = {acc[i][0][r] + bias4[0], acc[i][1][r] + bias4[1], acc[i][2][r] + bias4[2], acc[i][3][r] + bias4[3]};
+                    if (EPI == EPI_BIAS_GELU) {
+#pragma unroll
+                        for (int c = 0; c < 4; c++) v[c] = gelu_tanh_f(v[c]);
+                    } else if (EPI == EPI_BIAS_SILU) {
+#pragma unroll
+                        for (int c = 0; c < 4; c++) v[c] = v[c] / (1.0f + __expf(-v[c]));
+                    } else if (EPI == EPI_GATE_RESID) {
+                        f32x4_t g4;
+#pragma unroll
+                        for (int c = 0; c < 4; c++) g4[c] = m >= second_from ? gate_last[c] : gate_first[c];
+                        if (!few) {
+                            g4 = *reinterpret_cast<const f32x4_t*>(epi.gate + (long long)(min(m, M - 1) / rpb) * epi.gate_ld + n);
+                            arrived(g4);  // (in here, or the others wait as well)
+                        }
+                        const f32x4_t r4 = rows[READS ? i : 0][r];
+#pragma unroll
+                        for (int c = 0; c < 4; c++) v[c] = fmaf(g4[c], v[c], r4[c]);
+                    } else if (EPI == EPI_BIAS_ROWADD) {
+                        const f32x4_t t4 = rows[READS ? i : 0][r];
+                        v[0] += t4[0]; v[1] += t4[1]; v[2] += t4[2]; v[3] += t4[3];
+                    } else if (EPI == EPI_QKV_NORM && third < 2) {
+                        qk_norm4(v, make_float4(norm_w[0], norm_w[1], norm_w[2], norm_w[3]));
+                    }
+                    const long long idx = (long long)m * ldc + n;
+                    if (m < M) {
+                        if (OUT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(pr.out) + idx) = make_float4(v[0], v[1], v[2], v[3]);
+                        else *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(pr.out) + idx) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+                    }
+                }
+            return;
+        }
         const int valid = N - n0;  // (element by element: columns of this lane's four that exist, if fewer than four)
-        auto four = [&](const float* p) {
-            if (WHOLE_ROWS) return *reinterpret_cast<const float4*>(p);
-            return make_float4(p[0], valid > 1 ? p[1] : 0.f, valid > 2 ? p[2] : 0.f, valid > 3 ? p[3] : 0.f);
-        };
+        auto four = [&](const float* p) { return make_float4(p[0], valid > 1 ? p[1] : 0.f, valid > 2 ? p[2] : 0.f, valid > 3 ? p[3] : 0.f); };
         float bias4[4] = {0.f, 0.f, 0.f, 0.f};
         if (epi.bias)
 #pragma unroll
             for (int c = 0; c < 4; c++)
-                if (WHOLE_ROWS || c < valid) bias4[c] = epi.bias[n0 + c];
+                if (c < valid) bias4[c] = epi.bias[n0 + c];
+        const int third_e = EPI == EPI_QKV_NORM ? n0 / epi.gate_ld : 0;
         float4 norm_w = make_float4(1.f, 1.f, 1.f, 1.f);
-        const int third = EPI == EPI_QKV_NORM ? n0 / epi.gate_ld : 0;
-        if (EPI == EPI_QKV_NORM && third < 2) norm_w = *reinterpret_cast<const float4*>((third == 0 ? epi.gate : epi.resid) + (n0 & 63));
+        if (EPI == EPI_QKV_NORM && third_e < 2) norm_w = *reinterpret_cast<const float4*>((third_e == 0 ? epi.gate : epi.resid) + (n0 & 63));
 #pragma unroll
         for (int i = 0; i < TI; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int m = m_blk + wm * (TM / WM) + i * 16 + 4 * lg + r;  // (uniform over the 16 lanes that share a head)
+                const int m = m_wave + i * 16 + 4 * lg + r;
                 if (m >= M) continue;
                 const long long idx = (long long)m * ldc + n0;
                 float v[4];
@@ -839,20 +969,15 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
                 } else if (EPI == EPI_BIAS_ROWADD) {
                     const float4 t4 = four(epi.table + (long long)(m % rpb) * epi.gate_ld + n0);
                     v[0] += t4.x; v[1] += t4.y; v[2] += t4.z; v[3] += t4.w;
-                } else if (EPI == EPI_QKV_NORM && third < 2) {
+                } else if (EPI == EPI_QKV_NORM && third_e < 2) {
                     qk_norm4(v, norm_w);
                 }
-                if (WHOLE_ROWS) {
-                    if (OUT_F32) *reinterpret_cast<float4*>(reinterpret_cast<float*>(pr.out) + idx) = make_float4(v[0], v[1], v[2], v[3]);
-                    else *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(pr.out) + idx) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-                } else {
 #pragma unroll
-                    for (int c = 0; c < 4; c++)
-                        if (c < valid) {
-                            if (OUT_F32) reinterpret_cast<float*>(pr.out)[idx + c] = v[c];
-                            else reinterpret_cast<bf16_t*>(pr.out)[idx + c] = f32_to_bf16(v[c]);
-                        }
-                }
+                for (int c = 0; c < 4; c++)
+                    if (c < valid) {
+                        if (OUT_F32) reinterpret_cast<float*>(pr.out)[idx + c] = v[c];
+                        else reinterpret_cast<bf16_t*>(pr.out)[idx + c] = f32_to_bf16(v[c]);
+                    }
             }
     };
 
@@ -868,13 +993,16 @@ __global__ void __launch_bounds__(WM* WN * 64, MW) gemm_bf16_ring_kernel(const P
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         operands(next.A, next.Wp, next.tiled);
+        request(pr);
         fill_ring();
         epilogue(pr);
         k_loop();
         wait_vmcnt<0>();
+        request(next);
         epilogue(next);
         return;
     }
+    request(pr);
     wait_vmcnt<0>();
     epilogue(pr);
 }
