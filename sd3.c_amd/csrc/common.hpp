@@ -343,7 +343,7 @@ struct GemmF32Problem {
     int lda, ldw, n0, ldc, M, N, K;
     GemmEpilogueArgs ea;
     bool a_pieces = false;    // A: a matrix of pieces (pieces.hpp), in all problems of the launch and where gemm_f32_takes_a_pieces
-    bool out_pieces = false;  // EPI_BIAS_GELU: the output as a matrix of pieces of ldc columns
+    bool out_pieces = false;  // EPI_BIAS_GELU, A in pieces: the output as a matrix of pieces of ldc columns
 };
 bool gemm_f32_takes_a_pieces(const float* W, int ldw, int n0, int N, int K);
 int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st);

@@ -189,7 +189,7 @@ __device__ __forceinline__ void store_cols(float* p, const float (&v)[NJ]) {
 // m0: the lane's first row, n: its first column. Everything that is to be read is requested before the first store and waited for together: row by row, each behind the other's store,
 // 16 rows were 16 trips to memory. With the gate, 10656 x 768 x 768: tiles of 128x128 93 -> 84 us, of
 // 64x64 132 -> 116; 333 x 1536 x 1536 25.7 -> 23.5.
-// LEAN: row by row all the same, for the 256x128 tiles of the kernel that splits A itself, whose K loop spills registers beside anything else (K = 6144 370 -> 486 us). PIECES: the output may be one of pieces.
+// LEAN: row by row all the same, for the 256x128 tiles of the kernel that splits A itself, whose K loop spills registers beside anything else (K = 6144 370 -> 486 us). PIECES: the output may be one of pieces (A comes in them).
 template <int TI, int NJ, int EPI, bool PIECES, bool LEAN = false>
 __device__ __forceinline__ void store_tile(const TileProb& pr, const f32x4_t (&acc)[TI][NJ], int m0, int n) {
     asm volatile("" : "+v"(m0), "+v"(n));  // (or addresses are formed in front of the K loop and held through it)
@@ -1115,7 +1115,7 @@ int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st
         const GemmF32Problem& q = probs[i];
         if (q.M <= 0 || q.N <= 0) continue;
         if (q.K <= 0) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: K must be positive");
-        if (q.a_pieces != a_pieces || (a_pieces && !gemm_f32_takes_a_pieces(q.W, q.ldw, q.n0, q.N, q.K)) || (q.out_pieces && (epi != EPI_BIAS_GELU || !whole_chunks(q))))
+        if (q.a_pieces != a_pieces || (a_pieces && !gemm_f32_takes_a_pieces(q.W, q.ldw, q.n0, q.N, q.K)) || (q.out_pieces && (epi != EPI_BIAS_GELU || !a_pieces)))
             return fail(SD3_ERR_INVALID_ARG, "gemm_f32: operands or outputs in pieces that this launch does not take");
         if (epi == EPI_QKV_NORM && (!a_pieces || q.n0 || q.N % 192))
             return fail(SD3_ERR_INVALID_ARG, "gemm_f32: the norms of q and k are for A in pieces and heads of 64");
@@ -1155,8 +1155,6 @@ int gemm_f32_grouped(const GemmF32Problem* probs, int n, int epi, hipStream_t st
         }
     }
     if (whole_k_tiles(set, m) && f32_by_pieces(layers.l, m) && !g_gemm_f32_no_pieces) {
-        for (int i = 0; i < m; i++)
-            if (set.p[i].out_pieces) return fail(SD3_ERR_INVALID_ARG, "gemm_f32: no output in pieces from the kernel that splits A itself");
         const int shape = g_gemm_f32_tile >= 0 ? g_gemm_f32_tile : pick_f32_piece_tile(layers.l, m, cus);
         switch (epi) {
             case EPI_BIAS: return launch_pieces_shape<EPI_BIAS>(shape, set, m, st);
