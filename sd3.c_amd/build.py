@@ -17,7 +17,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-saniti
 # the attention kernel's running-maximum chains carry no NaNs by construction; without this flag every fmaxf is preceded
 # by a canonicalising v_max of each operand
 EXTRA_FLAGS = {"attention_bf16.hip": ["-fno-honor-nans"]}
-DEPS = [os.path.join(CSRC, h) for h in ("common.hpp", "device.hpp", "offsets.hpp", "passengers.hpp", "pieces.hpp", "tiles_f32.hpp")] + [os.path.join(os.path.dirname(HERE), "include", "sd3_hip.h")]
+DEPS = [os.path.join(CSRC, h) for h in ("common.hpp", "device.hpp", "offsets.hpp", "passengers.hpp", "pieces.hpp", "tiles_f32.hpp", "workspace.hpp")] + [os.path.join(os.path.dirname(HERE), "include", "sd3_hip.h")]
 
 
 def _stale(target, deps):

@@ -13,6 +13,7 @@
 
 #include "common.hpp"
 #include "pieces.hpp"
+#include "workspace.hpp"
 
 namespace sd3 {
 
@@ -84,8 +85,7 @@ struct sd3_ctx {
     std::unordered_map<std::string, std::pair<const float*, long long>> params;
     std::map<std::pair<const float*, int>, PackedWeight> packed;
     std::map<std::tuple<int, int, int, int, int>, float*> pos_tables;  // (C, max, base, h, w) -> cropped table
-    void* ws = nullptr;
-    size_t ws_bytes = 0;
+    sd3::Workspace ws;
     void* static_scratch = nullptr;  // this device's address of the fixed scratch array (resolved when the context is created)
     long long copies_built = 0;  // derived weight copies built so far (sd3_weights_copies_built)
     bool no_alloc = false;  // set for the duration of a call that must not allocate: a missing derived weight copy is then an error
@@ -130,15 +130,19 @@ struct Bump {
 };
 
 // Marks the end of an enqueueing call on the context's stream (see sd3_ctx::order_event). Nothing is recorded while the stream
-// is being captured into a graph: the event would become part of the capture, and replays are ordered by the caller.
-void record_order(sd3_ctx* ctx) {
+// is being captured into a graph: the event would become part of the capture, and replays are ordered by the caller. The graph
+// holds the address of the workspace, if the call uses it.
+void record_order(sd3_ctx* ctx, bool uses_workspace) {
     if (!ctx->order_event) return;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) {
         (void)hipGetLastError();
         return;
     }
-    if (cap != hipStreamCaptureStatusNone) return;
+    if (cap != hipStreamCaptureStatusNone) {
+        if (uses_workspace) ctx->ws.captured();
+        return;
+    }
     if (hipEventRecord(ctx->order_event, ctx->stream) == hipSuccess) ctx->order_pending = true;
     else (void)hipGetLastError();
 }
@@ -149,26 +153,10 @@ int wait_idle(sd3_ctx* ctx) {
 }
 struct OrderScope {  // records the order event when an enqueueing entry point returns, on every path
     sd3_ctx* ctx;
-    explicit OrderScope(sd3_ctx* c) : ctx(c) {}
-    ~OrderScope() { record_order(ctx); }
+    bool uses_workspace;
+    explicit OrderScope(sd3_ctx* c, bool uses_workspace_ = true) : ctx(c), uses_workspace(uses_workspace_) {}
+    ~OrderScope() { record_order(ctx, uses_workspace); }
 };
-
-int ensure_workspace(sd3_ctx* ctx, size_t bytes) {
-    if (bytes <= ctx->ws_bytes) return SD3_OK;
-    if (ctx->ws) {
-        SD3_HIP_TRY(hipStreamSynchronize(ctx->stream));
-        SD3_HIP_TRY(hipFree(ctx->ws));
-        ctx->ws = nullptr;
-        ctx->ws_bytes = 0;
-    }
-    hipError_t e = hipMalloc(&ctx->ws, bytes);
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        return fail(SD3_ERR_OOM, "workspace of %zu bytes: %s", bytes, hipGetErrorString(e));
-    }
-    ctx->ws_bytes = bytes;
-    return SD3_OK;
-}
 
 int get_packed(sd3_ctx* ctx, const float* w, long long K, long long N, int kind, const void** out) {
     auto key = std::make_pair(w, kind);
@@ -320,23 +308,12 @@ size_t block_workspace_bytes(const Dims& d, int prec, Pieces pieces = {}) {
     return b.off;
 }
 
-// Room for `front` bytes and a block's intermediates behind them. Operands in pieces are larger: where they don't fit, in a capture that what there is would do for or for lack of
-// memory, *pieces becomes none.
+// Room for `front` bytes and a block's intermediates behind them. Operands in pieces are larger: where they can't be had (Workspace::prefer), *pieces becomes none.
 int ensure_block_workspace(sd3_ctx* ctx, size_t front, const Dims& d, int prec, Pieces* pieces) {
-    const size_t plain = front + block_workspace_bytes(d, prec), bytes = front + block_workspace_bytes(d, prec, *pieces);
-    if (bytes == plain || bytes <= ctx->ws_bytes) return ensure_workspace(ctx, bytes);
-    if (plain <= ctx->ws_bytes) {
-        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(ctx->stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
-            (void)hipGetLastError();
-            *pieces = Pieces{};
-            return SD3_OK;
-        }
-    }
-    const int rc = ensure_workspace(ctx, bytes);
-    if (rc != SD3_ERR_OOM) return rc;
-    *pieces = Pieces{};
-    return ensure_workspace(ctx, plain);
+    bool had = false;
+    SD3_TRY(ctx->ws.prefer(ctx->stream, front + block_workspace_bytes(d, prec), front + block_workspace_bytes(d, prec, *pieces), &had));
+    if (!had) *pieces = Pieces{};
+    return SD3_OK;
 }
 
 // One linear layer: out = epilogue(A @ W + b). fp32: W used in place; bf16: the packed copy.
@@ -987,7 +964,7 @@ int sd3_ctx_destroy(sd3_ctx* ctx) {
         (void)wait_idle(ctx);
         for (auto& kv : ctx->packed) (void)hipFree(kv.second.ptr);
         for (auto& kv : ctx->pos_tables) (void)hipFree(kv.second);
-        if (ctx->ws) (void)hipFree(ctx->ws);
+        ctx->ws.release();
         for (auto& p : ctx->prof) {
             (void)hipEventDestroy(p.a);
             (void)hipEventDestroy(p.b);
@@ -1143,7 +1120,7 @@ int sd3_dit_block_w(sd3_ctx* ctx, const float* y, float* c, float* x, const sd3_
     OrderScope order(ctx);
     Pieces pieces = pieces_of(d, precision, *w);
     SD3_TRY(ensure_block_workspace(ctx, 0, d, precision, &pieces));
-    Bump ws(ctx->ws, ctx->ws_bytes);
+    Bump ws(ctx->ws.get(), ctx->ws.bytes());
     return run_block(ctx, precision, y, c, x, *w, d, pieces, nullptr, nullptr, ws);
 }
 
@@ -1177,7 +1154,7 @@ int sd3_dit_block_static(sd3_ctx* ctx, const float* y, float* c, float* x, const
     DeviceGuard g(ctx->device);
     if (!g.ok) return fail(SD3_ERR_HIP, "cannot select device %d", ctx->device);
     if (!ctx->static_scratch) return fail(SD3_ERR_HIP, "dit_block_static: the fixed scratch array has no address on device %d", ctx->device);
-    OrderScope order(ctx);  // (records an event that exists since the context was created: no allocation)
+    OrderScope order(ctx, false);  // (records an event that exists since the context was created: no allocation)
     Bump ws(ctx->static_scratch, SD3_STATIC_SCRATCH_BYTES);
     ctx->no_alloc = true;
     Pieces pieces = pieces_of(d, precision, w);
@@ -1275,7 +1252,7 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     }
     SD3_TRY(ensure_block_workspace(ctx, probe.off, dmax, precision, &any));
     if (!any.rows) pieces.assign(num_layers, Pieces{});
-    Bump ws(ctx->ws, ctx->ws_bytes);
+    Bump ws(ctx->ws.get(), ctx->ws.bytes());
     layout(ws, &temb, &h1, &h2, &yt, &yp, &y, &c, &x, &cap_in, &patches, &ada_all, &ada_out, &tokens);
     const size_t block_ws_off = ws.off;
 
@@ -1358,7 +1335,7 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     }
     // ---- blocks (modules.cpp:1687-1718)
     for (int l = 0; l < num_layers; l++) {
-        Bump bws(ctx->ws, ctx->ws_bytes);
+        Bump bws(ctx->ws.get(), ctx->ws.bytes());
         bws.off = block_ws_off;
         const float* base = ada_all + (size_t)l * B * 15 * C;
         AdaCarry carry;
@@ -1397,7 +1374,7 @@ static int dit_forward_impl(sd3_ctx* ctx, const float* pooled, const float* capt
     }
     // ---- output layer: LN(eps 1e-5), chunk 0 = scale, chunk 1 = shift, projection, tokens -> pixels (modules.cpp:1721-1752)
     {
-        Bump bws(ctx->ws, ctx->ws_bytes);
+        Bump bws(ctx->ws.get(), ctx->ws.bytes());
         bws.off = block_ws_off;
         void* x_hid = bws.take<char>((size_t)B * Tx * C * (bf ? 2 : 4));
         SD3_TRY(ln_mod(ctx, x, x_hid, nullptr, ada_out + C, ada_out, nullptr, nullptr, 2 * C, 1e-5f, B, Tx, C, bf));

@@ -4,10 +4,12 @@
 context's workspace grows. Blocks between the two sizes are computed both ways."""
 import numpy as np
 import pytest
+import torch
 
 from gpu_util import M, dev, dev_params, host
 from sd3_c_amd import lib as L
-from sd3_c_amd.params import block_param_shapes, synthetic_params_numpy
+from sd3_c_amd.config import DiTConfig
+from sd3_c_amd.params import block_param_shapes, dit_param_shapes, synthetic_params_numpy
 
 pytestmark = pytest.mark.gpu
 
@@ -84,3 +86,43 @@ def test_values_without_pieces(what):
     (ca, xa), (cb, xb) = _both_ways(1, 77, 1100, C, 24, 2, False, False, spoil)
     assert np.isfinite(xa).all() == (what == "scales")
     assert np.array_equal(xa, xb, equal_nan=True) and np.array_equal(ca, cb, equal_nan=True)
+
+
+@pytest.mark.parametrize("warm", ["pieces", "plain"])
+def test_captured_forwards_and_eager_ones_of_the_same_sizes(warm):
+    """A captured forward with operands in pieces, and one in a workspace that holds the layout without them only (as it is after a call that there was no memory for
+    more for), replayed behind eager calls of the same sizes: these leave the workspace where it is, with the bits of an eager forward throughout."""
+    cfg = DiTConfig(num_layers=2, dual_attention_layers=(0,), pooled_dim=64, captions_dim=64, in_channels=16, emb_dim=512, attn_heads=8, mlp_expand=2, patch_size=2,
+                    pos_embed_max_size=64, base_height=32, use_qk_norm=True)
+    g = torch.Generator(device="cuda").manual_seed(41)
+    P = {n: (1 if "rmsnorm" in n else 0) + 0.02 * torch.randn(s, device="cuda", generator=g) for n, s in dit_param_shapes(cfg).items()}
+    B, Tc, H, W = 2, 9, 80, 84   # 3378 rows of 512
+    lat = torch.randn((B, cfg.in_channels, H, W), device="cuda", generator=g)
+    captions = torch.randn((B, Tc, cfg.captions_dim), device="cuda", generator=g)
+    args = (torch.randn((B, cfg.pooled_dim), device="cuda", generator=g), captions, lat, torch.full((B,), 300.0, device="cuda"))
+    want = M.Denoiser(P, cfg, "fp32")(*args)
+    torch.cuda.synchronize()
+    den, out, eager = M.Denoiser(P, cfg, "fp32"), torch.empty_like(lat), torch.empty_like(lat)
+    L.check(L.load().sd3_tune(b"gemm_f32_no_pieces", int(warm == "plain")))
+    try:
+        den(*args, out=out)
+    finally:
+        L.check(L.load().sd3_tune(b"gemm_f32_no_pieces", 0))
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=side):
+        den(*args, out=out)
+    eager.zero_()   # (the runtime takes memory of its own at first launches)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+    free = torch.cuda.mem_get_info()[0]
+    for _ in range(3):
+        out.zero_()
+        eager.zero_()
+        den(*args, out=eager)
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free and torch.equal(eager, want)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
