@@ -412,6 +412,8 @@ struct QkNormJob {
     long long rows;
 };
 int qk_norm_rows(const QkNormJob* jobs, int n, float eps, int heads, int hs, int ld, hipStream_t st);
+// Whether these go by whole chunks (head_squares, head_factor); else the sums have another order
+bool qk_norm_by_chunks(const QkNormJob* jobs, int n, int hs, int ld);
 int unary_op(const float* in, float* out, long long n, int act, hipStream_t st);
 int add_op(const float* a, const float* b, float* out, long long n, hipStream_t st);
 int add_silu_op(const float* a, const float* b, float* out, long long n, hipStream_t st);

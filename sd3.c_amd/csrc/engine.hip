@@ -539,14 +539,16 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
                                      {c, c_hid, nullptr, c_shift, c_scale, nullptr, nullptr, ldc_ada, B, Tc}};
         SD3_TRY(ln_mod_pair(ctx, ln1, 2, 1e-6f, C, ln_out));
     }
-    bool fused_norm;
+    // The per-head RMSNorm of q and k (modules.cpp:1396-1399, 1420-1423) runs in the projection's epilogue, on the fp32 accumulators, in the bf16 path, so that the
+    // attention kernel streams K tiles straight into LDS, and with heads of 64 in fp32 where the inputs come in pieces and the norms would go by whole chunks: whether the
+    // inputs come in pieces depends on the batch, and a row's bits must not.
+    const QkNormJob norms[3] = {{(float*)x_qkv, w.x_rms_q, w.x_rms_k, mx}, {(float*)c_qkv, w.c_rms_q, w.c_rms_k, mc}, {(float*)x_qkv2, w.x2_rms_q, w.x2_rms_k, mx}};
+    const int n_norms = d.dual ? 3 : 2;
+    const bool fused_norm = d.qk && (bf || (pieces.rows && d.HS == 64 && qk_norm_by_chunks(norms, n_norms, d.HS, 3 * C)));
     {
-        // the per-head RMSNorm of q and k (modules.cpp:1396-1399, 1420-1423) runs in the projection's epilogue, on the fp32 accumulators, in the bf16 path, so that the
-        // attention kernel streams K tiles straight into LDS, and with heads of 64 in fp32 where the inputs come in pieces
         GemmEpilogueArgs nx, nc;
         nx.gate = w.x_rms_q; nx.resid = w.x_rms_k;
         nc.gate = w.c_rms_q; nc.resid = w.c_rms_k;
-        fused_norm = d.qk && (bf || (pieces.rows && d.HS == 64));
         GemmEpilogueArgs n2;
         n2.gate = w.x2_rms_q; n2.resid = w.x2_rms_k;
         // the dual branch's projection reads the other output of the same LayerNorm pass: same kind, same launch
@@ -558,10 +560,7 @@ int run_block(sd3_ctx* ctx, int prec, const float* y, float* c, float* x, const 
 
     // ---- joint attention over [context ; latent] (modules.cpp:1427-1432); qk-norm in place first where the projection has left it
     auto seg_ptr = [&](void* base, int third) -> void* { return (char*)base + (size_t)third * C * es; };
-    if (d.qk && !fused_norm) {
-        const QkNormJob norms[3] = {{(float*)x_qkv, w.x_rms_q, w.x_rms_k, mx}, {(float*)c_qkv, w.c_rms_q, w.c_rms_k, mc}, {(float*)x_qkv2, w.x2_rms_q, w.x2_rms_k, mx}};
-        SD3_TRY(qk_norm_rows(norms, d.dual ? 3 : 2, 1e-6f, d.NH, d.HS, 3 * C, st));
-    }
+    if (d.qk && !fused_norm) SD3_TRY(qk_norm_rows(norms, n_norms, 1e-6f, d.NH, d.HS, 3 * C, st));
     AttnSegments joint{}, dual_set{};
     joint.out_pieces = dual_set.out_pieces = pieces.att;
     joint.q[0] = c_qkv; joint.k[0] = seg_ptr(c_qkv, 1); joint.v[0] = seg_ptr(c_qkv, 2); joint.out[0] = d.discard ? nullptr : c_att;

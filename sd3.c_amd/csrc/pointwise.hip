@@ -329,11 +329,15 @@ __global__ void __launch_bounds__(256) qk_norm_kernel(const QkNormDev jobs, floa
     }
 }
 
-int qk_norm_rows(const QkNormJob* jobs, int n, float eps, int heads, int hs, int ld, hipStream_t st) {
+bool qk_norm_by_chunks(const QkNormJob* jobs, int n, int hs, int ld) {
     auto al = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    bool vec = (hs == 64 || hs == 128) && ld % 4 == 0 && n <= 3;
-    for (int i = 0; i < n; i++) vec = vec && al(jobs[i].qkv) && al(jobs[i].wq) && al(jobs[i].wk);
-    if (!vec) {
+    bool chunks = (hs == 64 || hs == 128) && ld % 4 == 0 && n <= 3;
+    for (int i = 0; i < n; i++) chunks = chunks && al(jobs[i].qkv) && al(jobs[i].wq) && al(jobs[i].wk);
+    return chunks;
+}
+
+int qk_norm_rows(const QkNormJob* jobs, int n, float eps, int heads, int hs, int ld, hipStream_t st) {
+    if (!qk_norm_by_chunks(jobs, n, hs, ld)) {
         for (int i = 0; i < n; i++) {
             SD3_TRY(rmsnorm_rows(jobs[i].qkv, jobs[i].qkv, jobs[i].wq, nullptr, eps, jobs[i].rows, heads, hs, ld, ld, st));
             float* k = jobs[i].qkv + (long long)heads * hs;

@@ -126,3 +126,34 @@ def test_captured_forwards_and_eager_ones_of_the_same_sizes(warm):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("norm_off", [0, 1])
+@pytest.mark.parametrize("B,Tc,Tx,C,NH,E,dual,qk", [
+    (2, 30, 400, 1536, 24, 2, False, True),    # 0.66e6 values alone, 1.3e6 together: LayerNorm's outputs in pieces
+    (3, 41, 471, 1536, 24, 2, True, True),     # 0.79e6 and 2.4e6: all of them; attention by pieces, 288 workgroups of 128 queries one after the other
+    (5, 10, 390, 1024, 16, 4, False, True),    # attention on the fp32 instruction
+    (4, 25, 300, 1536, 12, 2, False, True),    # heads of 128
+    (4, 25, 300, 1536, 24, 2, False, False),   # no norms
+])
+def test_an_element_alone_and_in_a_batch(norm_off, B, Tc, Tx, C, NH, E, dual, qk):
+    """Whether operands come in pieces depends on the rows of the whole batch, an element's bits do not, also where a norm's weights lie at any float."""
+    rng = np.random.Generator(np.random.Philox(Tx))
+    P = dev_params(synthetic_params_numpy(block_param_shapes(C, E, dual, qk, False, C // NH), 13, 0.05, 0.05))
+    if norm_off and qk:
+        for n in [n for n in P if "rmsnorm" in n][:1]:
+            moved = torch.empty(P[n].numel() + norm_off, device="cuda")[norm_off:]
+            moved.copy_(P[n].flatten())
+            P[n] = moved.view(P[n].shape)
+            assert P[n].data_ptr() % 16
+    y, c, x = (rng.standard_normal(s, dtype=np.float32) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
+    assert (Tc + Tx) * C < 1.0e6 < B * (Tc + Tx) * C
+
+    def run(b0, b1):
+        cg, xg = M.Dit_block(dev(y[b0:b1]), dev(c[b0:b1].copy()), dev(x[b0:b1].copy()), P, b1 - b0, Tc, Tx, C, NH, E, dual, qk, False, precision="fp32")
+        return host(cg), host(xg)
+
+    cg, xg = run(0, B)
+    for b in range(B):
+        c1, x1 = run(b, b + 1)
+        assert np.array_equal(cg[b:b + 1], c1) and np.array_equal(xg[b:b + 1], x1)
