@@ -10,18 +10,18 @@ from sd3_c_amd.params import block_param_shapes, synthetic_params_numpy
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tile", [0, 64064, 128, 256128, 256])
+@pytest.mark.parametrize("tile", [0, 64064, 64128, 128064, 128, 128256, 256128, 192, 192256, 256])
 @pytest.mark.parametrize("Tc,Tx", [(3, 7), (15, 33), (64, 65), (77, 200), (130, 256)])
 def test_gates_of_rows_of_several_batch_elements(tile, Tc, Tx):
     """Wavefronts have 16, 32, 64 or 128 consecutive rows: up to 18 elements of 7 rows, boundaries inside of them and between them; whole tiles of 256 rows (the persistent kernel's
-    form without conditions) and the last ones of a matrix."""
-    B, C, NH = 5, 256, 4
+    form without conditions) and the last ones of a matrix. (Tiles of 256x192 have no norms in their epilogue, and 48 columns a wavefront.)"""
+    B, C, NH, qk = 5, 256, 4, tile != 192
     rng = np.random.Generator(np.random.Philox(Tx))
-    P = dev_params(synthetic_params_numpy(block_param_shapes(C, 4, True, True, False, C // NH), 5, 0.05, 0.05))
+    P = dev_params(synthetic_params_numpy(block_param_shapes(C, 4, True, qk, False, C // NH), 5, 0.05, 0.05))
     y, c, x = (rng.standard_normal(s, dtype=np.float32) for s in ((B, C), (B, Tc, C), (B, Tx, C)))
 
     def run(b0, b1):
-        cg, xg = M.Dit_block(dev(y[b0:b1]), dev(c[b0:b1].copy()), dev(x[b0:b1].copy()), P, b1 - b0, Tc, Tx, C, NH, 4, True, True, False, precision="bf16")
+        cg, xg = M.Dit_block(dev(y[b0:b1]), dev(c[b0:b1].copy()), dev(x[b0:b1].copy()), P, b1 - b0, Tc, Tx, C, NH, 4, True, qk, False, precision="bf16")
         return host(cg), host(xg)
 
     L.check(L.load().sd3_tune(b"gemm_bf16_tile", tile))
