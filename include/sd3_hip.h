@@ -140,6 +140,10 @@ int sd3_weights_clear(sd3_ctx* ctx);
 /* Number of derived weight copies the context has built since it was created (bf16 / fp8 / transposed copies, one per
  * weight and kind): lets a caller or a test see whether a call re-used the existing copies or built new ones. */
 int sd3_weights_copies_built(sd3_ctx* ctx, long long* count);
+/* Number of fp32 products that the context has launched (or recorded into a graph) so far on an operand that was written as bf16
+ * pieces by what produced it; their results have the same bits as those of the others. Which operands are depends on the sizes, on the
+ * weights' addresses and on whether there is memory for the pieces (6 bytes a value instead of 4). */
+int sd3_operand_pieces_launches(sd3_ctx* ctx, long long* count);
 /* Rebuilds, from the current contents of the bound tensors, every derived copy a forward of `precision` uses (bf16: the
  * K-contiguous bf16 copies of the GEMM weights, the bf16 copies of the adaLN weights and of the patch-conv weight; fp32: the
  * transposed patch-conv weight). Optional before a first forward (copies are otherwise built on first use, inside that

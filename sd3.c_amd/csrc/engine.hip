@@ -88,6 +88,7 @@ struct sd3_ctx {
     sd3::Workspace ws;
     void* static_scratch = nullptr;  // this device's address of the fixed scratch array (resolved when the context is created)
     long long copies_built = 0;  // derived weight copies built so far (sd3_weights_copies_built)
+    long long piece_launches = 0;  // fp32 products of operands in pieces so far (sd3_operand_pieces_launches)
     bool no_alloc = false;  // set for the duration of a call that must not allocate: a missing derived weight copy is then an error
     // optional per-kernel-class timing with HIP events on the context's stream
     bool prof_on = false;
@@ -361,6 +362,7 @@ int linear_pair(sd3_ctx* ctx, int prec, const LayerCall* calls, int n, int out_f
             m++;
         }
         if (m == 0) return SD3_OK;
+        if (probs[0].a_pieces) ctx->piece_launches++;
         ProfScope ps(ctx, SD3_PROF_GEMM, flop);
         return gemm_f32_grouped(probs, m, epi, ctx->stream);
     }
@@ -1029,6 +1031,11 @@ int sd3_weights_forget(sd3_ctx* ctx, const float* ptr) {
 int sd3_weights_copies_built(sd3_ctx* ctx, long long* count) {
     NOTNULL(ctx); NOTNULL(count);
     *count = ctx->copies_built;
+    return SD3_OK;
+}
+int sd3_operand_pieces_launches(sd3_ctx* ctx, long long* count) {
+    NOTNULL(ctx); NOTNULL(count);
+    *count = ctx->piece_launches;
     return SD3_OK;
 }
 int sd3_weights_prepare(sd3_ctx* ctx, int precision) {

@@ -45,6 +45,7 @@ SIGNATURES = {
     "sd3_weights_forget": [vp, vp],
     "sd3_weights_clear": [vp],
     "sd3_weights_copies_built": [vp, C.POINTER(cll)],
+    "sd3_operand_pieces_launches": [vp, C.POINTER(cll)],
     "sd3_weights_prepare": [vp, ci],
     "sd3_dit_block": [vp, vp, vp, vp, cs] + [ci] * 10,
     "sd3_dit_block_static": [vp, vp, vp, vp, cs] + [ci] * 10,

@@ -273,6 +273,12 @@ class Context:
         L.call("sd3_weights_copies_built", self._h, C.byref(n))
         return n.value
 
+    def operand_pieces_launches(self):
+        """fp32 products launched by this context so far on operands that came as bf16 pieces."""
+        n = C.c_longlong(0)
+        L.call("sd3_operand_pieces_launches", self._h, C.byref(n))
+        return n.value
+
     def clear(self):
         L.call("sd3_weights_clear", self._h)
         self._keep = {}

@@ -1,7 +1,7 @@
 """fp32 blocks whose operands are written as bf16 pieces by what produces them: the same bits as from products that split fp32 operands themselves.
 
 `sd3_dit_block_static` has a fixed 64 MiB for its intermediates and goes without the pieces where these, six bytes a value instead of four, do not fit; the
-context's workspace grows. Blocks between the two sizes are computed both ways."""
+context's workspace grows. Blocks between the two sizes are computed both ways, and the context tells which of its products had operands in pieces."""
 import numpy as np
 import pytest
 import torch
@@ -23,6 +23,12 @@ def _plain_and_pieces_bytes(B, Tc, Tx, C, E, dual):
     return plain, qkv + 6 * C * (rows + B * Tx) + (6 if wide else 4) * (C * rows + E * C * rows)
 
 
+def _products(B, Tc, Tx, C, dual):
+    """How many of a block's products have operands in pieces: q|k|v and the first MLP layers; attention's outputs and the second MLP layers too"""
+    values = B * (Tc + Tx) * C
+    return 0 if values < 1.0e6 else 2 if values < 1.7e6 else 4 + dual
+
+
 def _both_ways(B, Tc, Tx, C, NH, E, dual, discard, spoil=None):
     plain, pieces = _plain_and_pieces_bytes(B, Tc, Tx, C, E, dual)
     limit = 64 << 20
@@ -36,9 +42,11 @@ def _both_ways(B, Tc, Tx, C, NH, E, dual, discard, spoil=None):
     try:
         ctx.bind(dev_params(P))
         out = []
-        for run in (ctx.block, ctx.block_static):
+        for run, products in ((ctx.block, _products(B, Tc, Tx, C, dual)), (ctx.block_static, 0)):
             cg, xg = dev(c.copy()), dev(x.copy())
+            before = ctx.operand_pieces_launches()
             run(dev(y), cg, xg, B, Tc, Tx, C, NH, E, dual, True, discard, precision="fp32")
+            assert ctx.operand_pieces_launches() - before == products
             out.append((host(cg), host(xg)))
         return out
     finally:
@@ -112,6 +120,8 @@ def test_captured_forwards_and_eager_ones_of_the_same_sizes(warm):
     torch.cuda.synchronize()
     with torch.cuda.graph(graph, stream=side):
         den(*args, out=out)
+    launched = den.ctx.operand_pieces_launches()
+    assert launched == (4 * 2 + 1) * 2 if warm == "pieces" else launched == 0   # (the warm call and the captured one, a dual block and a plain one)
     eager.zero_()   # (the runtime takes memory of its own at first launches)
     graph.replay()
     torch.cuda.synchronize()
@@ -126,6 +136,7 @@ def test_captured_forwards_and_eager_ones_of_the_same_sizes(warm):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+    assert (den.ctx.operand_pieces_launches() > launched) == (warm == "pieces")
 
 
 @pytest.mark.parametrize("norm_off", [0, 1])
@@ -153,7 +164,12 @@ def test_an_element_alone_and_in_a_batch(norm_off, B, Tc, Tx, C, NH, E, dual, qk
         cg, xg = M.Dit_block(dev(y[b0:b1]), dev(c[b0:b1].copy()), dev(x[b0:b1].copy()), P, b1 - b0, Tc, Tx, C, NH, E, dual, qk, False, precision="fp32")
         return host(cg), host(xg)
 
+    launched = M.shared_context(torch.device("cuda:0")).operand_pieces_launches
+    before = launched()
     cg, xg = run(0, B)
+    assert launched() - before == _products(B, Tc, Tx, C, dual)
     for b in range(B):
+        before = launched()
         c1, x1 = run(b, b + 1)
+        assert launched() == before
         assert np.array_equal(cg[b:b + 1], c1) and np.array_equal(xg[b:b + 1], x1)
