@@ -29,7 +29,15 @@ def _products(B, Tc, Tx, C, dual):
     return 0 if values < 1.0e6 else 2 if values < 1.7e6 else 4 + dual
 
 
-def _both_ways(B, Tc, Tx, C, NH, E, dual, discard, spoil=None):
+def _at(a, off):
+    """`a` on the GPU, `off` floats behind a multiple of 16 bytes"""
+    t = torch.empty(a.size + off, device="cuda")[off:].view(a.shape)
+    t.copy_(torch.from_numpy(a))
+    assert t.data_ptr() % 16 == 4 * off
+    return t
+
+
+def _both_ways(B, Tc, Tx, C, NH, E, dual, discard, spoil=None, off=0):
     plain, pieces = _plain_and_pieces_bytes(B, Tc, Tx, C, E, dual)
     limit = 64 << 20
     assert plain + (1 << 19) < limit < pieces  # (room for the modulation vectors, and the case tells the two apart)
@@ -43,7 +51,7 @@ def _both_ways(B, Tc, Tx, C, NH, E, dual, discard, spoil=None):
         ctx.bind(dev_params(P))
         out = []
         for run, products in ((ctx.block, _products(B, Tc, Tx, C, dual)), (ctx.block_static, 0)):
-            cg, xg = dev(c.copy()), dev(x.copy())
+            cg, xg = _at(c, off), _at(x, off)
             before = ctx.operand_pieces_launches()
             run(dev(y), cg, xg, B, Tc, Tx, C, NH, E, dual, True, discard, precision="fp32")
             assert ctx.operand_pieces_launches() - before == products
@@ -77,8 +85,17 @@ def test_the_same_bits_for_every_tile_shape(tile):
     assert np.array_equal(xa, xb) and np.array_equal(ca, cb)
 
 
+@pytest.mark.parametrize("B,Tc,Tx,C,NH,E,dual", [(1, 77, 1100, 1536, 24, 2, False), (1, 20, 930, 1536, 24, 2, True), (2, 15, 1701, 512, 8, 2, False)])
+def test_the_same_bits_with_streams_at_any_float(B, Tc, Tx, C, NH, E, dual):
+    """Rows of x and c that are not on 16 bytes go through the LayerNorm that writes its pieces value by value."""
+    (ca, xa), (cb, xb) = _both_ways(B, Tc, Tx, C, NH, E, dual, False, off=1)
+    assert np.isfinite(xa).all()
+    assert np.array_equal(xa, xb) and np.array_equal(ca, cb)
+
+
+@pytest.mark.parametrize("off", [0, 3])
 @pytest.mark.parametrize("what", ["scales", "tokens"])
-def test_values_without_pieces(what):
+def test_values_without_pieces(what, off):
     """Infinities, NaNs and values from 2^112 on in LayerNorm's, attention's and the MLP's outputs are formed anew by the fp32 instruction, from the bits that stand in the pieces' place."""
     C = 1536
 
@@ -91,7 +108,7 @@ def test_values_without_pieces(what):
             if "ada" in n and n.endswith(".bias"):
                 q[1 * C + 7] = 2.0 ** 115   # the scale of LayerNorm's channel 7 in front of q|k|v: values, too, and what attention makes of them
                 q[4 * C + 9] = -2.0 ** 115  # ... in front of the MLP: some of the hidden values
-    (ca, xa), (cb, xb) = _both_ways(1, 77, 1100, C, 24, 2, False, False, spoil)
+    (ca, xa), (cb, xb) = _both_ways(1, 77, 1100, C, 24, 2, False, False, spoil, off)
     assert np.isfinite(xa).all() == (what == "scales")
     assert np.array_equal(xa, xb, equal_nan=True) and np.array_equal(ca, cb, equal_nan=True)
 
